@@ -99,6 +99,7 @@ SYMBOLS = {
     "flare_causal_join": (C.c_int, [C.c_int32, C.c_int32, C.c_int64, C.c_int32, C.POINTER(_P), C.POINTER(_P), _P, _P]),
     "flare_causal_linear_workspace_bytes": (C.c_int, [C.POINTER(FlareCausalLinearDesc), C.POINTER(_SZ)]),
     "flare_causal_linear_fwd": (C.c_int, [C.POINTER(FlareCausalLinearDesc), _P, _P, _P, _P, _P, _SZ, _P]),
+    "flare_causal_linear_bwd": (C.c_int, [C.POINTER(FlareCausalLinearDesc), _P, _P, _P, _P, C.POINTER(C.c_int64), _P, _P, _P, _P, _P, _SZ, _P]),
     "flare_mlp_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_io_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), C.c_int32, C.c_int32, _P, _P, C.c_int32,
                                    _P, _P, _P, _P, _P, _P, _P, _P]),

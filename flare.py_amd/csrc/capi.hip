@@ -870,6 +870,63 @@ int flare_causal_linear_workspace_bytes(const FlareCausalLinearDesc* desc, size_
     return FLARE_OK;
 }
 
+namespace {
+
+// A [B,H,N,width] operand of a causal linear launch: its pointer and strides as the caller has them.
+struct ClOp { const void* p; const int64_t* s; };
+
+// Pointer and strides as the kernels take them; `rev` walks the token axis backwards (the last token first).
+const void* cl_op(const ClOp& o, int N, int dtype, bool rev, int64_t out[3])
+{
+    for (int i = 0; i < 3; ++i) out[i] = o.s[i];
+    if (!rev) return o.p;
+    out[2] = -o.s[2];
+    return static_cast<const char*>(o.p) + (int64_t)(N - 1) * o.s[2] * esize(dtype);
+}
+
+bool cl_aligned(const ClOp& o) { return strides_mult8(o.s) && aligned16(o.p); }
+
+bool cl_mfma(const FlareCausalLinearDesc* d, int Dk, int Dv)
+{
+    return !(d->flags & FLARE_FLAG_FORCE_GENERIC) && flare::causal_linear_mfma_supported(d->dtype, Dk, Dv);
+}
+
+flare::CausalLinearArgs cl_args(const FlareCausalLinearDesc* d, const CausalLinearPlan& p, int Dk, int Dv, const ClOp& q, const ClOp& k,
+                                const ClOp& v, const ClOp& y, void* states, bool rev)
+{
+    flare::CausalLinearArgs a;
+    memset(&a, 0, sizeof(a));
+    a.q = cl_op(q, d->N, d->dtype, rev, a.qs);
+    a.k = cl_op(k, d->N, d->dtype, rev, a.ks);
+    a.v = cl_op(v, d->N, d->dtype, rev, a.vs);
+    a.y = const_cast<void*>(cl_op(y, d->N, d->dtype, rev, a.ys));
+    a.states = static_cast<float*>(states);
+    a.B = d->B; a.H = d->H; a.N = d->N; a.Dk = Dk; a.Dv = Dv;
+    a.n_segs = p.n_segs; a.seg_len = p.seg_len;
+    a.inv_n = 1.0f / (float)d->N;
+    return a;
+}
+
+// 16-byte aligned rows of the sizes the matrix-core kernels take go there, everything else to the fp32 FMA kernels
+hipError_t cl_run(const FlareCausalLinearDesc* d, const CausalLinearPlan& p, int Dk, int Dv, const ClOp& q, const ClOp& k, const ClOp& v,
+                  const ClOp& y, void* states, bool rev, hipStream_t st)
+{
+    const flare::CausalLinearArgs a = cl_args(d, p, Dk, Dv, q, k, v, y, states, rev);
+    if (cl_mfma(d, Dk, Dv) && cl_aligned(q) && cl_aligned(k) && cl_aligned(v) && cl_aligned(y))
+        return flare::launch_causal_linear_mfma(a, d->dtype, 3, st);
+    return flare::launch_causal_linear(a, d->dtype, st);
+}
+
+int cl_check_workspace(const CausalLinearPlan& p, const void* workspace, size_t bytes)
+{
+    if (!workspace) return fail(FLARE_EWORKSPACE, "workspace is NULL");
+    if (bytes < p.total) return fail(FLARE_EWORKSPACE, "workspace has %zu bytes, %zu needed", bytes, p.total);
+    if (reinterpret_cast<uintptr_t>(workspace) % 4) return fail(FLARE_EINVAL, "workspace must be 4-byte aligned");
+    return FLARE_OK;
+}
+
+}  // namespace
+
 int flare_causal_linear_fwd(const FlareCausalLinearDesc* desc, const void* q, const void* k, const void* v,
                             void* y, void* workspace, size_t workspace_bytes, void* stream)
 {
@@ -877,26 +934,73 @@ int flare_causal_linear_fwd(const FlareCausalLinearDesc* desc, const void* q, co
     if (rc != FLARE_OK) return rc;
     if (!q || !k || !v || !y) return fail(FLARE_EINVAL, "q, k, v, y must not be NULL");
     const CausalLinearPlan p = plan_causal_linear(desc);
-    if (!workspace) return fail(FLARE_EWORKSPACE, "workspace is NULL");
-    if (workspace_bytes < p.total)
-        return fail(FLARE_EWORKSPACE, "workspace has %zu bytes, %zu needed", workspace_bytes, p.total);
-    if (reinterpret_cast<uintptr_t>(workspace) % 4) return fail(FLARE_EINVAL, "workspace must be 4-byte aligned");
-    flare::CausalLinearArgs a;
-    memset(&a, 0, sizeof(a));
-    a.q = q; a.k = k; a.v = v; a.y = y;
-    a.states = static_cast<float*>(workspace);
-    a.B = desc->B; a.H = desc->H; a.N = desc->N; a.Dk = desc->Dk; a.Dv = desc->Dv;
-    a.n_segs = p.n_segs; a.seg_len = p.seg_len;
-    a.inv_n = 1.0f / (float)desc->N;
-    for (int i = 0; i < 3; ++i) {
-        a.qs[i] = desc->q_stride[i]; a.ks[i] = desc->k_stride[i]; a.vs[i] = desc->v_stride[i]; a.ys[i] = desc->y_stride[i];
+    rc = cl_check_workspace(p, workspace, workspace_bytes);
+    if (rc != FLARE_OK) return rc;
+    return hip_status(cl_run(desc, p, desc->Dk, desc->Dv, {q, desc->q_stride}, {k, desc->k_stride}, {v, desc->v_stride},
+                             {y, desc->y_stride}, workspace, false, static_cast<hipStream_t>(stream)), "causal linear launch");
+}
+
+int flare_causal_linear_bwd(const FlareCausalLinearDesc* desc, const void* q, const void* k, const void* v, const void* gy,
+                            const int64_t gy_stride[3], const void* fwd_workspace, void* dq, void* dk, void* dv, void* workspace,
+                            size_t workspace_bytes, void* stream)
+{
+    int rc = check_causal_linear_desc(desc);
+    if (rc != FLARE_OK) return rc;
+    if (!q || !k || !v || !gy || !gy_stride) return fail(FLARE_EINVAL, "q, k, v, gy and gy_stride must not be NULL");
+    if (gy_stride[2] < desc->Dv) return fail(FLARE_EINVAL, "gy row stride %lld < row width %d", (long long)gy_stride[2], desc->Dv);
+    const CausalLinearPlan p = plan_causal_linear(desc);
+    rc = cl_check_workspace(p, workspace, workspace_bytes);
+    if (rc != FLARE_OK) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int H = desc->H, N = desc->N, Dk = desc->Dk, Dv = desc->Dv;
+    const int64_t sk[3] = {(int64_t)H * N * Dk, (int64_t)N * Dk, Dk}, sv[3] = {(int64_t)H * N * Dv, (int64_t)N * Dv, Dv};
+    const ClOp oq = {q, desc->q_stride}, ok = {k, desc->k_stride}, ov = {v, desc->v_stride}, og = {gy, gy_stride};
+    const ClOp odq = {dq, sk}, odk = {dk, sk}, odv = {dv, sv};
+    // Dk == Dv on the matrix cores: the three gradients need two running states, both square.  sum k v^T is the forward's
+    // own (its exclusive prefix is what the forward left in its workspace); sum q gy^T over the tokens behind serves dk
+    // (transposed) and dv, in one launch where the 16-bit kernel takes them.
+    const bool square = Dk == Dv && cl_mfma(desc, Dk, Dv) && cl_aligned(oq) && cl_aligned(ok) && cl_aligned(ov) && cl_aligned(og) &&
+                        (!dq || aligned16(dq)) && (!dk || aligned16(dk)) && (!dv || aligned16(dv));
+    hipError_t e = hipSuccess;
+    if (dq) {
+        if (square && fwd_workspace) {
+            flare::CausalLinearArgs a = cl_args(desc, p, Dv, Dk, og, ov, ok, odq, const_cast<void*>(fwd_workspace), false);
+            a.slot_t = 1;
+            e = flare::launch_causal_linear_mfma(a, desc->dtype, 2, st);
+        } else {
+            e = cl_run(desc, p, Dv, Dk, og, ov, ok, odq, workspace, false, st);
+        }
+        if (e != hipSuccess) return hip_status(e, "causal linear dq launch");
     }
-    // 16-bit inputs of the sizes the matrix-core kernels take go there when every row is 16-byte aligned
-    const bool mfma = !(desc->flags & FLARE_FLAG_FORCE_GENERIC) && flare::causal_linear_mfma_supported(desc->dtype, desc->Dk, desc->Dv) &&
-                      strides_mult8(desc->q_stride) && strides_mult8(desc->k_stride) && strides_mult8(desc->v_stride) &&
-                      strides_mult8(desc->y_stride) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(y);
-    if (mfma) return hip_status(flare::launch_causal_linear_mfma(a, desc->dtype, static_cast<hipStream_t>(stream)), "causal linear launch");
-    return hip_status(flare::launch_causal_linear(a, desc->dtype, static_cast<hipStream_t>(stream)), "causal linear launch");
+    if (square && dk && dv) {
+        flare::CausalLinearArgs a = cl_args(desc, p, Dk, Dv, ok, oq, og, odv, workspace, true);
+        const bool both = flare::causal_linear_dkv_supported(desc->dtype, Dk, Dv);
+        e = flare::launch_causal_linear_mfma(a, desc->dtype, both ? 1 : 3, st);
+        if (e != hipSuccess) return hip_status(e, "causal linear dv launch");
+        if (both) {
+            flare::CausalLinearDkvArgs f;
+            memset(&f, 0, sizeof(f));
+            f.q = cl_op(oq, N, desc->dtype, true, f.qs);
+            f.k = cl_op(ok, N, desc->dtype, true, f.ks);
+            f.v = cl_op(ov, N, desc->dtype, true, f.vs);
+            f.gy = cl_op(og, N, desc->dtype, true, f.gs);
+            f.dk = const_cast<void*>(cl_op(odk, N, desc->dtype, true, f.dks));
+            f.dv = const_cast<void*>(cl_op(odv, N, desc->dtype, true, f.dvs));
+            f.states = static_cast<const float*>(workspace);
+            f.B = desc->B; f.H = H; f.N = N; f.D = Dk;
+            f.n_segs = p.n_segs; f.seg_len = p.seg_len;
+            f.inv_n = a.inv_n;
+            e = flare::launch_causal_linear_dkv(f, desc->dtype, st);
+        } else {
+            a = cl_args(desc, p, Dv, Dk, ov, og, oq, odk, workspace, true);
+            a.slot_t = 1;
+            e = flare::launch_causal_linear_mfma(a, desc->dtype, 2, st);
+        }
+        return hip_status(e, "causal linear dk launch");
+    }
+    if (dk) e = cl_run(desc, p, Dv, Dk, ov, og, oq, odk, workspace, true, st);
+    if (e == hipSuccess && dv) e = cl_run(desc, p, Dk, Dv, ok, oq, og, odv, workspace, true, st);
+    return hip_status(e, "causal linear dk / dv launch");
 }
 
 static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const float* w_in, const float* b_in, int out_dim,

@@ -120,8 +120,10 @@ __global__ __launch_bounds__(256, 2) void causal_linear_mfma_kernel(CausalLinear
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                U[itw][dt][r] = STATE_ONLY ? 0.f : slot[(int64_t)(16 * (w * ITW + itw) + 4 * g + r) * DV + 16 * dt + c16];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * (w * ITW + itw) + 4 * g + r, d = 16 * dt + c16;
+                U[itw][dt][r] = STATE_ONLY ? 0.f : slot[a.slot_t ? d * DK + i : i * DV + d];
+            }
 
     // one register set: the next tile is requested at the top of an iteration and handed to LDS at its bottom.
     // Rows past the end of the segment repeat its last row (no branch around a load) and are staged as zeros.
@@ -280,6 +282,204 @@ __global__ __launch_bounds__(256, 2) void causal_linear_mfma_kernel(CausalLinear
     }
 }
 
+// ---- dk and dv of the backward, 16-bit, Dk == Dv == D -----------------------------------------------------------------
+//   dk_tau = (1/N) sum_{t >= tau} <v_tau, gy_t> q_t,   dv_tau = (1/N) sum_{t >= tau} <k_tau, q_t> gy_t
+// Both run over the reversed token axis (the launch argument's token strides are negative) with the same running state
+// R = sum q_t gy_t^T: dv uses it as the forward uses S, dk uses its transpose.  One launch stages every Q and GY tile once
+// for both gradients and for the state's update, and reads the token's own k and v rows straight from global memory:
+// six [N,D] arrays cross HBM instead of the eight of two output launches (and the pair needs one state pass, not two).
+// Bound by memory: 403 MB in 79 us (5.1 TB/s, the rate of a plain copy here) at B=4, H=8, N=16,384, D=64 bf16, where two
+// output launches with a state pass each took 154 us, and flipping the inputs and outputs in memory for them 412 us more.
+// R is published once, in the operand order of dv's product; dk's operand (rows i, contraction over d) is read back
+// from it by transposed reads: the entries hold four consecutive i of one d in 8 contiguous bytes.
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_linear_dkv_kernel(CausalLinearDkvArgs a)
+{
+    constexpr int KD = D / 32, DT = D / 16, ITW = DT / 4;
+    constexpr int RS = D + kPad;                      // LDS row stride in elements
+    constexpr int PT = kTile * (D / 8) / 256;         // 16-byte chunks of a tile per thread
+    using M_ = Ml<T>;
+
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    uint16_t* qt = reinterpret_cast<uint16_t*>(smem);            // [64][RS]
+    uint16_t* gt = qt + kTile * RS;                               // [64][RS]
+    u32x4* sop = reinterpret_cast<u32x4*>(gt + kTile * RS);       // [DT][KD][64]: R^T / N as A operands
+
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+    const int seg = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
+    const uint16_t* q = (const uint16_t*)a.q + b * a.qs[0] + h * a.qs[1];
+    const uint16_t* k = (const uint16_t*)a.k + b * a.ks[0] + h * a.ks[1];
+    const uint16_t* v = (const uint16_t*)a.v + b * a.vs[0] + h * a.vs[1];
+    const uint16_t* gy = (const uint16_t*)a.gy + b * a.gs[0] + h * a.gs[1];
+    uint16_t* dk = (uint16_t*)a.dk + b * a.dks[0] + h * a.dks[1];
+    uint16_t* dv = (uint16_t*)a.dv + b * a.dvs[0] + h * a.dvs[1];
+    const float* slot = a.states + ((int64_t)bh * a.n_segs + seg) * D * D;
+    const int n_lo = seg * a.seg_len, n_hi = min(a.N, n_lo + a.seg_len);
+    const int tiles = (n_hi - n_lo + kTile - 1) / kTile;
+
+    f32x4 U[ITW][DT];
+#pragma unroll
+    for (int itw = 0; itw < ITW; ++itw)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) U[itw][dt][r] = slot[(16 * (w * ITW + itw) + 4 * g + r) * D + 16 * dt + c16];
+
+    u32x4 qr[PT], gr[PT], kn[KD], vn[KD], kc[KD], vc[KD];
+    auto fetch = [&](int n0) {
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            const int c = tid + i * 256, tok = c / (D / 8), ch = c % (D / 8);
+            const int64_t n = min(n0 + tok, n_hi - 1);
+            qr[i] = *reinterpret_cast<const u32x4*>(q + n * a.qs[2] + ch * 8);
+            gr[i] = *reinterpret_cast<const u32x4*>(gy + n * a.gs[2] + ch * 8);
+        }
+        const int64_t n = min(n0 + 16 * w + c16, n_hi - 1);
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) {
+            kn[kd] = *reinterpret_cast<const u32x4*>(k + n * a.ks[2] + 32 * kd + 8 * g);
+            vn[kd] = *reinterpret_cast<const u32x4*>(v + n * a.vs[2] + 32 * kd + 8 * g);
+        }
+    };
+    auto stage = [&](int n0) {
+        const u32x4 z4 = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            const int c = tid + i * 256, tok = c / (D / 8), ch = c % (D / 8);
+            const bool in = n0 + tok < n_hi;
+            *reinterpret_cast<u32x4*>(qt + tok * RS + ch * 8) = in ? qr[i] : z4;
+            *reinterpret_cast<u32x4*>(gt + tok * RS + ch * 8) = in ? gr[i] : z4;
+        }
+    };
+    // as the forward's publish: entry of lane (gl, cl) of tile (dt, kd) = R[32 kd + 8 gl + e][16 dt + cl] / N, e = 0..7
+    auto publish = [&]() {
+#pragma unroll
+        for (int itw = 0; itw < ITW; ++itw) {
+            const int it = w * ITW + itw, kd = it >> 1, gl = 2 * (it & 1) + (g >> 1);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const f32x4 u = U[itw][dt] * a.inv_n;
+                uint8_t* e = reinterpret_cast<uint8_t*>(sop + (dt * KD + kd) * 64 + gl * 16 + c16) + 8 * (g & 1);
+                *reinterpret_cast<uint2*>(e) = make_uint2(M_::pack2(u[0], u[1]), M_::pack2(u[2], u[3]));
+            }
+        }
+    };
+    auto tr32 = [&](const uint16_t* tile, int bl, int col) {
+        const uint2 lo = tr16(tile + (16 * bl + 4 * g + (c16 >> 2)) * RS + col + 4 * (c16 & 3));
+        const uint2 hi = tr16(tile + (16 * bl + 16 + 4 * g + (c16 >> 2)) * RS + col + 4 * (c16 & 3));
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    };
+    // R[16 it + c16][32 kd + 8 g + e], e = 0..7: rows i, contraction over d, from the published entries
+    auto rrow = [&](int it, int kd) {
+        auto piece = [&](int d) {       // the 8 bytes of R[16 it + 4 (c16 & 3) .. + 3][d]
+            const int i = 16 * it + 4 * (c16 & 3);
+            return tr16(reinterpret_cast<const uint8_t*>(sop + ((d >> 4) * KD + (i >> 5)) * 64 + ((i & 31) >> 3) * 16 + (d & 15)) + 2 * (i & 7));
+        };
+        const uint2 lo = piece(32 * kd + 8 * g + (c16 >> 2)), hi = piece(32 * kd + 8 * g + 4 + (c16 >> 2));
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    };
+    // (masked scores of the wave's 16 tokens against the tile's) x value tile, for one of the two gradients: own = the
+    // tokens' own rows, key / val = the staged tiles
+    auto intra = [&](const uint16_t* key, const uint16_t* val, const u32x4 (&own)[KD], f32x4 (&acc)[DT]) {
+        const f32x4 zf = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = zf;
+        auto block_scores = [&](int bl) {
+            f32x4 s = zf;
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd)
+                s = M_::mma32(*reinterpret_cast<const u32x4*>(key + (16 * bl + c16) * RS + 32 * kd + 8 * g), own[kd], s);
+            if (bl == w) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[r] = 4 * g + r <= c16 ? s[r] : 0.f;
+            }
+            return make_uint2(M_::pack2(s[0], s[1]), M_::pack2(s[2], s[3]));
+        };
+#pragma unroll
+        for (int bl = 0; bl < 4; bl += 2) {
+            if (bl > w) break;      // uniform over the wave
+            const uint2 p0 = block_scores(bl);
+            uint2 p1 = make_uint2(0u, 0u);
+            if (bl + 1 <= w) p1 = block_scores(bl + 1);
+            const u32x4 pb = {p0.x, p0.y, p1.x, p1.y};
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[dt] = M_::mma32(tr32(val, bl, 16 * dt), pb, acc[dt]);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] *= a.inv_n;
+    };
+
+    if (tiles > 0) {
+        fetch(n_lo);
+        stage(n_lo);
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) { kc[kd] = kn[kd]; vc[kd] = vn[kd]; }
+        publish();
+    }
+    __syncthreads();
+
+    int n0 = n_lo;
+    for (int t = 0; t < tiles; ++t, n0 += kTile) {
+        fetch(n0 + kTile);      // unconditional: past the end the last rows are read again and never used
+        uint2 dvp[DT], dkp[DT];
+        f32x4 acc[DT];
+        intra(qt, gt, kc, acc);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd) acc[dt] = M_::mma32(sop[(dt * KD + kd) * 64 + lane], kc[kd], acc[dt]);
+            dvp[dt] = make_uint2(M_::pack2(acc[dt][0], acc[dt][1]), M_::pack2(acc[dt][2], acc[dt][3]));
+        }
+        intra(gt, qt, vc, acc);
+#pragma unroll
+        for (int it = 0; it < DT; ++it) {
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd) acc[it] = M_::mma32(rrow(it, kd), vc[kd], acc[it]);
+            dkp[it] = make_uint2(M_::pack2(acc[it][0], acc[it][1]), M_::pack2(acc[it][2], acc[it][3]));
+        }
+        // R += Q^T GY over the 64 tokens of the staged tiles, for the wave's rows of R
+#pragma unroll
+        for (int bl = 0; bl < 4; bl += 2) {
+            u32x4 gop[DT];
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) gop[dt] = tr32(gt, bl, 16 * dt);
+#pragma unroll
+            for (int itw = 0; itw < ITW; ++itw) {
+                const u32x4 qop = tr32(qt, bl, 16 * (w * ITW + itw));
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) U[itw][dt] = M_::mma32(qop, gop[dt], U[itw][dt]);
+            }
+        }
+        // the next tile's rows are waited for ahead of the conditional stores (see the forward)
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        const int64_t n = n0 + 16 * w + c16;
+        if (n < n_hi) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                *reinterpret_cast<uint2*>(dk + n * a.dks[2] + 16 * dt + 4 * g) = dkp[dt];
+                *reinterpret_cast<uint2*>(dv + n * a.dvs[2] + 16 * dt + 4 * g) = dvp[dt];
+            }
+        }
+        __syncthreads();        // everyone is done with this tile's rows and state operands
+        stage(n0 + kTile);
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) { kc[kd] = kn[kd]; vc[kd] = vn[kd]; }
+        publish();
+        __syncthreads();
+    }
+}
+
+template <typename T, int D>
+hipError_t launch_dkv(const CausalLinearDkvArgs& a, hipStream_t st)
+{
+    auto kern = causal_linear_dkv_kernel<T, D>;
+    constexpr size_t lds = lds_bytes<D, D, false>();
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3(a.n_segs, a.B * a.H), dim3(256), lds, st, a);
+    return hipGetLastError();
+}
+
 // ---- fp32 inputs: the same scheme on v_mfma_f32_16x16x4_f32 ------------------------------------------------------
 // A: lane (row c16, k = g) one float, B: lane (column c16, k = g) one float, accumulators as above.  A product over Dk
 // takes Dk/4 instructions; the k-slot of lane group g in instruction j is feature g Dk/4 + j, so that a lane's share of a
@@ -321,8 +521,10 @@ __global__ __launch_bounds__(256, 2) void causal_linear_f32_kernel(CausalLinearA
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                U[itw][dt][r] = STATE_ONLY ? 0.f : slot[(int64_t)(16 * (w * ITW + itw) + 4 * g + r) * DV + 16 * dt + c16];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * (w * ITW + itw) + 4 * g + r, d = 16 * dt + c16;
+                U[itw][dt][r] = STATE_ONLY ? 0.f : slot[a.slot_t ? d * DK + i : i * DV + d];
+            }
 
     f32x4 kr[KPT], vr[VPT], qn[QL / 4], qc[QL / 4];
     auto fetch = [&](int n0) {
@@ -462,7 +664,7 @@ __global__ __launch_bounds__(256, 2) void causal_linear_f32_kernel(CausalLinearA
 }
 
 template <int DK, int DV>
-hipError_t launch_f32_dd(const CausalLinearArgs& a, hipStream_t st)
+hipError_t launch_f32_dd(const CausalLinearArgs& a, int phases, hipStream_t st)
 {
     const int BH = a.B * a.H;
     auto state_k = causal_linear_f32_kernel<DK, DV, true>;
@@ -472,24 +674,26 @@ hipError_t launch_f32_dd(const CausalLinearArgs& a, hipStream_t st)
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(out_k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_o);
     if (e != hipSuccess) return e;
-    if (a.n_segs > 1) hipLaunchKernelGGL(state_k, dim3(a.n_segs - 1, BH), dim3(256), lds_s, st, a);
-    e = launch_causal_linear_prefix(a, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(out_k, dim3(a.n_segs, BH), dim3(256), lds_o, st, a);
+    if (phases & 1) {
+        if (a.n_segs > 1) hipLaunchKernelGGL(state_k, dim3(a.n_segs - 1, BH), dim3(256), lds_s, st, a);
+        e = launch_causal_linear_prefix(a, st);
+        if (e != hipSuccess) return e;
+    }
+    if (phases & 2) hipLaunchKernelGGL(out_k, dim3(a.n_segs, BH), dim3(256), lds_o, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_f32(const CausalLinearArgs& a, hipStream_t st)
+hipError_t launch_f32(const CausalLinearArgs& a, int phases, hipStream_t st)
 {
-    if (a.Dk == 64 && a.Dv == 32) return launch_f32_dd<64, 32>(a, st);
-    if (a.Dk == 64 && a.Dv == 64) return launch_f32_dd<64, 64>(a, st);
-    if (a.Dk == 128 && a.Dv == 32) return launch_f32_dd<128, 32>(a, st);
-    if (a.Dk == 128 && a.Dv == 64) return launch_f32_dd<128, 64>(a, st);
+    if (a.Dk == 64 && a.Dv == 32) return launch_f32_dd<64, 32>(a, phases, st);
+    if (a.Dk == 64 && a.Dv == 64) return launch_f32_dd<64, 64>(a, phases, st);
+    if (a.Dk == 128 && a.Dv == 32) return launch_f32_dd<128, 32>(a, phases, st);
+    if (a.Dk == 128 && a.Dv == 64) return launch_f32_dd<128, 64>(a, phases, st);
     return hipErrorInvalidValue;
 }
 
 template <typename T, int DK, int DV>
-hipError_t launch_dd(const CausalLinearArgs& a, hipStream_t st)
+hipError_t launch_dd(const CausalLinearArgs& a, int phases, hipStream_t st)
 {
     const int BH = a.B * a.H;
     auto state_k = causal_linear_mfma_kernel<T, DK, DV, true>;
@@ -499,29 +703,31 @@ hipError_t launch_dd(const CausalLinearArgs& a, hipStream_t st)
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(out_k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_o);
     if (e != hipSuccess) return e;
-    if (a.n_segs > 1) hipLaunchKernelGGL(state_k, dim3(a.n_segs - 1, BH), dim3(256), lds_s, st, a);
-    e = launch_causal_linear_prefix(a, st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(out_k, dim3(a.n_segs, BH), dim3(256), lds_o, st, a);
+    if (phases & 1) {
+        if (a.n_segs > 1) hipLaunchKernelGGL(state_k, dim3(a.n_segs - 1, BH), dim3(256), lds_s, st, a);
+        e = launch_causal_linear_prefix(a, st);
+        if (e != hipSuccess) return e;
+    }
+    if (phases & 2) hipLaunchKernelGGL(out_k, dim3(a.n_segs, BH), dim3(256), lds_o, st, a);
     return hipGetLastError();
 }
 
 template <typename T, int DK>
-hipError_t launch_d(const CausalLinearArgs& a, hipStream_t st)
+hipError_t launch_d(const CausalLinearArgs& a, int phases, hipStream_t st)
 {
     switch (a.Dv) {
-        case 32:  return launch_dd<T, DK, 32>(a, st);
-        case 64:  return launch_dd<T, DK, 64>(a, st);
-        case 128: return launch_dd<T, DK, 128>(a, st);
+        case 32:  return launch_dd<T, DK, 32>(a, phases, st);
+        case 64:  return launch_dd<T, DK, 64>(a, phases, st);
+        case 128: return launch_dd<T, DK, 128>(a, phases, st);
         default:  return hipErrorInvalidValue;
     }
 }
 
 template <typename T>
-hipError_t launch_t(const CausalLinearArgs& a, hipStream_t st)
+hipError_t launch_t(const CausalLinearArgs& a, int phases, hipStream_t st)
 {
-    if (a.Dk == 64) return launch_d<T, 64>(a, st);
-    if (a.Dk == 128) return launch_d<T, 128>(a, st);
+    if (a.Dk == 64) return launch_d<T, 64>(a, phases, st);
+    if (a.Dk == 128) return launch_d<T, 128>(a, phases, st);
     return hipErrorInvalidValue;
 }
 
@@ -533,10 +739,19 @@ bool causal_linear_mfma_supported(int dtype, int Dk, int Dv)
     return (dtype == 1 || dtype == 2) && (Dk == 64 || Dk == 128) && (Dv == 32 || Dv == 64 || Dv == 128);
 }
 
-hipError_t launch_causal_linear_mfma(const CausalLinearArgs& a, int dtype, hipStream_t st)
+hipError_t launch_causal_linear_mfma(const CausalLinearArgs& a, int dtype, int phases, hipStream_t st)
 {
-    if (dtype == 0) return launch_f32(a, st);
-    return dtype == 1 ? launch_t<bf16_t>(a, st) : launch_t<f16_t>(a, st);
+    if (dtype == 0) return launch_f32(a, phases, st);
+    return dtype == 1 ? launch_t<bf16_t>(a, phases, st) : launch_t<f16_t>(a, phases, st);
+}
+
+// D = 64 only: at 128 the running state, both gradients' accumulators and the rows in flight spill 97 of 256 registers
+bool causal_linear_dkv_supported(int dtype, int Dk, int Dv) { return (dtype == 1 || dtype == 2) && Dk == 64 && Dv == 64; }
+
+hipError_t launch_causal_linear_dkv(const CausalLinearDkvArgs& a, int dtype, hipStream_t st)
+{
+    if (a.D != 64) return hipErrorInvalidValue;
+    return dtype == 1 ? launch_dkv<bf16_t, 64>(a, st) : launch_dkv<f16_t, 64>(a, st);
 }
 
 }  // namespace flare

@@ -228,7 +228,18 @@ struct CausalLinearArgs {
     int B, H, N, Dk, Dv;
     int n_segs, seg_len;   // seg_len is a multiple of the 64-token tile
     float inv_n;           // 1 / N
-    int64_t qs[3], ks[3], vs[3], ys[3];
+    int slot_t;            // 1: the slots hold the transposed states [Dv][Dk] (outputs only; matrix-core kernels)
+    int64_t qs[3], ks[3], vs[3], ys[3];   // a token stride may be negative: the token axis reversed
+};
+
+// dk and dv of causal linear attention in one launch (causal_linear_mfma.hip); every token stride is the reversed one
+struct CausalLinearDkvArgs {
+    const void* q; const void* k; const void* v; const void* gy; void* dk; void* dv;
+    const float* states;   // [B*H, n_segs, D, D]: sum of q_t gy_t^T over the segments behind (exclusive prefix)
+    int B, H, N, D;
+    int n_segs, seg_len;
+    float inv_n;
+    int64_t qs[3], ks[3], vs[3], gs[3], dks[3], dvs[3];
 };
 
 struct MlpArgs {
@@ -362,7 +373,9 @@ hipError_t launch_causal_linear(const CausalLinearArgs& a, int dtype, hipStream_
 hipError_t launch_causal_linear_prefix(const CausalLinearArgs& a, hipStream_t st);   // exclusive prefix over the segment states
 // matrix-core kernels (causal_linear_mfma.hip): 16-bit inputs, Dk in {64, 128}, Dv in {32, 64, 128}
 bool       causal_linear_mfma_supported(int dtype, int Dk, int Dv);
-hipError_t launch_causal_linear_mfma(const CausalLinearArgs& a, int dtype, hipStream_t st);
+hipError_t launch_causal_linear_mfma(const CausalLinearArgs& a, int dtype, int phases, hipStream_t st);   // bit 0: states and prefix, bit 1: outputs
+bool       causal_linear_dkv_supported(int dtype, int Dk, int Dv);
+hipError_t launch_causal_linear_dkv(const CausalLinearDkvArgs& a, int dtype, hipStream_t st);
 
 hipError_t launch_triple_state(const TripleArgs& a, int dtype, hipStream_t st);
 hipError_t launch_triple_merge(const TripleArgs& a, hipStream_t st);

@@ -1109,7 +1109,19 @@ def flare_causal_decode_step(q, k_t, v_t, state, scale: float = 1.0, inplace: bo
 # --------------------------------------------------------------------------------------
 # causal linear attention
 # --------------------------------------------------------------------------------------
+def _causal_linear_desc(q, k, v, y, n_segs=0, force_generic=False):
+    B, H, N, Dk = q.shape
+    d = _lib.FlareCausalLinearDesc()
+    d.B, d.H, d.N, d.Dk, d.Dv = B, H, N, Dk, v.shape[-1]
+    d.dtype = _dtype_code(q)
+    d.n_segs = int(n_segs)
+    d.flags = _lib.FLAG_FORCE_GENERIC if force_generic else 0
+    d.q_stride, d.k_stride, d.v_stride, d.y_stride = _s3(q), _s3(k), _s3(v), _s3(y)
+    return d
+
+
 def _causal_linear_forward(q, k, v, n_segs: int = 0, force_generic: bool = False):
+    """(y, the launch's workspace: the segments' states, which the backward starts from)."""
     _require_cuda(q, k, v)
     lib = _lib.load()
     if q.dim() != 4 or q.shape != k.shape:
@@ -1119,15 +1131,9 @@ def _causal_linear_forward(q, k, v, n_segs: int = 0, force_generic: bool = False
         raise ValueError(f"V must have shape ({B}, {H}, {N}, Dv). Got V.shape={tuple(v.shape)}")
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError("Q, K, V must share one dtype")
-    Dv = v.shape[-1]
     q, k, v = _rows_last_contig(q), _rows_last_contig(k), _rows_last_contig(v)
-    y = torch.empty((B, H, N, Dv), dtype=q.dtype, device=q.device)
-    d = _lib.FlareCausalLinearDesc()
-    d.B, d.H, d.N, d.Dk, d.Dv = B, H, N, Dk, Dv
-    d.dtype = _dtype_code(q)
-    d.n_segs = int(n_segs)
-    d.flags = _lib.FLAG_FORCE_GENERIC if force_generic else 0
-    d.q_stride, d.k_stride, d.v_stride, d.y_stride = _s3(q), _s3(k), _s3(v), _s3(y)
+    y = torch.empty((B, H, N, v.shape[-1]), dtype=q.dtype, device=q.device)
+    d = _causal_linear_desc(q, k, v, y, n_segs, force_generic)
     with _on_device(q.device):
         need = C.c_size_t(0)
         _lib.check(lib.flare_causal_linear_workspace_bytes(C.byref(d), C.byref(need)),
@@ -1136,34 +1142,38 @@ def _causal_linear_forward(q, k, v, n_segs: int = 0, force_generic: bool = False
         rc = lib.flare_causal_linear_fwd(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(y), _ptr(ws), ws.numel(),
                                          C.c_void_p(_stream_ptr(q.device)))
     _lib.check(rc, "flare_causal_linear_fwd")
-    return y
+    return y, ws
 
 
 class _CausalLinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v):
-        ctx.save_for_backward(q, k, v)
-        return _causal_linear_forward(q, k, v)
+        q, k, v = _rows_last_contig(q), _rows_last_contig(k), _rows_last_contig(v)
+        y, ws = _causal_linear_forward(q, k, v)
+        ctx.save_for_backward(q, k, v, ws)
+        return y
 
     @staticmethod
     @once_differentiable
     def backward(ctx, gy):
-        # Every gradient is a causal linear attention again (the same kernels):
-        #   dq_t   = (1/N) sum_{tau <= t} <gy_t, v_tau> k_tau   = CL(gy, v, k)
-        #   dk_tau = (1/N) sum_{t >= tau} <v_tau, gy_t> q_t     = CL(v, gy, q) with the token axis reversed
-        #   dv_tau = (1/N) sum_{t >= tau} <k_tau, q_t> gy_t     = CL(k, q, gy) with the token axis reversed
-        q, k, v = ctx.saved_tensors
+        # Every gradient is a causal linear attention again (the same kernels, the last two over the reversed token axis):
+        #   dq_t   = (1/N) sum_{tau <= t} <gy_t, v_tau> k_tau
+        #   dk_tau = (1/N) sum_{t >= tau} <v_tau, gy_t> q_t
+        #   dv_tau = (1/N) sum_{t >= tau} <k_tau, q_t> gy_t
+        q, k, v, fwd_ws = ctx.saved_tensors
         gy = gy.to(q.dtype)
-        need = ctx.needs_input_grad
-        gq = _causal_linear_forward(gy, v, k) if need[0] else None
-        gk = gv = None
-        if need[1] or need[2]:
-            qr, kr, vr, gr = (t.flip(2) for t in (q, k, v, gy))
-            if need[1]:
-                gk = _causal_linear_forward(vr, gr, qr).flip(2)
-            if need[2]:
-                gv = _causal_linear_forward(kr, qr, gr).flip(2)
-        return gq, gk, gv
+        if gy.stride(-1) != 1 or any(s % 8 for s in gy.stride()[:3]) or gy.data_ptr() % 16 or gy.stride(2) < gy.shape[-1]:
+            gy = gy.contiguous()
+        grads = [torch.empty(t.shape, dtype=q.dtype, device=q.device) if need else None
+                 for t, need in zip((q, k, v), ctx.needs_input_grad)]
+        ws = torch.empty_like(fwd_ws)
+        d = _causal_linear_desc(q, k, v, v)
+        with _on_device(q.device):
+            rc = _lib.load().flare_causal_linear_bwd(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(gy), _s3(gy), _ptr(fwd_ws),
+                                                     *(_ptr(t) for t in grads), _ptr(ws), ws.numel(),
+                                                     C.c_void_p(_stream_ptr(q.device)))
+        _lib.check(rc, "flare_causal_linear_bwd")
+        return tuple(grads)
 
 
 def causal_linear_attention(q, k, v, n_segs: int = 0, force_generic: bool = False):
@@ -1174,7 +1184,7 @@ def causal_linear_attention(q, k, v, n_segs: int = 0, force_generic: bool = Fals
     force_generic=True, as fp32 FMA loops."""
     if n_segs == 0 and not force_generic and torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
         return _CausalLinearFn.apply(q, k, v)
-    return _causal_linear_forward(q, k, v, n_segs, force_generic)
+    return _causal_linear_forward(q, k, v, n_segs, force_generic)[0]
 
 
 class CausalLinear:

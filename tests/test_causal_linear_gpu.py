@@ -157,3 +157,29 @@ def test_gradients_through_the_same_kernels(dev, shape, dtype, tol):
     for a, b in ((qd, qr), (kd, kr), (vd, vr)):
         assert a.grad.dtype == dtype and a.grad.shape == b.grad.shape
         assert O.rel_l2(a.grad, b.grad) <= tol
+
+
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16), (128, torch.bfloat16), (64, torch.float32)])
+def test_gradients_of_square_heads(dev, N, D, dtype):
+    """Dk == Dv: dq starts from the forward's states (transposed), dk and dv share one state over the reversed tokens (one
+    launch for 16-bit heads of 64).  Edges of the 64-token tile, strided views, against fp64 autograd; 16-bit operands are
+    rounded twice on the way (scores, state): 2^-8 and 2^-11 per operand, so 2^-6 and 2^-9 with room, fp32 1e-5."""
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(N + D)
+    x = torch.randn(3, B, N, H * D, generator=g).to(dtype)
+    gy = torch.randn(B, N, H * D, generator=g).to(dtype)
+    heads = lambda t: t.view(B, N, H, D).permute(0, 2, 1, 3)
+    xd = [t.to(dev).requires_grad_(True) for t in x]
+    y = F.CausalLinear.apply(*(heads(t) for t in xd))
+    grads = torch.autograd.grad(y, xd, heads(gy.to(dev)))
+    xr = [t.double().requires_grad_(True) for t in x]
+    want = torch.autograd.grad(O.causal_linear_closed_form(*(heads(t) for t in xr)), xr, heads(gy.double()))
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -6, torch.float16: 2.0 ** -9}[dtype]
+    for a, b in zip(grads, want):
+        assert O.rel_l2(a, b) <= tol
+    # one gradient alone takes the separate launches: the same values up to the order of the sums
+    for i in range(3):
+        xi = [t.detach().requires_grad_(j == i) for j, t in enumerate(xd)]
+        (one,) = torch.autograd.grad(F.CausalLinear.apply(*(heads(t) for t in xi)), [xi[i]], heads(gy.to(dev)))
+        assert O.rel_l2(one, want[i]) <= tol
