@@ -344,7 +344,7 @@ int check_triple_desc(const FlareTripleDesc* d)
     return FLARE_OK;
 }
 
-struct TriplePlan { bool mfma; int n_splits, n_parts, tokens_per_split; size_t per_split, off_kk, total; };
+struct TriplePlan { bool mfma, d32; int n_splits, n_parts, tokens_per_split; size_t per_split, off_kk, off_tab, total; };
 
 bool strides_mult4(const int64_t* s) { return s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0; }
 bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
@@ -360,8 +360,14 @@ TriplePlan plan_triple(const FlareTripleDesc* d)
 {
     TriplePlan p;
     p.mfma = triple_wants_mfma(d);
+    // head dims of 32: one block of the state instead of eight, where every row of the inputs is 16-byte aligned
+    p.d32 = p.mfma && flare::triple32_supported(d->dtype, d->Dq, d->Dv) && strides_mult8(d->k1_stride) && strides_mult8(d->k2_stride) &&
+            strides_mult8(d->v_stride) && strides_mult8(d->q1_stride) && strides_mult8(d->q2_stride);
     int s = d->n_splits;
-    if (s <= 0) {
+    if (s <= 0 && p.d32) {
+        const int tps = flare::triple32_tokens_per_split(d->N, (int64_t)d->B * d->H);
+        s = (d->N + tps - 1) / tps;
+    } else if (s <= 0) {
         // about two workgroups per compute unit: more splits only add partials to write and merge (the matrix-core
         // state kernel runs one workgroup per split and 16 x 16 x 16 block of the state)
         const int64_t nb = p.mfma ? (int64_t)(d->Dq / 16) * (d->Dv / 16) * (d->Dq / 16) : 1;
@@ -370,18 +376,38 @@ TriplePlan plan_triple(const FlareTripleDesc* d)
         if (s < 1) s = 1;
     }
     int64_t tps = ((int64_t)d->N + s - 1) / s;
-    tps = ((tps + 63) / 64) * 64;
+    tps = p.d32 ? (tps + 127) / 128 * 128 : (tps + 63) / 64 * 64;
     p.tokens_per_split = (int)tps;
     p.n_splits = (int)(((int64_t)d->N + tps - 1) / tps);
     p.n_parts = p.n_splits;
     // sized for whichever kernel family ends up running (misaligned pointers demote to the fp32 kernels)
     p.per_split = flare::triple_partial_floats(d->Dq, d->Dv, false);
     if (p.mfma) p.per_split = std::max(p.per_split, flare::triple_partial_floats(d->Dq, d->Dv, true));
+    if (p.d32) p.per_split = std::max(p.per_split, flare::kTriple32Partial);
     const size_t bh = (size_t)d->B * d->H;
     p.off_kk = bh * p.n_parts * p.per_split * 4;
     p.off_kk = (p.off_kk + 255) & ~(size_t)255;
-    p.total = p.off_kk + bh * d->Dq * d->Dq * 4;
+    p.off_tab = (p.off_kk + bh * d->Dq * d->Dq * 4 + 255) & ~(size_t)255;
+    p.total = p.off_tab + (p.d32 ? bh * flare::triple32_table_bytes() : 0);
     return p;
+}
+
+bool out_strides32(const int64_t* s, const void* p) { return strides_mult8(s) && aligned16(p); }
+
+// Split partials of one state contraction, by the widest kernel the operands' alignment allows.
+struct TripleStateRun { flare::TripleArgs a; bool d32; };
+
+hipError_t triple_state_run(const FlareTripleDesc* d, const TriplePlan& p, const void* k1, const void* k2, const void* v, void* part,
+                            TripleStateRun* r, hipStream_t st)
+{
+    flare::TripleArgs& a = r->a;
+    a.k1 = k1; a.k2 = k2; a.v = v;
+    a.part = static_cast<float*>(part);
+    const bool mfma = p.mfma && aligned8(k1) && aligned8(k2) && aligned8(v);
+    r->d32 = p.d32 && aligned16(k1) && aligned16(k2) && aligned16(v);
+    a.diag_parts = mfma ? 1 : 0;
+    if (r->d32) return flare::launch_triple_state32(a, d->dtype, st);
+    return mfma ? flare::launch_triple_state_mfma(a, d->dtype, st) : flare::launch_triple_state(a, d->dtype, st);
 }
 
 void fill_triple_args(flare::TripleArgs& a, const FlareTripleDesc* d, const TriplePlan& p)
@@ -1209,6 +1235,64 @@ int flare_triple_workspace_bytes(const FlareTripleDesc* desc, size_t* bytes)
     return FLARE_OK;
 }
 
+namespace {
+
+// state (and kk) from the inputs; tab: where the 32-wide kernels leave the state's operand table (or NULL), *made says whether they did
+int triple_state_impl(const FlareTripleDesc* desc, const TriplePlan& p, const void* k1, const void* k2, const void* v, float* state,
+                      float* kk, void* workspace, uint16_t* tab, bool* made, hipStream_t st)
+{
+    TripleStateRun r;
+    fill_triple_args(r.a, desc, p);
+    r.a.state = state; r.a.kk = kk;
+    hipError_t e = triple_state_run(desc, p, k1, k2, v, workspace, &r, st);
+    if (e != hipSuccess) return hip_status(e, "triple state launch");
+    *made = r.d32 && tab;
+    if (!r.d32) return hip_status(flare::launch_triple_merge(r.a, st), "triple merge launch");
+    flare::Triple32MergeArgs m;
+    memset(&m, 0, sizeof(m));
+    m.part = r.a.part; m.BH = desc->B * desc->H; m.n_parts = p.n_parts; m.inv_n = 1.0f / (float)desc->N;
+    m.state = state; m.kk = desc->normalize ? kk : nullptr; m.tab = tab;
+    return hip_status(flare::launch_triple_merge32(m, desc->dtype, st), "triple merge launch");
+}
+
+int triple_out_impl(const FlareTripleDesc* desc, const TriplePlan& p, const void* q1, const void* q2, const float* state, const float* kk,
+                    const uint16_t* tab, void* out, hipStream_t st)
+{
+    if (p.d32 && aligned16(q1) && aligned16(q2) && out_strides32(desc->o_stride, out) && desc->H <= 65535) {
+        flare::Triple32OutArgs o;
+        memset(&o, 0, sizeof(o));
+        o.n_ops = 1; o.B = desc->B; o.H = desc->H; o.N = desc->N;
+        o.feature_map = desc->feature_map; o.normalize = desc->normalize;
+        o.op[0].q1 = q1; o.op[0].q2 = q2; o.op[0].out = out; o.op[0].tab = tab; o.op[0].state = state; o.op[0].kk = kk;
+        for (int i = 0; i < 3; ++i) { o.op[0].q1s[i] = desc->q1_stride[i]; o.op[0].q2s[i] = desc->q2_stride[i]; o.op[0].os[i] = desc->o_stride[i]; }
+        return hip_status(flare::launch_triple_out32(o, desc->dtype, st), "triple out launch");
+    }
+    flare::TripleArgs a;
+    fill_triple_args(a, desc, p);
+    a.q1 = q1; a.q2 = q2; a.out = out; a.state = const_cast<float*>(state); a.kk = const_cast<float*>(kk);
+    const bool mfma = p.mfma && aligned8(q1) && aligned8(q2) && aligned8(out) && strides_mult4(desc->o_stride);
+    return hip_status(mfma ? flare::launch_triple_out_mfma(a, desc->dtype, st) : flare::launch_triple_out(a, desc->dtype, st),
+                      "triple out launch");
+}
+
+int triple_check_workspace(const void* workspace, size_t have, size_t need)
+{
+    if (!workspace) return fail(FLARE_EWORKSPACE, "workspace is NULL");
+    if (have < need) return fail(FLARE_EWORKSPACE, "workspace has %zu bytes, %zu needed", have, need);
+    return FLARE_OK;
+}
+
+// Workspace of the backward behind the state contraction's own: the 32-wide kernels' five operand tables, or dS and the
+// exchanged copies of S and dS (fp32).
+size_t triple_bwd_extra(const FlareTripleDesc* d, const TriplePlan& p)
+{
+    const size_t bh = (size_t)d->B * d->H;
+    const size_t copies = 5 * bh * d->Dq * d->Dq * d->Dq * 4;
+    return p.d32 ? std::max(copies, 5 * bh * flare::triple32_table_bytes()) : copies;
+}
+
+}  // namespace
+
 int flare_triple_state_fwd(const FlareTripleDesc* desc, const void* k1, const void* k2, const void* v,
                            float* state, float* kk_state, void* workspace, size_t workspace_bytes,
                            void* stream)
@@ -1217,21 +1301,11 @@ int flare_triple_state_fwd(const FlareTripleDesc* desc, const void* k1, const vo
     if (rc != FLARE_OK) return rc;
     if (!k1 || !k2 || !v || !state) return fail(FLARE_EINVAL, "k1, k2, v and state must not be NULL");
     if (desc->normalize && !kk_state) return fail(FLARE_EINVAL, "kk_state is required when normalize != 0");
-    if (!workspace) return fail(FLARE_EWORKSPACE, "workspace is NULL");
     const TriplePlan p = plan_triple(desc);
-    if (workspace_bytes < p.total)
-        return fail(FLARE_EWORKSPACE, "workspace has %zu bytes, %zu needed", workspace_bytes, p.total);
-    flare::TripleArgs a;
-    fill_triple_args(a, desc, p);
-    a.k1 = k1; a.k2 = k2; a.v = v; a.state = state; a.kk = kk_state;
-    a.part = static_cast<float*>(workspace);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool mfma = p.mfma && aligned8(k1) && aligned8(k2) && aligned8(v);
-    if (mfma) a.n_parts = p.n_parts;
-    a.diag_parts = mfma ? 1 : 0;
-    hipError_t e = mfma ? flare::launch_triple_state_mfma(a, desc->dtype, st) : flare::launch_triple_state(a, desc->dtype, st);
-    if (e != hipSuccess) return hip_status(e, "triple state launch");
-    return hip_status(flare::launch_triple_merge(a, st), "triple merge launch");
+    rc = triple_check_workspace(workspace, workspace_bytes, p.total);
+    if (rc != FLARE_OK) return rc;
+    bool made;
+    return triple_state_impl(desc, p, k1, k2, v, state, kk_state, workspace, nullptr, &made, static_cast<hipStream_t>(stream));
 }
 
 int flare_triple_out_fwd(const FlareTripleDesc* desc, const void* q1, const void* q2, const float* state,
@@ -1241,14 +1315,7 @@ int flare_triple_out_fwd(const FlareTripleDesc* desc, const void* q1, const void
     if (rc != FLARE_OK) return rc;
     if (!q1 || !q2 || !state || !out) return fail(FLARE_EINVAL, "q1, q2, state and out must not be NULL");
     if (desc->normalize && !kk_state) return fail(FLARE_EINVAL, "kk_state is required when normalize != 0");
-    const TriplePlan p = plan_triple(desc);
-    flare::TripleArgs a;
-    fill_triple_args(a, desc, p);
-    a.q1 = q1; a.q2 = q2; a.out = out; a.state = const_cast<float*>(state); a.kk = const_cast<float*>(kk_state);
-    const bool mfma = p.mfma && aligned8(q1) && aligned8(q2) && aligned8(out) && strides_mult4(desc->o_stride);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    return hip_status(mfma ? flare::launch_triple_out_mfma(a, desc->dtype, st) : flare::launch_triple_out(a, desc->dtype, st),
-                      "triple out launch");
+    return triple_out_impl(desc, plan_triple(desc), q1, q2, state, kk_state, nullptr, out, static_cast<hipStream_t>(stream));
 }
 
 int flare_triple_fwd(const FlareTripleDesc* desc, const void* q1, const void* q2, const void* k1,
@@ -1259,14 +1326,103 @@ int flare_triple_fwd(const FlareTripleDesc* desc, const void* q1, const void* q2
     if (rc != FLARE_OK) return rc;
     if (!q1 || !q2 || !k1 || !k2 || !v || !state || !out)
         return fail(FLARE_EINVAL, "q1, q2, k1, k2, v, state and out must not be NULL");
-    if (!workspace) return fail(FLARE_EWORKSPACE, "workspace is NULL");
     const TriplePlan p = plan_triple(desc);
-    if (workspace_bytes < p.total)
-        return fail(FLARE_EWORKSPACE, "workspace has %zu bytes, %zu needed", workspace_bytes, p.total);
-    float* kk = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.off_kk);
-    rc = flare_triple_state_fwd(desc, k1, k2, v, state, kk, workspace, workspace_bytes, stream);
+    rc = triple_check_workspace(workspace, workspace_bytes, p.total);
     if (rc != FLARE_OK) return rc;
-    return flare_triple_out_fwd(desc, q1, q2, state, kk, out, stream);
+    float* kk = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.off_kk);
+    uint16_t* tab = p.d32 && aligned16(workspace) ? reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + p.off_tab) : nullptr;
+    bool made = false;
+    rc = triple_state_impl(desc, p, k1, k2, v, state, kk, workspace, tab, &made, static_cast<hipStream_t>(stream));
+    if (rc != FLARE_OK) return rc;
+    return triple_out_impl(desc, p, q1, q2, state, kk, made ? tab : nullptr, out, static_cast<hipStream_t>(stream));
+}
+
+int flare_triple_bwd_workspace_bytes(const FlareTripleDesc* desc, size_t* bytes)
+{
+    if (!bytes) return fail(FLARE_EINVAL, "bytes is NULL");
+    int rc = check_triple_desc(desc);
+    if (rc != FLARE_OK) return rc;
+    const TriplePlan p = plan_triple(desc);
+    *bytes = ((p.total + 255) & ~(size_t)255) + triple_bwd_extra(desc, p);
+    return FLARE_OK;
+}
+
+int flare_triple_bwd(const FlareTripleDesc* desc, const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
+                     const float* state, const float* dstate, const void* dout, void* dq1, void* dq2, void* dk1, void* dk2,
+                     void* dv, void* workspace, size_t workspace_bytes, void* stream)
+{
+    int rc = check_triple_desc(desc);
+    if (rc != FLARE_OK) return rc;
+    if (!q1 || !q2 || !k1 || !k2 || !v || !state || !dout || !dq1 || !dq2 || !dk1 || !dk2 || !dv)
+        return fail(FLARE_EINVAL, "q1, q2, k1, k2, v, state, dout and the gradients must not be NULL");
+    if (desc->Dq != desc->Dv) return fail(FLARE_EUNSUPPORTED, "the backward's contractions need Dq == Dv (got %d, %d)", desc->Dq, desc->Dv);
+    if (desc->feature_map || desc->normalize) return fail(FLARE_EUNSUPPORTED, "the backward takes neither a feature map nor the normaliser");
+    const TriplePlan p0 = plan_triple(desc);
+    const size_t base = (p0.total + 255) & ~(size_t)255;
+    rc = triple_check_workspace(workspace, workspace_bytes, base + triple_bwd_extra(desc, p0));
+    if (rc != FLARE_OK) return rc;
+    if (!aligned16(workspace)) return fail(FLARE_EINVAL, "workspace must be 16-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int B = desc->B, H = desc->H, N = desc->N, D = desc->Dq;
+    const size_t bh = (size_t)B * H;
+    const float inv_n = 1.0f / (float)N;
+    const int64_t cs[3] = {(int64_t)H * N * D, (int64_t)N * D, D};      // gradients are contiguous
+    // dS = (1/N) sum_n q1 dO q2, shaped as a state contraction of (q1, q2, dO)
+    FlareTripleDesc ds = *desc;
+    for (int i = 0; i < 3; ++i) { ds.k1_stride[i] = desc->q1_stride[i]; ds.k2_stride[i] = desc->q2_stride[i]; ds.v_stride[i] = desc->o_stride[i]; }
+    TriplePlan p = p0;                   // same sizes, same strides in another order
+    TripleStateRun r;
+    fill_triple_args(r.a, &ds, p);
+    p.mfma = triple_wants_mfma(&ds) && triple_wants_mfma(desc) && strides_mult4(desc->o_stride);
+    p.d32 = p0.d32 && strides_mult8(desc->o_stride) && aligned16(q1) && aligned16(q2) && aligned16(k1) && aligned16(k2) && aligned16(v) &&
+            aligned16(dout) && aligned16(dq1) && aligned16(dq2) && aligned16(dk1) && aligned16(dk2) && aligned16(dv) && (int64_t)H * 5 <= 65535;
+    float* dS = reinterpret_cast<float*>(static_cast<char*>(workspace) + base);
+    r.a.state = dS;
+    hipError_t e = triple_state_run(&ds, p, q1, q2, dout, workspace, &r, st);
+    if (e != hipSuccess) return hip_status(e, "triple dstate launch");
+    struct Op { const void* a; const int64_t* as; const void* b; const int64_t* bs; void* out; };
+    //                 dq1: dO, q2       dq2: q1, dO       dk1: v, k2       dk2: k1, v       dv: k1, k2
+    const Op ops[5] = {{dout, desc->o_stride, q2, desc->q2_stride, dq1}, {q1, desc->q1_stride, dout, desc->o_stride, dq2},
+                       {v, desc->v_stride, k2, desc->k2_stride, dk1}, {k1, desc->k1_stride, v, desc->v_stride, dk2},
+                       {k1, desc->k1_stride, k2, desc->k2_stride, dv}};
+    if (r.d32) {
+        const size_t tb = bh * flare::triple32_table_bytes();
+        uint16_t* t[5];                  // tables of S_ji, S_kj, dS_ji, dS_kj, dS
+        for (int i = 0; i < 5; ++i) t[i] = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + base + i * tb);
+        flare::Triple32MergeArgs m;
+        memset(&m, 0, sizeof(m));
+        m.part = r.a.part; m.BH = (int)bh; m.n_parts = p.n_parts; m.inv_n = inv_n; m.dstate = dstate;
+        m.fwd_state = state; m.fwd_tab_ji = t[0]; m.fwd_tab_kj = t[1]; m.tab_ji = t[2]; m.tab_kj = t[3]; m.tab = t[4];
+        e = flare::launch_triple_merge32(m, desc->dtype, st);
+        if (e != hipSuccess) return hip_status(e, "triple merge launch");
+        flare::Triple32OutArgs o;
+        memset(&o, 0, sizeof(o));
+        o.n_ops = 5; o.B = B; o.H = H; o.N = N;
+        for (int i = 0; i < 5; ++i) {
+            flare::Triple32OutOp& x = o.op[i];
+            x.q1 = ops[i].a; x.q2 = ops[i].b; x.out = ops[i].out; x.tab = t[i];
+            for (int c = 0; c < 3; ++c) { x.q1s[c] = ops[i].as[c]; x.q2s[c] = ops[i].bs[c]; x.os[c] = cs[c]; }
+        }
+        return hip_status(flare::launch_triple_out32(o, desc->dtype, st), "triple gradient launch");
+    }
+    e = flare::launch_triple_merge(r.a, st);
+    if (e != hipSuccess) return hip_status(e, "triple merge launch");
+    const size_t ns = bh * D * D * D;
+    float *s_ji = dS + ns, *s_kj = dS + 2 * ns, *d_ji = dS + 3 * ns, *d_kj = dS + 4 * ns;
+    e = flare::launch_triple_permute(const_cast<float*>(state), nullptr, 0.f, s_ji, s_kj, (int)bh, D, st);
+    if (e == hipSuccess) e = flare::launch_triple_permute(dS, dstate, inv_n, d_ji, d_kj, (int)bh, D, st);
+    if (e != hipSuccess) return hip_status(e, "triple permute launch");
+    const float* states[5] = {s_ji, s_kj, d_ji, d_kj, dS};
+    for (int i = 0; i < 5; ++i) {
+        FlareTripleDesc od = *desc;
+        for (int c = 0; c < 3; ++c) { od.q1_stride[c] = od.k1_stride[c] = ops[i].as[c]; od.q2_stride[c] = od.k2_stride[c] = ops[i].bs[c]; od.v_stride[c] = od.o_stride[c] = cs[c]; }
+        TriplePlan op = p0;
+        op.mfma = triple_wants_mfma(&od);
+        op.d32 = false;
+        rc = triple_out_impl(&od, op, ops[i].a, ops[i].b, states[i], nullptr, nullptr, ops[i].out, st);
+        if (rc != FLARE_OK) return rc;
+    }
+    return FLARE_OK;
 }
 
 }  // extern "C"

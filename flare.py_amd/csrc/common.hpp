@@ -170,6 +170,34 @@ __host__ __device__ inline size_t triple_partial_floats(int Dq, int Dv, bool dia
     return diag ? (size_t)(Dq / 16) * (Dv / 16) * (Dq / 16) * 4352 : (size_t)Dq * Dv * Dq + (size_t)Dq * Dq;
 }
 
+// Head dims of 32 (triple32_mfma.hip): floats of one split partial, 32 diagonals of 32 x 32 and the normaliser's tile
+constexpr size_t kTriple32Partial = 32768 + 1024;
+struct Triple32MergeArgs {
+    const float* part;                    // [BH, n_parts, kTriple32Partial]
+    int BH, n_parts;
+    float inv_n;
+    float* state; float* kk;              // [BH,32,32,32] and [BH,32,32] out, or null
+    const float* dstate;                  // [BH,32,32,32] or null: dstate / N is added to the sums
+    uint16_t* tab;                        // 16-bit operand tables of the sums, or null: as they are,
+    uint16_t* tab_ji; uint16_t* tab_kj;   // with the first two / the last two indices exchanged
+    const float* fwd_state;               // the forward's state or null: its two exchanged tables
+    uint16_t* fwd_tab_ji; uint16_t* fwd_tab_kj;
+};
+struct Triple32OutOp {
+    const void* q1; const void* q2; void* out;
+    const uint16_t* tab;                  // the state's operand table, or null: built from
+    const float* state;                   // the fp32 state
+    const float* kk;
+    int64_t q1s[3], q2s[3], os[3];
+};
+struct Triple32OutArgs {
+    Triple32OutOp op[5];
+    int n_ops;
+    int B, H, N;
+    int feature_map, normalize;
+    int tokens_per_wg;                    // set by the launcher
+};
+
 struct MixerBwdArgs {
     const void* q; const void* k; const void* v; const void* y; const void* dy;
     const float* z;          // [B,H,M,D] forward latent summary
@@ -388,5 +416,14 @@ hipError_t launch_triple_out_f32_mfma(const TripleArgs& a, hipStream_t st);
 bool       triple_mfma_supported(int dtype, int Dq, int Dv);
 hipError_t launch_triple_state_mfma(const TripleArgs& a, int dtype, hipStream_t st);
 hipError_t launch_triple_out_mfma(const TripleArgs& a, int dtype, hipStream_t st);
+// 16-bit head dims of 32 as one 32 x 32 x 32 block (triple32_mfma.hip): rows 16-byte aligned
+bool       triple32_supported(int dtype, int Dq, int Dv);
+size_t     triple32_table_bytes();        // of one (b,h)
+int        triple32_tokens_per_split(int64_t N, int64_t BH);
+hipError_t launch_triple_state32(const TripleArgs& a, int dtype, hipStream_t st);
+hipError_t launch_triple_merge32(const Triple32MergeArgs& a, int dtype, hipStream_t st);
+hipError_t launch_triple_out32(Triple32OutArgs& a, int dtype, hipStream_t st);
+// s += add * inv_n (add may be null), and s with its first two / last two indices exchanged; s, add, ji, kj [BH,D,D,D] fp32
+hipError_t launch_triple_permute(float* s, const float* add, float inv_n, float* ji, float* kj, int BH, int D, hipStream_t st);
 
 }  // namespace flare

@@ -129,6 +129,19 @@ __global__ __launch_bounds__(kThreads) void triple_merge_kernel(TripleArgs a)
     }
 }
 
+// One thread per element (i, j, k) of a state: s (+ add / N, written back) into its two copies with exchanged indices.
+__global__ __launch_bounds__(kThreads) void triple_permute_kernel(float* s, const float* add, float inv_n, float* ji, float* kj, int BH, int D)
+{
+    const size_t ns = (size_t)D * D * D, idx = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (idx >= ns * BH) return;
+    const size_t bh = idx / ns;
+    const int e = (int)(idx - bh * ns), i = e / (D * D), j = e / D % D, k = e % D;
+    float x = s[idx];
+    if (add) s[idx] = x = x + add[idx] * inv_n;
+    ji[bh * ns + ((size_t)j * D + i) * D + k] = x;
+    kj[bh * ns + ((size_t)i * D + k) * D + j] = x;
+}
+
 constexpr int kOutLdsFloats = 8192;
 
 // One thread per token; state rows staged through LDS IB rows at a time (broadcast reads).
@@ -261,6 +274,13 @@ hipError_t launch_triple_out(const TripleArgs& a, int dtype, hipStream_t st)
         case 1: return out_launch<bf16_t>(a, st);
         default: return out_launch<f16_t>(a, st);
     }
+}
+
+hipError_t launch_triple_permute(float* s, const float* add, float inv_n, float* ji, float* kj, int BH, int D, hipStream_t st)
+{
+    const size_t n = (size_t)BH * D * D * D;
+    hipLaunchKernelGGL(triple_permute_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, s, add, inv_n, ji, kj, BH, D);
+    return hipGetLastError();
 }
 
 }  // namespace flare

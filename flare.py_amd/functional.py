@@ -1199,6 +1199,17 @@ class CausalLinear:
 # --------------------------------------------------------------------------------------
 # triple attention
 # --------------------------------------------------------------------------------------
+def _triple_desc(q1, q2, k1, k2, v, out, feature_map=False, normalize=False, n_splits=0):
+    d = FlareTripleDesc()
+    d.B, d.H, d.N, d.Dq = q1.shape
+    d.Dv = v.shape[-1]
+    d.dtype = _dtype_code(q1)
+    d.feature_map, d.normalize, d.n_splits = int(feature_map), int(normalize), int(n_splits)
+    d.q1_stride, d.q2_stride, d.k1_stride, d.k2_stride = _s3(q1), _s3(q2), _s3(k1), _s3(k2)
+    d.v_stride, d.o_stride = _s3(v), _s3(out)
+    return d
+
+
 def _triple_forward(q1, q2, k1, k2, v, feature_map: bool, normalize: bool, n_splits: int = 0):
     _require_cuda(q1, q2, k1, k2, v)
     lib = _lib.load()
@@ -1225,14 +1236,7 @@ def _triple_forward(q1, q2, k1, k2, v, feature_map: bool, normalize: bool, n_spl
         return state[:, :, :Dq, :Dv, :Dq].contiguous(), out[..., :Dv].contiguous()
     state = torch.empty((B, H, Dq, Dv, Dq), dtype=torch.float32, device=q1.device)
     out = torch.empty((B, H, N, Dv), dtype=q1.dtype, device=q1.device)
-    d = FlareTripleDesc()
-    d.B, d.H, d.N, d.Dq, d.Dv = B, H, N, Dq, Dv
-    d.dtype = _dtype_code(q1)
-    d.feature_map = 1 if feature_map else 0
-    d.normalize = 1 if normalize else 0
-    d.n_splits = int(n_splits)
-    d.q1_stride, d.q2_stride, d.k1_stride, d.k2_stride = _s3(q1), _s3(q2), _s3(k1), _s3(k2)
-    d.v_stride, d.o_stride = _s3(v), _s3(out)
+    d = _triple_desc(q1, q2, k1, k2, v, out, feature_map, normalize, n_splits)
     need = C.c_size_t(0)
     _lib.check(lib.flare_triple_workspace_bytes(C.byref(d), C.byref(need)), "flare_triple_workspace_bytes")
     ws = torch.empty(max(int(need.value), 16), dtype=torch.uint8, device=q1.device)
@@ -1243,68 +1247,15 @@ def _triple_forward(q1, q2, k1, k2, v, feature_map: bool, normalize: bool, n_spl
     return state, out
 
 
-def _triple_desc(a, b, vlike, out):
-    B, H, N, Dq = a.shape
-    d = FlareTripleDesc()
-    d.B, d.H, d.N, d.Dq, d.Dv = B, H, N, Dq, vlike.shape[-1]
-    d.dtype = _dtype_code(a)
-    d.q1_stride = d.k1_stride = _s3(a)
-    d.q2_stride = d.k2_stride = _s3(b)
-    d.v_stride = _s3(vlike)
-    d.o_stride = _s3(out if out is not None else vlike)
-    return d
-
-
-def _triple_state_launch(k1, k2, v):
-    """state [B,H,Dq,Dv,Dq] fp32 = (1/N) sum_n k1[n,i] v[n,j] k2[n,k]  (flare_triple_state_fwd)."""
-    lib = _lib.load()
-    k1, k2, v = (_rows_last_contig(t) for t in (k1, k2, v))
-    B, H, N, Dq = k1.shape
-    state = torch.empty((B, H, Dq, v.shape[-1], Dq), dtype=torch.float32, device=k1.device)
-    d = _triple_desc(k1, k2, v, None)
-    need = C.c_size_t(0)
-    _lib.check(lib.flare_triple_workspace_bytes(C.byref(d), C.byref(need)), "flare_triple_workspace_bytes")
-    ws = torch.empty(max(int(need.value), 16), dtype=torch.uint8, device=k1.device)
-    with _on_device(k1.device):
-        rc = lib.flare_triple_state_fwd(C.byref(d), _ptr(k1), _ptr(k2), _ptr(v), _ptr(state), None, _ptr(ws), ws.numel(),
-                                        C.c_void_p(_stream_ptr(k1.device)))
-    _lib.check(rc, "flare_triple_state_fwd")
-    return state
-
-
-def _triple_out_launch(q1, q2, state):
-    """out [B,H,N,Dv] = sum_{i,k} q1[n,i] state[i,j,k] q2[n,k]  (flare_triple_out_fwd)."""
-    lib = _lib.load()
-    q1, q2 = _rows_last_contig(q1), _rows_last_contig(q2)
-    state = state.to(torch.float32).contiguous()
-    B, H, N, Dq = q1.shape
-    out = torch.empty((B, H, N, state.shape[3]), dtype=q1.dtype, device=q1.device)
-    d = _triple_desc(q1, q2, out, out)
-    with _on_device(q1.device):
-        rc = lib.flare_triple_out_fwd(C.byref(d), _ptr(q1), _ptr(q2), _ptr(state), None, _ptr(out),
-                                      C.c_void_p(_stream_ptr(q1.device)))
-    _lib.check(rc, "flare_triple_out_fwd")
-    return out
-
-
-def _triple_state(k1, k2, v):
-    """state [B,H,Dq,Dv,Dq] fp32 = (1/N) sum_n k1[n,i] v[n,j] k2[n,k]."""
-    return _triple_state_launch(k1, k2, v)
-
-
-def _triple_out(q1, q2, state, out_dtype=None):
-    """out [B,H,N,Dv] = sum_{i,k} q1[n,i] state[i,j,k] q2[n,k]."""
-    out = _triple_out_launch(q1, q2, state)
-    return out if out_dtype is None else out.to(out_dtype)
-
-
 class _TripleFn(torch.autograd.Function):
     """(STATE, O) = triple attention with the gradients of lra/models/triton/triple.py:124-135.  Every
     gradient is again a state or an output contraction, so for Dq == Dv the backward runs on the
-    same two HIP kernels with permuted states; otherwise it is the reference's einsum formulas."""
+    HIP kernels of the forward with permuted states (flare_triple_bwd); otherwise it is the reference's einsum formulas."""
 
     @staticmethod
     def forward(ctx, q1, q2, k1, k2, v):
+        ctx.set_materialize_grads(False)
+        q1, q2, k1, k2, v = (_rows_last_contig(t) for t in (q1, q2, k1, k2, v))
         state, out = _triple_forward(q1, q2, k1, k2, v, False, False)
         ctx.save_for_backward(q1, q2, k1, k2, v, state)
         return state, out
@@ -1318,17 +1269,20 @@ class _TripleFn(torch.autograd.Function):
         if dout is None:
             dout = torch.zeros_like(v)
         if q1.shape[-1] == v.shape[-1]:
-            do = dout.to(dt)
-            dq1 = _triple_out(do, q2, state.permute(0, 1, 3, 2, 4))        # sum_{j,k} dO[n,j] S[i,j,k] q2[n,k]
-            dq2 = _triple_out(q1, do, state.permute(0, 1, 2, 4, 3))        # sum_{i,j} q1[n,i] S[i,j,k] dO[n,j]
-            ds = _triple_state(q1, q2, do) * float(N)                      # sum_n q1[n,i] dO[n,j] q2[n,k]
+            lib = _lib.load()
+            do = _rows_last_contig(dout.to(dt))
+            grads = [torch.empty(t.shape, dtype=dt, device=t.device) for t in (q1, q2, k1, k2, v)]
             if dstate is not None:
-                ds = ds + dstate.float()
-            ds = ds / N
-            dk1 = _triple_out(v, k2, ds.permute(0, 1, 3, 2, 4))
-            dk2 = _triple_out(k1, v, ds.permute(0, 1, 2, 4, 3))
-            dv = _triple_out(k1, k2, ds)
-            return dq1, dq2, dk1, dk2, dv
+                dstate = dstate.to(torch.float32).contiguous()
+            d = _triple_desc(q1, q2, k1, k2, v, do)
+            need = C.c_size_t(0)
+            _lib.check(lib.flare_triple_bwd_workspace_bytes(C.byref(d), C.byref(need)), "flare_triple_bwd_workspace_bytes")
+            ws = torch.empty(int(need.value), dtype=torch.uint8, device=q1.device)
+            with _on_device(q1.device):
+                rc = lib.flare_triple_bwd(C.byref(d), _ptr(q1), _ptr(q2), _ptr(k1), _ptr(k2), _ptr(v), _ptr(state), _ptr(dstate),
+                                          _ptr(do), *(_ptr(g) for g in grads), _ptr(ws), ws.numel(), C.c_void_p(_stream_ptr(q1.device)))
+            _lib.check(rc, "flare_triple_bwd")
+            return tuple(grads)
         f = lambda t: t.float()
         do = f(dout)
         dq1 = torch.einsum("bhnj,bhijk,bhnk->bhni", do, state, f(q2))

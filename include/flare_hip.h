@@ -430,6 +430,15 @@ int flare_triple_fwd(const FlareTripleDesc* desc, const void* q1, const void* q2
                      const void* k1, const void* k2, const void* v, float* state, void* out,
                      void* workspace, size_t workspace_bytes, void* stream);
 
+int flare_triple_bwd_workspace_bytes(const FlareTripleDesc* desc, size_t* bytes);
+
+/* Gradients of flare_triple_fwd without feature map and normaliser (lra/models/triton/triple.py:124-135), Dq == Dv: every one
+ * is a state or an output contraction again.  state: the forward's (fp32 [B,H,D,D,D]); dstate: the gradient of it, or NULL;
+ * dout: [B,H,N,D] with desc's o_stride; dq1, dq2, dk1, dk2, dv: [B,H,N,D] contiguous. */
+int flare_triple_bwd(const FlareTripleDesc* desc, const void* q1, const void* q2, const void* k1, const void* k2,
+                     const void* v, const float* state, const float* dstate, const void* dout, void* dq1, void* dq2,
+                     void* dk1, void* dk2, void* dv, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

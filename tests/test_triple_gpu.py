@@ -206,3 +206,35 @@ def test_16bit_kernels_with_one_or_two_tokens_against_the_conditioning_bound(dev
         sub = (2.0 ** -24 * v.abs().mean(2))[:, :, None, :, None] if dtype == torch.float16 else 0.0
         excess = (st.double().cpu() - sr).abs() - 2 * eps * mag_state - sub
         assert float(excess.max()) <= 0.0, float(excess.max())
+
+
+@pytest.mark.parametrize("N", [1, 15, 127, 128, 129, 513, 3000])
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -7), (torch.float16, 2.0 ** -10)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_head_dim_32_forward_and_backward(dev, N, dtype, tol, strided):
+    """The 32 x 32 x 32 kernels at the edges of their tiles (128 tokens staged, 64 per wave pass): state, output (with and
+    without the normaliser and the in-kernel map), and the five gradients incl. one that flows into the state.  Positive
+    features and values, so that no sum cancels and each result carries at most the rounding of its operands, of the
+    product k1 k2 and of the result (three half-ulps: 2^-9 bf16, 2^-12 f16 each); gradients see one more."""
+    B, H, D = 2, 2, 32
+    g = torch.Generator().manual_seed(N)
+    def mk():
+        t = (torch.rand(B, N, H, D, generator=g) + 0.25).to(dtype)
+        return t.permute(0, 2, 1, 3) if strided else t.permute(0, 2, 1, 3).contiguous()
+    ins, go = [mk() for _ in range(5)], mk()
+    gs = torch.rand(B, H, D, D, D, generator=g)
+    onto = lambda t: t.transpose(1, 2).to(dev).transpose(1, 2) if strided else t.to(dev)
+    for fm, norm in ((None, False), ("elu", True)):
+        st, out = F.triple_attention(*[onto(t) for t in ins], feature_map=fm, normalize=norm)
+        sr, orf = O.triple_einsum(*[t.float() for t in ins], feature_map=fm == "elu", normalize=norm, dtype=torch.float64)
+        assert O.rel_l2(st, sr) <= tol and O.rel_l2(out, orf) <= tol
+    dins = [onto(t).requires_grad_(True) for t in ins]
+    st, out = F.TripleAttentionFunction.apply(*dins)
+    rins = [t.double().requires_grad_(True) for t in ins]
+    sr, orf = O.triple_einsum(*rins, dtype=torch.float64)
+    for with_state in (False, True):
+        roots = ((out, onto(go), orf, go.double()),) + (((st, gs.to(dev), sr, gs.double()),) if with_state else ())
+        got = torch.autograd.grad([r[0] for r in roots], dins, [r[1] for r in roots], retain_graph=True)
+        want = torch.autograd.grad([r[2] for r in roots], rins, [r[3] for r in roots], retain_graph=True)
+        for a, b in zip(got, want):
+            assert O.rel_l2(a, b) <= 1.5 * tol
