@@ -249,28 +249,60 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
 }
 
 // dz = sum of the split partials, Delta_m = <dz_m, z_m>  (MODE 0);  dq = scale * sum of the split partials  (MODE 1).
-// One thread per (b, h, m); fixed order.
-template <int MODE>
-__global__ __launch_bounds__(256) void bwd_f32_merge_kernel(MixerBwdArgs a)
+// Thread = four channels of a row; W waves share the partials (wave w takes w, w + W, ...) and meet in LDS in wave order (bit-
+// stable); W = 8 above eight partials, else 1, for the reason given at the forward's merge.
+template <int MODE, int W>
+__global__ __launch_bounds__(512) void bwd_f32_merge_kernel(MixerBwdArgs a)
 {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;      // (b*H + h)*M + m
-    if (r >= (int64_t)a.B * a.H * a.M) return;
+    constexpr int U = 8;
+    __shared__ f32x4 red[8][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave % W;
+    const int dq4 = a.D / 4;                                               // threads per row: 4, 8 or 16
+    const int64_t t = ((int64_t)blockIdx.x * (8 / W) + wave / W) * 64 + lane, rows = (int64_t)a.B * a.H * a.M;
+    const bool live = t < rows * dq4;
+    const int64_t r = live ? t / dq4 : rows - 1;                           // (b*H + h)*M + m
+    const int d = (int)(t % dq4) * 4;
     const int64_t bh = r / a.M;
     const int m = (int)(r % a.M);
     const int P = MODE == 0 ? a.n_splits0 : a.n_splits;
-    float delta = 0.f;
-    for (int d = 0; d < a.D; d += 4) {
-        f32x4 s = zero4f();
-        for (int p = 0; p < P; ++p) s += *reinterpret_cast<const f32x4*>(a.part + ((bh * P + p) * a.M + m) * a.D + d);
-        if (MODE == 0) {
-            *reinterpret_cast<f32x4*>(a.dz + r * a.D + d) = s;
-            const f32x4 zz = *reinterpret_cast<const f32x4*>(a.z + r * a.D + d);
-            delta += s[0] * zz[0] + s[1] * zz[1] + s[2] * zz[2] + s[3] * zz[3];
-        } else {
-            *reinterpret_cast<f32x4*>(a.dq + r * a.D + d) = s * a.scale;
+    const float* p0 = a.part + (bh * P * a.M + m) * a.D + d;
+    const int64_t sp = (int64_t)a.M * a.D;
+    f32x4 s = zero4f();
+    for (int p = w; p < P; p += W * U) {
+        f32x4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u] = zero4f();
+            if (p + W * u < P) v[u] = *reinterpret_cast<const f32x4*>(p0 + (p + W * u) * sp);
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
     }
-    if (MODE == 0) a.delta_lat[r] = delta;
+    if constexpr (W > 1) {
+        red[wave][lane] = s;
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (int i = 1; i < W; ++i) s += red[wave + i][lane];
+    }
+    if (MODE == 0) {
+        const f32x4 zz = *reinterpret_cast<const f32x4*>(a.z + r * a.D + d);
+        float delta = s[0] * zz[0] + s[1] * zz[1] + s[2] * zz[2] + s[3] * zz[3];
+        for (int o = 1; o < dq4; o <<= 1) delta += __shfl_xor(delta, o);   // the threads of a row are neighbours
+        if (live) {
+            *reinterpret_cast<f32x4*>(a.dz + r * a.D + d) = s;
+            if (d == 0) a.delta_lat[r] = delta;
+        }
+    } else if (live) {
+        *reinterpret_cast<f32x4*>(a.dq + r * a.D + d) = s * a.scale;
+    }
+}
+
+template <int MODE>
+void merge_launch_f32(const MixerBwdArgs& a, int64_t items, hipStream_t st)
+{
+    if ((MODE == 0 ? a.n_splits0 : a.n_splits) > 8) hipLaunchKernelGGL((bwd_f32_merge_kernel<MODE, 8>), dim3((unsigned)((items + 63) / 64)), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((bwd_f32_merge_kernel<MODE, 1>), dim3((unsigned)((items + 511) / 512)), dim3(512), 0, st, a);
 }
 
 // Delta_m = <dz_m, z_m> of a dz that the caller hands in (gather half): one thread per (b, h, m).
@@ -456,7 +488,7 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
     } else {
         if (a.drop_thr != 0) hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 0, 0, true>), dim3(a.n_splits0 * mblocks, a.H, a.B), dim3(256), 0, st, a);
         else                 hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 0, 0, false>), dim3(a.n_splits0 * mblocks, a.H, a.B), dim3(256), 0, st, a);
-        hipLaunchKernelGGL(bwd_f32_merge_kernel<0>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, a);
+        merge_launch_f32<0>(a, rows * (D / 4), st);
     }
     // token pass, in chunks of latents when their operands do not fit the LDS
     const int mc = tok_chunk(a.M, D);
@@ -476,7 +508,7 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
     }
     if (a.drop_thr != 0) hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 1, HALF, true>), dim3(a.n_splits * mblocks1, a.H, a.B), dim3(256), 0, st, a);
     else                 hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 1, HALF, false>), dim3(a.n_splits * mblocks1, a.H, a.B), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(bwd_f32_merge_kernel<1>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, a);
+    merge_launch_f32<1>(a, rows * (D / 4), st);
     return hipGetLastError();
 }
 

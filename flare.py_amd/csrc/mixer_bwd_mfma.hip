@@ -508,12 +508,16 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
 }
 
 // MODE 0: dz = sum of partials, Delta_m = <dz_m, z_m>;  MODE 1: dq = scale * sum of partials.
-// One thread per (b,h,m) and four channels; the partials are summed in split order (bit-stable).
-template <int MODE>
-__global__ __launch_bounds__(256) void bwd_merge_kernel(MixerBwdArgs a)
+// Thread = four channels of a row; W waves share the partials (wave w takes w, w + W, ...) and meet in LDS in wave order (bit-
+// stable); W = 8 above eight partials, else 1, for the reason given at the forward's merge.
+template <int MODE, int W>
+__global__ __launch_bounds__(512) void bwd_merge_kernel(MixerBwdArgs a)
 {
+    constexpr int U = 8;
+    __shared__ f32x4 red[8][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave % W;
     const int dq4 = a.D / 4;                                       // threads per row: 4, 8 or 16
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t t = ((int64_t)blockIdx.x * (8 / W) + wave / W) * 64 + lane;
     const int64_t rows = (int64_t)a.B * a.H * a.M;
     const bool live = t < rows * dq4;
     const int64_t r = live ? t / dq4 : rows - 1;                   // (b*H + h)*M + m
@@ -523,8 +527,23 @@ __global__ __launch_bounds__(256) void bwd_merge_kernel(MixerBwdArgs a)
     const float* p0 = a.part + (bh * a.n_splits * a.M + m) * a.D + d;
     const int64_t sp = (int64_t)a.M * a.D;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8      // eight loads in flight; the additions keep the split order
-    for (int p = 0; p < a.n_splits; ++p) s += *reinterpret_cast<const f32x4*>(p0 + p * sp);
+    for (int p = w; p < a.n_splits; p += W * U) {
+        f32x4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (p + W * u < a.n_splits) v[u] = *reinterpret_cast<const f32x4*>(p0 + (p + W * u) * sp);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
+    }
+    if constexpr (W > 1) {
+        red[wave][lane] = s;
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (int i = 1; i < W; ++i) s += red[wave + i][lane];
+    }
     if (MODE == 0) {
         const f32x4 zz = *reinterpret_cast<const f32x4*>(a.z + r * a.D + d);
         float delta = s[0] * zz[0] + s[1] * zz[1] + s[2] * zz[2] + s[3] * zz[3];
@@ -537,6 +556,13 @@ __global__ __launch_bounds__(256) void bwd_merge_kernel(MixerBwdArgs a)
     } else if (live) {
         *reinterpret_cast<f32x4*>(a.dq + r * a.D + d) = s * a.scale;
     }
+}
+
+template <int MODE>
+void merge_launch(const MixerBwdArgs& a, int64_t items, hipStream_t st)
+{
+    if (a.n_splits > 8) hipLaunchKernelGGL((bwd_merge_kernel<MODE, 8>), dim3((unsigned)((items + 63) / 64)), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((bwd_merge_kernel<MODE, 1>), dim3((unsigned)((items + 511) / 512)), dim3(512), 0, st, a);
 }
 
 // The halves of the mixer differentiated alone run the whole mixer's kernels with the other half's softmax weights
@@ -908,7 +934,7 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
     if (a.half != 1) {      // the gather half is handed dz
         e = dz32 ? launch_bwd_dz32(a0, st) : lat_launch<T, D, 0, DROPK>(a0, st);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(bwd_merge_kernel<0>, dim3((unsigned)((lat * (D / 4) + 255) / 256)), dim3(256), 0, st, a0);
+        merge_launch<0>(a0, lat * (D / 4), st);
     }
     // the token pass on the 32x32x16 product takes the (b,h) of the unshifted one-exponential form; the kernel below
     // then only works on the others (normally none: its workgroups return at once)
@@ -945,7 +971,7 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
     }
     e = dq32 ? launch_bwd_dq32(a, st) : lat_launch<T, D, 1, DROPK>(a, st);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bwd_merge_kernel<1>, dim3((unsigned)((lat * (D / 4) + 255) / 256)), dim3(256), 0, st, a);
+    merge_launch<1>(a, lat * (D / 4), st);
     return hipGetLastError();
 }
 

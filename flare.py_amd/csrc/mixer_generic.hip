@@ -92,59 +92,81 @@ __global__ __launch_bounds__(kGatherThreads) void gather_generic_kernel(MixerArg
     }
 }
 
-// Fixed-order merge of the split-N partials: bit-stable for a given n_parts.
-// One thread per (b,h,m,d); partials are visited in batches of 8 so that the loads of a batch
-// are all in flight before the first is consumed.
-__global__ __launch_bounds__(256) void gather_merge_kernel(MixerArgs a)
+// z and lse from the split-N partials: thread = V consecutive channels of one row; W waves of a workgroup share the partials
+// of the same 64 items (wave w takes w, w + W, ...), each with its own running maximum, and meet in LDS in wave order, so a
+// split count gives the same bits every time.  Few rows come with many partials (the splits fill the device), and then
+// the chain of loads over them is what it costs: W = 8 (B=1, H=4, N=500,001, M=256, D=16 f16 forward + backward, three merges: 683 -> 653 us).  Up to eight partials one wave has all its loads in flight at once and
+// more waves would only come and go: W = 1 (B=4, H=8, M=256, D=64, 8 partials: 209 us for the whole mixer, 221 with W = 8).
+template <int V, int W>
+__global__ __launch_bounds__(512) void gather_merge_kernel(MixerArgs a)
 {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = (int64_t)a.B * a.H * a.M * a.D;
-    if (idx >= total) return;
-    const int d = idx % a.D;
-    const int64_t r = idx / a.D;          // (b*H + h)*M + m
-    const int m = r % a.M;
-    const int64_t bh = r / a.M;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    constexpr int U = 8;
+    __shared__ float sm[8][64], sl[8][64];
+    __shared__ vec sacc[8][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave % W;
+    const int dv = a.D / V;                                        // items of a row
+    const int64_t total = (int64_t)a.B * a.H * a.M * dv;
+    const int64_t idx = ((int64_t)blockIdx.x * (8 / W) + wave / W) * 64 + lane;
+    const bool live = idx < total;
+    const int64_t r = (live ? idx : total - 1) / dv;               // (b*H + h)*M + m
+    const int d = (int)((live ? idx : total - 1) % dv) * V;
+    const int64_t m = r % a.M, bh = r / a.M;
     const int P = a.n_parts;
     const float* __restrict__ pm = a.part_m + bh * P * a.M + m;
     const float* __restrict__ pl = a.part_l + bh * P * a.M + m;
     const float* __restrict__ pa = a.part_acc + (bh * P * a.M + m) * a.D + d;
-    const int64_t sm = a.M, sa = (int64_t)a.M * a.D;
-    constexpr int U = 8;
+    const int64_t rs = a.M, as = (int64_t)a.M * a.D;
 
-    float mx = kNegBig;
-    int p = 0;
-    for (; p + U <= P; p += U) {
-        float t[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) t[u] = pm[(p + u) * sm];
-#pragma unroll
-        for (int u = 0; u < U; ++u) mx = fmaxf(mx, t[u]);
-    }
-    for (; p < P; ++p) mx = fmaxf(mx, pm[p * sm]);
-
-    float l = 0.f, acc = 0.f;
-    p = 0;
-    for (; p + U <= P; p += U) {
-        float tm[U], tl[U], ta[U];
+    float mx = kNegBig, l = 0.f;
+    vec acc = {};
+    for (int p0 = w; p0 < P; p0 += W * U) {
+        float tm[U], tl[U];
+        vec ta[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            tm[u] = pm[(p + u) * sm];
-            tl[u] = pl[(p + u) * sm];
-            ta[u] = pa[(p + u) * sa];
+            const int p = p0 + W * u;
+            const int pc = p < P ? p : p0;
+            tm[u] = p < P ? pm[pc * rs] : kNegBig;
+            tl[u] = p < P ? pl[pc * rs] : 0.f;
+            ta[u] = *reinterpret_cast<const vec*>(pa + pc * as);
         }
+        float nm = mx;
+#pragma unroll
+        for (int u = 0; u < U; ++u) nm = fmaxf(nm, tm[u]);
+        const float sc = fast_exp2(mx - nm);
+        l *= sc;
+        acc *= sc;
+        mx = nm;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const float w = fast_exp2(tm[u] - mx);
-            l = fmaf(tl[u], w, l);
-            acc = fmaf(ta[u], w, acc);
+            if (p0 + W * u >= P) break;
+            const float wt = fast_exp2(tm[u] - mx);
+            l = fmaf(tl[u], wt, l);
+            acc += ta[u] * wt;
         }
     }
-    for (; p < P; ++p) {
-        const float w = fast_exp2(pm[p * sm] - mx);
-        l = fmaf(pl[p * sm], w, l);
-        acc = fmaf(pa[p * sa], w, acc);
+    if constexpr (W > 1) {
+        sm[wave][lane] = mx;
+        sl[wave][lane] = l;
+        sacc[wave][lane] = acc;
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (int i = 0; i < W; ++i) mx = fmaxf(mx, sm[wave + i][lane]);
+        l = 0.f;
+        acc = vec{};
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            const float wt = fast_exp2(sm[wave + i][lane] - mx);
+            l = fmaf(sl[wave + i][lane], wt, l);
+            acc += sacc[wave + i][lane] * wt;
+        }
     }
-    a.z[idx] = l > 0.f ? acc / l : 0.f;
+    if (!live) return;
+    vec z = {};
+    if (l > 0.f) z = acc / l;
+    *reinterpret_cast<vec*>(a.z + r * a.D + d) = z;
     if (a.lse && d == 0) a.lse[r] = l > 0.f ? (mx + __log2f(l)) * kLn2 : -INFINITY;
 }
 
@@ -257,9 +279,14 @@ hipError_t launch_gather_generic(const MixerArgs& a, int dtype, hipStream_t st)
 
 hipError_t launch_gather_merge(const MixerArgs& a, hipStream_t st)
 {
-    const int64_t total = (int64_t)a.B * a.H * a.M * a.D;
-    dim3 grid((unsigned)((total + 255) / 256));
-    hipLaunchKernelGGL(gather_merge_kernel, grid, dim3(256), 0, st, a);
+    // four channels per thread where rows and arrays keep them 16-byte aligned (the generic kernels take any D and M)
+    const bool quad = a.D % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.part_acc) | reinterpret_cast<uintptr_t>(a.z)) & 15u) == 0;
+    const int64_t items = (int64_t)a.B * a.H * a.M * (quad ? a.D / 4 : a.D);
+    const auto launch = [&](auto kern, int w) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((items + 512 / w - 1) / (512 / w))), dim3(512), 0, st, a);
+    };
+    if (a.n_parts > 8) quad ? launch(gather_merge_kernel<4, 8>, 8) : launch(gather_merge_kernel<1, 8>, 8);
+    else               quad ? launch(gather_merge_kernel<4, 1>, 1) : launch(gather_merge_kernel<1, 1>, 1);
     return hipGetLastError();
 }
 

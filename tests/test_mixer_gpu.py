@@ -689,3 +689,12 @@ def test_fp32_scatter_takes_a_misaligned_z(dev):
     zo.copy_(z)
     assert zo.data_ptr() % 16 != 0
     assert O.rel_l2(F.flare_scatter(qd, kd, zo), F.flare_scatter(qd, kd, z)) <= 1e-6
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 16), (torch.float32, 7), (torch.bfloat16, 16), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("n_splits", [1, 8, 9, 64, 65])
+def test_merge_over_split_counts(dev, dtype, D, n_splits):
+    # eight waves share the partials, eight loads each: counts around one wave's, one round's and one more; a head dim that is
+    # no multiple of four takes the one-channel instance
+    q, k, v = make(2, 3, 65 * 256, 40 if dtype == torch.float32 else 64, D, dtype, seed=n_splits, kstd=3.0)
+    check(dev, q, k, v, n_splits=n_splits)
