@@ -63,6 +63,17 @@ class FlareMlpDesc(C.Structure):
     ]
 
 
+MLP_PACK_MAX = 16
+
+
+class FlareMlpPackDesc(C.Structure):
+    _fields_ = [
+        ("L", C.c_int32), ("C", C.c_int32), ("w_dtype", C.c_int32),
+        ("src", C.c_void_p * MLP_PACK_MAX), ("bsrc", C.c_void_p * MLP_PACK_MAX), ("ld", C.c_int64 * MLP_PACK_MAX),
+        ("rows", C.c_int32 * MLP_PACK_MAX), ("src_dtype", C.c_int32 * MLP_PACK_MAX), ("b_dtype", C.c_int32 * MLP_PACK_MAX),
+    ]
+
+
 class FlareTripleDesc(C.Structure):
     _fields_ = [
         ("B", C.c_int32), ("H", C.c_int32), ("N", C.c_int32), ("Dq", C.c_int32), ("Dv", C.c_int32),
@@ -107,6 +118,7 @@ SYMBOLS = {
     "flare_mlp_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_wgrad_partials": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(C.c_int32)]),
     "flare_mlp_wgrad": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P]),
+    "flare_mlp_pack": (C.c_int, [C.POINTER(FlareMlpPackDesc), _P, _P, _P, _P, _P]),
     "flare_mlp_expand_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_triple_workspace_bytes": (C.c_int, [C.POINTER(FlareTripleDesc), C.POINTER(_SZ)]),
     "flare_triple_state_fwd": (C.c_int, [C.POINTER(FlareTripleDesc), _P, _P, _P, _P, _P, _P, _SZ, _P]),

@@ -1226,6 +1226,34 @@ int flare_mlp_wgrad(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_str
     return hip_status(flare::launch_mlp_wgrad(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp weight-gradient launch");
 }
 
+static_assert(FLARE_MLP_PACK_MAX == flare::kMlpPackMax, "header and kernel argument block disagree");
+
+int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img, float* bias, void* stream)
+{
+    if (!d) return fail(FLARE_EINVAL, "descriptor is NULL");
+    if (d->L < 1 || d->L > FLARE_MLP_PACK_MAX) return fail(FLARE_EINVAL, "1 <= L <= %d required (got %d)", FLARE_MLP_PACK_MAX, d->L);
+    if (d->w_dtype != FLARE_DT_BF16 && d->w_dtype != FLARE_DT_F16) return fail(FLARE_EINVAL, "w_dtype must be bf16 or f16");
+    if (!flare::mlp_mfma_supported(d->w_dtype, d->C)) return fail(FLARE_EUNSUPPORTED, "C=%d: only 32, 64 and 128 are supported", d->C);
+    if (!w || !bias) return fail(FLARE_EINVAL, "w and bias must not be NULL");
+    if (!w_img != !wt_img) return fail(FLARE_EINVAL, "w_img and wt_img come together");
+    const void* outs[] = {w, w_img, wt_img, bias};
+    for (const void* p : outs)
+        if (p && !aligned16(p)) return fail(FLARE_EINVAL, "every output must be 16-byte aligned");
+    flare::MlpPackArgs a;
+    memset(&a, 0, sizeof(a));
+    for (int l = 0; l < d->L; ++l) {
+        if (!d->src[l]) return fail(FLARE_EINVAL, "src[%d] is NULL", l);
+        if (d->rows[l] < 1 || d->rows[l] > d->C || d->ld[l] < d->C) return fail(FLARE_EINVAL, "tile %d: 1 <= rows <= C and ld >= C required", l);
+        if (d->src_dtype[l] < FLARE_DT_F32 || d->src_dtype[l] > FLARE_DT_F16 || d->b_dtype[l] < FLARE_DT_F32 || d->b_dtype[l] > FLARE_DT_F16)
+            return fail(FLARE_EINVAL, "tile %d: unknown dtype", l);
+        a.src[l] = d->src[l]; a.bsrc[l] = d->bsrc[l]; a.ld[l] = d->ld[l]; a.rows[l] = d->rows[l];
+        a.src_dtype[l] = (int8_t)d->src_dtype[l]; a.b_dtype[l] = (int8_t)d->b_dtype[l];
+    }
+    a.w = static_cast<uint16_t*>(w); a.w_img = static_cast<uint16_t*>(w_img); a.wt_img = static_cast<uint16_t*>(wt_img);
+    a.bias = bias; a.L = d->L; a.C = d->C;
+    return hip_status(flare::launch_mlp_pack(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp pack launch");
+}
+
 int flare_triple_workspace_bytes(const FlareTripleDesc* desc, size_t* bytes)
 {
     if (!bytes) return fail(FLARE_EINVAL, "bytes is NULL");

@@ -330,6 +330,19 @@ struct MlpWgradArgs {
     int64_t tokens_per_wg;                      // set by the launcher
 };
 
+// Arguments of the packing kernel (mlp_pack.hip): up to 16 tiles, each read where its parameter lies.
+constexpr int kMlpPackMax = 16;
+struct MlpPackArgs {
+    const void* src[kMlpPackMax];               // element (0, 0) of every [out][in] tile
+    const void* bsrc[kMlpPackMax];              // its bias, or null (zeros)
+    int64_t ld[kMlpPackMax];                    // elements from one row of the tile to the next
+    int rows[kMlpPackMax];                      // rows (and bias elements) that exist; the others are zeros
+    int8_t src_dtype[kMlpPackMax], b_dtype[kMlpPackMax];
+    uint16_t* w; uint16_t* w_img; uint16_t* wt_img;      // [L,C,C]; the images may both be null
+    float* bias;                                // [L,C]
+    int L, C;
+};
+
 // Workgroups of the backward's dq pass (bwd_lat_kernel, MODE 1) that fit a compute unit: its instances with 16 or
 // 32 latents per wave at head dim 16, and with 16 at head dim 32, need few enough registers for three or four (measured:
 // 143 -> 119 us at M = 128, D = 16; 86 -> 74 us at M = 64, D = 16; 133 -> 106 us at M = 64, D = 32); squeezing the
@@ -395,6 +408,7 @@ hipError_t launch_mlp_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 int64_t    mlp_wgrad_tokens_per_wg(int64_t T, int C, int L);
 int        mlp_wgrad_partials(int64_t T, int C, int L);
 hipError_t launch_mlp_wgrad(const MlpWgradArgs& a, int w_dtype, hipStream_t st);
+hipError_t launch_mlp_pack(const MlpPackArgs& a, int w_dtype, hipStream_t st);
 
 int        causal_linear_tile();
 hipError_t launch_causal_linear(const CausalLinearArgs& a, int dtype, hipStream_t st);

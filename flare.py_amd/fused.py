@@ -34,7 +34,7 @@ from torch import nn
 from torch.autograd.function import once_differentiable
 
 from . import _lib
-from .functional import _autocast_dtype, _dtype_code, _on_device, _ptr, _stream_ptr
+from .functional import _DTYPES, _autocast_dtype, _dtype_code, _on_device, _ptr, _stream_ptr
 
 _SUPPORTED_C = (32, 64, 128)
 _ACTS = {"gelu": 0, "silu": 1}
@@ -244,12 +244,60 @@ def _shape_ok(width, mod, grad):
     return True
 
 
+def _readable(*ts):
+    """The packing launch reads these parameters where they lie (a tensor subclass may keep its values elsewhere)."""
+    return all(t is None or (type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype in _DTYPES
+                             and t.stride(-1) == 1 and (t.dim() == 1 or t.stride(0) >= t.shape[1])) for t in ts)
+
+
+def _pack_launch(Cdim, cd, tiles, dev, images):
+    """One flare_mlp_pack launch.  tiles: (weight, element offset of the tile, row stride, rows, bias or None, element offset)
+    each; returns (w [L,C,C], b [L,C], image of w, image of its transposes), the images None unless asked for."""
+    lib = _lib.load()
+    L = len(tiles)
+    d = _lib.FlareMlpPackDesc()
+    d.L, d.C, d.w_dtype = L, Cdim, _DTYPES[cd]
+    for l, (w, off, ld, rows, b, boff) in enumerate(tiles):
+        d.src[l], d.ld[l], d.rows[l], d.src_dtype[l] = w.data_ptr() + off * w.element_size(), ld, rows, _DTYPES[w.dtype]
+        if b is not None:
+            d.bsrc[l], d.b_dtype[l] = b.data_ptr() + boff * b.element_size(), _DTYPES[b.dtype]
+    ws = torch.empty(3 if images else 1, L, Cdim, Cdim, dtype=cd, device=dev)
+    bias = torch.empty(L, Cdim, dtype=torch.float32, device=dev)
+    with _on_device(dev):
+        rc = lib.flare_mlp_pack(C.byref(d), _ptr(ws), _ptr(ws[1]) if images else None, _ptr(ws[2]) if images else None, _ptr(bias),
+                                C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_pack")
+    return ws[0], bias, (ws[1] if images else None), (ws[2] if images else None)
+
+
+def _chain_tiles(layers):
+    """Tiles of a stack of Linears at most C x C, or None where the launch cannot read them."""
+    if not _readable(*(t for l in layers for t in (l.weight, l.bias))):
+        return None
+    return [(l.weight, 0, l.weight.stride(0), l.out_features, l.bias, 0) for l in layers]
+
+
+def _expand_tiles(f1, f2, E, Cdim):
+    if not _readable(f1.weight, f1.bias, f2.weight, f2.bias):
+        return None
+    w1, w2, tiles = f1.weight, f2.weight, []
+    for j in range(E):
+        tiles.append((w1, j * Cdim * w1.stride(0), w1.stride(0), Cdim, f1.bias, j * Cdim))
+        tiles.append((w2, j * Cdim, w2.stride(0), Cdim, f2.bias if j == 0 else None, 0))
+    return tiles
+
+
 def _packed(mod, layers, cd):
     """[L,C,C] weights in the compute dtype and [L,C] fp32 biases, cached on the module."""
     key = (cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
     cache = getattr(mod, "_flare_packed", None)
     if cache is not None and cache[0] == key:
         return cache[1], cache[2]
+    tiles = _chain_tiles(layers)
+    if tiles is not None:
+        w, b, _, _ = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, False)
+        mod._flare_packed = (key, w, b)
+        return w, b
     w = torch.stack([l.weight.detach() for l in layers]).to(cd).contiguous()
     Cdim = w.shape[-1]
     b = torch.stack([l.bias.detach().float() if l.bias is not None else w.new_zeros(Cdim, dtype=torch.float32) for l in layers]).contiguous()
@@ -267,6 +315,11 @@ def _packed_expand(mod, E, cd):
     if cache is not None and cache[0] == key:
         return cache[1], cache[2]
     Cdim = f1.in_features
+    tiles = _expand_tiles(f1, f2, E, Cdim)
+    if tiles is not None:
+        w, b, _, _ = _pack_launch(Cdim, cd, tiles, f1.weight.device, False)
+        mod._flare_packed = (key, w, b)
+        return w, b
     w1 = f1.weight.detach().to(cd).view(E, Cdim, Cdim)                       # [j][hidden row in chunk][in]
     w2 = f2.weight.detach().to(cd).view(Cdim, E, Cdim).permute(1, 0, 2)      # [j][out][hidden col in chunk]
     w = torch.stack([w1, w2], dim=1).reshape(2 * E, Cdim, Cdim).contiguous()
@@ -288,12 +341,16 @@ def _packed_io(mod, layers, cd, Cdim, in_dim, out_dim):
         return cache[1:]
     dev = layers[0].weight.device
     tiles = layers[1:] if in_dim else layers
-    w = torch.zeros(len(tiles), Cdim, Cdim, dtype=cd, device=dev)
-    b = torch.zeros(len(tiles), Cdim, dtype=torch.float32, device=dev)
-    for i, l in enumerate(tiles):
-        w[i, :l.out_features] = l.weight.detach().to(cd)
-        if l.bias is not None:
-            b[i, :l.out_features] = l.bias.detach().float()
+    packed = _chain_tiles(tiles)
+    if packed is not None:
+        w, b, _, _ = _pack_launch(Cdim, cd, packed, dev, False)
+    else:
+        w = torch.zeros(len(tiles), Cdim, Cdim, dtype=cd, device=dev)
+        b = torch.zeros(len(tiles), Cdim, dtype=torch.float32, device=dev)
+        for i, l in enumerate(tiles):
+            w[i, :l.out_features] = l.weight.detach().to(cd)
+            if l.bias is not None:
+                b[i, :l.out_features] = l.bias.detach().float()
     w_in = b_in = None
     if in_dim:
         w_in = torch.zeros(Cdim, 4, dtype=torch.float32, device=dev)
@@ -394,7 +451,7 @@ def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None):
     return fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype), fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype)
 
 
-def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0):
+def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False):
     lib = _lib.load()
     info = _layers_of(mod)
     layers, act_mask, add_mask, act = info
@@ -409,10 +466,10 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     if E:
         if x_head or y_head:
             raise ValueError("head-padded rows are not available for the expanding two-layer MLP")
-        w, b = _packed_expand(mod, E, cd)
+        w, b = _packed_train_expand(mod, E, cd)[:2] if train else _packed_expand(mod, E, cd)
         act_mask, add_mask = 1, 0
     else:
-        w, b = _packed(mod, layers, cd)
+        w, b = _packed_train(mod, layers, cd)[:2] if train else _packed(mod, layers, cd)
     x2 = x.reshape(-1, x.shape[-1])
     if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
@@ -495,8 +552,12 @@ def _packed_train(mod, layers, cd):
     cache = mod.__dict__.get("_flare_packed_train")
     if cache is not None and cache[0] == key:
         return cache[1:]
-    w, b = _packed(mod, layers, cd)
-    w_img, wt_img = mlp_weight_images(w)
+    tiles = _chain_tiles(layers)
+    if tiles is not None:
+        w, b, w_img, wt_img = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, True)
+    else:
+        w, b = _packed(mod, layers, cd)
+        w_img, wt_img = mlp_weight_images(w)
     mod.__dict__["_flare_packed_train"] = (key, w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
@@ -509,8 +570,12 @@ def _packed_train_expand(mod, E, cd):
     cache = mod.__dict__.get("_flare_packed_train")
     if cache is not None and cache[0] == key:
         return cache[1:]
-    w, b = _packed_expand(mod, E, cd)
-    w_img, wt_img = mlp_weight_images(w)
+    tiles = _expand_tiles(f1, f2, E, f1.in_features)
+    if tiles is not None:
+        w, b, w_img, wt_img = _pack_launch(f1.in_features, cd, tiles, f1.weight.device, True)
+    else:
+        w, b = _packed_expand(mod, E, cd)
+        w_img, wt_img = mlp_weight_images(w)
     mod.__dict__["_flare_packed_train"] = (key, w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
@@ -547,7 +612,7 @@ class _FusedMlpFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, mod, cd, norm, out_dtype, x, res, gamma, beta, *wb):
         with torch.no_grad():
-            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype)
+            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype, train=True)
         ctx.mod, ctx.cd, ctx.norm = mod, cd, norm
         # res and x one tensor: dy is added to dx inside the kernel.  (Two tensors over the same memory are not
         # enough: one of them may be detached, and then its path carries no gradient.)
@@ -647,8 +712,8 @@ class _FusedPairFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, mod_a, mod_b, cd, norm, out_dtype, x, gamma, beta, *wb):
         with torch.no_grad():
-            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype)
-            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype)
+            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, train=True)
+            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, train=True)
         ctx.mods, ctx.cd, ctx.norm = (mod_a, mod_b), cd, norm
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)

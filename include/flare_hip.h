@@ -399,6 +399,20 @@ int flare_mlp_bwd_partial_rows(const FlareMlpDesc* desc, int32_t* rows);
 int flare_mlp_wgrad_partials(const FlareMlpDesc* desc, int32_t* parts);
 int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                     float* dw_part, float* db_part, float* dw, float* db, void* stream);
+/* The operands of the launches above from the parameters, in one launch.  Tile l is the [out][in] block at src[l] with ld[l] elements
+ * between its rows, of which rows[l] (1 .. C) exist and the others are taken as zeros; bsrc[l] (or NULL: zeros) holds rows[l] bias
+ * elements.  Each has its own element type.  Outputs: w [L,C,C] in w_dtype, bias [L,C] fp32, and, unless both are NULL, w_img and
+ * wt_img [L,C,C], the images flare_mlp_bwd reads.  1 <= L <= FLARE_MLP_PACK_MAX. */
+#define FLARE_MLP_PACK_MAX 16
+typedef struct {
+    int32_t L, C, w_dtype;
+    const void* src[FLARE_MLP_PACK_MAX];
+    const void* bsrc[FLARE_MLP_PACK_MAX];
+    int64_t ld[FLARE_MLP_PACK_MAX];
+    int32_t rows[FLARE_MLP_PACK_MAX], src_dtype[FLARE_MLP_PACK_MAX], b_dtype[FLARE_MLP_PACK_MAX];
+} FlareMlpPackDesc;
+int flare_mlp_pack(const FlareMlpPackDesc* desc, void* w, void* w_img, void* wt_img, float* bias, void* stream);
+
 /* Backward of flare_mlp_fwd with FLARE_MLP_EXPAND (y = res + W2 act(W1 norm(x) + b1) + b2, hidden width E C run as E
  * chunks; desc as for the forward: L = 2 E tiles, flags = FLARE_MLP_EXPAND; w_img, wt_img: LDS images of the 2 E tiles
  * and of their transposes, bias [2E,C] as for the forward).  Outputs as flare_mlp_bwd, with the rows for the weight

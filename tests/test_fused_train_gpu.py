@@ -459,3 +459,40 @@ def test_block_with_16bit_parameters_trains_fused(dev, dtype):
     for (n, p), (_, q) in zip(blk.named_parameters(), ref.named_parameters()):
         assert p.grad is not None and p.grad.dtype == dtype, n
         assert rel(p.grad, q.grad) <= 8e-2, n
+
+
+@pytest.mark.parametrize("C", [32, 64, 128])
+@pytest.mark.parametrize("cd", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("pd", [torch.float32, torch.bfloat16, torch.float16])
+def test_packed_operands_are_the_stacked_parameters(dev, C, cd, pd):
+    """The packing launch against torch's own stack and cast, bit for bit: rows at a stride and off the 16-byte grid, a missing
+    bias, a narrow last layer, the expanding MLP's tiles, special values."""
+    from flare_py_amd import fused
+
+    g = torch.Generator().manual_seed(C)
+    layers = [torch.nn.Linear(C, C, bias=i != 1) for i in range(3)] + [torch.nn.Linear(C, 3)]
+    for l in layers:
+        wide = torch.randn(l.out_features, C + 3, generator=g).mul_(100).to(dev, pd)
+        wide[0, 1], wide[0, 2], wide[1, 1] = float("inf"), 1e-7, -0.0
+        l.weight = torch.nn.Parameter(wide[:, 1:1 + C])
+        if l.bias is not None:
+            l.bias = torch.nn.Parameter(torch.randn(l.out_features + 1, generator=g).to(dev, pd)[1:])
+    w, b, img, img_t = fused._pack_launch(C, cd, fused._chain_tiles(layers), dev, True)
+    ref = torch.zeros(4, C, C, dtype=cd, device=dev)
+    refb = torch.zeros(4, C, device=dev)
+    for i, l in enumerate(layers):
+        ref[i, :l.out_features] = l.weight.detach().to(cd)
+        if l.bias is not None:
+            refb[i, :l.out_features] = l.bias.detach().float()
+    assert torch.equal(w, ref) and torch.equal(b, refb)
+    assert torch.equal(img.view_as(ref), fused.mlp_weight_image(ref).view_as(ref))
+    assert torch.equal(img_t.view_as(ref), fused.mlp_weight_image(ref.transpose(1, 2).contiguous()).view_as(ref))
+
+    E = 3
+    f1, f2 = torch.nn.Linear(C, E * C).to(dev, pd), torch.nn.Linear(E * C, C).to(dev, pd)
+    w, b, _, _ = fused._pack_launch(C, cd, fused._expand_tiles(f1, f2, E, C), dev, False)
+    for j in range(E):
+        assert torch.equal(w[2 * j], f1.weight.detach()[j * C:(j + 1) * C].to(cd))
+        assert torch.equal(w[2 * j + 1], f2.weight.detach()[:, j * C:(j + 1) * C].to(cd))
+        assert torch.equal(b[2 * j], f1.bias.detach()[j * C:(j + 1) * C].float())
+        assert torch.equal(b[2 * j + 1], f2.bias.detach().float() if j == 0 else torch.zeros(C, device=dev))
