@@ -18,6 +18,7 @@ FLAG_FORCE_GENERIC = 1
 FLAG_MFMA16 = 2
 FLAG_GRAD_LIKE_KV = 8
 MLP_EXPAND = 1
+MLP_W_TILED = 2
 MLP_BWD_ADD_DY = 1           # bits of flare_mlp_bwd's add_dy argument
 MLP_BWD_ACCUMULATE = 2
 ABI_VERSION = 2
@@ -71,6 +72,7 @@ class FlareMlpPackDesc(C.Structure):
         ("L", C.c_int32), ("C", C.c_int32), ("w_dtype", C.c_int32),
         ("src", C.c_void_p * MLP_PACK_MAX), ("bsrc", C.c_void_p * MLP_PACK_MAX), ("ld", C.c_int64 * MLP_PACK_MAX),
         ("rows", C.c_int32 * MLP_PACK_MAX), ("src_dtype", C.c_int32 * MLP_PACK_MAX), ("b_dtype", C.c_int32 * MLP_PACK_MAX),
+        ("tiled", C.c_int32),
     ]
 
 
@@ -118,6 +120,9 @@ SYMBOLS = {
     "flare_mlp_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_wgrad_partials": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(C.c_int32)]),
     "flare_mlp_wgrad": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P]),
+    "flare_mlp_wgrad_norm": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, C.c_int32, _P, _P]),
+    "flare_mlp_few": (C.c_int, [C.POINTER(FlareMlpDesc)]),
+    "flare_mlp_few_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_pack": (C.c_int, [C.POINTER(FlareMlpPackDesc), _P, _P, _P, _P, _P]),
     "flare_mlp_expand_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_triple_workspace_bytes": (C.c_int, [C.POINTER(FlareTripleDesc), C.POINTER(_SZ)]),

@@ -1083,7 +1083,17 @@ static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const flo
     a.in_dim = in_dim; a.in_act = in_act ? 1 : 0; a.w_in = w_in; a.b_in = b_in; a.out_dim = out_dim;
     a.x_head = x_head; a.y_head = y_head;
     a.xs = d->x_stride; a.rs = d->res_stride; a.ys = d->y_stride;
+    if (d->flags & FLARE_MLP_W_TILED) {
+        if (in_dim || out_dim || !flare_mlp_few(d)) return fail(FLARE_EUNSUPPORTED, "tiled weights: only where flare_mlp_few says so");
+        return hip_status(flare::launch_mlp_few(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token launch");
+    }
     return hip_status(flare::launch_mlp_mfma(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp launch");
+}
+
+int flare_mlp_few(const FlareMlpDesc* d)
+{
+    return d && d->T >= 1 && !(d->flags & FLARE_MLP_EXPAND) && flare::mlp_mfma_supported(d->w_dtype, d->C) && flare::mlp_few_ok(d->T, d->C, d->L)
+               ? flare::mlp_few_bwd_rows(d->T) : 0;
 }
 
 int flare_mlp_fwd(const FlareMlpDesc* d, const void* x, const void* w, const float* bias, const float* gamma,
@@ -1132,9 +1142,9 @@ static int check_mlp_bwd_common(const FlareMlpDesc* d, const void* x, const void
     return FLARE_OK;
 }
 
-int flare_mlp_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
-                  const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
-                  void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream)
+static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
+                        const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
+                        void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream, bool few, const void* dy2)
 {
     int rc = check_mlp_bwd_common(d, x, dy, w_img, wt_img, bias, gamma, beta, dx, dn, stats, gb_part, gb);
     if (rc != FLARE_OK) return rc;
@@ -1146,7 +1156,7 @@ int flare_mlp_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const vo
     if (!aligned16(a_in) || !aligned16(g_out)) return fail(FLARE_EINVAL, "every buffer must be 16-byte aligned");
     flare::MlpBwdArgs a;
     memset(&a, 0, sizeof(a));
-    a.x = x; a.dy = dy; a.dx = dx;
+    a.x = x; a.dy = dy; a.dy2 = dy2; a.dx = dx;
     a.w = static_cast<const uint16_t*>(w_img); a.wt = static_cast<const uint16_t*>(wt_img);
     a.bias = bias; a.gamma = gamma; a.beta = beta;
     a.a_in = static_cast<uint16_t*>(a_in); a.g_out = static_cast<uint16_t*>(g_out);
@@ -1157,7 +1167,25 @@ int flare_mlp_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const vo
     if (add_dy & ~(FLARE_MLP_BWD_ADD_DY | FLARE_MLP_BWD_ACCUMULATE)) return fail(FLARE_EINVAL, "add_dy holds unknown bits (got %d)", add_dy);
     a.add_dy = add_dy;
     a.xs = d->x_stride; a.dys = d->y_stride; a.dxs = d->C;
+    if (few) return hip_status(flare::launch_mlp_few_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token backward launch");
     return hip_status(flare::launch_mlp_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp backward launch");
+}
+
+int flare_mlp_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
+                  const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
+                  void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream)
+{
+    return mlp_bwd_impl(d, x, dy, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, dn, stats, gb_part, gb, stream, false, nullptr);
+}
+
+int flare_mlp_few_bwd(const FlareMlpDesc* d, const void* x, const void* dy_a, const void* dy_b, const void* w_img, const void* wt_img,
+                      const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in, void* g_out,
+                      float* gb_part, void* stream)
+{
+    if (!flare_mlp_few(d)) return fail(FLARE_EUNSUPPORTED, "the few-token launch runs only where flare_mlp_few says so");
+    if (dy_b && !aligned16(dy_b)) return fail(FLARE_EINVAL, "dy_b must be 16-byte aligned");
+    // the shared checks ask for dn and stats, which this launch does without
+    return mlp_bwd_impl(d, x, dy_a, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, gb_part, gb_part, gb_part, nullptr, stream, true, dy_b);
 }
 
 int flare_mlp_expand_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
@@ -1208,6 +1236,12 @@ int flare_mlp_wgrad_partials(const FlareMlpDesc* d, int32_t* parts)
 int flare_mlp_wgrad(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                     float* dw_part, float* db_part, float* dw, float* db, void* stream)
 {
+    return flare_mlp_wgrad_norm(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, nullptr, 0, nullptr, stream);
+}
+
+int flare_mlp_wgrad_norm(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                         float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream)
+{
     int rc = check_wgrad_desc(d);
     if (rc != FLARE_OK) return rc;
     if (!a_in || !g_out || !dw_part) return fail(FLARE_EINVAL, "a_in, g_out and dw_part must not be NULL");
@@ -1222,6 +1256,9 @@ int flare_mlp_wgrad(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_str
     a.a_in = static_cast<const uint16_t*>(a_in); a.g_out = static_cast<const uint16_t*>(g_out);
     a.a_lstride = a_layer_stride; a.g_lstride = g_layer_stride;
     a.dw_part = dw_part; a.db_part = db_part; a.dw = dw; a.db = db;
+    if (gb && (!gb_part || gb_rows < 1 || !aligned16(gb_part) || !aligned16(gb)))
+        return fail(FLARE_EINVAL, "gb needs gb_part with gb_rows >= 1, both 16-byte aligned");
+    a.gb_part = gb ? gb_part : nullptr; a.gb_rows = gb_rows; a.gb = gb;
     a.T = d->T; a.C = d->C; a.L = d->L;
     return hip_status(flare::launch_mlp_wgrad(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp weight-gradient launch");
 }
@@ -1235,7 +1272,8 @@ int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img
     if (d->w_dtype != FLARE_DT_BF16 && d->w_dtype != FLARE_DT_F16) return fail(FLARE_EINVAL, "w_dtype must be bf16 or f16");
     if (!flare::mlp_mfma_supported(d->w_dtype, d->C)) return fail(FLARE_EUNSUPPORTED, "C=%d: only 32, 64 and 128 are supported", d->C);
     if (!w || !bias) return fail(FLARE_EINVAL, "w and bias must not be NULL");
-    if (!w_img != !wt_img) return fail(FLARE_EINVAL, "w_img and wt_img come together");
+    if (d->tiled ? w_img != nullptr : !w_img != !wt_img)
+        return fail(FLARE_EINVAL, "w_img and wt_img come together; tiled operands have no w_img");
     const void* outs[] = {w, w_img, wt_img, bias};
     for (const void* p : outs)
         if (p && !aligned16(p)) return fail(FLARE_EINVAL, "every output must be 16-byte aligned");
@@ -1250,7 +1288,7 @@ int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img
         a.src_dtype[l] = (int8_t)d->src_dtype[l]; a.b_dtype[l] = (int8_t)d->b_dtype[l];
     }
     a.w = static_cast<uint16_t*>(w); a.w_img = static_cast<uint16_t*>(w_img); a.wt_img = static_cast<uint16_t*>(wt_img);
-    a.bias = bias; a.L = d->L; a.C = d->C;
+    a.bias = bias; a.L = d->L; a.C = d->C; a.tiled = d->tiled ? 1 : 0;
     return hip_status(flare::launch_mlp_pack(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp pack launch");
 }
 

@@ -295,6 +295,7 @@ struct MlpArgs {
 // backward of the fused MLP chain (mlp_bwd_mfma.hip)
 struct MlpBwdArgs {
     const void* x; const void* dy; void* dx;    // [T,C] rows: the forward's input, the gradient of its output, the gradient of x
+    const void* dy2;                            // few-token launch only: gradient of the second chain's output (tiles L .. 2 L - 1), or null
     const uint16_t* w; const uint16_t* wt;      // [L,C,C] 16-bit weights [out][in] and their transposes [in][out]
     const float* bias;                          // [L,C] or null
     const float* gamma; const float* beta;      // [C] norm parameters (beta may be null)
@@ -325,6 +326,8 @@ struct MlpWgradArgs {
     float* dw_part;                             // [parts,L,C,C] out: partial dW_l[out][in] per token range
     float* db_part;                             // [parts,L,C] out or null: partial db_l
     float* dw; float* db;                       // [L,C,C], [L,C] out or null: the partials summed in index order
+    const float* gb_part; float* gb;            // or null: the norm's partial rows [gb_rows,2,C] of the backward, summed by the same launch
+    int gb_rows;
     int64_t T;
     int C, L;
     int64_t tokens_per_wg;                      // set by the launcher
@@ -341,6 +344,7 @@ struct MlpPackArgs {
     uint16_t* w; uint16_t* w_img; uint16_t* wt_img;      // [L,C,C]; the images may both be null
     float* bias;                                // [L,C]
     int L, C;
+    int tiled;                                  // 1: w and wt_img in the few-token kernels' operand order (wt_img may be null)
 };
 
 // Workgroups of the backward's dq pass (bwd_lat_kernel, MODE 1) that fit a compute unit: its instances with 16 or
@@ -408,6 +412,11 @@ hipError_t launch_mlp_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 int64_t    mlp_wgrad_tokens_per_wg(int64_t T, int C, int L);
 int        mlp_wgrad_partials(int64_t T, int C, int L);
 hipError_t launch_mlp_wgrad(const MlpWgradArgs& a, int w_dtype, hipStream_t st);
+// launches of few tokens (mlp_few_mfma.hip): chain and head-padded modes, one or two chains
+bool       mlp_few_ok(int64_t T, int C, int L);
+int        mlp_few_bwd_rows(int64_t T);
+hipError_t launch_mlp_few(const MlpArgs& a, int w_dtype, hipStream_t st);
+hipError_t launch_mlp_few_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_mlp_pack(const MlpPackArgs& a, int w_dtype, hipStream_t st);
 
 int        causal_linear_tile();

@@ -19,19 +19,24 @@ __device__ __forceinline__ float load_as_float(const void* p, int64_t i, int dt)
     return (float)static_cast<const _Float16*>(p)[i];
 }
 
-// thread = four consecutive 16-bit outputs of one array: blockIdx.z = 0 the tiles, 1 their images, 2 the transposes' images
+// thread = four consecutive 16-bit outputs of one array: blockIdx.z = 0 the tiles, 1 their images, 2 the transposes' images;
+// a.tiled: 0 the tiles, 1 the transposes, both with every matrix operand's 64 lanes x 16 bytes in one piece
 template <typename V>
 __global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPackArgs a)
 {
     typedef V vec4 __attribute__((ext_vector_type(4)));
     const int l = blockIdx.y, what = blockIdx.z;
     const int C = a.C;
-    V* out = reinterpret_cast<V*>(what == 0 ? a.w : what == 1 ? a.w_img : a.wt_img);
+    V* out = reinterpret_cast<V*>(what == 0 ? a.w : what == 1 && !a.tiled ? a.w_img : a.wt_img);
+    const bool transposed = what == (a.tiled ? 1 : 2);
     const int e = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
     if (out && e < C * C) {
-        const int row = e / C, rem = e % C;
+        int row = e / C, rem = e % C;
         int col = rem;
-        if (what > 0) {
+        if (a.tiled) {      // [C / 16 row blocks][C / 32 k-steps][4 lane groups][16 rows][8 columns]
+            row = e / (16 * C) * 16 + (e >> 3) % 16;
+            col = e % (16 * C) / 512 * 32 + (e >> 7) % 4 * 8 + (e & 7);
+        } else if (what > 0) {
             const int key = (row & 15) >> (C == 128 ? 0 : C == 64 ? 1 : 2);
             const int c = (rem >> 3) ^ key, half = (rem >> 2) & 1;
             col = 8 * (4 * (c >> 2) + 2 * half + ((c & 3) >> 1)) + 4 * (c & 1);
@@ -39,7 +44,7 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPackArgs a)
         vec4 v;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int r = what == 2 ? col + j : row, k = what == 2 ? row : col + j;      // [out][in] element of the tile
+            const int r = transposed ? col + j : row, k = transposed ? row : col + j;      // [out][in] element of the tile
             v[j] = r < a.rows[l] ? (V)load_as_float(a.src[l], (int64_t)r * a.ld[l] + k, a.src_dtype[l]) : (V)0.f;
         }
         *reinterpret_cast<vec4*>(out + (size_t)l * C * C + e) = v;
@@ -54,7 +59,7 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPackArgs a)
 
 hipError_t launch_mlp_pack(const MlpPackArgs& a, int w_dtype, hipStream_t st)
 {
-    const dim3 grid((unsigned)((a.C * a.C / 4 + 255) / 256), (unsigned)a.L, a.w_img ? 3 : 1);
+    const dim3 grid((unsigned)((a.C * a.C / 4 + 255) / 256), (unsigned)a.L, a.tiled ? (a.wt_img ? 2 : 1) : a.w_img ? 3 : 1);
     if (w_dtype == 1) hipLaunchKernelGGL(mlp_pack_kernel<__bf16>, grid, dim3(256), 0, st, a);
     else              hipLaunchKernelGGL(mlp_pack_kernel<_Float16>, grid, dim3(256), 0, st, a);
     return hipGetLastError();

@@ -196,28 +196,40 @@ __global__ __launch_bounds__(64 * WO * WI * WK) void mlp_wgrad_kernel(MlpWgradAr
     }
 }
 
-// out[i] = sum over p of part[p][i].  Thread (x, y) of a 64 x 4 workgroup: four outputs, the partials p = y, y + 4,
-// ... with four loads in flight; the four y meet in LDS.  The order of the additions is fixed.
-__global__ __launch_bounds__(256) void sum_parts_kernel(const float* part, int parts, int64_t n, float* out)
+// Up to three sums over partial results in one launch: out[i] = sum over p of part[p][i].  A workgroup owns 4 X outputs of one
+// job: thread (x, y) adds the partials p = y, y + Y, ... of four outputs with four loads in flight (X Y = 256), the Y meet in
+// LDS.  The order of the additions is fixed.  Wide jobs (the weights) take X = 64, narrow ones (biases, norm parameters, whose
+// partials are many) X = 16.  Every sum was a launch of its own before: three of the nine launches of a chain's backward.
+struct SumJob { const float* part; float* out; int64_t n; int parts, first, x; };     // first: its first workgroup
+struct SumJobs { SumJob j[3]; int n; };
+__global__ __launch_bounds__(256) void sum_parts_kernel(SumJobs jobs)
 {
-    __shared__ f32x4 red[4][64];
-    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-    const int64_t i = ((int64_t)blockIdx.x * 64 + x) * 4;
+    __shared__ f32x4 red[256];
+    int k = 0;
+    while (k + 1 < jobs.n && (int)blockIdx.x >= jobs.j[k + 1].first) ++k;
+    const SumJob job = jobs.j[k];
+    const int X = job.x, Y = 256 / X;
+    const int x = (int)threadIdx.x % X, y = (int)threadIdx.x / X;
+    const int64_t n = job.n, i = ((int64_t)((int)blockIdx.x - job.first) * X + x) * 4;
+    const float* part = job.part;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
     if (i < n) {
         int p = y;
-        for (; p + 12 < parts; p += 16) {
+        for (; p + 3 * Y < job.parts; p += 4 * Y) {
             const f32x4 v0 = *reinterpret_cast<const f32x4*>(part + (size_t)p * n + i);
-            const f32x4 v1 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + 4) * n + i);
-            const f32x4 v2 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + 8) * n + i);
-            const f32x4 v3 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + 12) * n + i);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + Y) * n + i);
+            const f32x4 v2 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + 2 * Y) * n + i);
+            const f32x4 v3 = *reinterpret_cast<const f32x4*>(part + (size_t)(p + 3 * Y) * n + i);
             s += (v0 + v1) + (v2 + v3);
         }
-        for (; p < parts; p += 4) s += *reinterpret_cast<const f32x4*>(part + (size_t)p * n + i);
+        for (; p < job.parts; p += Y) s += *reinterpret_cast<const f32x4*>(part + (size_t)p * n + i);
     }
-    red[y][x] = s;
+    red[threadIdx.x] = s;
     __syncthreads();
-    if (y == 0 && i < n) *reinterpret_cast<f32x4*>(out + i) = (red[0][x] + red[1][x]) + (red[2][x] + red[3][x]);
+    if (y == 0 && i < n) {
+        for (int q = 1; q < Y; ++q) s += red[q * X + x];
+        *reinterpret_cast<f32x4*>(job.out + i) = s;
+    }
 }
 
 template <int C> struct WgradShape;
@@ -253,14 +265,15 @@ int wgrad_wk(int C) { return C == 128 ? 1 : C == 64 ? 2 : 8; }
 
 }  // namespace
 
-// Tokens per workgroup: at least one workgroup per compute unit over all layers, between 1024 and 4096 tokens (more,
+// Tokens per workgroup: at least one workgroup per compute unit over all layers, between 256 and 4096 tokens (more,
 // smaller ranges only add partial results to write and sum: measured at 262,144 tokens x 5 layers), a multiple of the
-// kernel's token tile.
+// kernel's token tile.  The lower end is for small meshes, where a workgroup's walk over its tiles is all there is to wait for:
+// 4096 tokens x 5 layers took 17.9 us in ranges of 1024, 7.3 us in ranges of 256.
 int64_t mlp_wgrad_tokens_per_wg(int64_t T, int C, int L)
 {
     const int64_t kt = 32 * wgrad_wk(C);
     int64_t want = (T * L + (int64_t)device_cus() - 1) / (int64_t)device_cus();
-    want = std::min<int64_t>(std::max<int64_t>(want, 1024), 4096);
+    want = std::min<int64_t>(std::max<int64_t>(want, 256), 4096);
     return (want + kt - 1) / kt * kt;
 }
 
@@ -278,15 +291,18 @@ hipError_t launch_mlp_wgrad(const MlpWgradArgs& a0, int w_dtype, hipStream_t st)
     hipError_t e = w_dtype == 1 ? launch_t<bf16_t>(a, st) : launch_t<f16_t>(a, st);
     if (e != hipSuccess) return e;
     const int parts = mlp_wgrad_partials(a.T, a.C, a.L);
-    if (a.dw) {
-        const int64_t n = (int64_t)a.L * a.C * a.C;
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n / 4 + 63) / 64)), dim3(256), 0, st, a.dw_part, parts, n, a.dw);
-        e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    if (a.db && a.db_part) {
-        const int64_t n = (int64_t)a.L * a.C;
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n / 4 + 63) / 64)), dim3(256), 0, st, a.db_part, parts, n, a.db);
+    SumJobs jobs{};
+    int blocks = 0;
+    auto add = [&](const float* part, float* out, int64_t n, int np, int x) {
+        if (!part || !out) return;
+        jobs.j[jobs.n++] = SumJob{part, out, n, np, blocks, x};
+        blocks += (int)((n / 4 + x - 1) / x);
+    };
+    add(a.dw_part, a.dw, (int64_t)a.L * a.C * a.C, parts, 64);
+    add(a.db_part, a.db, (int64_t)a.L * a.C, parts, 16);
+    add(a.gb_part, a.gb, 2 * (int64_t)a.C, a.gb_rows, 16);
+    if (blocks > 0) {
+        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)blocks), dim3(256), 0, st, jobs);
         e = hipGetLastError();
     }
     return e;

@@ -120,6 +120,7 @@ def _io_dims(mod, layers):
 
 
 _BWD_MAX_LAYERS = {32: 8, 64: 8, 128: 5}      # the backward keeps every layer's slopes in registers
+_FEW_TOKENS = {32: 16384, 64: 16384, 128: 12288}
 
 
 class _SubChain:
@@ -250,9 +251,10 @@ def _readable(*ts):
                              and t.stride(-1) == 1 and (t.dim() == 1 or t.stride(0) >= t.shape[1])) for t in ts)
 
 
-def _pack_launch(Cdim, cd, tiles, dev, images):
+def _pack_launch(Cdim, cd, tiles, dev, images, tiled=False):
     """One flare_mlp_pack launch.  tiles: (weight, element offset of the tile, row stride, rows, bias or None, element offset)
-    each; returns (w [L,C,C], b [L,C], image of w, image of its transposes), the images None unless asked for."""
+    each; returns (w [L,C,C], b [L,C], image of w, image of its transposes), the images None unless asked for.  tiled: w and the
+    last result in the few-token kernels' operand order, no image of w."""
     lib = _lib.load()
     L = len(tiles)
     d = _lib.FlareMlpPackDesc()
@@ -261,13 +263,15 @@ def _pack_launch(Cdim, cd, tiles, dev, images):
         d.src[l], d.ld[l], d.rows[l], d.src_dtype[l] = w.data_ptr() + off * w.element_size(), ld, rows, _DTYPES[w.dtype]
         if b is not None:
             d.bsrc[l], d.b_dtype[l] = b.data_ptr() + boff * b.element_size(), _DTYPES[b.dtype]
-    ws = torch.empty(3 if images else 1, L, Cdim, Cdim, dtype=cd, device=dev)
+    d.tiled = int(tiled)
+    ws = torch.empty(1 if not images else 2 if tiled else 3, L, Cdim, Cdim, dtype=cd, device=dev)
     bias = torch.empty(L, Cdim, dtype=torch.float32, device=dev)
     with _on_device(dev):
-        rc = lib.flare_mlp_pack(C.byref(d), _ptr(ws), _ptr(ws[1]) if images else None, _ptr(ws[2]) if images else None, _ptr(bias),
-                                C.c_void_p(_stream_ptr(dev)))
+        img = ws[1] if images and not tiled else None
+        img_t = ws[-1] if images else None
+        rc = lib.flare_mlp_pack(C.byref(d), _ptr(ws), _ptr(img), _ptr(img_t), _ptr(bias), C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_pack")
-    return ws[0], bias, (ws[1] if images else None), (ws[2] if images else None)
+    return ws[0], bias, img, img_t
 
 
 def _chain_tiles(layers):
@@ -285,6 +289,27 @@ def _expand_tiles(f1, f2, E, Cdim):
         tiles.append((w1, j * Cdim * w1.stride(0), w1.stride(0), Cdim, f1.bias, j * Cdim))
         tiles.append((w2, j * Cdim, w2.stride(0), Cdim, f2.bias if j == 0 else None, 0))
     return tiles
+
+
+def _few(T, Cdim, L):
+    """Rows of the norm's partial sums the few-token backward writes for such a launch, 0 where the other kernels serve it:
+    what flare_mlp_few answers, without a call into the library (every fused call asks)."""
+    return (T + 15) // 16 if 0 < T <= _FEW_TOKENS[Cdim] and L <= _BWD_MAX_LAYERS[Cdim] else 0
+
+
+def _packed_few(mod, layers, cd, train):
+    """(tiled w, fp32 biases, tiled transposes or None) of a chain for the few-token launches, cached on the module; None where
+    the packing launch cannot read the parameters.  A pair passes the layers of both stacks and the first stack's module."""
+    key = (cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
+    cache = mod.__dict__.get("_flare_packed_few")
+    if cache is not None and cache[0] == key and (cache[3] is not None or not train):
+        return cache[1:]
+    tiles = _chain_tiles(layers)
+    if tiles is None:
+        return None
+    w, b, _, wt = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, train, tiled=True)
+    mod.__dict__["_flare_packed_few"] = (key, w, b, wt)
+    return w, b, wt
 
 
 def _packed(mod, layers, cd):
@@ -390,20 +415,28 @@ def _fused_mlp_io(x, mod, cd, io, info, norm, out_dtype):
     return y
 
 
+def _vec32(p):
+    """A parameter vector as the launches read it: itself where it already is contiguous fp32 on the 16-byte grid."""
+    if p.dtype is torch.float32 and p.is_contiguous() and type(p) in (torch.Tensor, nn.Parameter) and p.data_ptr() % 16 == 0:
+        return p
+    v = p.detach().float().contiguous()
+    return v if v.data_ptr() % 16 == 0 else v.clone()
+
+
 def _norm_args(d, norm, x, Cdim):
     """Fill the descriptor's norm fields; returns (gamma, beta) fp32 tensors or None."""
     gamma = beta = None
     if norm is not None and not isinstance(norm, nn.Identity):
         if isinstance(norm, nn.LayerNorm):
             d.norm, d.eps = 1, float(norm.eps)
-            beta = None if norm.bias is None else norm.bias.detach().float().contiguous()
+            beta = None if norm.bias is None else _vec32(norm.bias)
         elif isinstance(norm, nn.RMSNorm):
             d.norm = 2
             d.eps = float(norm.eps) if norm.eps is not None else float(torch.finfo(x.dtype).eps)
         else:
             raise TypeError(f"unsupported norm {type(norm).__name__}")
-        gamma = (norm.weight.detach().float().contiguous() if getattr(norm, "weight", None) is not None
-                 else torch.ones(Cdim, dtype=torch.float32, device=x.device))
+        weight = norm.weight
+        gamma = _vec32(weight) if weight is not None else torch.ones(Cdim, dtype=torch.float32, device=x.device)
     return gamma, beta
 
 
@@ -435,10 +468,26 @@ def fused_mlp(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=
     return _fused_mlp_fwd(x, mod, cd, norm, res, out_dtype, x_head, y_head)
 
 
+def _pair_info(x, mod_a, mod_b, cd):
+    """(layers of both, act_mask, add_mask, act) where one few-token launch takes both stacks, else None: plain chains of
+    C x C layers, alike in length, masks and activation, and few enough tokens."""
+    Cdim = x.shape[-1]
+    infos = [_layers_of(m) for m in (mod_a, mod_b)]
+    if infos[0] is None or infos[1] is None or infos[0][1:] != infos[1][1:] or len(infos[0][0]) != len(infos[1][0]):
+        return None
+    layers = infos[0][0] + infos[1][0]
+    if len(layers) > _lib.MLP_PACK_MAX or any(l.in_features != Cdim or l.out_features != Cdim for l in layers):
+        return None
+    if not _few(x.numel() // Cdim, Cdim, len(infos[0][0])):
+        return None
+    return (layers, *infos[0][1:])
+
+
 def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None):
     """(mod_a(norm(x)), mod_b(norm(x))) as fused_mlp computes them, for two stacks that read the same rows through the
     same norm (a block's k and v projections).  With gradients enabled and both stacks plain chains of C x C layers the
-    pair is one autograd node whose backward sums the two gradients of x inside the second launch."""
+    pair is one autograd node whose backward sums the two gradients of x inside the second launch (few tokens: one backward
+    launch for both stacks)."""
     if torch.is_grad_enabled() and all(_train_subchain(m) is None and not _expand_factor(m, x.shape[-1]) for m in (mod_a, mod_b)):
         has_norm = norm is not None and not isinstance(norm, nn.Identity)
         gamma = getattr(norm, "weight", None) if has_norm else None
@@ -451,19 +500,35 @@ def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None):
     return fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype), fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype)
 
 
-def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False):
+def _forward_plan(mod):
+    """(_layers_of, _io_dims where an end is narrow else None, width, _expand_factor), kept like _layers_of."""
+    key = _structure_key(mod)
+    cached = mod.__dict__.get("_flare_fwd_plan")
+    if cached is None or cached[1] != key or cached[0][0] is not _layers_of(mod):
+        info = _layers_of(mod)
+        io = _io_dims(mod, info[0])
+        Cdim = info[0][0].in_features
+        cached = ((info, io if io is not None and (io[1] or io[2]) else None, Cdim, _expand_factor(mod, Cdim)), key)
+        mod.__dict__["_flare_fwd_plan"] = cached
+    return cached[0]
+
+
+def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False, operands=None):
     lib = _lib.load()
-    info = _layers_of(mod)
+    info, io, Cdim, E = _forward_plan(mod)
     layers, act_mask, add_mask, act = info
-    io = _io_dims(mod, layers)
-    if io is not None and (io[1] or io[2]):
+    if io is not None:
         y = _fused_mlp_io(x, mod, cd, io, info, norm, out_dtype)
         return y if res is None else res + y
-    Cdim = layers[0].in_features
     if x.shape[-1] != (Cdim // x_head * 16 if x_head else Cdim):
         raise ValueError(f"x rows are {x.shape[-1]} wide, expected {Cdim // x_head * 16 if x_head else Cdim}")
-    E = _expand_factor(mod, Cdim)
-    if E:
+    few = not E and bool(_few(x.numel() // x.shape[-1], Cdim, len(layers)))
+    if operands is None and few:
+        operands = _packed_few(mod, layers, cd, train)
+        few = operands is not None
+    if few:
+        w, b = operands[:2]
+    elif E:
         if x_head or y_head:
             raise ValueError("head-padded rows are not available for the expanding two-layer MLP")
         w, b = _packed_train_expand(mod, E, cd)[:2] if train else _packed_expand(mod, E, cd)
@@ -478,7 +543,7 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     y = torch.empty(*x.shape[:-1], ywidth, dtype=out_dtype, device=x.device)
     d = _lib.FlareMlpDesc()
     d.T, d.C, d.L = x2.shape[0], Cdim, w.shape[0]
-    d.flags = (_lib.MLP_EXPAND if E else 0) | ((x_head // 4) << 8) | ((y_head // 4) << 12)
+    d.flags = (_lib.MLP_EXPAND if E else _lib.MLP_W_TILED if few else 0) | ((x_head // 4) << 8) | ((y_head // 4) << 12)
     d.w_dtype, d.x_dtype, d.y_dtype = _dtype_code(w), _dtype_code(x2), _dtype_code(y)
     d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
     d.x_stride, d.y_stride = x2.stride(0), ywidth
@@ -580,10 +645,11 @@ def _packed_train_expand(mod, E, cd):
     return w, b, w_img, wt_img
 
 
-def _weight_grads(d, g_out, a_in, want_bias, L=None):
+def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None):
     """dW [L, C(out), C(in)] and db [L, C] (or None) in fp32 from the rows the backward launch left: one pass of
     flare_mlp_wgrad over both row arrays, partial results per token range summed in a fixed order.  g_out, a_in:
-    [L,T,C], or [T,C] for an array all L layers share."""
+    [L,T,C], or [T,C] for an array all L layers share.  gb, gsum: the norm's partial rows [rows,2,C], summed into gsum [2,C] by
+    the launch that sums the others."""
     lib = _lib.load()
     T, Cdim = g_out.shape[-2:]
     L = (g_out.shape[0] if g_out.dim() == 3 else a_in.shape[0]) if L is None else L
@@ -598,10 +664,10 @@ def _weight_grads(d, g_out, a_in, want_bias, L=None):
     dw = torch.empty(L, Cdim, Cdim, dtype=torch.float32, device=dev)
     db = torch.empty(L, Cdim, dtype=torch.float32, device=dev) if want_bias else None
     with _on_device(dev):
-        rc = lib.flare_mlp_wgrad(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
-                                 _ptr(g_out), T * Cdim if g_out.dim() == 3 else 0,
-                                 _ptr(dwp), _ptr(dbp), _ptr(dw), _ptr(db), C.c_void_p(_stream_ptr(dev)))
-    _lib.check(rc, "flare_mlp_wgrad")
+        rc = lib.flare_mlp_wgrad_norm(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
+                                      _ptr(g_out), T * Cdim if g_out.dim() == 3 else 0, _ptr(dwp), _ptr(dbp), _ptr(dw), _ptr(db),
+                                      _ptr(gb), 0 if gb is None else gb.shape[0], _ptr(gsum), C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_wgrad_norm")
     return dw, db
 
 
@@ -664,7 +730,13 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
     layers, act_mask, add_mask, act = _layers_of(mod)
     L = len(layers)
     Cdim = x.shape[-1]
-    _, b, w_img, wt_img = _packed_train(mod, layers, cd)
+    few = _few(x.numel() // Cdim, Cdim, L)
+    packed = _packed_few(mod, layers, cd, True) if few else None
+    if packed is not None:
+        w_img, b, wt_img = packed            # the tiled operands
+    else:
+        few = 0
+        _, b, w_img, wt_img = _packed_train(mod, layers, cd)
     x2 = x.reshape(-1, Cdim)
     if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
@@ -684,7 +756,10 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
     g_out = torch.empty(L, T, Cdim, dtype=cd, device=dev)
     dn = stats = gb = gsum = None
     any_bias = any(l.bias is not None for l in layers)
-    if d.norm:
+    if few and d.norm:
+        gb = torch.empty(few, 2, Cdim, dtype=torch.float32, device=dev)
+        gsum = torch.empty(2, Cdim, dtype=torch.float32, device=dev)
+    elif d.norm:
         rows = C.c_int32(0)
         _lib.check(lib.flare_mlp_bwd_partial_rows(C.byref(d), C.byref(rows)), "flare_mlp_bwd_partial_rows")
         dn = torch.empty(T, Cdim, dtype=cd, device=dev)
@@ -693,13 +768,53 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
         gsum = torch.empty(2, Cdim, dtype=torch.float32, device=dev)
     bits = (_lib.MLP_BWD_ADD_DY if res_is_x else 0) | (_lib.MLP_BWD_ACCUMULATE if dx_acc is not None else 0)
     with _on_device(dev):
-        rc = lib.flare_mlp_bwd(C.byref(d), _ptr(x2), _ptr(dy2), _ptr(w_img), _ptr(wt_img), _ptr(b), _ptr(gamma), _ptr(beta),
-                               bits, _ptr(dx), _ptr(a_in), _ptr(g_out), _ptr(dn), _ptr(stats), _ptr(gb),
-                               _ptr(gsum), C.c_void_p(_stream_ptr(dev)))
+        if few:
+            rc = lib.flare_mlp_few_bwd(C.byref(d), _ptr(x2), _ptr(dy2), None, _ptr(w_img), _ptr(wt_img), _ptr(b), _ptr(gamma), _ptr(beta),
+                                       bits, _ptr(dx), _ptr(a_in), _ptr(g_out), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
+        else:
+            rc = lib.flare_mlp_bwd(C.byref(d), _ptr(x2), _ptr(dy2), _ptr(w_img), _ptr(wt_img), _ptr(b), _ptr(gamma), _ptr(beta),
+                                   bits, _ptr(dx), _ptr(a_in), _ptr(g_out), _ptr(dn), _ptr(stats), _ptr(gb),
+                                   None, C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_bwd")
     # weight and bias gradients: one more launch over the rows the kernel left (16-bit products with fp32
-    # accumulation, as torch runs a Linear's backward under autocast); norm gradients: partial rows, summed by the launch
-    dW, db = _weight_grads(d, g_out, a_in, any_bias)                 # [L, out, in], [L, C] fp32
+    # accumulation, as torch runs a Linear's backward under autocast); norm gradients: partial rows, summed with the others
+    dW, db = _weight_grads(d, g_out, a_in, any_bias, gb=gb, gsum=gsum)                 # [L, out, in], [L, C] fp32
+    return dx, gsum, dW, db, layers
+
+
+def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb):
+    """Backward of both stacks of a pair in one launch: (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
+    None, the 2 L layers)."""
+    lib = _lib.load()
+    layers, act_mask, add_mask, act = _pair_info(x, mod_a, mod_b, cd)
+    w, b, wt = _packed_few(mod_a, layers, cd, True)
+    L2, Cdim, dev = len(layers), x.shape[-1], x.device
+    x2 = x.reshape(-1, Cdim)
+    if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
+        x2 = x2.contiguous()
+    da, db_ = _rows2d(dya, Cdim), _rows2d(dyb, Cdim)
+    if da.dtype != db_.dtype:
+        da, db_ = da.float(), db_.float()
+    if da.stride() != db_.stride():
+        da, db_ = da.contiguous(), db_.contiguous()
+    T = x2.shape[0]
+    d = _lib.FlareMlpDesc()
+    d.T, d.C, d.L = T, Cdim, L2 // 2
+    d.w_dtype, d.x_dtype, d.y_dtype = _dtype_code(w), _dtype_code(x2), _dtype_code(da)
+    d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
+    d.x_stride, d.y_stride = x2.stride(0), da.stride(0)
+    gamma, beta = _norm_args(d, norm, x, Cdim)
+    dx = torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
+    rows = torch.empty(2, L2, T, Cdim, dtype=cd, device=dev)         # a_in, g_out
+    gb = gsum = None
+    if d.norm:
+        gb = torch.empty(_few(T, Cdim, L2 // 2), 2, Cdim, dtype=torch.float32, device=dev)
+        gsum = torch.empty(2, Cdim, dtype=torch.float32, device=dev)
+    with _on_device(dev):
+        rc = lib.flare_mlp_few_bwd(C.byref(d), _ptr(x2), _ptr(da), _ptr(db_), _ptr(w), _ptr(wt), _ptr(b), _ptr(gamma), _ptr(beta),
+                                   0, _ptr(dx), _ptr(rows[0]), _ptr(rows[1]), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_few_bwd")
+    dW, db = _weight_grads(d, rows[1], rows[0], any(l.bias is not None for l in layers), gb=gb, gsum=gsum)
     return dx, gsum, dW, db, layers
 
 
@@ -712,8 +827,14 @@ class _FusedPairFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, mod_a, mod_b, cd, norm, out_dtype, x, gamma, beta, *wb):
         with torch.no_grad():
-            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, train=True)
-            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, train=True)
+            info = _pair_info(x, mod_a, mod_b, cd)
+            packed = None if info is None else _packed_few(mod_a, info[0], cd, True)
+            ctx.pair = packed is not None
+            n = len(info[0]) // 2 if ctx.pair else 0
+            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, train=True,
+                                operands=(packed[0][:n], packed[1][:n]) if ctx.pair else None)
+            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, train=True,
+                                operands=(packed[0][n:], packed[1][n:]) if ctx.pair else None)
         ctx.mods, ctx.cd, ctx.norm = (mod_a, mod_b), cd, norm
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)
@@ -727,11 +848,18 @@ class _FusedPairFn(torch.autograd.Function):
         if ctx.versions != tuple(None if t is None else t._version for t in ctx.params):
             raise RuntimeError("a parameter of the fused MLP was modified in place between its forward and its backward")
         mod_a, mod_b = ctx.mods
-        dx, gs_a, dWa, dba, la = _chain_backward(mod_a, ctx.cd, ctx.norm, x, dya, False)
-        dx, gs_b, dWb, dbb, lb = _chain_backward(mod_b, ctx.cd, ctx.norm, x, dyb, False, dx_acc=dx)
+        if ctx.pair:
+            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb)
+            n = len(layers) // 2
+            la, lb, dWa, dWb = layers[:n], layers[n:], dW[:n], dW[n:]
+            dba, dbb = (None, None) if db is None else (db[:n], db[n:])
+        else:
+            dx, gs_a, dWa, dba, la = _chain_backward(mod_a, ctx.cd, ctx.norm, x, dya, False)
+            dx, gs_b, dWb, dbb, lb = _chain_backward(mod_b, ctx.cd, ctx.norm, x, dyb, False, dx_acc=dx)
+            gs = None if gs_a is None else gs_a + gs_b
         need = ctx.needs_input_grad            # (mod_a, mod_b, cd, norm, out_dtype, x, gamma, beta, *wb)
         grads = [None, None, None, None, None, dx.view(x.shape) if need[5] else None]
-        grads += _norm_grads(ctx.norm, None if gs_a is None else gs_a + gs_b, need[6], need[7])
+        grads += _norm_grads(ctx.norm, gs, need[6], need[7])
         at = 8
         for layers, dW, db in ((la, dWa, dba), (lb, dWb, dbb)):
             n = len(layers)

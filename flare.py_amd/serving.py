@@ -51,7 +51,7 @@ class GraphedForward:
         baked into the graph)."""
         keep = []
         for m in self.module.modules():
-            for name in ("_flare_packed", "_q_cache"):
+            for name in ("_flare_packed", "_flare_packed_few", "_q_cache"):
                 c = getattr(m, name, None)
                 if c is not None:
                     keep.append(c)

@@ -76,7 +76,7 @@ class GraphedTrainStep:
     def _drop_operand_caches(self):
         """Forget the packed weights the warm-up left on the modules, so that the captured step packs them itself."""
         for m in self.module.modules():
-            for name in ("_flare_packed", "_flare_packed_train", "_q_cache"):
+            for name in ("_flare_packed", "_flare_packed_train", "_flare_packed_few", "_q_cache"):
                 m.__dict__.pop(name, None)
 
     def _capture(self, inputs):

@@ -388,6 +388,21 @@ int flare_mlp_io_fwd(const FlareMlpDesc* desc, int32_t in_dim, int32_t in_act, c
  *   ch = col / 8, j = col % 8, key = (row % 16) >> (C == 128 ? 0 : C == 64 ? 1 : 2)
  * (flare.py_amd/fused.py::mlp_weight_image builds them). */
 int flare_mlp_bwd_partial_rows(const FlareMlpDesc* desc, int32_t* rows);
+
+/* Launches of few tokens, on weights in an order of their own (flare_mlp_pack with tiled): element (row, col) of a tile at
+ *   ((row / 16 * (C / 32) + col / 32) * 4 + col % 32 / 8) * 128 + row % 16 * 8 + col % 8.
+ * flare_mlp_few: 0 where the kernels above serve the descriptor (T, C, L, w_dtype, flags are read), else the rows of gb_part that
+ * flare_mlp_few_bwd writes.  Forward: flare_mlp_fwd with FLARE_MLP_W_TILED in desc->flags (chain and head-padded rows).
+ * flare_mlp_few_bwd: as flare_mlp_bwd (flags == 0), w and wt the tiled weights and transposes, gb_part [rows,2,C] summed in the
+ * launch (no dn, no stats; flare_mlp_wgrad_norm adds the rows up).  With dy_b it differentiates two chains of equal L, masks and
+ * activation that read the same rows through the same norm (a block's k and v projections, pdebench/models/flare.py:139-140):
+ * chain a is tiles 0 .. L-1 and chain b tiles L .. 2L-1 of w / wt [2L,C,C] and bias [2L,C]; dy_a, dy_b share dtype and row
+ * stride; dx is the sum over both, a_in and g_out are [2L,T,C]. */
+#define FLARE_MLP_W_TILED 2
+int flare_mlp_few(const FlareMlpDesc* desc);
+int flare_mlp_few_bwd(const FlareMlpDesc* desc, const void* x, const void* dy_a, const void* dy_b, const void* w, const void* wt,
+                      const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in, void* g_out,
+                      float* gb_part, void* stream);
 /* Weight and bias gradients from the rows flare_mlp_bwd leaves, in one pass over both (the reference gets them from
  * torch's Linear backward: dW = dt^T s, db = column sums of dt; pdebench/models/flare.py:45-59 under autograd).
  * Only T, C, L and w_dtype of the descriptor are read.  a_in, g_out: L arrays of [T,C] rows in the weights' type,
@@ -399,10 +414,15 @@ int flare_mlp_bwd_partial_rows(const FlareMlpDesc* desc, int32_t* rows);
 int flare_mlp_wgrad_partials(const FlareMlpDesc* desc, int32_t* parts);
 int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                     float* dw_part, float* db_part, float* dw, float* db, void* stream);
+/* The same, with the norm's partial rows of the backward (gb_part [gb_rows,2,C]; pass its gb as NULL there) summed into gb [2,C] by
+ * the launch that sums the others; gb NULL: nothing. */
+int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                         float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream);
 /* The operands of the launches above from the parameters, in one launch.  Tile l is the [out][in] block at src[l] with ld[l] elements
  * between its rows, of which rows[l] (1 .. C) exist and the others are taken as zeros; bsrc[l] (or NULL: zeros) holds rows[l] bias
  * elements.  Each has its own element type.  Outputs: w [L,C,C] in w_dtype, bias [L,C] fp32, and, unless both are NULL, w_img and
- * wt_img [L,C,C], the images flare_mlp_bwd reads.  1 <= L <= FLARE_MLP_PACK_MAX. */
+ * wt_img [L,C,C], the images flare_mlp_bwd reads.  1 <= L <= FLARE_MLP_PACK_MAX.  tiled != 0: w and (unless NULL) wt_img receive
+ * the tiles and their transposes in the operand order of the few-token launches instead, w_img must be NULL. */
 #define FLARE_MLP_PACK_MAX 16
 typedef struct {
     int32_t L, C, w_dtype;
@@ -410,6 +430,7 @@ typedef struct {
     const void* bsrc[FLARE_MLP_PACK_MAX];
     int64_t ld[FLARE_MLP_PACK_MAX];
     int32_t rows[FLARE_MLP_PACK_MAX], src_dtype[FLARE_MLP_PACK_MAX], b_dtype[FLARE_MLP_PACK_MAX];
+    int32_t tiled;
 } FlareMlpPackDesc;
 int flare_mlp_pack(const FlareMlpPackDesc* desc, void* w, void* w_img, void* wt_img, float* bias, void* stream);
 

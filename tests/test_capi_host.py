@@ -344,3 +344,18 @@ def test_mlp_expand_bwd_validation():
     assert call() == _lib.FLARE_EINVAL and "FLARE_MLP_EXPAND" in _lib.last_error()
     m.flags, m.C = _lib.MLP_EXPAND, 96
     assert call() == _lib.FLARE_EUNSUPPORTED
+
+
+def test_few_token_limits_agree_with_the_library():
+    from flare_py_amd import fused
+
+    lib = _lib.load()
+    for Cdim in (32, 64, 128):
+        for L in (1, 5, 6, 8, 9):
+            for T in (1, 16, 17, 12288, 12289, 16384, 16385, 1 << 20):
+                m = _lib.FlareMlpDesc()
+                m.T, m.C, m.L, m.w_dtype = T, Cdim, L, _lib.DT_BF16
+                assert lib.flare_mlp_few(C.byref(m)) == fused._few(T, Cdim, L), (Cdim, L, T)
+    m.flags = _lib.MLP_EXPAND
+    m.T = 16
+    assert lib.flare_mlp_few(C.byref(m)) == 0

@@ -496,3 +496,34 @@ def test_packed_operands_are_the_stacked_parameters(dev, C, cd, pd):
         assert torch.equal(w[2 * j + 1], f2.weight.detach()[:, j * C:(j + 1) * C].to(cd))
         assert torch.equal(b[2 * j], f1.bias.detach()[j * C:(j + 1) * C].float())
         assert torch.equal(b[2 * j + 1], f2.bias.detach().float() if j == 0 else torch.zeros(C, device=dev))
+
+
+@pytest.mark.parametrize("C,num_layers,T", [(32, 6, 15), (64, 3, 17), (128, 3, 1), (128, 3, 4099), (64, 6, 16384)])
+@pytest.mark.parametrize("kind,dtype,act", [("ln", torch.bfloat16, "gelu"), ("rms", torch.float16, "silu"), (None, torch.bfloat16, "gelu")])
+def test_pair_of_chains_against_fp32_torch_layers(dev, C, num_layers, T, kind, dtype, act):
+    """Two stacks behind one norm in one launch each way: outputs and every gradient against fp32 autograd, at token counts
+    around the 16-token workgroup and at the end of the range."""
+    torch.manual_seed(T)
+    norm = {"ln": nn.LayerNorm, "rms": nn.RMSNorm, None: lambda c: nn.Identity()}[kind](C).to(dev)
+    mods = [ResidualMLP(C, C, C, num_layers=num_layers, act=act, input_residual=True, output_residual=True).to(dev) for _ in range(2)]
+    for p in norm.parameters():
+        p.data += 0.3 * torch.randn_like(p)
+    x = (torch.randn(T, C, device=dev) * 1.5 + 0.2).requires_grad_(True)
+    gys = [torch.randn(T, C, device=dev) for _ in range(2)]
+    params = [p for m in (norm, *mods) for p in m.parameters()]
+
+    def grads(ys):
+        return torch.autograd.grad(ys, [x, *params], [g.to(y.dtype) for g, y in zip(gys, ys)])
+
+    ref_y = [m(norm(x)) for m in mods]
+    ref = [y.detach() for y in ref_y] + list(grads(ref_y))
+    assert fused._pair_info(x, *mods, dtype) is not None
+    with torch.autocast("cuda", dtype=dtype):
+        ys = fused.fused_mlp_pair(x, *mods, dtype, norm=norm, out_dtype=dtype)
+        got = [y.detach() for y in ys] + list(grads(ys))
+        with torch.no_grad():
+            alone = [fused.fused_mlp(x, m, dtype, norm=norm, out_dtype=dtype) for m in mods]
+    for y, z in zip(ys, alone):
+        assert torch.equal(y, z)
+    for i, (a, b) in enumerate(zip(got, ref)):
+        assert rel(a.float(), b) <= 3e-2, i
