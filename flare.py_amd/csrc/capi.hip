@@ -5,6 +5,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 
 #include "common.hpp"
@@ -1290,6 +1291,63 @@ int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img
     a.w = static_cast<uint16_t*>(w); a.w_img = static_cast<uint16_t*>(w_img); a.wt_img = static_cast<uint16_t*>(wt_img);
     a.bias = bias; a.L = d->L; a.C = d->C; a.tiled = d->tiled ? 1 : 0;
     return hip_status(flare::launch_mlp_pack(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp pack launch");
+}
+
+static int check_rows(int64_t T, int32_t C, std::initializer_list<const void*> must, std::initializer_list<const void*> may)
+{
+    if (T < 1) return fail(FLARE_EINVAL, "T >= 1 required (got %lld)", (long long)T);
+    if (!flare::rows_f32_supported(C)) return fail(FLARE_EUNSUPPORTED, "C=%d: only 32, 64, 128 and 256 are supported", C);
+    for (const void* p : must)
+        if (!p) return fail(FLARE_EINVAL, "a required array is NULL");
+    for (const auto& l : {must, may})
+        for (const void* p : l)
+            if (p && !aligned16(p)) return fail(FLARE_EINVAL, "every array must be 16-byte aligned");
+    return FLARE_OK;
+}
+
+int flare_rows_parts(int64_t T, int32_t C, int32_t* parts)
+{
+    if (!parts) return fail(FLARE_EINVAL, "parts is NULL");
+    const int rc = check_rows(T, C, {}, {});
+    if (rc != FLARE_OK) return rc;
+    *parts = flare::rows_f32_parts(T, C);
+    return FLARE_OK;
+}
+
+int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const float* t, float* dt, float* copy, float* db_part,
+                       float* db, void* stream)
+{
+    const int rc = check_rows(T, C, {ds, db_part}, {t, dt, copy, db});
+    if (rc != FLARE_OK) return rc;
+    if (act < -1 || act > FLARE_ACT_SILU) return fail(FLARE_EINVAL, "unknown activation %d", act);
+    if (act >= 0 && (!t || !dt)) return fail(FLARE_EINVAL, "t and dt must not be NULL with an activation");
+    return hip_status(flare::launch_rows_act_bwd(act, ds, t, dt, copy, db_part, db, T, C, static_cast<hipStream_t>(stream)), "row activation backward launch");
+}
+
+int flare_rows_norm_fwd(int64_t T, int32_t C, int32_t norm, float eps, const float* x, const float* gamma, const float* beta,
+                        float* y, float* stats, void* stream)
+{
+    const int rc = check_rows(T, C, {x, y, stats}, {gamma, beta});
+    if (rc != FLARE_OK) return rc;
+    if (norm != FLARE_NORM_LAYER && norm != FLARE_NORM_RMS) return fail(FLARE_EINVAL, "unknown norm %d", norm);
+    if (!(eps >= 0.f)) return fail(FLARE_EINVAL, "eps must be >= 0");
+    flare::RowsNormArgs a;
+    memset(&a, 0, sizeof(a));
+    a.x = x; a.gamma = gamma; a.beta = beta; a.y = y; a.stats = stats; a.T = T; a.C = C; a.norm = norm; a.eps = eps;
+    return hip_status(flare::launch_rows_norm(a, static_cast<hipStream_t>(stream)), "row norm launch");
+}
+
+int flare_rows_norm_bwd(int64_t T, int32_t C, int32_t norm, const float* dy, const float* x, const float* stats, const float* gamma,
+                        const float* add, float* dx, float* gb_part, float* gb, void* stream)
+{
+    const int rc = check_rows(T, C, {dy, x, stats, dx, gb_part}, {gamma, add, gb});
+    if (rc != FLARE_OK) return rc;
+    if (norm != FLARE_NORM_LAYER && norm != FLARE_NORM_RMS) return fail(FLARE_EINVAL, "unknown norm %d", norm);
+    flare::RowsNormArgs a;
+    memset(&a, 0, sizeof(a));
+    a.x = x; a.dy = dy; a.add = add; a.gamma = gamma; a.y = dx; a.stats = const_cast<float*>(stats); a.gb_part = gb_part; a.gb = gb;
+    a.T = T; a.C = C; a.norm = norm;
+    return hip_status(flare::launch_rows_norm_bwd(a, static_cast<hipStream_t>(stream)), "row norm backward launch");
 }
 
 int flare_triple_workspace_bytes(const FlareTripleDesc* desc, size_t* bytes)

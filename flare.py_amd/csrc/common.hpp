@@ -347,6 +347,18 @@ struct MlpPackArgs {
     int tiled;                                  // 1: w and wt_img in the few-token kernels' operand order (wt_img may be null)
 };
 
+// Row passes of fp32 token-wise layers (rows_f32.hip)
+struct RowsNormArgs {
+    const float* x; const float* dy; const float* add;      // [T,C]; add (or null) joins dx
+    const float* gamma; const float* beta;                  // [C] or null
+    float* y;                                               // [T,C]: the norm's output, in the backward dx
+    float* stats;                                           // [T,2] mean and 1/std: written by the forward, read by the backward
+    float* gb_part; float* gb;                              // backward: [parts,2,C] and their sum [2,C] (or null)
+    int64_t T;
+    int C, norm;                                            // 1 LayerNorm, 2 RMSNorm
+    float eps;
+};
+
 // Workgroups of the backward's dq pass (bwd_lat_kernel, MODE 1) that fit a compute unit: its instances with 16 or
 // 32 latents per wave at head dim 16, and with 16 at head dim 32, need few enough registers for three or four (measured:
 // 143 -> 119 us at M = 128, D = 16; 86 -> 74 us at M = 64, D = 16; 133 -> 106 us at M = 64, D = 32); squeezing the
@@ -417,6 +429,12 @@ bool       mlp_few_ok(int64_t T, int C, int L);
 int        mlp_few_bwd_rows(int64_t T);
 hipError_t launch_mlp_few(const MlpArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_mlp_few_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
+hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts, hipStream_t st);   // n a multiple of 4
+bool       rows_f32_supported(int C);
+int        rows_f32_parts(int64_t T, int C);
+hipError_t launch_rows_act_bwd(int act, const float* ds, const float* t, float* dt, float* copy, float* part, float* db, int64_t T, int C, hipStream_t st);
+hipError_t launch_rows_norm(const RowsNormArgs& a, hipStream_t st);
+hipError_t launch_rows_norm_bwd(const RowsNormArgs& a, hipStream_t st);
 hipError_t launch_mlp_pack(const MlpPackArgs& a, int w_dtype, hipStream_t st);
 
 int        causal_linear_tile();

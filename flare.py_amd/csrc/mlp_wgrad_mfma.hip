@@ -284,6 +284,15 @@ int mlp_wgrad_partials(int64_t T, int C, int L)
     return (int)((T + per - 1) / per) * wgrad_wk(C);
 }
 
+hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts, hipStream_t st)
+{
+    SumJobs jobs{};
+    jobs.n = 1;
+    jobs.j[0] = SumJob{part, out, n, parts, 0, 4};        // few outputs, many partials: 64 ways over the partials
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n / 4 + 3) / 4)), dim3(256), 0, st, jobs);
+    return hipGetLastError();
+}
+
 hipError_t launch_mlp_wgrad(const MlpWgradArgs& a0, int w_dtype, hipStream_t st)
 {
     MlpWgradArgs a = a0;

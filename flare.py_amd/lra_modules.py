@@ -20,8 +20,8 @@ from torch import nn
 from torch.nn import functional as F
 
 from .functional import flare_multihead_mixer, triple_attention
-from . import fused
-from .modules import ResidualMLP, _lin, _norm
+from . import fused, rows
+from .modules import ResidualMLP, _chain_info, _lin, _mlp_block, _norm, _project
 
 __all__ = ["FLARE", "FLAREBlock", "TripleAttention", "TripleBlock", "make_kernel", "RotaryPositionalEmbeddings"]
 
@@ -93,7 +93,7 @@ class FLARE(nn.Module):
         if cd is not None:
             k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd)
         else:
-            xn = x if _norm is None else _norm(x)
+            xn = x if _norm is None else rows.norm(_norm, x) if _chain_info(self.k_proj, x) is not None else _norm(x)
             k, v = self.k_proj(xn), self.v_proj(xn)
         k = k.view(B, N, self.num_heads, self.head_dim).permute(0, 2, 1, 3)
         v = v.view(B, N, self.num_heads, self.head_dim).permute(0, 2, 1, 3)
@@ -104,6 +104,8 @@ class FLARE(nn.Module):
         y = y.permute(0, 2, 1, 3).reshape(B, N, C)
         if cd is not None and pdrop == 0.0:
             return fused.fused_mlp(y, self.out_proj, cd, res=_res, out_dtype=(x if _res is None else _res).dtype)
+        if pdrop == 0.0:
+            return _project(self.out_proj, y, _res)
         y = F.dropout(_lin(self.out_proj, y), p=pdrop)
         return y if _res is None else _res + y
 
@@ -128,7 +130,7 @@ class FLAREBlock(nn.Module):
         cd = fused.compute_dtype(x, self.mlp)
         if cd is not None:
             return fused.fused_mlp(x, self.mlp, cd, norm=self.norm2, res=x)
-        return x + self.mlp(self.norm2(x))
+        return _mlp_block(self.mlp, self.norm2, x)
 
 
 # ---- feature maps ("kernels") applied to q1, q2, k1, k2 --------------------------------------

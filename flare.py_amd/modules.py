@@ -18,7 +18,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
-from . import fused
+from . import fused, rows
 from .functional import flare_multihead_mixer
 
 __all__ = ["ResidualMLP", "FLARE", "FLAREBlock", "FinalLayer", "FLAREModel"]
@@ -57,18 +57,13 @@ class _LinearLongRows(torch.autograd.Function):
             dx = dy @ w
         dy2, x2 = dy.reshape(-1, w.shape[0]), x.reshape(-1, w.shape[1])
         if ctx.needs_input_grad[1]:
-            T = x2.shape[0]
-            S = next(s for s in (64, 32, 16, 8, 4, 2, 1) if T % s == 0)
-            if S > 1:
-                dw = torch.bmm(dy2.view(S, T // S, -1).transpose(1, 2), x2.view(S, T // S, -1)).sum(0)
-            else:
-                dw = dy2.t() @ x2
+            dw = rows.weight_grad(dy2, x2)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = dy2.sum(0)
         return dx, dw, db
 
 
-_LONG_ROWS = 4096      # rows from which the sliced weight gradient pays (below, one product is as fast)
+_LONG_ROWS = rows.LONG_ROWS      # rows from which the sliced weight gradient pays (below, one product is as fast)
 
 
 def _lin(layer: nn.Linear, x):
@@ -78,6 +73,31 @@ def _lin(layer: nn.Linear, x):
             and max(layer.in_features, layer.out_features) <= 1024):
         return _LinearLongRows.apply(x, layer.weight, layer.bias)
     return layer(x)
+
+
+def _chain_info(mod, x):
+    return rows.chain_info(mod, x, _LONG_ROWS)
+
+
+def _project(layer: nn.Linear, y, res):
+    """[res +] layer(y)."""
+    info = _chain_info(layer, y)
+    if info is not None and (res is None or rows.res_ok(res, y)):
+        return rows.chain(layer, y, info, res=res)
+    y = _lin(layer, y)
+    return y if res is None else res + y
+
+
+def _mlp_block(mlp, norm, x):
+    """x + mlp(norm(x)) outside the fused 16-bit launches."""
+    info = _chain_info(mlp, x)
+    if info is not None and _plain_call(mlp):
+        return rows.chain(mlp, rows.norm(norm, x), info, res=x)
+    return x + mlp(norm(x))
+
+
+def _plain_call(mod):
+    return type(mod) is ResidualMLP and rows._plain(mod)
 
 
 class ResidualMLP(nn.Module):
@@ -101,6 +121,9 @@ class ResidualMLP(nn.Module):
         self.output_residual = output_residual and hidden_dim == out_dim
 
     def forward(self, x):
+        info = _chain_info(self, x)      # fp32 training over long rows: products with HIP row passes around them
+        if info is not None:
+            return rows.chain(self, x, info)
         if self.num_layers == -1:
             return x + _lin(self.fc, x) if self.residual else _lin(self.fc, x)
         h = self.act(_lin(self.fc1, x))
@@ -203,7 +226,7 @@ class FLARE(nn.Module):
             out_dtype = _res.dtype if _res is not None else x.dtype
             return fused.fused_mlp(y, self.out_proj, cd, res=_res, out_dtype=out_dtype), None
         if _norm is not None:
-            x = _norm(x)
+            x = rows.norm(_norm, x) if _chain_info(self.k_proj, x) is not None else _norm(x)
         k = self._heads(self.k_proj(x))
         v = self._heads(self.v_proj(x))
         if self.qk_norm:
@@ -221,8 +244,7 @@ class FLARE(nn.Module):
             y = F.softmax(scores.transpose(-2, -1), dim=-1) @ z
 
         y = y.permute(0, 2, 1, 3).reshape(B, N, C)
-        y = _lin(self.out_proj, y)
-        return (y if _res is None else _res + y), scores
+        return _project(self.out_proj, y, _res), scores
 
 
 class FLAREBlock(nn.Module):
@@ -248,7 +270,7 @@ class FLAREBlock(nn.Module):
         if cd is not None:
             x = fused.fused_mlp(x, self.mlp, cd, norm=self.norm2, res=x)
         else:
-            x = x + self.mlp(self.norm2(x))
+            x = _mlp_block(self.mlp, self.norm2, x)
         return x, scores
 
 

@@ -418,6 +418,22 @@ int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_
  * the launch that sums the others; gb NULL: nothing. */
 int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream);
+/* Row passes around fp32 products in training: contiguous [T,C] rows on the 16-byte grid, C in {32, 64, 128, 256}; act -1 none, else
+ * FLARE_ACT_*; norm FLARE_NORM_LAYER or FLARE_NORM_RMS.
+ *   flare_rows_act_bwd   dt = ds act'(t), db [C] = its column sums (act -1: the column sums of ds, t and dt may be
+ *                        NULL); copy (or NULL) = ds
+ *   flare_rows_norm_fwd  y = norm(x) (gamma, beta may be NULL), stats [T,2] = mean (0 for RMS) and 1/std
+ *   flare_rows_norm_bwd  dx = [add] + the norm's gradient, gb [2,C] = dgamma, dbeta
+ * db_part [parts,C] and gb_part [parts,2,C] are scratch, parts from flare_rows_parts; db, gb may be NULL (the partial rows stay).
+ * Sums are taken in a fixed order. */
+int flare_rows_parts(int64_t T, int32_t C, int32_t* parts);
+int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const float* t, float* dt, float* copy, float* db_part,
+                       float* db, void* stream);
+int flare_rows_norm_fwd(int64_t T, int32_t C, int32_t norm, float eps, const float* x, const float* gamma, const float* beta,
+                        float* y, float* stats, void* stream);
+int flare_rows_norm_bwd(int64_t T, int32_t C, int32_t norm, const float* dy, const float* x, const float* stats, const float* gamma,
+                        const float* add, float* dx, float* gb_part, float* gb, void* stream);
+
 /* The operands of the launches above from the parameters, in one launch.  Tile l is the [out][in] block at src[l] with ld[l] elements
  * between its rows, of which rows[l] (1 .. C) exist and the others are taken as zeros; bsrc[l] (or NULL: zeros) holds rows[l] bias
  * elements.  Each has its own element type.  Outputs: w [L,C,C] in w_dtype, bias [L,C] fp32, and, unless both are NULL, w_img and

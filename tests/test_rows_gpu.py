@@ -1,0 +1,113 @@
+"""fp32 training of the token-wise layers through the row passes (rows.chain, rows.norm) against the same torch layers in fp64; the
+error may not exceed what torch's own fp32 layers show by more than half (sums in another order), with 1e-7 for results that
+torch happens to get exactly."""
+import copy
+
+import pytest
+import torch
+from torch import nn
+
+import flare_py_amd as F
+from flare_py_amd import modules, rows
+from flare_py_amd.modules import ResidualMLP
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float((a.double() - b).norm() / (b.norm() + 1e-300))
+
+
+def grads(fn, x, params, gy):
+    y = fn(x)
+    return [y.detach(), *torch.autograd.grad(y, [x, *params], gy)]
+
+
+def hold(got, t32, ref):
+    for i, (a, b, r) in enumerate(zip(got, t32, ref)):
+        assert rel(a, r) <= 1.5 * rel(b, r) + 1e-7, (i, rel(a, r), rel(b, r))
+
+
+@pytest.mark.parametrize("C,T,layers,act,ends", [(32, 4096, 3, "gelu", True), (64, 4097, 0, "silu", False), (128, 5003, 3, "gelu", True),
+                                                 (256, 4099, 1, "silu", True), (128, 70001, -1, "gelu", True)])
+def test_residual_mlp(dev, monkeypatch, C, T, layers, act, ends):
+    torch.manual_seed(C)
+    m = ResidualMLP(C, C, C, num_layers=layers, act=act, input_residual=ends, output_residual=ends).to(dev)
+    if layers > 0:
+        m.fcs[0].bias = None
+    for p in m.parameters():
+        p.data.mul_(2.0)
+    x = (torch.randn(T, C, device=dev) * 3).requires_grad_(True)
+    gy = torch.randn(T, C, device=dev)
+    m64, x64 = copy.deepcopy(m).double(), x.detach().double().requires_grad_(True)
+    ref = grads(m64, x64, list(m64.parameters()), gy.double())
+    assert rows.chain_info(m, x) is not None
+    got = grads(m, x, list(m.parameters()), gy)
+    monkeypatch.setattr(modules, "_LONG_ROWS", 1 << 62)
+    t32 = grads(m, x, list(m.parameters()), gy)
+    monkeypatch.undo()
+    hold(got, t32, ref)
+    again = grads(m, x, list(m.parameters()), gy)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("kind", [nn.LayerNorm, nn.RMSNorm])
+@pytest.mark.parametrize("C,T", [(32, 4096), (64, 4105), (128, 4097), (256, 33001)])
+def test_norm(dev, kind, C, T):
+    torch.manual_seed(T)
+    m = kind(C).to(dev)
+    for p in m.parameters():
+        p.data.add_(0.5 * torch.randn_like(p))
+    x = (torch.randn(T, C, device=dev) * 2 + 1).requires_grad_(True)
+    gy = torch.randn(T, C, device=dev)
+    m64, x64 = copy.deepcopy(m).double(), x.detach().double().requires_grad_(True)
+    m64.eps = m.eps if m.eps is not None else torch.finfo(torch.float32).eps
+    ref = grads(m64, x64, list(m64.parameters()), gy.double())
+    got = grads(lambda t: rows.norm(m, t), x, list(m.parameters()), gy)
+    hold(got, grads(m, x, list(m.parameters()), gy), ref)
+
+
+def test_strided_rows_frozen_parameters_and_hooks(dev):
+    torch.manual_seed(0)
+    m = ResidualMLP(64, 64, 64, num_layers=1, input_residual=True, output_residual=True).to(dev)
+    wide = torch.randn(2, 3000, 67, device=dev)
+    x = wide[..., 1:65]                                       # rows at a stride, off the 16-byte grid, no gradient asked for
+    m.fc1.bias.requires_grad_(False)
+    ref = m.double()(x.double())
+    ref.sum().backward()
+    want = [None if p.grad is None else p.grad.clone() for p in m.parameters()]
+    m.float().zero_grad(set_to_none=True)
+    y = m(x)
+    assert rel(y.detach(), ref.detach()) <= 1e-6
+    y.sum().backward()
+    for p, r in zip(m.parameters(), want):
+        assert (p.grad is None) == (r is None) and (r is None or rel(p.grad, r.double()) <= 1e-5)
+    assert rows.chain_info(m, x) is not None
+    seen = []
+    h = m.act.register_forward_hook(lambda *a: seen.append(1))
+    assert rows.chain_info(m, x) is None                      # a hook wants its layer called
+    m(x)
+    h.remove()
+    assert seen
+    m.fc2.weight.requires_grad_(False)
+    assert rows.chain_info(m, x) is None
+    with torch.no_grad():
+        assert rows.chain_info(m, x) is None
+
+
+@pytest.mark.parametrize("lra", [False, True])
+def test_block_against_torch_layers(dev, monkeypatch, lra):
+    from flare_py_amd import lra_modules
+
+    torch.manual_seed(1)
+    cls = lra_modules.FLAREBlock if lra else F.FLAREBlock
+    kw = {"kv_proj_hidden_dim": 64, "ffn_hidden_dim": 64} if lra else {}
+    m = cls(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev)
+    x = torch.randn(2, 2500, 64, device=dev, requires_grad=True)
+    gy = torch.randn(2, 2500, 64, device=dev)
+    run = (lambda t: m(t)) if lra else (lambda t: m(t)[0])
+    got = grads(run, x, list(m.parameters()), gy)
+    monkeypatch.setattr(modules, "_LONG_ROWS", 1 << 62)
+    t32 = grads(run, x, list(m.parameters()), gy)
+    for a, b in zip(got, t32):
+        assert rel(a, b.double()) <= 1e-5
