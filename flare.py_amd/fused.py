@@ -472,6 +472,8 @@ def _pair_info(x, mod_a, mod_b, cd):
     """(layers of both, act_mask, add_mask, act) where one few-token launch takes both stacks, else None: plain chains of
     C x C layers, alike in length, masks and activation, and few enough tokens."""
     Cdim = x.shape[-1]
+    if not 0 < x.numel() // Cdim <= _FEW_TOKENS[Cdim]:      # most calls end here: nothing else is looked at for them
+        return None
     infos = [_layers_of(m) for m in (mod_a, mod_b)]
     if infos[0] is None or infos[1] is None or infos[0][1:] != infos[1][1:] or len(infos[0][0]) != len(infos[1][0]):
         return None
@@ -504,7 +506,7 @@ def _forward_plan(mod):
     """(_layers_of, _io_dims where an end is narrow else None, width, _expand_factor), kept like _layers_of."""
     key = _structure_key(mod)
     cached = mod.__dict__.get("_flare_fwd_plan")
-    if cached is None or cached[1] != key or cached[0][0] is not _layers_of(mod):
+    if cached is None or cached[1] != key:
         info = _layers_of(mod)
         io = _io_dims(mod, info[0])
         Cdim = info[0][0].in_features

@@ -8,7 +8,7 @@ the start value of dx together (flare_rows_act_bwd), the product that adds W^T d
 the norms are one pass each way.
 
 Used where the modules' fp32 Linear layers already run as a once-differentiable function (gradients enabled, outside autocast,
-4096 rows or more); every other call keeps the torch layers.
+4096 rows or more) and the arrays are large enough (MIN_ELEMS); every other call keeps the torch layers.
 """
 from __future__ import annotations
 
@@ -22,6 +22,10 @@ from . import _lib, fused
 from .functional import _on_device, _ptr, _stream_ptr
 
 LONG_ROWS = 4096      # rows from which this pays (below, launches are what counts and the torch layers have as few)
+# Elements of a row array from which an eager step waits for the kernels (recorded into a graph it always does): below, the host's
+# enqueueing is what it costs, and a layer's node here enqueues a little more than torch's own nodes.  A block's step at 65,536 x 128
+# rows 3.35 -> 2.94 ms; at 8192 x 64, host-bound, 3.02 ms with torch's nodes and 3.21 ms with these.
+MIN_ELEMS = 6 << 20
 _WIDTHS = (32, 64, 128, 256)
 
 
@@ -47,6 +51,7 @@ def _param_ok(p):
 def _call_ok(x, long_rows):
     return (torch.is_grad_enabled() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype is torch.float32
             and x.shape[-1] in _WIDTHS and x.numel() // x.shape[-1] >= long_rows and not torch.is_autocast_enabled()
+            and (x.numel() >= MIN_ELEMS or torch.cuda.is_current_stream_capturing())
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 

@@ -14,6 +14,11 @@ from flare_py_amd.modules import ResidualMLP
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def every_size(monkeypatch):
+    monkeypatch.setattr(rows, "MIN_ELEMS", 0)
+
+
 def rel(a, b):
     return float((a.double() - b).norm() / (b.norm() + 1e-300))
 
@@ -45,7 +50,7 @@ def test_residual_mlp(dev, monkeypatch, C, T, layers, act, ends):
     got = grads(m, x, list(m.parameters()), gy)
     monkeypatch.setattr(modules, "_LONG_ROWS", 1 << 62)
     t32 = grads(m, x, list(m.parameters()), gy)
-    monkeypatch.undo()
+    monkeypatch.setattr(modules, "_LONG_ROWS", rows.LONG_ROWS)
     hold(got, t32, ref)
     again = grads(m, x, list(m.parameters()), gy)
     assert all(torch.equal(a, b) for a, b in zip(got, again))
@@ -111,3 +116,10 @@ def test_block_against_torch_layers(dev, monkeypatch, lra):
     t32 = grads(run, x, list(m.parameters()), gy)
     for a, b in zip(got, t32):
         assert rel(a, b.double()) <= 1e-5
+
+
+def test_small_arrays_keep_the_torch_layers_outside_a_capture(dev, monkeypatch):
+    monkeypatch.undo()
+    m = ResidualMLP(64, 64, 64, num_layers=1, input_residual=True, output_residual=True).to(dev)
+    assert rows.chain_info(m, torch.randn(8192, 64, device=dev)) is None
+    assert rows.chain_info(m, torch.empty(rows.MIN_ELEMS // 64, 64, device=dev)) is not None
