@@ -297,6 +297,16 @@ def _few(T, Cdim, L):
     return (T + 15) // 16 if 0 < T <= _FEW_TOKENS[Cdim] and L <= _BWD_MAX_LAYERS[Cdim] else 0
 
 
+def drop_operands(mod):
+    """Forget the packed weights kept for mod, and for the chain between its narrow ends: that chain's copies live on an object that
+    is no submodule, and a walk over module.modules() alone passes them by."""
+    sub = mod.__dict__.get("_flare_subchain")
+    for m in (mod, None if sub is None else sub[0]):
+        if m is not None:
+            for name in ("_flare_packed", "_flare_packed_train", "_flare_packed_few"):
+                m.__dict__.pop(name, None)
+
+
 def _packed_few(mod, layers, cd, train):
     """(tiled w, fp32 biases, tiled transposes or None) of a chain for the few-token launches, cached on the module; None where
     the packing launch cannot read the parameters.  A pair passes the layers of both stacks and the first stack's module."""

@@ -33,6 +33,8 @@ import contextlib
 
 import torch
 
+from . import fused
+
 __all__ = ["GraphedTrainStep"]
 
 
@@ -76,8 +78,8 @@ class GraphedTrainStep:
     def _drop_operand_caches(self):
         """Forget the packed weights the warm-up left on the modules, so that the captured step packs them itself."""
         for m in self.module.modules():
-            for name in ("_flare_packed", "_flare_packed_train", "_flare_packed_few", "_q_cache"):
-                m.__dict__.pop(name, None)
+            fused.drop_operands(m)
+            m.__dict__.pop("_q_cache", None)
 
     def _capture(self, inputs):
         self._check()

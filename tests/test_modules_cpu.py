@@ -208,3 +208,36 @@ def test_linear_with_sliced_weight_gradient_equals_linear():
     # the dispatcher only takes it in training, on a GPU, outside autocast, over many rows
     lin = torch.nn.Linear(8, 8)
     assert modules._lin(lin, torch.randn(5000, 8)).grad_fn.name() != "_LinearLongRowsBackward"
+
+
+def test_a_captured_step_packs_the_chain_between_narrow_ends_itself(monkeypatch):
+    """Dropping the packed weights reaches those of in_proj / out_proj, whose C x C layers are packed on an object of their own:
+    kept, a captured step would record no packing launch and replay old weights."""
+    from flare_py_amd import fused, train_graph
+
+    packs = []
+
+    def launch(Cdim, cd, tiles, dev, images, tiled=False):
+        packs.append(len(tiles))
+        w = torch.zeros(len(tiles), Cdim, Cdim, dtype=cd)
+        return w, torch.zeros(len(tiles), Cdim), w, w
+
+    monkeypatch.setattr(fused, "_pack_launch", launch)
+    monkeypatch.setattr(fused, "_readable", lambda *ts: True)
+    m = FLAREModel(**KW)
+    stacks = [fused._train_subchain(m.in_proj), fused._train_subchain(m.out_proj[1]), m.blocks[0].mlp]
+    step = train_graph.GraphedTrainStep(m, None)
+
+    def pack_all():
+        packs.clear()
+        for mod in stacks:
+            layers = fused._layers_of(mod)[0]
+            fused._packed(mod, layers, torch.bfloat16)
+            fused._packed_train(mod, layers, torch.bfloat16)
+            fused._packed_few(mod, layers, torch.bfloat16, True)
+        return len(packs)
+
+    assert all(mod is not None for mod in stacks)
+    assert pack_all() == 9 and pack_all() == 0       # packed once, then kept
+    step._drop_operand_caches()
+    assert pack_all() == 9

@@ -65,6 +65,25 @@ def test_replays_equal_eager_steps_across_parameter_updates(dev, kind, ac):
     assert len(step._graphs) == 1
 
 
+@pytest.mark.parametrize("N", [600, 9000])          # the few-token launches and the many-token ones
+def test_replays_of_a_whole_model_equal_eager_steps_across_parameter_updates(dev, N):
+    """The lift and the head have a narrow end each: the square layers between are packed apart from the other stacks."""
+    torch.manual_seed(14)
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=2, num_heads=4, num_latents=32).to(dev).train()
+    params = list(m.parameters())
+    opt = torch.optim.SGD(params, lr=5e-2)
+    step = F.GraphedTrainStep(m, _mse, autocast_dtype=torch.bfloat16)
+    for it in range(4):
+        x, t = torch.randn(2, N, 3, device=dev), torch.randn(2, N, 1, device=dev)
+        loss_e, grads_e = _eager(m, (), x, t, torch.bfloat16)
+        loss_g = step(x, t).clone()
+        assert torch.equal(loss_g, loss_e), it
+        for (n, p), ge in zip(m.named_parameters(), grads_e):
+            assert torch.equal(p.grad, ge), (n, it)
+        opt.step()
+    assert len(step._graphs) == 1
+
+
 def test_new_shapes_and_replaced_parameters_are_captured_again(dev):
     torch.manual_seed(12)
     blk = _lra_block(dev)
