@@ -76,7 +76,9 @@ class GraphedTrainStep:
         return loss
 
     def _drop_operand_caches(self):
-        """Forget the packed weights the warm-up left on the modules, so that the captured step packs them itself."""
+        """Forget the packed weights the warm-up left on the modules, so that the captured step packs them itself; likewise the
+        16-bit copies of parameters that torch keeps while a caller's own autocast region is open around the call."""
+        torch.clear_autocast_cache()
         for m in self.module.modules():
             fused.drop_operands(m)
             m.__dict__.pop("_q_cache", None)

@@ -241,3 +241,20 @@ def test_a_captured_step_packs_the_chain_between_narrow_ends_itself(monkeypatch)
     assert pack_all() == 9 and pack_all() == 0       # packed once, then kept
     step._drop_operand_caches()
     assert pack_all() == 9
+
+
+def test_a_captured_step_casts_the_parameters_itself_inside_a_callers_autocast():
+    """torch keeps its casts of parameters until the outermost autocast region ends, whatever happens to the parameters."""
+    from flare_py_amd import train_graph
+
+    lin = torch.nn.Linear(4, 4)
+    step = train_graph.GraphedTrainStep(lin, None)
+    x = torch.randn(2, 4)
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        with torch.autocast("cpu", dtype=torch.bfloat16):
+            lin(x)
+        with torch.no_grad():
+            lin.weight.mul_(2.0)
+        step._drop_operand_caches()
+        y = lin(x)
+    assert torch.equal(y, torch.nn.functional.linear(x.bfloat16(), lin.weight.bfloat16(), lin.bias.bfloat16()))

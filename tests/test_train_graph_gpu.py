@@ -84,6 +84,21 @@ def test_replays_of_a_whole_model_equal_eager_steps_across_parameter_updates(dev
     assert len(step._graphs) == 1
 
 
+def test_a_step_captured_inside_the_callers_autocast_sees_parameter_updates(dev):
+    torch.manual_seed(15)
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev).train()
+    opt = torch.optim.SGD(m.parameters(), lr=5e-2)
+    step = F.GraphedTrainStep(m, _mse, autocast_dtype=torch.bfloat16)
+    for it in range(3):
+        x, t = torch.randn(2, 600, 3, device=dev), torch.randn(2, 600, 1, device=dev)
+        loss_e, grads_e = _eager(m, (), x, t, torch.bfloat16)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss_g = step(x, t).clone()
+        assert torch.equal(loss_g, loss_e), it
+        assert all(torch.equal(p.grad, g) for p, g in zip(m.parameters(), grads_e)), it
+        opt.step()
+
+
 def test_new_shapes_and_replaced_parameters_are_captured_again(dev):
     torch.manual_seed(12)
     blk = _lra_block(dev)
