@@ -938,9 +938,10 @@ flare::CausalLinearArgs cl_args(const FlareCausalLinearDesc* d, const CausalLine
 hipError_t cl_run(const FlareCausalLinearDesc* d, const CausalLinearPlan& p, int Dk, int Dv, const ClOp& q, const ClOp& k, const ClOp& v,
                   const ClOp& y, void* states, bool rev, hipStream_t st)
 {
-    const flare::CausalLinearArgs a = cl_args(d, p, Dk, Dv, q, k, v, y, states, rev);
-    if (cl_mfma(d, Dk, Dv) && cl_aligned(q) && cl_aligned(k) && cl_aligned(v) && cl_aligned(y))
-        return flare::launch_causal_linear_mfma(a, d->dtype, 3, st);
+    flare::CausalLinearArgs a = cl_args(d, p, Dk, Dv, q, k, v, y, states, rev);
+    const bool mfma = cl_mfma(d, Dk, Dv) && cl_aligned(q) && cl_aligned(k) && cl_aligned(v);
+    if (mfma && cl_aligned(y)) return flare::launch_causal_linear_mfma(a, d->dtype, 3, st);
+    a.keep_slots = mfma && Dk == Dv;      // a backward of these q, k, v takes the slots for the matrix-core kernels'
     return flare::launch_causal_linear(a, d->dtype, st);
 }
 

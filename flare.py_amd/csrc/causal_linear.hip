@@ -10,6 +10,10 @@
 // owns one output column j and a fixed set of rows, for both the output (rows = tokens) and the
 // state update (rows = key features), so the running state of a segment is read-modify-written
 // in place in the workspace by the thread that owns each element.
+//
+// A backward may start from the segment states its forward left (flare_causal_linear_bwd).  It can tell from q, k and v alone
+// that the matrix-core kernels took the forward, which only read their slots, but not where y was: for an output off the 16-byte
+// grid behind such inputs the slots are put back as they were (KEEP; 64 more registers, 18 % slower at Dk = Dv = 128, so only there).
 #include "common.hpp"
 
 namespace flare {
@@ -32,7 +36,7 @@ __device__ __forceinline__ void load_rows(float* dst, int dst_stride, const T* s
 
 // DVP = Dv rounded up to a power of two in 4..128.  Thread tid owns column j = tid % DVP and the
 // rows tg, tg + G, tg + 2G, ... with tg = tid / DVP, G = 256 / DVP.
-template <typename T, int DVP, bool STATE_ONLY>
+template <typename T, int DVP, bool STATE_ONLY, bool KEEP = false>
 __global__ __launch_bounds__(256) void causal_linear_kernel(CausalLinearArgs a)
 {
     constexpr int G = 256 / DVP;
@@ -58,6 +62,13 @@ __global__ __launch_bounds__(256) void causal_linear_kernel(CausalLinearArgs a)
     float sacc[RS];
 #pragma unroll
     for (int r = 0; r < RS; ++r) sacc[r] = 0.f;
+    if (KEEP && col) {
+#pragma unroll
+        for (int r = 0; r < RS; ++r) {
+            const int i = tg + r * G;
+            if (i < Dk) sacc[r] = S[(int64_t)i * Dv + j];
+        }
+    }
 
     for (int n0 = n_lo; n0 < n_hi; n0 += kTile) {
         __syncthreads();   // the previous tile's LDS reads are done
@@ -126,7 +137,7 @@ __global__ __launch_bounds__(256) void causal_linear_kernel(CausalLinearArgs a)
             }
         }
     }
-    if constexpr (STATE_ONLY) {
+    if constexpr (STATE_ONLY || KEEP) {      // every read of S is behind the last tile's barrier
         if (col) {
 #pragma unroll
             for (int r = 0; r < RS; ++r) {
@@ -171,6 +182,7 @@ hipError_t launch_dvp(const CausalLinearArgs& a, hipStream_t st)
     const int BH = a.B * a.H;
     auto state_k = causal_linear_kernel<T, DVP, true>;
     auto out_k = causal_linear_kernel<T, DVP, false>;
+    if constexpr (DVP >= 64) { if (a.keep_slots) out_k = causal_linear_kernel<T, DVP, false, true>; }
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(state_k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(out_k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -256,6 +256,7 @@ struct CausalLinearArgs {
     int B, H, N, Dk, Dv;
     int n_segs, seg_len;   // seg_len is a multiple of the 64-token tile
     float inv_n;           // 1 / N
+    int keep_slots;        // 1: the FMA kernels leave the slots as the prefix made them (Dv >= 64)
     int slot_t;            // 1: the slots hold the transposed states [Dv][Dk] (outputs only; matrix-core kernels)
     int64_t qs[3], ks[3], vs[3], ys[3];   // a token stride may be negative: the token axis reversed
 };

@@ -334,7 +334,7 @@ int flare_causal_linear_fwd(const FlareCausalLinearDesc* desc, const void* q, co
 /* Gradients of flare_causal_linear_fwd: dq, dk [B,H,N,Dk] and dv [B,H,N,Dv] contiguous, any of them NULL.  desc and q, k, v
  * as in the forward (y_stride is only checked), gy [B,H,N,Dv] with its own strides; the workspace is of
  * flare_causal_linear_workspace_bytes(desc) bytes.  fwd_workspace: the workspace the forward of the same descriptor and
- * operands was given, as it left it (Dk == Dv: dq then needs no state pass of its own), or NULL. */
+ * operands was given, as it left it (Dk == Dv: dq then needs no state pass of its own; whatever alignment y had), or NULL. */
 int flare_causal_linear_bwd(const FlareCausalLinearDesc* desc, const void* q, const void* k, const void* v, const void* gy,
                             const int64_t gy_stride[3], const void* fwd_workspace, void* dq, void* dk, void* dv,
                             void* workspace, size_t workspace_bytes, void* stream);

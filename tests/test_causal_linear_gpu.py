@@ -5,10 +5,13 @@ tests/test_oracle.py by the closed form tril(QK^T)V/N.  Tolerances: 1e-5 (fp32) 
 relative L2 on the same rounded inputs (the reference's own self-test uses allclose 1e-5 / 1e-3,
 causal_linear.py:455-457).
 """
+import ctypes as C
+
 import pytest
 import torch
 
 import flare_py_amd as F
+from flare_py_amd import _lib
 from oracle import flare_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -183,3 +186,39 @@ def test_gradients_of_square_heads(dev, N, D, dtype):
         xi = [t.detach().requires_grad_(j == i) for j, t in enumerate(xd)]
         (one,) = torch.autograd.grad(F.CausalLinear.apply(*(heads(t) for t in xi)), [xi[i]], heads(gy.to(dev)))
         assert O.rel_l2(one, want[i]) <= tol
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16), (64, torch.float32)])
+@pytest.mark.parametrize("how", ["aligned", "offset", "row stride"])
+def test_backward_takes_the_forwards_workspace_from_either_kernel(dev, D, dtype, how):
+    """The C interface: an output off the 16-byte grid sends the forward to the FMA kernels, its backward still starts dq from the
+    segment states it finds in the forward's workspace.  Segments of several tiles; tolerances as above."""
+    B, H, N = 1, 2, 1000
+    g = torch.Generator().manual_seed(D)
+    q, k, v, gy = (torch.randn(B, H, N, D, generator=g).to(dtype) for _ in range(4))
+    qd, kd, vd, gd = (t.to(dev) for t in (q, k, v, gy))
+    stride = D + (1 if how == "row stride" else 0)
+    flat = torch.empty(B * H * N * stride + 16, dtype=dtype, device=dev)
+    y = flat[1 if how == "offset" else 0:].as_strided((B, H, N, D), (H * N * stride, N * stride, stride, 1))
+    lib = _lib.load()
+    d = _lib.FlareCausalLinearDesc()
+    d.B, d.H, d.N, d.Dk, d.Dv, d.n_segs = B, H, N, D, D, 3
+    d.dtype = {torch.float32: _lib.DT_F32, torch.bfloat16: _lib.DT_BF16, torch.float16: _lib.DT_F16}[dtype]
+    i3 = lambda t: _lib.I3(*t.stride()[:3])
+    d.q_stride, d.k_stride, d.v_stride, d.y_stride = i3(qd), i3(kd), i3(vd), i3(y)
+    need = C.c_size_t(0)
+    _lib.check(lib.flare_causal_linear_workspace_bytes(C.byref(d), C.byref(need)), "workspace")
+    fwd, ws = (torch.empty(need.value, dtype=torch.uint8, device=dev) for _ in range(2))
+    p = lambda t: C.c_void_p(t.data_ptr())
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib.flare_causal_linear_fwd(C.byref(d), p(qd), p(kd), p(vd), p(y), p(fwd), need.value, st), "forward")
+    grads = [torch.empty_like(t) for t in (qd, kd, vd)]
+    _lib.check(lib.flare_causal_linear_bwd(C.byref(d), p(qd), p(kd), p(vd), p(gd), i3(gd), p(fwd), *(p(t) for t in grads), p(ws),
+                                           need.value, st), "backward")
+    ref = [t.double().requires_grad_(True) for t in (q, k, v)]
+    yr = O.causal_linear_closed_form(*ref)
+    want = torch.autograd.grad(yr, ref, gy.double())
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -6, torch.float16: 2.0 ** -9}[dtype]
+    assert O.rel_l2(y, yr.detach()) <= tol
+    for name, a, b in zip(("dq", "dk", "dv"), grads, want):
+        assert O.rel_l2(a, b) <= tol, name
