@@ -1150,6 +1150,9 @@ class _CausalLinearFn(torch.autograd.Function):
     def forward(ctx, q, k, v):
         q, k, v = _rows_last_contig(q), _rows_last_contig(k), _rows_last_contig(v)
         y, ws = _causal_linear_forward(q, k, v)
+        # rows off the 16-byte grid took the FMA kernels, which leave other states behind: the backward, which may get these tensors
+        # back on another grid (a saved-tensor hook), must not start from them
+        ctx.states = not any(t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]) for t in (q, k, v))
         ctx.save_for_backward(q, k, v, ws)
         return y
 
@@ -1161,6 +1164,7 @@ class _CausalLinearFn(torch.autograd.Function):
         #   dk_tau = (1/N) sum_{t >= tau} <v_tau, gy_t> q_t
         #   dv_tau = (1/N) sum_{t >= tau} <k_tau, q_t> gy_t
         q, k, v, fwd_ws = ctx.saved_tensors
+        q, k, v = _rows_last_contig(q), _rows_last_contig(k), _rows_last_contig(v)
         gy = gy.to(q.dtype)
         if gy.stride(-1) != 1 or any(s % 8 for s in gy.stride()[:3]) or gy.data_ptr() % 16 or gy.stride(2) < gy.shape[-1]:
             gy = gy.contiguous()
@@ -1169,8 +1173,8 @@ class _CausalLinearFn(torch.autograd.Function):
         ws = torch.empty_like(fwd_ws)
         d = _causal_linear_desc(q, k, v, v)
         with _on_device(q.device):
-            rc = _lib.load().flare_causal_linear_bwd(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(gy), _s3(gy), _ptr(fwd_ws),
-                                                     *(_ptr(t) for t in grads), _ptr(ws), ws.numel(),
+            rc = _lib.load().flare_causal_linear_bwd(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(gy), _s3(gy),
+                                                     _ptr(fwd_ws) if ctx.states else None, *(_ptr(t) for t in grads), _ptr(ws), ws.numel(),
                                                      C.c_void_p(_stream_ptr(q.device)))
         _lib.check(rc, "flare_causal_linear_bwd")
         return tuple(grads)

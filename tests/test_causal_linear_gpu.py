@@ -222,3 +222,24 @@ def test_backward_takes_the_forwards_workspace_from_either_kernel(dev, D, dtype,
     assert O.rel_l2(y, yr.detach()) <= tol
     for name, a, b in zip(("dq", "dk", "dv"), grads, want):
         assert O.rel_l2(a, b) <= tol, name
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (64, torch.float32)])
+def test_gradients_when_saved_tensors_come_back_on_another_grid(dev, D, dtype):
+    """Rows off the 16-byte grid send the forward to the FMA kernels; a saved-tensor hook (offloading, say) may hand the backward
+    aligned copies of them, or copies in another memory order.  As many heads as it takes for segments of several tiles."""
+    B, H, N = 64, 16, 200
+    g = torch.Generator().manual_seed(D)
+    wide = torch.randn(3, B, H, N, D + 8, generator=g).to(dtype)
+    gy = torch.randn(B, H, N, D, generator=g).to(dtype)
+    xr = [t[..., 1:D + 1].double().requires_grad_(True) for t in wide]
+    want = torch.autograd.grad(O.causal_linear_closed_form(*xr), xr, gy.double())
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -6}[dtype]
+    for unpack in (torch.clone, lambda t: t.transpose(0, -1).contiguous().transpose(0, -1)):
+        xd = [t.to(dev)[..., 1:D + 1].requires_grad_(True) for t in wide]
+        assert xd[0].data_ptr() % 16 != 0
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = F.CausalLinear.apply(*xd)
+        got = torch.autograd.grad(y, xd, gy.to(dev))
+        for a, b in zip(got, want):
+            assert O.rel_l2(a, b) <= tol
