@@ -1267,7 +1267,9 @@ class _TripleFn(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dstate, dout):
-        q1, q2, k1, k2, v, state = ctx.saved_tensors
+        *rows, state = ctx.saved_tensors
+        q1, q2, k1, k2, v = (_rows_last_contig(t) for t in rows)      # a saved-tensor hook may change the memory order
+        state = state.contiguous()
         N = q1.shape[2]
         dt = q1.dtype
         if dout is None:

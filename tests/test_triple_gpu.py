@@ -238,3 +238,19 @@ def test_head_dim_32_forward_and_backward(dev, N, dtype, tol, strided):
         want = torch.autograd.grad([r[2] for r in roots], rins, [r[3] for r in roots], retain_graph=True)
         for a, b in zip(got, want):
             assert O.rel_l2(a, b) <= 1.5 * tol
+
+
+@pytest.mark.parametrize("D,dtype,tol", [(32, torch.float16, 2.0 ** -9), (16, torch.bfloat16, 2.0 ** -6), (24, torch.float32, 1e-5)])
+def test_gradients_when_saved_tensors_come_back_in_another_memory_order(dev, D, dtype, tol):
+    """A saved-tensor hook owes the backward the values, not the strides."""
+    g = torch.Generator().manual_seed(D)
+    ins = [(torch.rand(1, 2, 200, D, generator=g) + 0.25).to(dtype) for _ in range(5)]
+    go = (torch.rand(1, 2, 200, D, generator=g) + 0.25).to(dtype)
+    dins = [t.to(dev).requires_grad_(True) for t in ins]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.transpose(-1, -2).contiguous().transpose(-1, -2)):
+        _, out = F.TripleAttentionFunction.apply(*dins)
+    got = torch.autograd.grad(out, dins, go.to(dev))
+    rins = [t.double().requires_grad_(True) for t in ins]
+    want = torch.autograd.grad(O.triple_einsum(*rins, dtype=torch.float64)[1], rins, go.double())
+    for a, b in zip(got, want):
+        assert O.rel_l2(a, b) <= tol
