@@ -112,7 +112,8 @@ class _LinearLongRowsPass(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dy):
-        s, w, t = ctx.saved_tensors
+        s, w, t = ctx.saved_tensors                          # through saved-tensor hooks in any memory order
+        s, t = _rows(s, s.shape[-1]), None if t is None else _rows(t, t.shape[-1])
         act, T, width, dev = ctx.act, s.shape[0], s.shape[1], s.device
         _, _, need_x, need_w, need_b, need_res = ctx.needs_input_grad
         ds = _rows(dy, width)
@@ -162,6 +163,7 @@ class _NormFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, dy):
         x2, stats, gamma = ctx.saved_tensors
+        x2, stats = _rows(x2, x2.shape[-1]), stats.contiguous()
         T, width = x2.shape
         need = ctx.needs_input_grad            # (kind, eps, x, gamma, beta)
         dx = torch.empty_like(x2)

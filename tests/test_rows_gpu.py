@@ -123,3 +123,20 @@ def test_small_arrays_keep_the_torch_layers_outside_a_capture(dev, monkeypatch):
     m = ResidualMLP(64, 64, 64, num_layers=1, input_residual=True, output_residual=True).to(dev)
     assert rows.chain_info(m, torch.randn(8192, 64, device=dev)) is None
     assert rows.chain_info(m, torch.empty(rows.MIN_ELEMS // 64, 64, device=dev)) is not None
+
+
+def test_saved_tensors_may_come_back_in_another_memory_order(dev):
+    """A saved-tensor hook owes the backward the values, not the strides."""
+    torch.manual_seed(2)
+    m, n = ResidualMLP(64, 64, 64, num_layers=1, input_residual=True, output_residual=True).to(dev), nn.LayerNorm(64).to(dev)
+    x = torch.randn(4096, 64, device=dev, requires_grad=True)
+    gy = torch.randn(4096, 64, device=dev)
+    params = [*m.parameters(), *n.parameters()]
+    run = lambda t: m(rows.norm(n, t))
+    want = grads(run, x, params, gy)
+    assert rows.chain_info(m, x) is not None
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.t().contiguous().t() if t.dim() == 2 else t):
+        y = run(x)
+    got = [y.detach(), *torch.autograd.grad(y, [x, *params], gy)]
+    for a, b in zip(got, want):
+        assert rel(a, b.double()) <= 1e-6
