@@ -21,10 +21,12 @@ from torch.autograd.function import once_differentiable
 from . import _lib, fused
 from .functional import _on_device, _ptr, _stream_ptr
 
-LONG_ROWS = 4096      # rows from which this pays (below, launches are what counts and the torch layers have as few)
-# Elements of a row array from which an eager step waits for the kernels (recorded into a graph it always does): below, the host's
-# enqueueing is what it costs, and a layer's node here enqueues a little more than torch's own nodes.  A block's step at 65,536 x 128
-# rows 3.35 -> 2.94 ms; at 8192 x 64, host-bound, 3.02 ms with torch's nodes and 3.21 ms with these.
+LONG_ROWS = 4096      # rows from which the modules' fp32 Linear layers slice their weight gradient (below, one product is as fast)
+# Elements of a row array from which a step waits for the kernels: below, the host's enqueueing is what it costs, and a layer's node
+# here enqueues a little more than torch's own nodes.  A sequence block's step, torch's nodes / these, us: 64 channels, 8192 rows
+# 2755 / 2831, 65,536 rows (4 Mi) 2800 / 2846, 98,304 rows (6 Mi) 3100 / 2839, 131,072 rows 3850 / 3072; 128 channels, 32,768 rows
+# (4 Mi) 2647 / 2700, 49,152 rows (6 Mi) 3214 / 2745, 65,536 rows 3180 / 2754.  A step recorded into a graph has no host to wait for,
+# but follows the same rule: its replays give the results of the eager step bit for bit.
 MIN_ELEMS = 6 << 20
 _WIDTHS = (32, 64, 128, 256)
 
@@ -51,7 +53,7 @@ def _param_ok(p):
 def _call_ok(x, long_rows):
     return (torch.is_grad_enabled() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype is torch.float32
             and x.shape[-1] in _WIDTHS and x.numel() // x.shape[-1] >= long_rows and not torch.is_autocast_enabled()
-            and (x.numel() >= MIN_ELEMS or torch.cuda.is_current_stream_capturing())
+            and x.numel() >= MIN_ELEMS
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 

@@ -23,7 +23,7 @@ def _eager(blk, extra, x, t, ac):
     params = [p for p in blk.parameters()]
     for p in params:
         p.grad = None
-    with torch.autocast("cuda", dtype=ac):
+    with torch.autocast("cuda", dtype=ac or torch.bfloat16, enabled=ac is not None):
         out = blk(x, *extra)
     loss = _mse(out, t)
     loss.backward()
@@ -82,6 +82,28 @@ def test_replays_of_a_whole_model_equal_eager_steps_across_parameter_updates(dev
             assert torch.equal(p.grad, ge), (n, it)
         opt.step()
     assert len(step._graphs) == 1
+
+
+@pytest.mark.parametrize("kind,B,N", [("pde", 2, 2500), ("lra_masked", 8, 4000), ("pde", 1, 100000)])
+def test_fp32_replays_equal_eager_steps_across_parameter_updates(dev, kind, B, N):
+    """Long row arrays in fp32, on either side of the size from which the HIP row passes take the token-wise layers: the recorded
+    step runs the kernels of the eager one."""
+    torch.manual_seed(16)
+    C = 64
+    blk = modules.FLAREBlock(channel_dim=C, num_heads=4, num_latents=32).to(dev).train() if kind == "pde" else _lra_block(dev)
+    extra = () if kind == "pde" else ((torch.arange(N)[None, :] < torch.arange(B)[:, None] * (N // B) + N // B).to(dev),)
+    opt = torch.optim.SGD(blk.parameters(), lr=5e-2)
+    step = F.GraphedTrainStep(blk, _mse)
+    for it in range(4):
+        x, t = torch.randn(B, N, C, device=dev), torch.randn(B, N, C, device=dev)
+        loss_e, grads_e = _eager(blk, extra, x, t, None)
+        loss_g = step(x, *extra, t).clone()
+        assert torch.equal(loss_g, loss_e), it
+        for (n, p), ge in zip(blk.named_parameters(), grads_e):
+            assert torch.equal(p.grad, ge), (n, it)
+        opt.zero_grad(set_to_none=True)
+        step(x, *extra, t)
+        opt.step()
 
 
 def test_a_step_captured_inside_the_callers_autocast_sees_parameter_updates(dev):
