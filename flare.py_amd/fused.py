@@ -297,6 +297,17 @@ def _few(T, Cdim, L):
     return (T + 15) // 16 if 0 < T <= _FEW_TOKENS[Cdim] and L <= _BWD_MAX_LAYERS[Cdim] else 0
 
 
+def _param_key(layers):
+    """What packed copies of these layers' parameters depend on: an in-place change moves a version, another tensor an address.
+    Read from the layers' own tables where the parameters are there (see _structure_key)."""
+    key = []
+    for l in layers:
+        p = l._parameters
+        w, b = p["weight"] if "weight" in p else l.weight, p["bias"] if "bias" in p else l.bias
+        key.append((w.data_ptr(), w._version) if b is None else (w.data_ptr(), w._version, b.data_ptr(), b._version))
+    return tuple(key)
+
+
 def drop_operands(mod):
     """Forget the packed weights kept for mod, and for the chain between its narrow ends: that chain's copies live on an object that
     is no submodule, and a walk over module.modules() alone passes them by."""
@@ -310,7 +321,7 @@ def drop_operands(mod):
 def _packed_few(mod, layers, cd, train):
     """(tiled w, fp32 biases, tiled transposes or None) of a chain for the few-token launches, cached on the module; None where
     the packing launch cannot read the parameters.  A pair passes the layers of both stacks and the first stack's module."""
-    key = (cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
+    key = (cd, _param_key(layers))
     cache = mod.__dict__.get("_flare_packed_few")
     if cache is not None and cache[0] == key and (cache[3] is not None or not train):
         return cache[1:]
@@ -324,7 +335,7 @@ def _packed_few(mod, layers, cd, train):
 
 def _packed(mod, layers, cd):
     """[L,C,C] weights in the compute dtype and [L,C] fp32 biases, cached on the module."""
-    key = (cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
+    key = (cd, _param_key(layers))
     cache = getattr(mod, "_flare_packed", None)
     if cache is not None and cache[0] == key:
         return cache[1], cache[2]
@@ -344,8 +355,7 @@ def _packed_expand(mod, E, cd):
     """Tiles W1[0:C], W2[:,0:C], W1[C:2C], W2[:,C:2C], ... as [2E,C,C] and bias rows b1[0:C], b2, b1[C:2C], 0, ...
     (the layout FLARE_MLP_EXPAND asks for), cached on the module."""
     f1, f2 = mod.fc1, mod.fc2
-    key = ("expand", cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version)
-                               for l in (f1, f2)))
+    key = ("expand", cd, _param_key((f1, f2)))
     cache = getattr(mod, "_flare_packed", None)
     if cache is not None and cache[0] == key:
         return cache[1], cache[2]
@@ -370,7 +380,7 @@ def _packed_expand(mod, E, cd):
 def _packed_io(mod, layers, cd, Cdim, in_dim, out_dim):
     """Tiles of a stack with a narrow first and/or last layer: (w [L,C,C], b [L,C], w_in [C,4] fp32, b_in [C]),
     the narrow last layer zero-padded to C rows; cached on the module."""
-    key = ("io", cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
+    key = ("io", cd, _param_key(layers))
     cache = getattr(mod, "_flare_packed", None)
     if cache is not None and cache[0] == key:
         return cache[1:]
@@ -625,7 +635,7 @@ def mlp_weight_images(w):
 def _packed_train(mod, layers, cd):
     """(w [L,C,C] for the forward launch, images of the weights and of their transposes for the backward, fp32 biases
     [L,C]), cached on the module until a parameter changes."""
-    key = ("train", cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version) for l in layers))
+    key = ("train", cd, _param_key(layers))
     cache = mod.__dict__.get("_flare_packed_train")
     if cache is not None and cache[0] == key:
         return cache[1:]
@@ -642,8 +652,7 @@ def _packed_train(mod, layers, cd):
 def _packed_train_expand(mod, E, cd):
     """The same for the expanding two-layer MLP: its 2 E tiles (see _packed_expand) and their transposes as images."""
     f1, f2 = mod.fc1, mod.fc2
-    key = ("train-expand", cd, tuple((l.weight.data_ptr(), l.weight._version, None if l.bias is None else l.bias._version)
-                                     for l in (f1, f2)))
+    key = ("train-expand", cd, _param_key((f1, f2)))
     cache = mod.__dict__.get("_flare_packed_train")
     if cache is not None and cache[0] == key:
         return cache[1:]

@@ -258,3 +258,38 @@ def test_a_captured_step_casts_the_parameters_itself_inside_a_callers_autocast()
         step._drop_operand_caches()
         y = lin(x)
     assert torch.equal(y, torch.nn.functional.linear(x.bfloat16(), lin.weight.bfloat16(), lin.bias.bfloat16()))
+
+
+def test_packed_copies_follow_a_bias_that_is_replaced_alone(monkeypatch):
+    """A new bias tensor starts at the version count of the old one: its address has to tell them apart, in every packed copy."""
+    from flare_py_amd import fused
+
+    packs = []
+
+    def launch(Cdim, cd, tiles, dev, images, tiled=False):
+        packs.append([float(t[4].detach().sum()) for t in tiles if t[4] is not None])
+        w = torch.zeros(len(tiles), Cdim, Cdim, dtype=cd)
+        return w, torch.zeros(len(tiles), Cdim), w, w
+
+    monkeypatch.setattr(fused, "_pack_launch", launch)
+    monkeypatch.setattr(fused, "_readable", lambda *ts: True)
+    a, b = (ResidualMLP(32, 32, 32, num_layers=0, input_residual=True, output_residual=True) for _ in range(2))
+    wide, lift = ResidualMLP(32, 64, 32, num_layers=0), ResidualMLP(3, 32, 32, num_layers=0)
+    la, lb = fused._layers_of(a)[0], fused._layers_of(b)[0]
+    cd = torch.bfloat16
+    calls = {"chain": lambda: fused._packed(a, la, cd), "training": lambda: fused._packed_train(a, la, cd),
+             "few tokens": lambda: fused._packed_few(a, la, cd, True), "pair": lambda: fused._packed_few(a, la + lb, cd, True),
+             "expanding": lambda: fused._packed_expand(wide, 2, cd), "expanding, training": lambda: fused._packed_train_expand(wide, 2, cd),
+             "narrow": lambda: fused._packed_io(lift, fused._layers_of(lift)[0], cd, 32, 3, 0)}
+    for what, call in calls.items():
+        owner = {"pair": b, "narrow": lift}.get(what, wide if what.startswith("expanding") else a)
+        call()
+        packs.clear()
+        call()
+        assert not packs, what
+        owner.fc2.bias = torch.nn.Parameter(torch.full((32,), 5.0))
+        call()
+        assert len(packs) == 1 and 160.0 in packs[0], what
+        owner.fc2.bias.data = torch.full((32,), 7.0)
+        call()
+        assert len(packs) == 2 and 224.0 in packs[1], what
