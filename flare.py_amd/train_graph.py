@@ -18,8 +18,8 @@ What the caller has to know:
   its gradient in `.grad` the same way.
 * The 16-bit operand copies of the weights are packed inside the captured step from the parameters' own storage, so
   an optimizer that updates the parameters in place between calls is seen by the next replay.  Replacing a
-  parameter tensor (`load_state_dict(assign=True)`, `.to()`, a new `nn.Parameter`) is detected by address and leads
-  to a new capture.
+  parameter tensor (`load_state_dict(assign=True)`, `.to()`, a new `nn.Parameter`), a frozen one too, is detected by
+  address and leads to a new capture, and so does freezing or unfreezing one.
 * Attention dropout of the sequence-benchmark modules draws its seed on the host, where a replay would repeat it:
   modules with `attn_drop > 0` in training mode are refused.  torch's own dropout is capture-safe.
 * Capture fails when an autograd graph of an earlier eager step on another stream is still alive (a kept loss tensor
@@ -55,13 +55,23 @@ class GraphedTrainStep:
             return contextlib.nullcontext()
         return torch.autocast("cuda", dtype=self.autocast_dtype)
 
-    def _params(self):
-        return [p for p in self.module.parameters() if p.requires_grad]
+    def _parameters(self, mods):
+        """(parameters that ask for gradients; what the recorded step depends on: where every parameter lies, a frozen one too, and
+        which get gradients).  One walk: this is the host's share of a replay."""
+        params, key, seen = [], [], set()
+        for m in mods:
+            for t in m._parameters.values():
+                if t is not None and id(t) not in seen:
+                    seen.add(id(t))
+                    key.append((t.data_ptr(), t.requires_grad))
+                    if t.requires_grad:
+                        params.append(t)
+        return params, key
 
-    def _check(self):
+    def _check(self, mods):
         if not self.module.training:
             raise RuntimeError("GraphedTrainStep captures training steps: call module.train() first")
-        for m in self.module.modules():
+        for m in mods:
             if float(getattr(m, "attn_drop_p", 0.0) or 0.0) > 0.0:
                 raise RuntimeError("GraphedTrainStep: attention dropout draws its seed on the host, a replay would repeat "
                                    "the same keep mask every step; train this module eagerly or with attn_drop = 0")
@@ -83,9 +93,7 @@ class GraphedTrainStep:
             fused.drop_operands(m)
             m.__dict__.pop("_q_cache", None)
 
-    def _capture(self, inputs):
-        self._check()
-        params = self._params()
+    def _capture(self, inputs, params):
         dev = inputs[0].device
         static_inputs = [t.detach().clone().requires_grad_(t.requires_grad) if isinstance(t, torch.Tensor) else t for t in inputs]
         side = torch.cuda.Stream(device=dev)
@@ -100,7 +108,7 @@ class GraphedTrainStep:
             loss = self._one_step(static_inputs, params).detach()   # no reference to the recorded autograd graph
         grads = [p.grad for p in params]
         self._drop_operand_caches()               # those of the capture live in the graph's pool: eager calls repack
-        return graph, static_inputs, loss, grads, tuple(p.data_ptr() for p in params)
+        return graph, static_inputs, loss, grads
 
     def __call__(self, *inputs):
         """inputs = the module's positional arguments followed by the target handed to loss_fn(output, target)."""
@@ -111,13 +119,13 @@ class GraphedTrainStep:
             raise ValueError("GraphedTrainStep replays HIP graphs: the tensors must live on a HIP device")
         key = tuple((tuple(t.shape), t.dtype, t.device.index) if isinstance(t, torch.Tensor) else ("const", t) for t in inputs)
         entry = self._graphs.get(key)
-        params = self._params()
-        if entry is not None and entry[4] != tuple(p.data_ptr() for p in params):
-            entry = None                          # a parameter tensor was replaced: the graph reads the old one
+        mods = list(self.module.modules())
+        self._check(mods)
+        params, reads = self._parameters(mods)
+        if entry is not None and entry[4] != reads:
+            entry = None                          # a parameter tensor was replaced (the graph reads the old one), frozen or unfrozen
         if entry is None:
-            entry = self._graphs[key] = self._capture(inputs)
-        else:
-            self._check()
+            entry = self._graphs[key] = (*self._capture(inputs, params), reads)
         graph, static_inputs, loss, grads, _ = entry
         with torch.no_grad():
             for s, t in zip(static_inputs, inputs):

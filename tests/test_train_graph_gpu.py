@@ -143,6 +143,31 @@ def test_new_shapes_and_replaced_parameters_are_captured_again(dev):
     assert not step._graphs
 
 
+def test_frozen_parameters_that_are_replaced_or_unfrozen_are_captured_again(dev):
+    torch.manual_seed(17)
+    blk = _lra_block(dev)
+    lin = blk.att.out_proj
+    lin.weight.requires_grad_(False)
+    step = F.GraphedTrainStep(blk, _mse, autocast_dtype=torch.bfloat16)
+    x, t = torch.randn(2, 256, 64, device=dev), torch.randn(2, 256, 64, device=dev)
+
+    def eager():
+        blk.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss = _mse(blk(x, None), t)
+        loss.backward()
+        return loss.detach().clone(), [None if p.grad is None else p.grad.clone() for p in blk.parameters()]
+
+    for change in (lambda: None, lambda: setattr(lin, "weight", torch.nn.Parameter(lin.weight.detach() * 0.5, requires_grad=False)),
+                   lambda: lin.weight.requires_grad_(True)):
+        change()
+        loss_e, grads_e = eager()
+        blk.zero_grad(set_to_none=True)
+        assert torch.equal(step(x, None, t), loss_e)
+        for p, g in zip(blk.parameters(), grads_e):
+            assert (p.grad is None) == (g is None) and (g is None or torch.equal(p.grad, g))
+
+
 def test_input_gradient_is_handed_to_the_callers_tensor(dev):
     torch.manual_seed(13)
     blk = _lra_block(dev)
