@@ -16,6 +16,7 @@ import ctypes as C
 
 import torch
 from torch import nn
+from torch.nn.modules import module as _module
 from torch.autograd.function import once_differentiable
 
 from . import _lib, fused
@@ -41,8 +42,9 @@ def weight_grad(dy2, x2):
 
 
 def _plain(m):
-    """No hooks: the module's own forward is all that calling it does."""
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    """No hooks, its own or global ones, and no forward replaced on the instance: its class's forward is all that calling it does."""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
+                or _module._has_any_global_hook())
 
 
 def _param_ok(p):

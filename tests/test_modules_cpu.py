@@ -293,3 +293,22 @@ def test_packed_copies_follow_a_bias_that_is_replaced_alone(monkeypatch):
         owner.fc2.bias.data = torch.full((32,), 7.0)
         call()
         assert len(packs) == 2 and 224.0 in packs[1], what
+
+
+def test_row_passes_leave_modules_alone_whose_call_does_more_than_their_class():
+    from flare_py_amd import rows
+
+    act = torch.nn.GELU(approximate="tanh")
+    assert rows._plain(act)
+    inner = act.forward
+    act.forward = lambda x: inner(x)                  # as offloading and wrapping libraries do
+    assert not rows._plain(act)
+    del act.forward
+    assert rows._plain(act)
+    reg = torch.nn.modules.module
+    for hook in (lambda: reg.register_module_forward_hook(lambda *a: None), lambda: reg.register_module_forward_pre_hook(lambda *a: None),
+                 lambda: reg.register_module_full_backward_hook(lambda *a: None)):
+        h = hook()
+        assert not rows._plain(act)
+        h.remove()
+        assert rows._plain(act)

@@ -140,3 +140,29 @@ def test_saved_tensors_may_come_back_in_another_memory_order(dev):
     got = [y.detach(), *torch.autograd.grad(y, [x, *params], gy)]
     for a, b in zip(got, want):
         assert rel(a, b.double()) <= 1e-6
+
+
+@pytest.mark.parametrize("lra", [False, True])
+@pytest.mark.parametrize("how", ["forward replaced", "global hook"])
+def test_replaced_forwards_and_global_hooks_are_called(dev, lra, how):
+    from flare_py_amd import lra_modules
+
+    cls = lra_modules.FLAREBlock if lra else F.FLAREBlock
+    kw = {"kv_proj_hidden_dim": 64, "ffn_hidden_dim": 64} if lra else {}
+    m = cls(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev)
+    x = torch.randn(2, 2500, 64, device=dev, requires_grad=True)
+    watched, seen = {m.norm1, m.norm2, m.mlp, m.mlp.act, m.att.k_proj.act}, set()
+    handle = None
+    if how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, *a: seen.add(mod))
+    else:
+        for mod in watched:
+            mod.forward = (lambda mod, f: lambda *a: (seen.add(mod), f(*a))[1])(mod, mod.forward)
+    try:
+        out = m(x)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert watched <= seen
+    (out if lra else out[0]).sum().backward()
+    assert bool(torch.isfinite(x.grad).all())
