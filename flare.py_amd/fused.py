@@ -294,7 +294,7 @@ def _expand_tiles(f1, f2, E, Cdim):
 def _few(T, Cdim, L):
     """Rows of the norm's partial sums the few-token backward writes for such a launch, 0 where the other kernels serve it:
     what flare_mlp_few answers, without a call into the library (every fused call asks)."""
-    return (T + 15) // 16 if 0 < T <= _FEW_TOKENS[Cdim] and L <= _BWD_MAX_LAYERS[Cdim] else 0
+    return (T + 15) // 16 if 0 < T <= _FEW_TOKENS.get(Cdim, 0) and L <= _BWD_MAX_LAYERS[Cdim] else 0
 
 
 def _param_key(layers):
@@ -492,7 +492,7 @@ def _pair_info(x, mod_a, mod_b, cd):
     """(layers of both, act_mask, add_mask, act) where one few-token launch takes both stacks, else None: plain chains of
     C x C layers, alike in length, masks and activation, and few enough tokens."""
     Cdim = x.shape[-1]
-    if not 0 < x.numel() // Cdim <= _FEW_TOKENS[Cdim]:      # most calls end here: nothing else is looked at for them
+    if not 0 < x.numel() // Cdim <= _FEW_TOKENS.get(Cdim, 0):      # most calls end here: nothing else is looked at for them
         return None
     infos = [_layers_of(m) for m in (mod_a, mod_b)]
     if infos[0] is None or infos[1] is None or infos[0][1:] != infos[1][1:] or len(infos[0][0]) != len(infos[1][0]):

@@ -359,3 +359,14 @@ def test_few_token_limits_agree_with_the_library():
     m.flags = _lib.MLP_EXPAND
     m.T = 16
     assert lib.flare_mlp_few(C.byref(m)) == 0
+
+
+def test_few_token_question_at_unsupported_widths():
+    """No, and no error either: the launch itself refuses them."""
+    from flare_py_amd import fused
+
+    for Cdim in (16, 96, 256):
+        m = _lib.FlareMlpDesc()
+        m.T, m.C, m.L, m.w_dtype = 16, Cdim, 1, _lib.DT_BF16
+        assert _lib.load().flare_mlp_few(C.byref(m)) == fused._few(16, Cdim, 1) == 0
+        assert fused._pair_info(torch.empty(16, Cdim), torch.nn.Linear(Cdim, Cdim), torch.nn.Linear(Cdim, Cdim), torch.bfloat16) is None
