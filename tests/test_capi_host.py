@@ -370,3 +370,203 @@ def test_few_token_question_at_unsupported_widths():
         m.T, m.C, m.L, m.w_dtype = 16, Cdim, 1, _lib.DT_BF16
         assert _lib.load().flare_mlp_few(C.byref(m)) == fused._few(16, Cdim, 1) == 0
         assert fused._pair_info(torch.empty(16, Cdim), torch.nn.Linear(Cdim, Cdim), torch.nn.Linear(Cdim, Cdim), torch.bfloat16) is None
+
+
+def _refused(rc, text, code=_lib.FLARE_EINVAL):
+    assert rc == code and text in _lib.last_error(), (rc, _lib.last_error())
+
+
+def test_causal_linear_bwd_validation():
+    lib = _lib.load()
+    d = _lib.FlareCausalLinearDesc()
+    d.B, d.H, d.N, d.Dk, d.Dv, d.dtype = 1, 2, 256, 64, 64, _lib.DT_BF16
+    d.q_stride = d.k_stride = d.v_stride = d.y_stride = _lib.I3(2 * 256 * 64, 256 * 64, 64)
+    need = C.c_size_t(0)
+    assert lib.flare_causal_linear_workspace_bytes(d, C.byref(need)) == _lib.FLARE_OK and need.value > 0
+    fake = C.c_void_p(4096)
+
+    def call(q=fake, gy=fake, gs=_lib.I3(2 * 256 * 64, 256 * 64, 64), ws=fake, have=need.value):
+        return lib.flare_causal_linear_bwd(d, q, fake, fake, gy, gs, None, fake, fake, fake, ws, have, None)
+
+    assert lib.flare_causal_linear_bwd(None, *([None] * 4), None, *([None] * 5), 0, None) == _lib.FLARE_EINVAL
+    _refused(call(q=None), "must not be NULL")
+    _refused(call(gy=None), "must not be NULL")
+    _refused(call(gs=None), "must not be NULL")
+    _refused(call(gs=_lib.I3(0, 0, 63)), "gy row stride")
+    _refused(call(ws=None), "workspace", _lib.FLARE_EWORKSPACE)
+    _refused(call(have=need.value - 1), "needed", _lib.FLARE_EWORKSPACE)
+    _refused(call(ws=C.c_void_p(4098)), "4-byte")
+    d.Dk = 129
+    _refused(call(), "at most 128", _lib.FLARE_EUNSUPPORTED)
+    d.Dk, d.v_stride = 64, _lib.I3(0, 0, 32)
+    _refused(call(), "v row stride")
+
+
+def test_triple_bwd_validation():
+    lib = _lib.load()
+    d = _lib.FlareTripleDesc()
+    d.B, d.H, d.N, d.Dq, d.Dv, d.dtype = 1, 2, 256, 32, 32, _lib.DT_F16
+    for n in ("q1", "q2", "k1", "k2", "v", "o"):
+        setattr(d, n + "_stride", _lib.I3(2 * 256 * 32, 256 * 32, 32))
+    need, fwd = C.c_size_t(0), C.c_size_t(0)
+    _refused(lib.flare_triple_bwd_workspace_bytes(d, None), "bytes is NULL")
+    assert lib.flare_triple_bwd_workspace_bytes(d, C.byref(need)) == _lib.FLARE_OK
+    assert lib.flare_triple_workspace_bytes(d, C.byref(fwd)) == _lib.FLARE_OK and need.value > fwd.value > 0
+    fake = C.c_void_p(4096)
+
+    def call(null=None, ws=fake, have=need.value):
+        ptrs = [None if i == null else fake for i in range(13)]
+        ptrs[6] = None                                     # dstate may be missing
+        return lib.flare_triple_bwd(d, *ptrs, ws, have, None)
+
+    for i in range(13):
+        if i != 6:
+            _refused(call(null=i), "must not be NULL")
+    _refused(call(ws=None), "workspace", _lib.FLARE_EWORKSPACE)
+    _refused(call(have=need.value - 1), "needed", _lib.FLARE_EWORKSPACE)
+    _refused(call(ws=C.c_void_p(4104)), "16-byte")
+    d.normalize = 1
+    _refused(call(), "neither a feature map nor the normaliser", _lib.FLARE_EUNSUPPORTED)
+    d.normalize, d.feature_map = 0, 1
+    _refused(call(), "neither a feature map nor the normaliser", _lib.FLARE_EUNSUPPORTED)
+    d.feature_map, d.Dv = 0, 16
+    _refused(call(), "Dq == Dv", _lib.FLARE_EUNSUPPORTED)
+    d.Dq = d.Dv = 65
+    _refused(call(), "at most 64", _lib.FLARE_EUNSUPPORTED)
+
+
+def test_mlp_few_bwd_and_tiled_forward_validation():
+    lib = _lib.load()
+    m = _lib.FlareMlpDesc()
+    m.T, m.C, m.L = 64, 128, 5
+    m.x_dtype = m.y_dtype = m.res_dtype = m.w_dtype = _lib.DT_BF16
+    m.norm, m.eps = 1, 1e-5
+    m.x_stride = m.y_stride = m.res_stride = 128
+    fake, odd = C.c_void_p(4096), C.c_void_p(4104)
+
+    def call(x=fake, dy_a=fake, dy_b=fake, gamma=fake, add=0, a_in=fake, gb=fake):
+        return lib.flare_mlp_few_bwd(m, x, dy_a, dy_b, fake, fake, fake, gamma, fake, add, fake, a_in, fake, gb, None)
+
+    assert lib.flare_mlp_few_bwd(None, *([None] * 8), 0, *([None] * 5)) == _lib.FLARE_EUNSUPPORTED
+    _refused(call(x=None), "must not be NULL")
+    _refused(call(dy_a=odd), "16-byte")
+    _refused(call(dy_b=odd), "dy_b")
+    _refused(call(gamma=None), "norm")
+    _refused(call(gb=None), "norm")
+    _refused(call(a_in=None), "a_in and g_out")
+    _refused(call(add=4), "unknown bits")
+    for field, value in (("T", 12289), ("T", 0), ("L", 6), ("C", 96), ("flags", _lib.MLP_EXPAND)):
+        keep = getattr(m, field)
+        setattr(m, field, value)
+        _refused(call(), "flare_mlp_few", _lib.FLARE_EUNSUPPORTED)
+        setattr(m, field, keep)
+    m.flags = _lib.MLP_W_TILED                                # the backward knows its operands' order without it
+    _refused(call(), "flags must be 0", _lib.FLARE_EUNSUPPORTED)
+
+    def forward():
+        return lib.flare_mlp_fwd(m, fake, fake, fake, fake, fake, fake, fake, None)
+
+    m.T = 12289
+    _refused(forward(), "flare_mlp_few", _lib.FLARE_EUNSUPPORTED)
+    m.T, m.L = 64, 6
+    _refused(forward(), "flare_mlp_few", _lib.FLARE_EUNSUPPORTED)
+    m.flags, m.L = _lib.MLP_W_TILED | _lib.MLP_EXPAND, 4
+    _refused(forward(), "flare_mlp_few", _lib.FLARE_EUNSUPPORTED)
+    m.flags, m.norm = _lib.MLP_W_TILED, 0
+    _refused(lib.flare_mlp_io_fwd(m, 3, 1, fake, fake, 0, fake, fake, fake, None, None, None, fake, None), "flare_mlp_few", _lib.FLARE_EUNSUPPORTED)
+
+
+def test_mlp_pack_validation():
+    lib = _lib.load()
+    fake, odd = C.c_void_p(4096), C.c_void_p(4104)
+
+    def desc(**kw):
+        d = _lib.FlareMlpPackDesc()
+        d.L, d.C, d.w_dtype = 2, 64, _lib.DT_BF16
+        for l in range(2):
+            d.src[l], d.ld[l], d.rows[l] = 4096, 64, 64
+        for k, v in kw.items():
+            if isinstance(v, tuple):
+                getattr(d, k)[v[0]] = v[1]
+            else:
+                setattr(d, k, v)
+        return d
+
+    def call(d, w=fake, img=None, img_t=None, bias=fake):
+        return lib.flare_mlp_pack(d, w, img, img_t, bias, None)
+
+    assert lib.flare_mlp_pack(None, *([None] * 5)) == _lib.FLARE_EINVAL
+    _refused(call(desc(L=0)), "1 <= L")
+    _refused(call(desc(L=_lib.MLP_PACK_MAX + 1)), "1 <= L")
+    _refused(call(desc(w_dtype=_lib.DT_F32)), "w_dtype")
+    _refused(call(desc(C=96)), "32, 64 and 128", _lib.FLARE_EUNSUPPORTED)
+    _refused(call(desc(), w=None), "must not be NULL")
+    _refused(call(desc(), bias=None), "must not be NULL")
+    _refused(call(desc(), img=fake), "come together")
+    _refused(call(desc(tiled=1), img=fake, img_t=fake), "come together")
+    _refused(call(desc(), w=odd), "16-byte")
+    _refused(call(desc(), img=fake, img_t=odd), "16-byte")
+    _refused(call(desc(src=(1, None))), "src[1] is NULL")
+    _refused(call(desc(rows=(0, 65))), "tile 0")
+    _refused(call(desc(rows=(1, 0))), "tile 1")
+    _refused(call(desc(ld=(1, 63))), "tile 1")
+    _refused(call(desc(src_dtype=(0, 3))), "unknown dtype")
+    _refused(call(desc(b_dtype=(1, -1))), "unknown dtype")
+
+
+def test_mlp_wgrad_norm_validation():
+    lib = _lib.load()
+    m = _lib.FlareMlpDesc()
+    m.T, m.C, m.L, m.w_dtype = 100, 64, 2, _lib.DT_BF16
+    fake, odd = C.c_void_p(4096), C.c_void_p(4104)
+
+    def call(part=fake, rows=7, gb=fake, a=fake):
+        return lib.flare_mlp_wgrad_norm(m, a, 0, fake, 0, fake, None, None, None, part, rows, gb, None)
+
+    _refused(call(a=None), "must not be NULL")
+    _refused(call(part=None), "gb needs gb_part")
+    _refused(call(rows=0), "gb needs gb_part")
+    _refused(call(part=odd), "16-byte")
+    _refused(call(gb=odd), "16-byte")
+
+
+def test_row_pass_validation():
+    lib = _lib.load()
+    fake, odd, n = C.c_void_p(4096), C.c_void_p(4104), C.c_int32(0)
+    assert lib.flare_rows_parts(1, 32, C.byref(n)) == _lib.FLARE_OK and n.value == 1
+    assert lib.flare_rows_parts(1 << 40, 256, C.byref(n)) == _lib.FLARE_OK and 1 <= n.value <= 4096
+    _refused(lib.flare_rows_parts(4, 32, None), "parts is NULL")
+    _refused(lib.flare_rows_parts(0, 32, C.byref(n)), "T >= 1")
+    _refused(lib.flare_rows_parts(4, 96, C.byref(n)), "only 32, 64, 128 and 256", _lib.FLARE_EUNSUPPORTED)
+
+    def act(T=4, width=64, kind=0, ds=fake, t=fake, dt=fake, part=fake):
+        return lib.flare_rows_act_bwd(T, width, kind, ds, t, dt, None, part, None, None)
+
+    _refused(act(T=0), "T >= 1")
+    _refused(act(width=48), "only 32", _lib.FLARE_EUNSUPPORTED)
+    _refused(act(kind=2), "unknown activation")
+    _refused(act(kind=-2), "unknown activation")
+    _refused(act(ds=None), "required array is NULL")
+    _refused(act(part=None), "required array is NULL")
+    _refused(act(t=None), "must not be NULL with an activation")
+    _refused(act(dt=None), "must not be NULL with an activation")
+    _refused(act(ds=odd), "16-byte")
+
+    def fwd(norm=1, eps=1e-5, x=fake, gamma=fake, stats=fake):
+        return lib.flare_rows_norm_fwd(4, 64, norm, eps, x, gamma, None, fake, stats, None)
+
+    _refused(fwd(norm=0), "unknown norm")
+    _refused(fwd(eps=-1.0), "eps")
+    _refused(fwd(eps=float("nan")), "eps")
+    _refused(fwd(x=None), "required array is NULL")
+    _refused(fwd(gamma=odd), "16-byte")
+    _refused(fwd(stats=None), "required array is NULL")
+
+    def bwd(norm=2, dy=fake, stats=fake, add=None, part=fake):
+        return lib.flare_rows_norm_bwd(4, 64, norm, dy, fake, stats, None, add, fake, part, None, None)
+
+    _refused(bwd(norm=3), "unknown norm")
+    _refused(bwd(dy=None), "required array is NULL")
+    _refused(bwd(stats=None), "required array is NULL")
+    _refused(bwd(part=None), "required array is NULL")
+    _refused(bwd(add=odd), "16-byte")

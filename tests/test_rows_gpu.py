@@ -166,3 +166,30 @@ def test_replaced_forwards_and_global_hooks_are_called(dev, lra, how):
     assert watched <= seen
     (out if lra else out[0]).sum().backward()
     assert bool(torch.isfinite(x.grad).all())
+
+
+@pytest.mark.parametrize("norm", [1, 2])
+@pytest.mark.parametrize("T,C", [(1, 32), (1000, 64), (4097, 256)])
+def test_norm_backward_adds_another_gradient(dev, norm, T, C):
+    """The C interface's optional gradient of x from another path (a residual's): added to dx, one rounding of the sum."""
+    import ctypes
+
+    from flare_py_amd import _lib
+
+    lib = _lib.load()
+    x, dy, add = (torch.randn(T, C, device=dev) for _ in range(3))
+    gamma = torch.rand(C, device=dev) + 0.5
+    y, stats = torch.empty_like(x), torch.empty(T, 2, device=dev)
+    p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib.flare_rows_norm_fwd(T, C, norm, 1e-5, p(x), p(gamma), None, p(y), p(stats), st), "forward")
+    part, gb = torch.empty(rows._parts(T, C), 2, C, device=dev), torch.empty(2, C, device=dev)
+    dx = {}
+    for a in (None, add):
+        dx[a is add] = torch.empty_like(x)
+        _lib.check(lib.flare_rows_norm_bwd(T, C, norm, p(dy), p(x), p(stats), p(gamma), p(a), p(dx[a is add]), p(part), p(gb), st), "backward")
+    assert torch.equal(dx[True], dx[False] + add)
+    xr = x.double().requires_grad_(True)
+    yr = (nn.functional.layer_norm(xr, (C,), gamma.double(), None, 1e-5) if norm == 1 else nn.functional.rms_norm(xr, (C,), gamma.double(), 1e-5))
+    (want,) = torch.autograd.grad(yr, xr, dy.double())
+    assert rel(y, yr.detach()) <= 1e-6 and rel(dx[False], want) <= 1e-6

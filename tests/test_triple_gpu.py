@@ -254,3 +254,33 @@ def test_gradients_when_saved_tensors_come_back_in_another_memory_order(dev, D, 
     want = torch.autograd.grad(O.triple_einsum(*rins, dtype=torch.float64)[1], rins, go.double())
     for a, b in zip(got, want):
         assert O.rel_l2(a, b) <= tol
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -7), (torch.float16, 2.0 ** -10)])
+@pytest.mark.parametrize("stride,offset", [(40, 0), (40, 4), (40, 1), (36, 0), (33, 0)])
+def test_head_dim_32_rows_off_the_grid(dev, dtype, tol, stride, offset):
+    """One operand after the other (and all of them) off the 16-byte grid of the 32 x 32 x 32 kernels: by 8 bytes (the 16 x 16 x 16
+    kernels' grid), by 2, or at a row stride of either grid or none.  Forward with and without normaliser, backward, bounds as above."""
+    B, H, N, D = 2, 2, 300, 32
+    g = torch.Generator().manual_seed(stride + offset)
+    ins = [(torch.rand(B, H, N, D, generator=g) + 0.25).to(dtype) for _ in range(6)]
+
+    def off(t):
+        wide = torch.zeros(B, H, N, stride, dtype=dtype, device=dev).view(-1)
+        buf = torch.cat([wide, wide[:8]])
+        v = buf.as_strided((B, H, N, D), (H * N * stride, N * stride, stride, 1), offset)
+        v.copy_(t)
+        return v
+
+    rins = [t.double().requires_grad_(True) for t in ins[:5]]
+    sr, orf = O.triple_einsum(*rins, dtype=torch.float64)
+    want = torch.autograd.grad(orf, rins, ins[5].double())
+    nr = O.triple_einsum(*[t.float() for t in ins[:5]], normalize=True, dtype=torch.float64)[1]
+    for which in [*range(6), None]:
+        ops = [off(t) if which in (i, None) else t.to(dev) for i, t in enumerate(ins)]
+        dins = [t.detach().requires_grad_(True) for t in ops[:5]]
+        st, out = F.TripleAttentionFunction.apply(*dins)
+        assert O.rel_l2(st.detach(), sr.detach()) <= tol and O.rel_l2(out.detach(), orf.detach()) <= tol, which
+        assert O.rel_l2(F.triple_attention(*ops[:5], normalize=True)[1], nr) <= tol, which
+        for a, b in zip(torch.autograd.grad(out, dins, ops[5]), want):
+            assert O.rel_l2(a, b) <= 1.5 * tol, which
