@@ -63,8 +63,6 @@ template <typename F> __device__ __forceinline__ void with_dtype(int dt, F&& f)
     else if (dt == 1) f(std::integral_constant<int, 1>{});
     else f(std::integral_constant<int, 2>{});
 }
-template <int DT> struct Raw4 { using type = uint2; };
-template <> struct Raw4<0> { using type = f32x4; };
 template <int DT> __device__ __forceinline__ f32x4 load4(const void* base, int64_t e)
 {
     if constexpr (DT == 0) {
@@ -166,9 +164,8 @@ __device__ __forceinline__ void row_stats(const f32x4 (&x)[C / 16], int norm, fl
     rstd = rsqrtf(tok_sum(ss) * (1.f / C) + eps);
 }
 
-// The layers run in a loop, not unrolled: a launch this short meets a cold instruction cache, and the code of five layers
-// takes longer to arrive than to run.  Registers cannot be indexed by the layer number, so the tiles turn by one place per
-// layer instead.  pin: the loads have returned here, and nothing inside the loop waits for memory.
+// The layers run in a loop: unrolled they took the same time, at a multiple of the code.  Registers cannot be indexed by the
+// layer number, so the tiles turn by one place per layer instead.  pin: the loads have returned here, and nothing inside the loop waits for memory.
 template <int N, int KS> __device__ __forceinline__ void turn(u32x4 (&r)[N][KS])
 {
 #pragma unroll

@@ -10,7 +10,8 @@ Fast path: when the Linear layers may run in bf16/f16 (autocast, or 16-bit weigh
 is 32, 64 or 128, FLAREBlock runs as four fused HIP launches around the mixer (norm1 + k_proj,
 norm1 + v_proj, out_proj + residual, norm2 + FFN + residual; see fused.py) instead of ~70 torch
 kernels; with gradients enabled the same launches are differentiable (fused._FusedMlpFn).  fp32
-without autocast uses the torch layers.
+without autocast uses the torch layers, in training over long row arrays with HIP row passes around the library's
+products (rows.py).
 """
 from __future__ import annotations
 

@@ -96,7 +96,8 @@ def _parts(T, width):
 
 class _LinearLongRowsPass(torch.autograd.Function):
     """[res +] ([x +] act(x W^T + b)); inputs (act or -1, add, x, w, b, res).  One node per layer, as with torch's layers, and
-    the forward is torch's own calls: the outputs do not depend on whether a call comes here."""
+    the forward is torch's own calls: a chain's outputs do not depend on whether a call comes here (a norm's in front of it do, in
+    rounding: _NormFn reduces in an order of its own)."""
 
     @staticmethod
     def forward(ctx, act, add, x, w, b, res):
