@@ -4,8 +4,8 @@
 // type and row count per tile), so nothing is stacked or converted beforehand.
 //
 // A few hundred KB: what it costs is the launch.  The same from torch calls (stack, cast, stack, two index expansions and
-// an indexed read) was six launches per stack; an 8-block model's training step on 4096 points packs 33 stacks
-// (4.27 -> 3.68 ms replayed, about 190 launches fewer).
+// an indexed read) was six launches per stack; an 8-block model's training step on 4096 points packs 34 stacks
+// (4.27 -> 3.68 ms replayed, about 190 launches fewer), a block's k and v stacks in one launch.
 #include "common.hpp"
 
 namespace flare {
