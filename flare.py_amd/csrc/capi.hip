@@ -1325,6 +1325,31 @@ int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const
     return hip_status(flare::launch_rows_act_bwd(act, ds, t, dt, copy, db_part, db, T, C, static_cast<hipStream_t>(stream)), "row activation backward launch");
 }
 
+int flare_rows_layer_bwd_parts(int64_t T, int32_t C, int32_t* parts)
+{
+    if (!parts) return fail(FLARE_EINVAL, "parts is NULL");
+    const int rc = check_rows(T, C, {}, {});
+    if (rc != FLARE_OK) return rc;
+    *parts = flare::rows_layer_bwd_supported(C) ? flare::rows_layer_bwd_parts(T) : 0;
+    return FLARE_OK;
+}
+
+int flare_rows_layer_bwd(int64_t T, int32_t C, int32_t act, int32_t add, const float* dy, const float* t, const float* x, const float* w,
+                         float* dx, float* dw_part, float* db_part, float* dw, float* db, void* stream)
+{
+    const int rc = check_rows(T, C, {dy, x, w, dw_part, dw}, {t, dx, db_part, db});
+    if (rc != FLARE_OK) return rc;
+    if (!flare::rows_layer_bwd_supported(C)) return fail(FLARE_EUNSUPPORTED, "C=%d: only 64 and 128 are supported", C);
+    if (act < -1 || act > FLARE_ACT_SILU) return fail(FLARE_EINVAL, "unknown activation %d", act);
+    if (act >= 0 && !t) return fail(FLARE_EINVAL, "t must not be NULL with an activation");
+    if (db && !db_part) return fail(FLARE_EINVAL, "db needs db_part");
+    flare::RowsLayerArgs a;
+    memset(&a, 0, sizeof(a));
+    a.dy = dy; a.t = t; a.x = x; a.w = w; a.dx = dx; a.dw_part = dw_part; a.db_part = db ? db_part : nullptr;
+    a.T = T; a.C = C; a.add = add;
+    return hip_status(flare::launch_rows_layer_bwd(act, a, dw, db, static_cast<hipStream_t>(stream)), "row layer backward launch");
+}
+
 int flare_rows_norm_fwd(int64_t T, int32_t C, int32_t norm, float eps, const float* x, const float* gamma, const float* beta,
                         float* y, float* stats, void* stream)
 {

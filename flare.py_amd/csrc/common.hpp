@@ -360,6 +360,16 @@ struct RowsNormArgs {
     float eps;
 };
 
+// Backward of one fp32 layer y = [x +] act(x W^T + b) in one pass (rows_layer_f32_mfma.hip)
+struct RowsLayerArgs {
+    const float* dy; const float* t; const float* x;        // [T,C]: the gradient of y, x W^T + b (act only), the input
+    const float* w;                                         // [C,C] (out, in)
+    float* dx;                                              // [T,C] or null
+    float* dw_part; float* db_part;                         // [parts,C,C] and [parts,C] (or null)
+    int64_t T, rows_per_wg;                                 // rows_per_wg: set by the launcher
+    int C, add;                                             // add: dx starts from dy
+};
+
 // Workgroups of the backward's dq pass (bwd_lat_kernel, MODE 1) that fit a compute unit: its instances with 16 or
 // 32 latents per wave at head dim 16, and with 16 at head dim 32, need few enough registers for three or four (measured:
 // 143 -> 119 us at M = 128, D = 16; 86 -> 74 us at M = 64, D = 16; 133 -> 106 us at M = 64, D = 32); squeezing the
@@ -431,6 +441,10 @@ int        mlp_few_bwd_rows(int64_t T);
 hipError_t launch_mlp_few(const MlpArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_mlp_few_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts, hipStream_t st);   // n a multiple of 4
+hipError_t launch_sum_layer_parts(const float* dw_part, float* dw, const float* db_part, float* db, int C, int parts, hipStream_t st);   // db may be null
+bool       rows_layer_bwd_supported(int C);
+int        rows_layer_bwd_parts(int64_t T);
+hipError_t launch_rows_layer_bwd(int act, const RowsLayerArgs& a, float* dw, float* db, hipStream_t st);
 bool       rows_f32_supported(int C);
 int        rows_f32_parts(int64_t T, int C);
 hipError_t launch_rows_act_bwd(int act, const float* ds, const float* t, float* dt, float* copy, float* part, float* db, int64_t T, int C, hipStream_t st);

@@ -9,37 +9,12 @@
 // A thread owns four consecutive channels, the same for all its rows, so the sums over rows stay in its registers; a
 // workgroup leaves one partial row, and the partial rows are added in a fixed order by one small launch.
 #include <algorithm>
-#include <type_traits>
 
-#include "common.hpp"
+#include "rows_f32.hpp"
 
 namespace flare {
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// GELU's gate 0.5 (1 + tanh u) is 1 / (1 + exp(-2 u)), 2 u = 1.5957691 x (1 + 0.044715 x^2): no cancellation for negative x.
-// gate = 1 / (1 + e), 1 - gate = e / (1 + e), e kept finite.
-template <int ACT> __device__ __forceinline__ float act_slope(float x)
-{
-    const float a = ACT == 1 ? 1.5957691216057308f * x * fmaf(0.044715f * x, x, 1.f) : x;
-    const float da = ACT == 1 ? 1.5957691216057308f * fmaf(3.f * 0.044715f * x, x, 1.f) : 1.f;
-    const float e = fminf(expf(-a), 3.0e38f), r = 1.f / (1.f + e);
-    return r * fmaf(x * (e * r), da, 1.f);
-}
-
-// act: -1 none, else FLARE_ACT_*
-template <typename F> hipError_t with_act(int act, F&& f)
-{
-    switch (act) {
-        case -1: f(std::integral_constant<int, 0>{}); break;
-        case 0:  f(std::integral_constant<int, 1>{}); break;
-        case 1:  f(std::integral_constant<int, 2>{}); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
 
 // the workgroup's sums over its rows -> one partial row: thread x % quads owns four channels
 template <int N>
@@ -173,7 +148,7 @@ int rows_f32_parts(int64_t T, int C)
 hipError_t launch_rows_act_bwd(int act, const float* ds, const float* t, float* dt, float* copy, float* part, float* db, int64_t T, int C, hipStream_t st)
 {
     const int parts = rows_f32_parts(T, C);
-    hipError_t e = with_act(act, [&](auto ac) {
+    hipError_t e = with_row_act(act, [&](auto ac) {
         hipLaunchKernelGGL(rows_act_bwd_kernel<decltype(ac)::value>, dim3((unsigned)parts), dim3(256), 0, st, (const f32x4*)ds,
                            (const f32x4*)t, (f32x4*)dt, (f32x4*)copy, T * C / 4, C / 4, part);
     });

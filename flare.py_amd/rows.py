@@ -3,9 +3,10 @@ around them.
 
 What torch runs as separate layers (pdebench/models/flare.py:45-59, 204-215) spends most of an fp32 training step outside the
 products: in the backward the activation, the bias gradients and the sums at the residuals each make passes of their own over
-[T,C], and the norms run far from the memory's rate.  Here a layer's backward is one pass that forms dt, the bias gradient and
-the start value of dx together (flare_rows_act_bwd), the product that adds W^T dt to it, and the sliced weight gradient;
-the norms are one pass each way.
+[T,C], and the norms run far from the memory's rate.  Here a layer's backward is one pass over the rows (flare_rows_layer_bwd:
+slope, both products and the bias sums); at the widths that kernel does not take, a pass that forms dt, the bias gradient and the
+start value of dx together (flare_rows_act_bwd), the product that adds W^T dt to it, and the sliced weight gradient.  The norms are
+one pass each way.
 
 Used where the modules' fp32 Linear layers already run as a once-differentiable function (gradients enabled, outside autocast,
 4096 rows or more) and the arrays are large enough (MIN_ELEMS); every other call keeps the torch layers.
@@ -23,12 +24,14 @@ from . import _lib, fused
 from .functional import _on_device, _ptr, _stream_ptr
 
 LONG_ROWS = 4096      # rows from which the modules' fp32 Linear layers slice their weight gradient (below, one product is as fast)
-# Elements of a row array from which a step waits for the kernels: below, the host's enqueueing is what it costs, and a layer's node
-# here enqueues a little more than torch's own nodes.  A sequence block's step, torch's nodes / these, us: 64 channels, 8192 rows
-# 2755 / 2831, 65,536 rows (4 Mi) 2800 / 2846, 98,304 rows (6 Mi) 3100 / 2839, 131,072 rows 3850 / 3072; 128 channels, 32,768 rows
-# (4 Mi) 2647 / 2700, 49,152 rows (6 Mi) 3214 / 2745, 65,536 rows 3180 / 2754.  A step recorded into a graph has no host to wait for,
-# but follows the same rule: its replays give the results of the eager step bit for bit.
-MIN_ELEMS = 6 << 20
+# Elements of a row array from which these nodes pay, at the widths whose layer backward is one pass (_ONE_PASS): a layer enqueues less
+# than torch's own nodes, so they win from the smallest arrays on.  A sequence block's step, torch's nodes / these, us: 64 channels,
+# 8192 rows (0.5 Mi) 3047 / 2298, 16,384 rows 3066 / 2259, 98,304 rows (6 Mi) 3083 / 2273, 131,072 rows 3846 / 2341; 128 channels,
+# 8192 rows 2946 / 2122, 65,536 rows 3176 / 2173, 131,072 rows 5548 / 3869.  The other widths keep the separate passes, which enqueue
+# a little more than torch's nodes do: there the line is where a step waits for the kernels (6 Mi).  A step recorded into a graph has
+# no host to wait for, but follows the same rule: its replays give the results of the eager step bit for bit.
+MIN_ELEMS = 5 << 17
+_ONE_PASS = (64, 128)
 _WIDTHS = (32, 64, 128, 256)
 
 
@@ -55,7 +58,7 @@ def _param_ok(p):
 def _call_ok(x, long_rows):
     return (torch.is_grad_enabled() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype is torch.float32
             and x.shape[-1] in _WIDTHS and x.numel() // x.shape[-1] >= long_rows and not torch.is_autocast_enabled()
-            and x.numel() >= MIN_ELEMS
+            and x.numel() >= (MIN_ELEMS if x.shape[-1] in _ONE_PASS else 10 * MIN_ELEMS)
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
@@ -94,6 +97,14 @@ def _parts(T, width):
     return n.value
 
 
+def _layer_parts(T, width):
+    """Partial results of flare_rows_layer_bwd, 0 where the separate passes serve the width."""
+    n = C.c_int32(0)
+    if width in _ONE_PASS:
+        _lib.check(_lib.load().flare_rows_layer_bwd_parts(T, width, C.byref(n)), "flare_rows_layer_bwd_parts")
+    return n.value
+
+
 class _LinearLongRowsPass(torch.autograd.Function):
     """[res +] ([x +] act(x W^T + b)); inputs (act or -1, add, x, w, b, res).  One node per layer, as with torch's layers, and
     the forward is torch's own calls: a chain's outputs do not depend on whether a call comes here (a norm's in front of it do, in
@@ -122,6 +133,19 @@ class _LinearLongRowsPass(torch.autograd.Function):
         act, T, width, dev = ctx.act, s.shape[0], s.shape[1], s.device
         _, _, need_x, need_w, need_b, need_res = ctx.needs_input_grad
         ds = _rows(dy, width)
+        w = w.contiguous()
+        parts = _layer_parts(T, width) if need_w and w.data_ptr() % 16 == 0 else 0
+        if parts:
+            dx = torch.empty_like(ds) if need_x else None
+            part = torch.empty(parts, width + 1, width, dtype=torch.float32, device=dev)
+            dw = torch.empty(width, width, dtype=torch.float32, device=dev)
+            db = torch.empty(width, dtype=torch.float32, device=dev) if need_b else None
+            at = part.data_ptr()
+            with _on_device(dev):
+                rc = _lib.load().flare_rows_layer_bwd(T, width, act, ctx.add, _ptr(ds), _ptr(t), _ptr(s), _ptr(w), _ptr(dx), at, at + 4 * parts * width * width,
+                                                      _ptr(dw), _ptr(db), C.c_void_p(_stream_ptr(dev)))
+            _lib.check(rc, "flare_rows_layer_bwd")
+            return None, None, None if dx is None else dx.view(dy.shape), dw, db, dy if need_res else None
         dt = torch.empty_like(ds) if act >= 0 else ds
         dx = torch.empty_like(ds) if ctx.add and need_x else None
         db = torch.empty(width, dtype=torch.float32, device=dev) if need_b else None

@@ -429,6 +429,11 @@ int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_l
 int flare_rows_parts(int64_t T, int32_t C, int32_t* parts);
 int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const float* t, float* dt, float* copy, float* db_part,
                        float* db, void* stream);
+/* Backward of one layer y = [x +] act(x W^T + b) in one pass (C in {64, 128}; flare_rows_layer_bwd_parts answers 0 for the others):
+ * dx = [dy if add] + (dy act'(t)) W (or NULL), dw [C,C] (out, in), db [C] (or NULL).  dw_part [parts,C,C] and db_part [parts,C] are scratch. */
+int flare_rows_layer_bwd_parts(int64_t T, int32_t C, int32_t* parts);
+int flare_rows_layer_bwd(int64_t T, int32_t C, int32_t act, int32_t add, const float* dy, const float* t, const float* x, const float* w,
+                         float* dx, float* dw_part, float* db_part, float* dw, float* db, void* stream);
 int flare_rows_norm_fwd(int64_t T, int32_t C, int32_t norm, float eps, const float* x, const float* gamma, const float* beta,
                         float* y, float* stats, void* stream);
 int flare_rows_norm_bwd(int64_t T, int32_t C, int32_t norm, const float* dy, const float* x, const float* stats, const float* gamma,

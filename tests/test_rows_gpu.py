@@ -193,3 +193,39 @@ def test_norm_backward_adds_another_gradient(dev, norm, T, C):
     yr = (nn.functional.layer_norm(xr, (C,), gamma.double(), None, 1e-5) if norm == 1 else nn.functional.rms_norm(xr, (C,), gamma.double(), 1e-5))
     (want,) = torch.autograd.grad(yr, xr, dy.double())
     assert rel(y, yr.detach()) <= 1e-6 and rel(dx[False], want) <= 1e-6
+
+
+@pytest.mark.parametrize("act", [-1, 0, 1])
+@pytest.mark.parametrize("T,C", [(1, 64), (15, 128), (64, 64), (65, 128), (177, 64), (4111, 128), (16384, 128), (16385, 64), (33000, 128), (40000, 64)])
+def test_layer_backward_in_one_pass(dev, act, T, C):
+    """flare_rows_layer_bwd against the layer's gradients in fp64: around a workgroup's least rows, the tile, the 16-row step and the
+    first row counts that give every compute unit more than one tile.  Bound per result: 2e-6 of its norm, several times what sums of
+    C (dx) or T (dw, db) products rounded in fp32 show."""
+    import ctypes
+
+    from flare_py_amd import _lib
+
+    lib = _lib.load()
+    torch.manual_seed(T)
+    dy, x = torch.randn(T, C, device=dev), torch.randn(T, C, device=dev)
+    w, b = torch.randn(C, C, device=dev) * C ** -0.5, torch.randn(C, device=dev)
+    t = torch.nn.functional.linear(x, w, b) * 2
+    n = ctypes.c_int32(0)
+    _lib.check(lib.flare_rows_layer_bwd_parts(T, C, ctypes.byref(n)), "parts")
+    assert 1 <= n.value <= 4096
+    t64 = t.double().requires_grad_(True)
+    f = (lambda v: v, lambda v: nn.functional.gelu(v, approximate="tanh"), nn.functional.silu)[act + 1]
+    (dt,) = torch.autograd.grad(f(t64), t64, dy.double())
+    p = lambda v: None if v is None else ctypes.c_void_p(v.data_ptr())
+    for add, want_x, want_b in ((0, True, True), (1, True, False), (0, False, True)):
+        guard = torch.full((T + 64, C), 7.0, device=dev)
+        dx, dw, db = guard[:T] if want_x else None, torch.empty_like(w), torch.empty_like(b) if want_b else None
+        pw, pb = torch.empty(n.value, C, C, device=dev), torch.empty(n.value, C, device=dev)
+        _lib.check(lib.flare_rows_layer_bwd(T, C, act, add, p(dy), p(t) if act >= 0 else None, p(x), p(w), p(dx), p(pw), p(pb), p(dw), p(db),
+                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "flare_rows_layer_bwd")
+        assert rel(dw, dt.t() @ x.double()) <= 2e-6
+        if want_b:
+            assert rel(db, dt.sum(0)) <= 2e-6 * max(1.0, float(dt.norm() / dt.sum(0).norm()))
+        if want_x:
+            assert rel(dx, dt @ w.double() + (dy.double() if add else 0)) <= 2e-6
+            assert bool((guard[T:] == 7.0).all())
