@@ -64,6 +64,13 @@ class FlareMlpDesc(C.Structure):
     ]
 
 
+class FlareBlockDesc(C.Structure):
+    _fields_ = [
+        ("mlp", FlareMlpDesc * 4), ("mixer", FlareMixerDesc),
+        ("w", C.c_void_p * 4), ("b", C.c_void_p * 4), ("gamma", C.c_void_p * 4), ("beta", C.c_void_p * 4), ("q", C.c_void_p),
+    ]
+
+
 MLP_PACK_MAX = 16
 
 
@@ -116,6 +123,8 @@ SYMBOLS = {
     "flare_mlp_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_io_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), C.c_int32, C.c_int32, _P, _P, C.c_int32,
                                    _P, _P, _P, _P, _P, _P, _P, _P]),
+    "flare_block_scratch_bytes": (C.c_int, [C.POINTER(FlareBlockDesc), C.POINTER(_SZ)]),
+    "flare_block_fwd": (C.c_int, [C.POINTER(FlareBlockDesc), _P, _P, _P, _SZ, _P]),
     "flare_mlp_bwd_partial_rows": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(C.c_int32)]),
     "flare_mlp_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_wgrad_partials": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(C.c_int32)]),

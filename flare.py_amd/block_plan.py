@@ -1,0 +1,174 @@
+"""A FLAREBlock's inference forward as one call into the library.
+
+Under autocast and without gradients the block is seven launches (norm + k projection, norm + v projection, three of the mixer,
+output projection + residual, norm + feed-forward + residual; pdebench/models/flare.py:107-215), and on small point clouds enqueueing
+them from Python is what it costs: five calls of 20 to 30 us each, most of it spent deciding again what the last call decided.
+An 8-block model of 64 channels on 3973 points: 1070 us a forward, 380 us
+through the plans (0.31 ms of kernels).  `forward` keeps what depends on the module and the shape only -- descriptors, the packed 16-bit weights the modules hold
+anyway, the layout of one scratch allocation -- and hands the rest to flare_block_fwd.  Nothing about an input is kept.
+
+A plan is made when a block meets a shape for the second time.  Every call compares what it was made from: the modules' structure,
+every parameter's address and version, the norms' eps, the mixer's scale.  Where any of it changed, a new plan is made, and calls a
+plan does not cover (hooks on the attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer
+pads itself) run the general path of modules.py.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import torch
+from torch import nn
+
+from . import _lib, functional, fused, rows
+
+_MAX_SHAPES = 8           # plans kept per block; a plan holds a descriptor of 0.5 KB and references to the module's packed weights
+_X_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
+class _Plans(dict):
+    """shape -> (key, plan).  A copy of a module, and one read back from a file, begins without plans: they hold addresses."""
+
+    def __deepcopy__(self, memo):
+        return _Plans()
+
+    def __reduce__(self):
+        return _Plans, ()
+
+
+class _Plan:
+    __slots__ = ("desc", "ref", "scratch", "keep")
+
+
+def _key(block):
+    """Everything a plan is made from, or None for a block that the general path serves."""
+    m = block._modules
+    att, mlp, n1, n2 = m["att"], m["mlp"], m["norm1"], m["norm2"]
+    if not rows._plain(att) or att.qk_norm or "latent_q" not in att._parameters:
+        return None
+    a = att._modules
+    layers, key = [], [att.attn_scale, att.num_heads, att.num_latents, att.head_dim]
+    for mod in (a["k_proj"], a["v_proj"], a["out_proj"], mlp):
+        info = fused._layers_of(mod)
+        if info is None:
+            return None
+        key.append(fused._structure_key(mod))
+        layers += info[0]
+    for n in (n1, n2):
+        p = n._parameters
+        for name in ("weight", "bias"):
+            t = p.get(name)
+            key.append(None if t is None else (t.data_ptr(), t._version))
+        key += (type(n), getattr(n, "eps", None))
+    if any("weight" not in l._parameters for l in layers):      # a parametrised weight is another tensor at every access
+        return None
+    q = att._parameters["latent_q"]
+    key.append((q.data_ptr(), q._version))
+    key.append(fused._param_key(layers))
+    return key
+
+
+def _mlp(mod, T, cd, x_dtype, y_dtype, x_stride, y_stride, norm=None, res=None, x_head=0, y_head=0):
+    """(descriptor, weights, biases, gamma, beta) of one launch of fused._fused_mlp_fwd, or None."""
+    info, io, Cdim, E = fused._forward_plan(mod)
+    layers, act_mask, add_mask, act = info
+    if io is not None or (E and (x_head or y_head)):
+        return None
+    few, w, b = False, None, None
+    if not E and fused._few(T, Cdim, len(layers)):
+        packed = fused._packed_few(mod, layers, cd, False)
+        if packed is not None:
+            few, (w, b) = True, packed[:2]
+    if w is None:
+        w, b = fused._packed_expand(mod, E, cd) if E else fused._packed(mod, layers, cd)
+    if E:
+        act_mask, add_mask = 1, 0
+    d = _lib.FlareMlpDesc()
+    d.T, d.C, d.L = T, Cdim, w.shape[0]
+    d.flags = (_lib.MLP_EXPAND if E else _lib.MLP_W_TILED if few else 0) | ((x_head // 4) << 8) | ((y_head // 4) << 12)
+    d.w_dtype, d.x_dtype, d.y_dtype = functional._DTYPES[cd], functional._DTYPES[x_dtype], functional._DTYPES[y_dtype]
+    d.act, d.act_mask, d.add_mask, d.x_stride, d.y_stride = act, act_mask, add_mask, x_stride, y_stride
+    gamma = beta = None
+    if norm is not None:
+        gamma, beta = norm._parameters.get("weight"), norm._parameters.get("bias")
+        if gamma is None or any(t is not None and fused._vec32(t) is not t for t in (gamma, beta)):
+            return None                                   # a converted copy would have to follow its parameter
+        fused._norm_args(d, norm, torch.empty(0, dtype=x_dtype), Cdim)
+    if res is not None:
+        d.res_dtype, d.res_stride = functional._DTYPES[res], Cdim
+    return d, w, b, gamma, beta
+
+
+def _build(block, x, cd):
+    """A plan for inputs of x's shape and type, or None where the general path has to serve them."""
+    att, mlp = block.att, block.mlp
+    B, N, Cdim = x.shape
+    H, M, D = att.num_heads, att.num_latents, att.head_dim
+    if any(fused.compute_dtype(x, m) is not cd for m in (att.k_proj, att.v_proj, att.out_proj, mlp)):
+        return None
+    if M % 32 or D not in (4, 8, 16, 32, 64) or any(type(n) not in (nn.LayerNorm, nn.RMSNorm) for n in (block.norm1, block.norm2)):
+        return None
+    if any(p.device != x.device for mod in (att, mlp, block.norm1, block.norm2) for p in mod.parameters()):
+        return None
+    head = D if D in (4, 8) else 0                        # narrow heads: k, v and the mixer's rows padded to 16 columns
+    Dp, T = (16 if head else D), B * N
+    width = H * Dp
+    parts = [_mlp(att.k_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head),
+             _mlp(att.v_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head),
+             _mlp(att.out_proj, T, cd, cd, x.dtype, width, Cdim, res=x.dtype, x_head=head),
+             _mlp(mlp, T, cd, x.dtype, x.dtype, Cdim, Cdim, norm=block.norm2, res=x.dtype)]
+    if any(p is None for p in parts):
+        return None
+    q = att._cached_q(cd, Dp - D)
+    plan = _Plan()
+    d = plan.desc = _lib.FlareBlockDesc()
+    for i, (desc, w, b, gamma, beta) in enumerate(parts):
+        d.mlp[i], d.w[i], d.b[i] = desc, w.data_ptr(), b.data_ptr()
+        d.gamma[i], d.beta[i] = (None if t is None else t.data_ptr() for t in (gamma, beta))
+    d.q = q.data_ptr()
+    m = d.mixer
+    m.B, m.H, m.N, m.M, m.D, m.dtype, m.scale, m.flags = B, H, N, M, Dp, functional._DTYPES[cd], float(att.attn_scale), functional._extra_mixer_flags
+    m.q_stride = _lib.I3(0, M * Dp, Dp)
+    m.k_stride = m.v_stride = m.y_stride = _lib.I3(N * width, Dp, width)
+    n = C.c_size_t(0)
+    if _lib.load().flare_block_scratch_bytes(C.byref(d), C.byref(n)) != _lib.FLARE_OK:
+        return None
+    plan.ref, plan.scratch = C.byref(d), n.value
+    plan.keep = [q] + [t for p in parts for t in p[1:]]   # the parameters' packed copies, and the norms' vectors
+    return plan
+
+
+def forward(block, x):
+    """block(x) through a plan, or None: the general path serves the call."""
+    if torch.is_grad_enabled() or type(x) is not torch.Tensor or not x.is_cuda or not torch.is_autocast_enabled("cuda"):
+        return None
+    cd = torch.get_autocast_dtype("cuda")
+    if (cd not in (torch.bfloat16, torch.float16) or x.dtype not in _X_DTYPES or x.dim() != 3 or x.numel() == 0
+            or not x.is_contiguous() or x.data_ptr() % 16):
+        return None
+    plans = block.__dict__.get("_flare_plans")
+    if plans is None:
+        plans = block.__dict__["_flare_plans"] = _Plans()
+    dev = x.device
+    shape = (x.shape, x.dtype, cd, dev.index, functional._extra_mixer_flags)
+    entry = plans.get(shape)
+    if entry is None:
+        if len(plans) >= _MAX_SHAPES:
+            plans.clear()
+        plans[shape] = (None, None)
+        return None
+    key = _key(block)
+    if key is None:
+        return None
+    plan = entry[1]
+    if entry[0] != key:
+        plan = _build(block, x, cd)
+        plans[shape] = (key, plan)
+    if plan is None:
+        return None
+    y = torch.empty_like(x)
+    scratch = torch.empty(plan.scratch, dtype=torch.uint8, device=dev)
+    with functional._on_device(dev):
+        rc = _lib.load().flare_block_fwd(plan.ref, x.data_ptr(), y.data_ptr(), scratch.data_ptr(), plan.scratch, functional._stream_ptr(dev))
+    if rc:
+        _lib.check(rc, "flare_block_fwd")
+    return y

@@ -1111,6 +1111,65 @@ int flare_mlp_io_fwd(const FlareMlpDesc* d, int32_t in_dim, int32_t in_act, cons
     return mlp_fwd_impl(d, in_dim, in_act, w_in, b_in, out_dim, x, w, bias, gamma, beta, res, y, stream);
 }
 
+// Scratch of a block's forward: k rows, v rows, the mixer's output rows, the mixer's workspace with z at its tail.  The attention's result
+// takes the place of k and v, which nothing reads behind the mixer.
+struct BlockScratch { size_t k, v, y, x1, ws, ws_bytes, total; };
+static int plan_block(const FlareBlockDesc* d, BlockScratch* s)
+{
+    if (!d) return fail(FLARE_EINVAL, "descriptor must not be NULL");
+    const FlareMixerDesc& m = d->mixer;
+    const int rc = check_mixer_desc(&m);
+    if (rc != FLARE_OK) return rc;
+    const int64_t T = (int64_t)m.B * m.N, width = (int64_t)m.H * m.D;
+    if (m.dtype != FLARE_DT_BF16 && m.dtype != FLARE_DT_F16) return fail(FLARE_EUNSUPPORTED, "the mixer of a block runs in bf16 or f16");
+    for (const int64_t* st : {m.k_stride, m.v_stride, m.y_stride})
+        if (st[0] != m.N * width || st[1] != m.D || st[2] != width) return fail(FLARE_EINVAL, "k, v and y of a block are [B,N,H,D] rows");
+    for (int i = 0; i < 4; ++i) {
+        const FlareMlpDesc& f = d->mlp[i];
+        if (f.T != T || f.C != d->mlp[0].C) return fail(FLARE_EINVAL, "mlp %d: T and C must be the block's", i);
+        const bool from = i == 2, to = i < 2;      // reads / writes the mixer's rows
+        if (f.x_stride != (from ? width : f.C) || f.y_stride != (to ? width : f.C)) return fail(FLARE_EINVAL, "mlp %d: rows must be contiguous", i);
+        if (f.x_dtype != (from ? m.dtype : d->mlp[0].x_dtype) || f.y_dtype != (to ? m.dtype : d->mlp[0].x_dtype))
+            return fail(FLARE_EINVAL, "mlp %d: element types do not fit the block", i);
+        if (!to && (f.res_dtype != d->mlp[0].x_dtype || f.res_stride != f.C)) return fail(FLARE_EINVAL, "mlp %d: the residual must be the block's rows", i);
+    }
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t rows = up((size_t)T * width * 2);
+    if ((size_t)T * d->mlp[0].C * 4 > 2 * rows) return fail(FLARE_EINVAL, "H D of a block's mixer must be C or more");
+    s->x1 = s->k = 0; s->v = rows; s->y = 2 * rows; s->ws = 3 * rows;
+    s->ws_bytes = mixer_ws_bytes(&m);
+    s->total = s->ws + up(s->ws_bytes);
+    return FLARE_OK;
+}
+
+int flare_block_scratch_bytes(const FlareBlockDesc* d, size_t* bytes)
+{
+    if (!bytes) return fail(FLARE_EINVAL, "bytes is NULL");
+    BlockScratch s;
+    const int rc = plan_block(d, &s);
+    if (rc == FLARE_OK) *bytes = s.total;
+    return rc;
+}
+
+int flare_block_fwd(const FlareBlockDesc* d, const void* x, void* y, void* scratch, size_t scratch_bytes, void* stream)
+{
+    BlockScratch s;
+    int rc = plan_block(d, &s);
+    if (rc != FLARE_OK) return rc;
+    if (!x || !y) return fail(FLARE_EINVAL, "x and y must not be NULL");
+    if (!scratch || scratch_bytes < s.total || reinterpret_cast<uintptr_t>(scratch) % 256)
+        return fail(FLARE_EWORKSPACE, "scratch must hold %zu bytes, 256-byte aligned", s.total);
+    uint8_t* base = static_cast<uint8_t*>(scratch);
+    void *k = base + s.k, *v = base + s.v, *ym = base + s.y, *x1 = base + s.x1;
+    auto mlp = [&](int i, const void* in, const void* res, void* out) {
+        return flare_mlp_fwd(&d->mlp[i], in, d->w[i], d->b[i], d->gamma[i], d->beta[i], res, out, stream);
+    };
+    if ((rc = mlp(0, x, nullptr, k)) != FLARE_OK || (rc = mlp(1, x, nullptr, v)) != FLARE_OK) return rc;
+    if ((rc = flare_mixer_fwd(&d->mixer, d->q, k, v, nullptr, ym, nullptr, base + s.ws, s.ws_bytes, stream)) != FLARE_OK) return rc;
+    if ((rc = mlp(2, ym, x, x1)) != FLARE_OK) return rc;
+    return mlp(3, x1, x1, y);
+}
+
 int flare_mlp_bwd_partial_rows(const FlareMlpDesc* d, int32_t* rows)
 {
     if (!d || !rows) return fail(FLARE_EINVAL, "descriptor and rows must not be NULL");

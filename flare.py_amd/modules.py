@@ -19,7 +19,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
-from . import fused, rows
+from . import block_plan, fused, rows
 from .functional import flare_multihead_mixer
 
 __all__ = ["ResidualMLP", "FLARE", "FLAREBlock", "FinalLayer", "FLAREModel"]
@@ -266,6 +266,10 @@ class FLAREBlock(nn.Module):
                                num_layers=num_layers_ffn, act=act, input_residual=True, output_residual=True)
 
     def forward(self, x, return_scores: bool = False):
+        if not return_scores and type(self.att) is FLARE:
+            y = block_plan.forward(self, x)      # inference under autocast: the launches below from one call
+            if y is not None:
+                return y, None
         x, scores = self.att(x, return_scores=return_scores, _norm=self.norm1, _res=x)
         cd = fused.compute_dtype(x, self.mlp)
         if cd is not None:

@@ -366,6 +366,22 @@ int flare_mlp_io_fwd(const FlareMlpDesc* desc, int32_t in_dim, int32_t in_act, c
 #define FLARE_MLP_BWD_ADD_DY 1
 #define FLARE_MLP_BWD_ACCUMULATE 2
 
+/* One encoder block's forward as one call (pdebench/models/flare.py:107-215):  k, v = mlp[0](norm x), mlp[1](norm x);
+ * x1 = x + mlp[2](mixer(q, k, v));  y = x1 + mlp[3](norm x1).  mlp[i], w, b, gamma, beta: as flare_mlp_fwd takes them (residual types
+ * and strides of 2 and 3 included; x, x1, y share a type and are contiguous [T,C] rows, T = B N of the mixer); mixer: as
+ * flare_mixer_fwd takes it, with k, v and y as [B,N,H,D] rows in the scratch memory.  scratch: 256-byte aligned. */
+typedef struct FlareBlockDesc {
+    FlareMlpDesc mlp[4];
+    FlareMixerDesc mixer;
+    const void* w[4];
+    const float* b[4];
+    const float* gamma[4];
+    const float* beta[4];
+    const void* q;
+} FlareBlockDesc;
+int flare_block_scratch_bytes(const FlareBlockDesc* desc, size_t* bytes);
+int flare_block_fwd(const FlareBlockDesc* desc, const void* x, void* y, void* scratch, size_t scratch_bytes, void* stream);
+
 /* Backward of flare_mlp_fwd for the chain of C x C layers (desc->flags == 0; at most 8 layers, 5 at C = 128): what
  * torch autograd computes for  y = res + ResidualMLP(norm(x))  (pdebench/models/flare.py:45-59, 204-215) when
  * the reference trains a block.  One token-parallel launch recomputes the forward and walks the chain back;
