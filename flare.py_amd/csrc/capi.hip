@@ -1209,7 +1209,12 @@ static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, co
 {
     int rc = check_mlp_bwd_common(d, x, dy, w_img, wt_img, bias, gamma, beta, dx, dn, stats, gb_part, gb);
     if (rc != FLARE_OK) return rc;
-    if (d->flags != 0) return fail(FLARE_EUNSUPPORTED, "the backward covers the chain of C x C layers only (flags must be 0)");
+    const int x_head = few ? 4 * ((d->flags >> 8) & 15) : 0, y_head = few ? 4 * ((d->flags >> 12) & 15) : 0;
+    if (d->flags & ~(few ? 0xff00 : 0)) return fail(FLARE_EUNSUPPORTED, "the backward covers the chain of C x C layers only (flags must be 0)");
+    if (x_head > 8 || y_head > 8) return fail(FLARE_EINVAL, "head-padded rows need a head dim of 4 or 8");
+    const int64_t x_width = x_head ? 16 * (int64_t)(d->C / x_head) : d->C, y_width = y_head ? 16 * (int64_t)(d->C / y_head) : d->C;
+    if (d->x_stride < x_width || d->y_stride < y_width) return fail(FLARE_EINVAL, "x and dy rows must be as wide as their padded heads");
+    if ((x_head || y_head) && add_dy) return fail(FLARE_EUNSUPPORTED, "head-padded rows cannot be combined with bits of add_dy");
     if (d->L > flare::mlp_bwd_max_layers(d->C))
         return fail(FLARE_EUNSUPPORTED, "the backward keeps every layer's slopes in registers: at most %d layers at C=%d (got %d)",
                     flare::mlp_bwd_max_layers(d->C), d->C, d->L);
@@ -1227,7 +1232,8 @@ static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, co
     a.norm = d->norm; a.eps = d->eps; a.act = d->act; a.act_mask = d->act_mask; a.add_mask = d->add_mask;
     if (add_dy & ~(FLARE_MLP_BWD_ADD_DY | FLARE_MLP_BWD_ACCUMULATE)) return fail(FLARE_EINVAL, "add_dy holds unknown bits (got %d)", add_dy);
     a.add_dy = add_dy;
-    a.xs = d->x_stride; a.dys = d->y_stride; a.dxs = d->C;
+    a.xs = d->x_stride; a.dys = d->y_stride; a.dxs = x_width;
+    a.x_head = x_head; a.y_head = y_head;
     if (few) return hip_status(flare::launch_mlp_few_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token backward launch");
     return hip_status(flare::launch_mlp_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp backward launch");
 }

@@ -187,6 +187,18 @@ template <int N> __device__ __forceinline__ void pin(f32x4 (&r)[N])
     for (int l = 0; l < N; ++l) asm volatile("" : "+v"(r[l]));
 }
 
+// column of channels f = 16 ft + 4 g .. of a row: f itself, or 16 (f / head) + f % head in head-padded rows
+__device__ __forceinline__ int col_of(int head, int ft, int g)
+{
+    return head == 0 ? 16 * ft + 4 * g : head == 8 ? 32 * ft + 8 * g - 4 * (g & 1) : 64 * ft + 16 * g;
+}
+// the zeros of head-padded rows up to 16 columns, by the lane that holds the head's last four channels
+template <int DT> __device__ __forceinline__ void store_pad(void* base, int64_t e, int head, int g)
+{
+    const int nz = head == 0 ? 0 : head == 8 ? ((g & 1) ? 2 : 0) : 3;
+    for (int z = 1; z <= nz; ++z) store4<DT>(base, e + 4 * z, f32x4{0.f, 0.f, 0.f, 0.f});
+}
+
 // Forward.  LMAX: layers held in registers, L <= LMAX (the surplus tiles are the last one again: no branch around a load).
 template <typename T, int C, int LMAX>
 __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
@@ -204,17 +216,13 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
     const bool live = t < a.T;
     const int64_t tok = live ? t : a.T - 1;
 
-    // column of channel f = 16 ft + 4 g of a row: f itself, or 16 (f / head) + f % head in head-padded rows
-    auto col_of = [&](int head, int ft) {
-        return head == 0 ? 16 * ft + 4 * g : head == 8 ? 32 * ft + 8 * g - 4 * (g & 1) : 64 * ft + 16 * g;
-    };
     f32x4 x0[FT], own;
     with_dtype(a.x_dtype, [&](auto dc) {
         constexpr int DT = decltype(dc)::value;
-        own = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, w));
+        own = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, w, g));
         if (a.norm != 0) {
 #pragma unroll
-            for (int ft = 0; ft < FT; ++ft) x0[ft] = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, ft));
+            for (int ft = 0; ft < FT; ++ft) x0[ft] = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, ft, g));
         }
     });
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -268,11 +276,9 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
     if (live) {
         with_dtype(a.y_dtype, [&](auto dc) {
             constexpr int DT = decltype(dc)::value;
-            const int64_t e = tok * a.ys + col_of(a.y_head, w);
+            const int64_t e = tok * a.ys + col_of(a.y_head, w, g);
             store4<DT>(a.y, e, s);
-            // head-padded rows: zeros up to 16 columns, by the lane that holds the head's last four channels
-            const int nz = a.y_head == 0 ? 0 : a.y_head == 8 ? ((g & 1) ? 2 : 0) : 3;
-            for (int z = 1; z <= nz; ++z) store4<DT>(a.y, e + 4 * z, zero);
+            store_pad<DT>(a.y, e, a.y_head, g);
         });
     }
 }
@@ -301,10 +307,10 @@ __global__ __launch_bounds__(4 * C) void few_mlp_bwd_kernel(MlpBwdArgs a)
     f32x4 x0[FT], own, dy[CH];
     with_dtype(a.x_dtype, [&](auto dc) {
         constexpr int DT = decltype(dc)::value;
-        own = load4<DT>(a.x, tok * a.xs + ch0);
+        own = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, w, g));
         if (a.norm != 0) {
 #pragma unroll
-            for (int ft = 0; ft < FT; ++ft) x0[ft] = load4<DT>(a.x, tok * a.xs + 16 * ft + 4 * g);
+            for (int ft = 0; ft < FT; ++ft) x0[ft] = load4<DT>(a.x, tok * a.xs + col_of(a.x_head, ft, g));
         }
     });
     f32x4 gm = zero, bt = zero;
@@ -314,7 +320,7 @@ __global__ __launch_bounds__(4 * C) void few_mlp_bwd_kernel(MlpBwdArgs a)
     }
     with_dtype(a.dy_dtype, [&](auto dc) {
 #pragma unroll
-        for (int c = 0; c < CH; ++c) dy[c] = load4<decltype(dc)::value>(c == 0 ? a.dy : a.dy2, tok * a.dys + ch0);
+        for (int c = 0; c < CH; ++c) dy[c] = load4<decltype(dc)::value>(c == 0 ? a.dy : a.dy2, tok * a.dys + col_of(a.y_head, w, g));
     });
     u32x4 wr[LMAX][KS], wt[LMAX][KS];
     f32x4 bias[LMAX];
@@ -461,9 +467,10 @@ __global__ __launch_bounds__(4 * C) void few_mlp_bwd_kernel(MlpBwdArgs a)
         if (a.add_dy & 1) total += dy[0];
         with_dtype(a.dx_dtype, [&](auto dc) {
             constexpr int DT = decltype(dc)::value;
-            const int64_t e = tok * a.dxs + ch0;
+            const int64_t e = tok * a.dxs + col_of(a.x_head, w, g);
             if (a.add_dy & 2) total += load4<DT>(a.dx, e);        // dx holds another path's gradient of the same x
             store4<DT>(a.dx, e, total);
+            store_pad<DT>(a.dx, e, a.x_head, g);
         });
     }
 }

@@ -245,7 +245,7 @@ def _hip_backward_ok(q, k, v, key_mask, force_generic, drop=None) -> bool:
 
 
 def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None):
-    """dq, dk, dv from the HIP backward kernels (flare_mixer_bwd); drop = (p, seed) of the forward's attention dropout."""
+    """dq (fp32), dk, dv from the HIP backward kernels (flare_mixer_bwd); drop = (p, seed) of the forward's attention dropout."""
     lib = _lib.load()
     k, v = _rows_last_contig(k), _rows_last_contig(v)
     B, H, N, D = k.shape
@@ -275,8 +275,7 @@ def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None):
                                  _ptr(gy), _s3(gy), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), ws.numel(),
                                  C.c_void_p(_stream_ptr(k.device)))
     _lib.check(rc, "flare_mixer_bwd")
-    gq = dq.sum(0) if q.dim() == 3 else dq
-    return gq.to(q.dtype), dk, dv
+    return dq if q.dim() != 3 else dq[0] if B == 1 else dq.sum(0), dk, dv
 
 
 #: elements of one [B,H,M,T] fp32 temporary of the tiled gradients below (64 MiB); about six such temporaries are
@@ -437,9 +436,16 @@ def _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, km, gy, drop=None):
 
 
 class _MixerFn(torch.autograd.Function):
+    """q16: q as the kernels take it (cast for autocast, its heads filled up with zero columns to those of k and v), where that is
+    another tensor; the gradient then goes to q itself, in q's type and width, without the cast's and the padding's own nodes."""
+
     @staticmethod
-    def forward(ctx, q, k, v, scale, key_mask, n_splits, force_generic, token_major):
+    def forward(ctx, q, k, v, scale, key_mask, n_splits, force_generic, token_major, q16=None):
         ctx.scale, ctx.key_mask = scale, key_mask
+        ctx.q_dtype, ctx.q_width = q.dtype, q.shape[-1]
+        ctx.set_materialize_grads(False)      # z's gradient, which nobody reads, would be a launch
+        if q16 is not None:
+            q = q16
         ctx.hip = _hip_backward_ok(q, k, v, key_mask, force_generic)
         if ctx.hip:
             y, z, lse_lat, lse_tok = _mixer_forward(q, k, v, scale, key_mask, n_splits, force_generic, token_major, True)
@@ -458,6 +464,8 @@ class _MixerFn(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, gy, _gz):
+        if gy is None:
+            return (None,) * 9
         if ctx.hip:
             q, k, v, y, z, lse_lat, lse_tok = ctx.saved_tensors
             gq, gk, gv = _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, ctx.scale, ctx.key_mask, gy)
@@ -465,7 +473,16 @@ class _MixerFn(torch.autograd.Function):
             q, k, v, *stats = ctx.saved_tensors
             gq, gk, gv = _mixer_torch_grad(q, k, v, ctx.scale, ctx.key_mask, gy,
                                            stats=(stats[1], stats[0], stats[2]) if stats else None)
-        return gq, gk, gv, None, None, None, None, None
+        return gq[..., :ctx.q_width].to(ctx.q_dtype), gk, gv, None, None, None, None, None, None
+
+
+def mixer_narrow_heads(q, k, v, scale):
+    """y of the differentiable mixer for latents q [H,M,D] and 16-bit k, v [B,H,N,16] whose heads hold D channels followed by zeros (as
+    the projections write them); y is head-padded like them, token-major in memory."""
+    q16 = torch.zeros(*q.shape[:-1], k.shape[-1], dtype=k.dtype, device=k.device)
+    with torch.no_grad():
+        q16[..., :q.shape[-1]].copy_(q)
+    return _MixerFn.apply(q, k, v, float(scale), None, 0, False, True, q16)[0]
 
 
 class _MixerDropoutFn(torch.autograd.Function):
@@ -492,6 +509,7 @@ class _MixerDropoutFn(torch.autograd.Function):
         if ctx.hip:
             q, k, v, y, z, lse_lat, lse_tok = ctx.saved_tensors
             gq, gk, gv = _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, ctx.scale, ctx.key_mask, gy, ctx.drop)
+            gq = gq.to(q.dtype)
         else:
             q, k, v = ctx.saved_tensors
             gq, gk, gv = _mixer_torch_grad(q, k, v, ctx.scale, ctx.key_mask, gy, ctx.drop)
@@ -537,8 +555,10 @@ def flare_multihead_mixer(q, k, v, scale: float = 1.0, key_mask=None, return_z: 
     run forward and backward on the 16x16x32 kernels, fp32 problems on the fp32 matrix-core kernels.
     """
     ac = _autocast_dtype(k)
+    q_in = q
     if ac is not None:
         q, k, v = (t if t.dtype == ac else t.to(ac) for t in (q, k, v))
+    q_cast = q
     if dropout_p > 0.0:
         if not dropout_p < 1.0:
             raise ValueError("dropout_p must be in [0, 1)")
@@ -581,7 +601,10 @@ def flare_multihead_mixer(q, k, v, scale: float = 1.0, key_mask=None, return_z: 
         if token_major_out:
             y = y.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
     elif needs_grad:
-        y, z = _MixerFn.apply(q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out)
+        # the cast of the latents for autocast stays inside the function
+        cast = q is q_cast and q is not q_in and q_in.dtype == torch.float32
+        y, z = _MixerFn.apply(q_in if cast else q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out,
+                              q.detach() if cast else None)
     else:
         y, z = _mixer_forward(q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out)
     if pad:

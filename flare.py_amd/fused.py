@@ -22,8 +22,8 @@ projection of a FLAREBlock at the reference's default ratios) runs through `_Fus
 launch, and a backward that recomputes the chain per token tile in one launch (flare_mlp_bwd) and forms the
 parameter gradients from the rows it leaves with one more launch (flare_mlp_wgrad); the expanding two-layer MLP has a
 backward launch of its own (flare_mlp_expand_bwd).  A stack with a narrow first input or last output keeps that one
-layer as a torch layer while gradients are enabled and sends the C x C layers between through the same path; the
-head-padded variants have no backward.
+layer as a torch layer while gradients are enabled and sends the C x C layers between through the same path.
+Head-padded rows (narrow heads) have a backward in the few-token launches.
 """
 from __future__ import annotations
 
@@ -505,11 +505,26 @@ def _pair_info(x, mod_a, mod_b, cd):
     return (layers, *infos[0][1:])
 
 
-def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None):
+def narrow_train_ok(x, mod_a, mod_b, out):
+    """True where a training step may keep narrow heads padded between the projections, the mixer and the output projection: the
+    few-token launches differentiate head-padded rows (x: the rows the projections read; out: a Linear of their width)."""
+    info = _pair_info(x, mod_a, mod_b, None)
+    return (info is not None and isinstance(out, nn.Linear) and _train_subchain(mod_a) is None and _train_subchain(mod_b) is None
+            and out.in_features == out.out_features == x.shape[-1] and _chain_tiles(info[0] + [out]) is not None)
+
+
+def project_padded(y, out, cd, head, res, out_dtype):
+    """[res +] out(y) for rows y of padded heads, differentiable where narrow_train_ok() says so."""
+    if torch.is_grad_enabled():
+        return _fused_mlp_train(y, out, cd, None, res, out_dtype, head)
+    return fused_mlp(y, out, cd, res=res, out_dtype=out_dtype, x_head=head)
+
+
+def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None, y_head=0):
     """(mod_a(norm(x)), mod_b(norm(x))) as fused_mlp computes them, for two stacks that read the same rows through the
     same norm (a block's k and v projections).  With gradients enabled and both stacks plain chains of C x C layers the
     pair is one autograd node whose backward sums the two gradients of x inside the second launch (few tokens: one backward
-    launch for both stacks)."""
+    launch for both stacks).  y_head: as fused_mlp's, with gradients enabled where narrow_train_ok() says so."""
     if torch.is_grad_enabled() and all(_train_subchain(m) is None and not _expand_factor(m, x.shape[-1]) for m in (mod_a, mod_b)):
         has_norm = norm is not None and not isinstance(norm, nn.Identity)
         gamma = getattr(norm, "weight", None) if has_norm else None
@@ -518,8 +533,9 @@ def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None):
         for m in (mod_a, mod_b):
             layers = _layers_of(m)[0]
             wb += [l.weight for l in layers] + [l.bias for l in layers]
-        return _FusedPairFn.apply(mod_a, mod_b, cd, norm if has_norm else None, out_dtype, x, gamma, beta, *wb)
-    return fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype), fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype)
+        return _FusedPairFn.apply(mod_a, mod_b, cd, norm if has_norm else None, (out_dtype, y_head), x, gamma, beta, *wb)
+    return (fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head),
+            fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head))
 
 
 def _forward_plan(mod):
@@ -697,10 +713,11 @@ class _FusedMlpFn(torch.autograd.Function):
     (x, res, gamma, beta, w_0 .. w_{L-1}, b_0 .. b_{L-1}) with None where a tensor does not exist."""
 
     @staticmethod
-    def forward(ctx, mod, cd, norm, out_dtype, x, res, gamma, beta, *wb):
+    def forward(ctx, mod, cd, norm, fmt, x, res, gamma, beta, *wb):
+        out_dtype, x_head = fmt
         with torch.no_grad():
-            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype, train=True)
-        ctx.mod, ctx.cd, ctx.norm = mod, cd, norm
+            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype, x_head=x_head, train=True)
+        ctx.mod, ctx.cd, ctx.norm, ctx.x_head = mod, cd, norm, x_head
         # res and x one tensor: dy is added to dx inside the kernel.  (Two tensors over the same memory are not
         # enough: one of them may be detached, and then its path carries no gradient.)
         ctx.res_is_x = res is x
@@ -720,11 +737,11 @@ class _FusedMlpFn(torch.autograd.Function):
         if ctx.versions != tuple(None if t is None else t._version for t in ctx.params):
             raise RuntimeError("a parameter of the fused MLP was modified in place between its forward and its backward")
         mod, cd, norm = ctx.mod, ctx.cd, ctx.norm
-        if _expand_factor(mod, x.shape[-1]):
+        if not ctx.x_head and _expand_factor(mod, x.shape[-1]):
             return _backward_expand(ctx, dy, x, _expand_factor(mod, x.shape[-1]))
-        dx, gsum, dW, db, layers = _chain_backward(mod, cd, norm, x, dy, ctx.res_is_x)
+        dx, gsum, dW, db, layers = _chain_backward(mod, cd, norm, x, dy, ctx.res_is_x, x_head=ctx.x_head)
         L = len(layers)
-        need = ctx.needs_input_grad            # (mod, cd, norm, out_dtype, x, res, gamma, beta, *wb)
+        need = ctx.needs_input_grad            # (mod, cd, norm, fmt, x, res, gamma, beta, *wb)
         grads = [None, None, None, None]
         grads.append(dx.view(x.shape) if need[4] else None)
         grads.append(None if (not ctx.has_res or ctx.res_is_x or not need[5]) else dy)
@@ -743,22 +760,26 @@ def _norm_grads(norm, gsum, need_gamma, need_beta):
             gsum[1].to(norm.bias.dtype) if (need_beta and getattr(norm, "bias", None) is not None) else None]
 
 
-def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
+def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     """Backward of y = [x +] chain(norm(x)) for the chain of C x C layers: (dx [T,C], the norm's [2,C] sums or None,
     dW [L,out,in], db [L,C] or None, the layers).  dx_acc: a [T,C] gradient of the same x that another chain left
-    (x's dtype, contiguous); the kernel adds its result into it and it is returned as dx."""
+    (x's dtype, contiguous); the kernel adds its result into it and it is returned as dx.  x_head: rows of x and dx hold padded
+    heads (few tokens only)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _layers_of(mod)
     L = len(layers)
-    Cdim = x.shape[-1]
-    few = _few(x.numel() // Cdim, Cdim, L)
+    Cdim, xw = layers[0].in_features, x.shape[-1]
+    x = x.reshape(-1, xw)
+    few = _few(x.shape[0], Cdim, L)
     packed = _packed_few(mod, layers, cd, True) if few else None
     if packed is not None:
         w_img, b, wt_img = packed            # the tiled operands
+    elif x_head:
+        raise RuntimeError("head-padded rows have a backward in the few-token launches only")
     else:
         few = 0
         _, b, w_img, wt_img = _packed_train(mod, layers, cd)
-    x2 = x.reshape(-1, Cdim)
+    x2 = x
     if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
     dy2 = _rows2d(dy, Cdim)
@@ -769,10 +790,11 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
     d.w_dtype, d.x_dtype, d.y_dtype = _dtype_code(w_img), _dtype_code(x2), _dtype_code(dy2)
     d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
     d.x_stride, d.y_stride = x2.stride(0), dy2.stride(0)
+    d.flags = (x_head // 4) << 8
     gamma, beta = _norm_args(d, norm, x, Cdim)
     if dx_acc is not None and (dx_acc.shape != (T, Cdim) or dx_acc.dtype != x2.dtype or not dx_acc.is_contiguous()):
         raise ValueError("dx_acc must be a contiguous [T, C] tensor of x's dtype")
-    dx = dx_acc if dx_acc is not None else torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
+    dx = dx_acc if dx_acc is not None else torch.empty(T, xw, dtype=x2.dtype, device=dev)
     a_in = torch.empty(L, T, Cdim, dtype=cd, device=dev)
     g_out = torch.empty(L, T, Cdim, dtype=cd, device=dev)
     dn = stats = gb = gsum = None
@@ -803,8 +825,8 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None):
     return dx, gsum, dW, db, layers
 
 
-def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb):
-    """Backward of both stacks of a pair in one launch: (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
+def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0):
+    """Backward of both stacks of a pair in one launch (y_head: dya and dyb are rows of padded heads): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
     None, the 2 L layers)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _pair_info(x, mod_a, mod_b, cd)
@@ -813,7 +835,8 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb):
     x2 = x.reshape(-1, Cdim)
     if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
-    da, db_ = _rows2d(dya, Cdim), _rows2d(dyb, Cdim)
+    yw = Cdim // y_head * 16 if y_head else Cdim
+    da, db_ = _rows2d(dya, yw), _rows2d(dyb, yw)
     if da.dtype != db_.dtype:
         da, db_ = da.float(), db_.float()
     if da.stride() != db_.stride():
@@ -824,6 +847,7 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb):
     d.w_dtype, d.x_dtype, d.y_dtype = _dtype_code(w), _dtype_code(x2), _dtype_code(da)
     d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
     d.x_stride, d.y_stride = x2.stride(0), da.stride(0)
+    d.flags = (y_head // 4) << 12
     gamma, beta = _norm_args(d, norm, x, Cdim)
     dx = torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
     rows = torch.empty(2, L2, T, Cdim, dtype=cd, device=dev)         # a_in, g_out
@@ -846,17 +870,20 @@ class _FusedPairFn(torch.autograd.Function):
     [T, C] arrays.  Inputs: (x, gamma, beta, weights and biases of a, weights and biases of b)."""
 
     @staticmethod
-    def forward(ctx, mod_a, mod_b, cd, norm, out_dtype, x, gamma, beta, *wb):
+    def forward(ctx, mod_a, mod_b, cd, norm, fmt, x, gamma, beta, *wb):
+        out_dtype, y_head = fmt
         with torch.no_grad():
             info = _pair_info(x, mod_a, mod_b, cd)
             packed = None if info is None else _packed_few(mod_a, info[0], cd, True)
             ctx.pair = packed is not None
             n = len(info[0]) // 2 if ctx.pair else 0
-            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, train=True,
+            if y_head and not ctx.pair:
+                raise ValueError("head-padded rows have no backward here: call under torch.no_grad()")
+            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
                                 operands=(packed[0][:n], packed[1][:n]) if ctx.pair else None)
-            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, train=True,
+            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
                                 operands=(packed[0][n:], packed[1][n:]) if ctx.pair else None)
-        ctx.mods, ctx.cd, ctx.norm = (mod_a, mod_b), cd, norm
+        ctx.mods, ctx.cd, ctx.norm, ctx.y_head = (mod_a, mod_b), cd, norm, y_head
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)
         ctx.save_for_backward(x)
@@ -870,7 +897,7 @@ class _FusedPairFn(torch.autograd.Function):
             raise RuntimeError("a parameter of the fused MLP was modified in place between its forward and its backward")
         mod_a, mod_b = ctx.mods
         if ctx.pair:
-            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb)
+            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb, ctx.y_head)
             n = len(layers) // 2
             la, lb, dWa, dWb = layers[:n], layers[n:], dW[:n], dW[n:]
             dba, dbb = (None, None) if db is None else (db[:n], db[n:])
@@ -878,7 +905,7 @@ class _FusedPairFn(torch.autograd.Function):
             dx, gs_a, dWa, dba, la = _chain_backward(mod_a, ctx.cd, ctx.norm, x, dya, False)
             dx, gs_b, dWb, dbb, lb = _chain_backward(mod_b, ctx.cd, ctx.norm, x, dyb, False, dx_acc=dx)
             gs = None if gs_a is None else gs_a + gs_b
-        need = ctx.needs_input_grad            # (mod_a, mod_b, cd, norm, out_dtype, x, gamma, beta, *wb)
+        need = ctx.needs_input_grad            # (mod_a, mod_b, cd, norm, fmt, x, gamma, beta, *wb)
         grads = [None, None, None, None, None, dx.view(x.shape) if need[5] else None]
         grads += _norm_grads(ctx.norm, gs, need[6], need[7])
         at = 8
@@ -939,7 +966,7 @@ def _backward_expand(ctx, dy, x, E):
     _lib.check(rc, "flare_mlp_expand_bwd")
     dW1, db1 = _weight_grads(d, dt, n_row, f1.bias is not None)          # [E, C(hidden chunk), C(in)], [E, C]
     dW2, db2 = _weight_grads(d, dy_row, h, f2.bias is not None, L=E)     # [E, C(out), C(hidden chunk)], [E, C] (E equal rows)
-    need = ctx.needs_input_grad            # (mod, cd, norm, out_dtype, x, res, gamma, beta, w1, w2, b1, b2)
+    need = ctx.needs_input_grad            # (mod, cd, norm, fmt, x, res, gamma, beta, w1, w2, b1, b2)
     grads = [None, None, None, None]
     grads.append(dx.view(x.shape) if need[4] else None)
     grads.append(None if (not ctx.has_res or ctx.res_is_x or not need[5]) else dy)
@@ -955,10 +982,10 @@ def _backward_expand(ctx, dy, x, E):
     return tuple(grads)
 
 
-def _fused_mlp_train(x, mod, cd, norm, res, out_dtype):
+def _fused_mlp_train(x, mod, cd, norm, res, out_dtype, x_head=0):
     layers = _layers_of(mod)[0]
     has_norm = norm is not None and not isinstance(norm, nn.Identity)
     gamma = getattr(norm, "weight", None) if has_norm else None
     beta = getattr(norm, "bias", None) if has_norm else None
     wb = [l.weight for l in layers] + [l.bias for l in layers]
-    return _FusedMlpFn.apply(mod, cd, norm if has_norm else None, out_dtype, x, res, gamma, beta, *wb)
+    return _FusedMlpFn.apply(mod, cd, norm if has_norm else None, (out_dtype, x_head), x, res, gamma, beta, *wb)

@@ -20,7 +20,7 @@ from torch import nn
 from torch.nn import functional as F
 
 from . import block_plan, fused, rows
-from .functional import flare_multihead_mixer
+from .functional import flare_multihead_mixer, mixer_narrow_heads
 
 __all__ = ["ResidualMLP", "FLARE", "FLAREBlock", "FinalLayer", "FLAREModel"]
 
@@ -198,21 +198,25 @@ class FLARE(nn.Module):
         q = self.latent_q.view(self.num_heads, self.num_latents, self.head_dim)
         cd = self._fusable(x, return_scores)
         D = self.head_dim
-        # (head-padded rows have no backward: with gradients enabled the generic fused branch pads inside the mixer)
-        narrow = (cd is not None and not torch.is_grad_enabled() and D in (4, 8) and self.num_latents % 32 == 0 and not self.qk_norm
+        # narrow heads: the projections write k, v head-padded to 16 columns, which is what the mixer's matrix-core kernels take, and
+        # the output projection reads the mixer's padded rows: no copies between
+        narrow = (cd is not None and D in (4, 8) and self.num_latents % 32 == 0 and not self.qk_norm
                   # head-padded rows exist for the chain of square layers only: an expanding two-layer k/v projection
                   # takes the generic fused branch below, where the mixer pads the heads itself
-                  and not fused._expand_factor(self.k_proj, C) and not fused._expand_factor(self.v_proj, C))
+                  and not fused._expand_factor(self.k_proj, C) and not fused._expand_factor(self.v_proj, C)
+                  # with gradients enabled they exist where the few-token launches run
+                  and (not torch.is_grad_enabled() or fused.narrow_train_ok(x, self.k_proj, self.v_proj, self.out_proj)))
         if narrow:
-            # narrow heads: the projections write k, v head-padded to 16 columns, which is what the mixer's
-            # matrix-core kernels take, and the output projection reads the mixer's padded rows: no copies between
             H = self.num_heads
-            k = fused.fused_mlp(x, self.k_proj, cd, norm=_norm, out_dtype=cd, y_head=D).view(B, N, H, 16).permute(0, 2, 1, 3)
-            v = fused.fused_mlp(x, self.v_proj, cd, norm=_norm, out_dtype=cd, y_head=D).view(B, N, H, 16).permute(0, 2, 1, 3)
-            y = flare_multihead_mixer(self._cached_q(cd, 16 - D), k, v, scale=self.attn_scale, token_major_out=True)
+            k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd, y_head=D)
+            k, v = (t.view(B, N, H, 16).permute(0, 2, 1, 3) for t in (k, v))
+            if torch.is_grad_enabled():
+                y = mixer_narrow_heads(q, k, v, self.attn_scale)
+            else:
+                y = flare_multihead_mixer(self._cached_q(cd, 16 - D), k, v, scale=self.attn_scale, token_major_out=True)
             y = y.permute(0, 2, 1, 3).reshape(B, N, H * 16)          # a view: the kernel laid y out as [B,N,H,16]
             out_dtype = _res.dtype if _res is not None else x.dtype
-            return fused.fused_mlp(y, self.out_proj, cd, res=_res, out_dtype=out_dtype, x_head=D), None
+            return fused.project_padded(y, self.out_proj, cd, D, _res, out_dtype), None
         if cd is not None:
             k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd)
             k, v = self._heads(k), self._heads(v)

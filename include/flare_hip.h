@@ -409,7 +409,7 @@ int flare_mlp_bwd_partial_rows(const FlareMlpDesc* desc, int32_t* rows);
  *   ((row / 16 * (C / 32) + col / 32) * 4 + col % 32 / 8) * 128 + row % 16 * 8 + col % 8.
  * flare_mlp_few: 0 where the kernels above serve the descriptor (T, C, L, w_dtype, flags are read), else the rows of gb_part that
  * flare_mlp_few_bwd writes.  Forward: flare_mlp_fwd with FLARE_MLP_W_TILED in desc->flags (chain and head-padded rows).
- * flare_mlp_few_bwd: as flare_mlp_bwd (flags == 0), w and wt the tiled weights and transposes, gb_part [rows,2,C] summed in the
+ * flare_mlp_few_bwd: as flare_mlp_bwd (flags: head-padded rows only, FLARE_MLP_X_HEAD for x and dx, FLARE_MLP_Y_HEAD for dy), w and wt the tiled weights and transposes, gb_part [rows,2,C] summed in the
  * launch (no dn, no stats; flare_mlp_wgrad_norm adds the rows up).  With dy_b it differentiates two chains of equal L, masks and
  * activation that read the same rows through the same norm (a block's k and v projections, pdebench/models/flare.py:139-140):
  * chain a is tiles 0 .. L-1 and chain b tiles L .. 2L-1 of w / wt [2L,C,C] and bias [2L,C]; dy_a, dy_b share dtype and row

@@ -13,6 +13,7 @@ from torch import nn
 import flare_py_amd as F
 from flare_py_amd import fused
 from flare_py_amd.modules import ResidualMLP
+from oracle import flare_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -527,3 +528,47 @@ def test_pair_of_chains_against_fp32_torch_layers(dev, C, num_layers, T, kind, d
         assert torch.equal(y, z)
     for i, (a, b) in enumerate(zip(got, ref)):
         assert rel(a.float(), b) <= 3e-2, i
+
+
+@pytest.mark.parametrize("C,H,B,N", [(32, 8, 2, 7), (64, 16, 1, 17), (64, 8, 1, 1), (64, 8, 2, 2001), (32, 4, 1, 16384)])
+@pytest.mark.parametrize("cd,rms", [(torch.bfloat16, False), (torch.float16, True)])
+def test_narrow_heads_stay_padded_in_training(dev, monkeypatch, C, H, B, N, cd, rms):
+    """Head dims of 4 and 8 with gradients: the projections write padded rows, the mixer's and the projections' backwards read and write
+    them.  Outputs and gradients are as near to the fp64 oracle as those of the path that pads inside the mixer (a quarter more is
+    room for another order of the same roundings; 2e-3 for results that both get to 16-bit precision)."""
+    torch.manual_seed(N)
+    blk = F.FLAREBlock(channel_dim=C, num_heads=H, num_latents=32, rmsnorm=rms).to(dev)
+    for l in blk.modules():
+        if isinstance(l, nn.Linear):
+            l.reset_parameters()
+    x = torch.randn(B, N, C, device=dev, requires_grad=True)
+    gy = torch.randn(B, N, C, device=dev)
+    assert fused.narrow_train_ok(x, blk.att.k_proj, blk.att.v_proj, blk.att.out_proj)
+
+    def step():
+        with torch.autocast("cuda", dtype=cd):
+            y = blk(x)[0]
+        return [y.detach(), *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
+
+    got = step()
+    monkeypatch.setattr(fused, "narrow_train_ok", lambda *a: False)
+    other = step()
+    sd = {k: v.detach().cpu().double().requires_grad_(True) for k, v in blk.state_dict().items()}
+    x64 = x.detach().cpu().double().requires_grad_(True)
+    y64 = O.flare_block(sd, "", x64, H, rmsnorm=rms)
+    want = [y64.detach(), *torch.autograd.grad(y64, [x64, *(sd[n] for n, _ in blk.named_parameters())], gy.cpu().double())]
+    for i, (a, b, r) in enumerate(zip(got, other, want)):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        ea, eb = (float((t.cpu().double() - r).norm() / (r.norm() + 1e-300)) for t in (a, b))
+        assert ea <= 1.25 * eb + 2e-3, (i, ea, eb)
+
+
+def test_padded_rows_beyond_the_few_token_launches_are_refused(dev):
+    m = ResidualMLP(64, 64, 64, num_layers=1).to(dev)
+    x = torch.randn(16385, 64, device=dev, requires_grad=True)
+    assert not fused.narrow_train_ok(x, m, m, nn.Linear(64, 64).to(dev))
+    with pytest.raises(ValueError, match="head-padded"):
+        fused.fused_mlp_pair(x, m, m, torch.bfloat16, out_dtype=torch.bfloat16, y_head=8)
+    y = fused.project_padded(torch.randn(16385, 128, device=dev), nn.Linear(64, 64).to(dev), torch.bfloat16, 8, None, torch.float32)
+    with pytest.raises(RuntimeError, match="head-padded"):
+        y.sum().backward()
