@@ -132,6 +132,8 @@ SYMBOLS = {
     "flare_mlp_wgrad_norm": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, C.c_int32, _P, _P]),
     "flare_mlp_few": (C.c_int, [C.POINTER(FlareMlpDesc)]),
     "flare_mlp_few_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
+    "flare_mlp_few_bwd_res": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
+    "flare_mlp_few_pair_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_act_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_layer_bwd_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),

@@ -118,6 +118,13 @@ def _build(block, x, cd):
              _mlp(mlp, T, cd, x.dtype, x.dtype, Cdim, Cdim, norm=block.norm2, res=x.dtype)]
     if any(p is None for p in parts):
         return None
+    # few tokens: the projections' weights in one piece, so that one launch serves both
+    info = fused._pair_info(x, att.k_proj, att.v_proj, cd)
+    packed = None if info is None else fused._packed_few(att.k_proj, info[0], cd, False)
+    if packed is not None:
+        n = len(info[0]) // 2
+        parts[0] = (parts[0][0], packed[0][:n], packed[1][:n], *parts[0][3:])
+        parts[1] = (parts[1][0], packed[0][n:], packed[1][n:], *parts[1][3:])
     q = att._cached_q(cd, Dp - D)
     plan = _Plan()
     d = plan.desc = _lib.FlareBlockDesc()

@@ -1033,7 +1033,7 @@ int flare_causal_linear_bwd(const FlareCausalLinearDesc* desc, const void* q, co
 
 static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const float* w_in, const float* b_in, int out_dim,
                         const void* x, const void* w, const float* bias, const float* gamma, const float* beta,
-                        const void* res, void* y, void* stream)
+                        const void* res, void* y, void* y2, void* stream)
 {
     if (!d) return fail(FLARE_EINVAL, "descriptor is NULL");
     if (d->T < 1 || d->L < 1 || d->L > 16) return fail(FLARE_EINVAL, "T >= 1 and 1 <= L <= 16 required (got %lld, %d)", (long long)d->T, d->L);
@@ -1073,7 +1073,7 @@ static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const flo
         return fail(FLARE_EINVAL, "w, bias, gamma, beta must be 16-byte aligned");
     flare::MlpArgs a;
     memset(&a, 0, sizeof(a));
-    a.x = x; a.res = res; a.y = y; a.w = static_cast<const uint16_t*>(w); a.bias = bias; a.gamma = gamma; a.beta = beta;
+    a.x = x; a.res = res; a.y = y; a.y2 = y2; a.w = static_cast<const uint16_t*>(w); a.bias = bias; a.gamma = gamma; a.beta = beta;
     a.T = d->T; a.C = d->C; a.L = d->L;
     a.x_dtype = d->x_dtype; a.res_dtype = d->res_dtype; a.y_dtype = d->y_dtype;
     a.norm = d->norm; a.eps = d->eps; a.act = d->act; a.act_mask = d->act_mask; a.add_mask = d->add_mask;
@@ -1092,6 +1092,14 @@ static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const flo
     return hip_status(flare::launch_mlp_mfma(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp launch");
 }
 
+int flare_mlp_few_pair_fwd(const FlareMlpDesc* d, const void* x, const void* w, const float* bias, const float* gamma, const float* beta,
+                           void* y_a, void* y_b, void* stream)
+{
+    if (!d || !(d->flags & FLARE_MLP_W_TILED)) return fail(FLARE_EINVAL, "a pair of chains takes tiled weights");
+    if (!y_b || !aligned16(y_b)) return fail(FLARE_EINVAL, "y_b must be 16-byte aligned and not NULL");
+    return mlp_fwd_impl(d, 0, 0, nullptr, nullptr, 0, x, w, bias, gamma, beta, nullptr, y_a, y_b, stream);
+}
+
 int flare_mlp_few(const FlareMlpDesc* d)
 {
     return d && d->T >= 1 && !(d->flags & FLARE_MLP_EXPAND) && flare::mlp_mfma_supported(d->w_dtype, d->C) && flare::mlp_few_ok(d->T, d->C, d->L)
@@ -1101,14 +1109,14 @@ int flare_mlp_few(const FlareMlpDesc* d)
 int flare_mlp_fwd(const FlareMlpDesc* d, const void* x, const void* w, const float* bias, const float* gamma,
                   const float* beta, const void* res, void* y, void* stream)
 {
-    return mlp_fwd_impl(d, 0, 0, nullptr, nullptr, 0, x, w, bias, gamma, beta, res, y, stream);
+    return mlp_fwd_impl(d, 0, 0, nullptr, nullptr, 0, x, w, bias, gamma, beta, res, y, nullptr, stream);
 }
 
 int flare_mlp_io_fwd(const FlareMlpDesc* d, int32_t in_dim, int32_t in_act, const float* w_in, const float* b_in,
                      int32_t out_dim, const void* x, const void* w, const float* bias, const float* gamma,
                      const float* beta, const void* res, void* y, void* stream)
 {
-    return mlp_fwd_impl(d, in_dim, in_act, w_in, b_in, out_dim, x, w, bias, gamma, beta, res, y, stream);
+    return mlp_fwd_impl(d, in_dim, in_act, w_in, b_in, out_dim, x, w, bias, gamma, beta, res, y, nullptr, stream);
 }
 
 // Scratch of a block's forward: k rows, v rows, the mixer's output rows, the mixer's workspace with z at its tail.  The attention's result
@@ -1164,7 +1172,14 @@ int flare_block_fwd(const FlareBlockDesc* d, const void* x, void* y, void* scrat
     auto mlp = [&](int i, const void* in, const void* res, void* out) {
         return flare_mlp_fwd(&d->mlp[i], in, d->w[i], d->b[i], d->gamma[i], d->beta[i], res, out, stream);
     };
-    if ((rc = mlp(0, x, nullptr, k)) != FLARE_OK || (rc = mlp(1, x, nullptr, v)) != FLARE_OK) return rc;
+    // few tokens: both projections in one launch where their weights lie in one piece
+    const FlareMlpDesc &dk = d->mlp[0], &dv = d->mlp[1];
+    if ((dk.flags & FLARE_MLP_W_TILED) && memcmp(&dk, &dv, sizeof(dk)) == 0 && d->gamma[0] == d->gamma[1] && d->beta[0] == d->beta[1] &&
+        static_cast<const uint16_t*>(d->w[0]) + (size_t)dk.L * dk.C * dk.C == d->w[1] && d->b[0] && d->b[0] + (size_t)dk.L * dk.C == d->b[1])
+        rc = flare_mlp_few_pair_fwd(&dk, x, d->w[0], d->b[0], d->gamma[0], d->beta[0], k, v, stream);
+    else if ((rc = mlp(0, x, nullptr, k)) == FLARE_OK)
+        rc = mlp(1, x, nullptr, v);
+    if (rc != FLARE_OK) return rc;
     if ((rc = flare_mixer_fwd(&d->mixer, d->q, k, v, nullptr, ym, nullptr, base + s.ws, s.ws_bytes, stream)) != FLARE_OK) return rc;
     if ((rc = mlp(2, ym, x, x1)) != FLARE_OK) return rc;
     return mlp(3, x1, x1, y);
@@ -1205,7 +1220,8 @@ static int check_mlp_bwd_common(const FlareMlpDesc* d, const void* x, const void
 
 static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
                         const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
-                        void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream, bool few, const void* dy2)
+                        void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream, bool few, const void* dy2,
+                        const void* dres)
 {
     int rc = check_mlp_bwd_common(d, x, dy, w_img, wt_img, bias, gamma, beta, dx, dn, stats, gb_part, gb);
     if (rc != FLARE_OK) return rc;
@@ -1222,7 +1238,7 @@ static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, co
     if (!aligned16(a_in) || !aligned16(g_out)) return fail(FLARE_EINVAL, "every buffer must be 16-byte aligned");
     flare::MlpBwdArgs a;
     memset(&a, 0, sizeof(a));
-    a.x = x; a.dy = dy; a.dy2 = dy2; a.dx = dx;
+    a.x = x; a.dy = dy; a.dy2 = dy2; a.dres = dres; a.dx = dx;
     a.w = static_cast<const uint16_t*>(w_img); a.wt = static_cast<const uint16_t*>(wt_img);
     a.bias = bias; a.gamma = gamma; a.beta = beta;
     a.a_in = static_cast<uint16_t*>(a_in); a.g_out = static_cast<uint16_t*>(g_out);
@@ -1242,17 +1258,25 @@ int flare_mlp_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const vo
                   const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
                   void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream)
 {
-    return mlp_bwd_impl(d, x, dy, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, dn, stats, gb_part, gb, stream, false, nullptr);
+    return mlp_bwd_impl(d, x, dy, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, dn, stats, gb_part, gb, stream, false, nullptr, nullptr);
 }
 
 int flare_mlp_few_bwd(const FlareMlpDesc* d, const void* x, const void* dy_a, const void* dy_b, const void* w_img, const void* wt_img,
                       const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in, void* g_out,
                       float* gb_part, void* stream)
 {
+    return flare_mlp_few_bwd_res(d, x, dy_a, dy_b, nullptr, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, gb_part, stream);
+}
+
+int flare_mlp_few_bwd_res(const FlareMlpDesc* d, const void* x, const void* dy_a, const void* dy_b, const void* dres, const void* w_img,
+                          const void* wt_img, const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx,
+                          void* a_in, void* g_out, float* gb_part, void* stream)
+{
+    if (dres && (!aligned16(dres) || (d && ((d->flags >> 8) & 15)))) return fail(FLARE_EINVAL, "dres must be 16-byte aligned rows, not next to padded heads of x");
     if (!flare_mlp_few(d)) return fail(FLARE_EUNSUPPORTED, "the few-token launch runs only where flare_mlp_few says so");
     if (dy_b && !aligned16(dy_b)) return fail(FLARE_EINVAL, "dy_b must be 16-byte aligned");
     // the shared checks ask for dn and stats, which this launch does without
-    return mlp_bwd_impl(d, x, dy_a, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, gb_part, gb_part, gb_part, nullptr, stream, true, dy_b);
+    return mlp_bwd_impl(d, x, dy_a, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, gb_part, gb_part, gb_part, nullptr, stream, true, dy_b, dres);
 }
 
 int flare_mlp_expand_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,

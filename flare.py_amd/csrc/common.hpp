@@ -273,6 +273,7 @@ struct CausalLinearDkvArgs {
 
 struct MlpArgs {
     const void* x; const void* res; void* y;   // [T,C] rows; res may be null
+    void* y2;                                   // few-token launch only: a second chain's output (tiles and biases L .. 2 L - 1), or null
     const uint16_t* w;                          // [L,C,C] 16-bit weights, row-major [out][in]
     const float* bias;                          // [L,C] or null
     const float* gamma; const float* beta;      // [C] norm parameters (beta may be null)
@@ -297,6 +298,7 @@ struct MlpArgs {
 struct MlpBwdArgs {
     const void* x; const void* dy; void* dx;    // [T,C] rows: the forward's input, the gradient of its output, the gradient of x
     const void* dy2;                            // few-token launch only: gradient of the second chain's output (tiles L .. 2 L - 1), or null
+    const void* dres;                           // few-token launch only: [T,C] rows of dx's type that are added to dx, or null
     int x_head, y_head;                         // few-token launch only: as MlpArgs, for the rows of x and dx / of dy
     const uint16_t* w; const uint16_t* wt;      // [L,C,C] 16-bit weights [out][in] and their transposes [in][out]
     const float* bias;                          // [L,C] or null

@@ -9,6 +9,8 @@
 // requested at the very start, straight into registers, and a layer is one LDS exchange of the 16 x C activations (each wave
 // writes its 16 channels in B-operand order, one barrier, everybody reads all of them) and C / 32 products.  The price is
 // that every 16 tokens read all weights again from the L2, which is what ends the range this is used in.
+// Two chains that read the same rows (a block's k and v projections) are one launch each way: with the
+// forward pair, one packing launch a block and the residual's gradient added here, the step of 8 blocks went from 1689 to 1608 us.
 // 4096 tokens, C = 128, five layers, in a replayed graph: forward 17.3 -> 9.1 us, backward 37.6 + 8.6 + 4.6 (norm sums) -> 16.2
 // us, two chains of it 102 -> 27 us; the 8-block model's training step 3.68 -> 1.81 ms (with one launch for the sums over
 // partial results and 256-token ranges in mlp_wgrad_mfma.hip).
@@ -211,6 +213,7 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
     const int L = a.L;
     const bool has_bias = a.bias != nullptr;
     const int ch0 = 16 * w + 4 * g;                               // this lane's four channels of the stream
+    const int chain = blockIdx.y;                                 // 1: the second chain of a pair
 
     const int64_t t = (int64_t)blockIdx.x * 16 + c16;
     const bool live = t < a.T;
@@ -235,7 +238,7 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
     f32x4 bias[LMAX];
 #pragma unroll
     for (int l = 0; l < LMAX; ++l) {
-        const size_t tile = l < L ? l : L - 1;
+        const size_t tile = (size_t)chain * L + (l < L ? l : L - 1);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) wr[l][ks] = operand<C>(a.w, tile, w, ks, lane);
         // a missing bias reads the weights instead (any mapped memory will do) and is replaced by zeros where it is used
@@ -277,8 +280,9 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
         with_dtype(a.y_dtype, [&](auto dc) {
             constexpr int DT = decltype(dc)::value;
             const int64_t e = tok * a.ys + col_of(a.y_head, w, g);
-            store4<DT>(a.y, e, s);
-            store_pad<DT>(a.y, e, a.y_head, g);
+            void* y = chain ? a.y2 : a.y;
+            store4<DT>(y, e, s);
+            store_pad<DT>(y, e, a.y_head, g);
         });
     }
 }
@@ -468,6 +472,7 @@ __global__ __launch_bounds__(4 * C) void few_mlp_bwd_kernel(MlpBwdArgs a)
         with_dtype(a.dx_dtype, [&](auto dc) {
             constexpr int DT = decltype(dc)::value;
             const int64_t e = tok * a.dxs + col_of(a.x_head, w, g);
+            if (a.dres) total += load4<DT>(a.dres, e);            // another path's gradient of x (a residual's)
             if (a.add_dy & 2) total += load4<DT>(a.dx, e);        // dx holds another path's gradient of the same x
             store4<DT>(a.dx, e, total);
             store_pad<DT>(a.dx, e, a.x_head, g);
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(4 * C) void few_mlp_bwd_kernel(MlpBwdArgs a)
 template <typename T, int C, int LMAX>
 hipError_t fwd_l(const MlpArgs& a, hipStream_t st)
 {
-    const dim3 grid((unsigned)((a.T + 15) / 16));
+    const dim3 grid((unsigned)((a.T + 15) / 16), a.y2 ? 2 : 1);
     hipLaunchKernelGGL((few_mlp_mfma_kernel<T, C, LMAX>), grid, dim3(4 * C), 0, st, a);
     return hipGetLastError();
 }

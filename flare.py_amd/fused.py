@@ -513,6 +513,46 @@ def narrow_train_ok(x, mod_a, mod_b, out):
             and out.in_features == out.out_features == x.shape[-1] and _chain_tiles(info[0] + [out]) is not None)
 
 
+def _pair_packs(x, mod_a, mod_b):
+    info = _pair_info(x, mod_a, mod_b, None)
+    return info is not None and _chain_tiles(info[0]) is not None
+
+
+def prepack(x, cd, *stacks):
+    """The packed operands of several stacks that the few-token launches of one training step will ask for (a tuple of modules shares
+    a packing: a pair), from one packing launch instead of one each.  Does nothing where they are not all plain chains at few
+    tokens, or where fewer than two of them have to be packed again."""
+    Cdim = x.shape[-1]
+    if not 0 < x.numel() // Cdim <= _FEW_TOKENS.get(Cdim, 0):
+        return
+    stale, tiles, at = [], [], 0
+    for mods in stacks:
+        layers = []
+        for m in mods:
+            info = _layers_of(m)
+            if (info is None or len(info[0]) > _BWD_MAX_LAYERS[Cdim] or _train_subchain(m) is not None
+                    or any(l.in_features != Cdim or l.out_features != Cdim for l in info[0])):
+                return
+            layers += info[0]
+        if len(mods) == 2 and _pair_info(x, *mods, cd) is None:
+            return
+        key = (cd, _param_key(layers))
+        cache = mods[0].__dict__.get("_flare_packed_few")
+        if cache is not None and cache[0] == key and cache[3] is not None:
+            continue
+        t = _chain_tiles(layers)
+        if t is None:
+            return
+        stale.append((mods[0], key, at, at + len(t)))
+        tiles += t
+        at += len(t)
+    if len(stale) < 2 or at > _lib.MLP_PACK_MAX:
+        return
+    w, b, _, wt = _pack_launch(Cdim, cd, tiles, x.device, True, tiled=True)
+    for mod, key, lo, hi in stale:
+        mod.__dict__["_flare_packed_few"] = (key, w[lo:hi], b[lo:hi], wt[lo:hi])
+
+
 def project_padded(y, out, cd, head, res, out_dtype):
     """[res +] out(y) for rows y of padded heads, differentiable where narrow_train_ok() says so."""
     if torch.is_grad_enabled():
@@ -520,11 +560,13 @@ def project_padded(y, out, cd, head, res, out_dtype):
     return fused_mlp(y, out, cd, res=res, out_dtype=out_dtype, x_head=head)
 
 
-def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None, y_head=0):
+def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None, y_head=0, with_res=False):
     """(mod_a(norm(x)), mod_b(norm(x))) as fused_mlp computes them, for two stacks that read the same rows through the
     same norm (a block's k and v projections).  With gradients enabled and both stacks plain chains of C x C layers the
     pair is one autograd node whose backward sums the two gradients of x inside the second launch (few tokens: one backward
-    launch for both stacks).  y_head: as fused_mlp's, with gradients enabled where narrow_train_ok() says so."""
+    launch for both stacks).  y_head: as fused_mlp's, with gradients enabled where narrow_train_ok() says so.
+    with_res: a third result, x as the block's residual is to read it: where one launch is the pair's backward, that path's gradient
+    is added there, and not by a launch over three [T, C] arrays."""
     if torch.is_grad_enabled() and all(_train_subchain(m) is None and not _expand_factor(m, x.shape[-1]) for m in (mod_a, mod_b)):
         has_norm = norm is not None and not isinstance(norm, nn.Identity)
         gamma = getattr(norm, "weight", None) if has_norm else None
@@ -533,9 +575,12 @@ def fused_mlp_pair(x, mod_a, mod_b, cd, norm=None, out_dtype=None, y_head=0):
         for m in (mod_a, mod_b):
             layers = _layers_of(m)[0]
             wb += [l.weight for l in layers] + [l.bias for l in layers]
-        return _FusedPairFn.apply(mod_a, mod_b, cd, norm if has_norm else None, (out_dtype, y_head), x, gamma, beta, *wb)
-    return (fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head),
-            fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head))
+        through = with_res and x.requires_grad and type(x) is torch.Tensor and _pair_packs(x, mod_a, mod_b)
+        out = _FusedPairFn.apply(mod_a, mod_b, cd, norm if has_norm else None, (out_dtype, y_head, through), x, gamma, beta, *wb)
+        return out if through or not with_res else (*out, x)
+    out = (fused_mlp(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head),
+           fused_mlp(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head))
+    return (*out, x) if with_res else out
 
 
 def _forward_plan(mod):
@@ -551,7 +596,9 @@ def _forward_plan(mod):
     return cached[0]
 
 
-def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False, operands=None):
+def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False, operands=None, pair=None):
+    """pair: a list that the two chains of a few-token pair pass through (operands: their halves of one packing): the first one's
+    launch is left to the second."""
     lib = _lib.load()
     info, io, Cdim, E = _forward_plan(mod)
     layers, act_mask, add_mask, act = info
@@ -592,6 +639,15 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
         if r2.stride(-1) != 1 or r2.stride(0) % 4 or r2.data_ptr() % 16:
             r2 = r2.contiguous()
         d.res_dtype, d.res_stride = _dtype_code(r2), r2.stride(0)
+    if pair is not None:
+        pair.append((w, b, y))
+        if len(pair) == 2:
+            (w, b, ya), _ = pair
+            with _on_device(x.device):
+                rc = lib.flare_mlp_few_pair_fwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(b), _ptr(gamma), _ptr(beta), _ptr(ya), _ptr(y),
+                                                C.c_void_p(_stream_ptr(x.device)))
+            _lib.check(rc, "flare_mlp_few_pair_fwd")
+        return y
     with _on_device(x.device):
         rc = lib.flare_mlp_fwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(b), _ptr(gamma), _ptr(beta), _ptr(r2), _ptr(y),
                                C.c_void_p(_stream_ptr(x.device)))
@@ -825,8 +881,9 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     return dx, gsum, dW, db, layers
 
 
-def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0):
-    """Backward of both stacks of a pair in one launch (y_head: dya and dyb are rows of padded heads): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
+def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None):
+    """Backward of both stacks of a pair in one launch (y_head: dya and dyb are rows of padded heads; dres: another gradient of x,
+    added to dx): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
     None, the 2 L layers)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _pair_info(x, mod_a, mod_b, cd)
@@ -855,10 +912,15 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0):
     if d.norm:
         gb = torch.empty(_few(T, Cdim, L2 // 2), 2, Cdim, dtype=torch.float32, device=dev)
         gsum = torch.empty(2, Cdim, dtype=torch.float32, device=dev)
+    r2 = None
+    if dres is not None:
+        r2 = dres.reshape(-1, Cdim)
+        if r2.dtype != x2.dtype or not r2.is_contiguous() or r2.data_ptr() % 16:
+            r2 = r2.to(x2.dtype, copy=True, memory_format=torch.contiguous_format)
     with _on_device(dev):
-        rc = lib.flare_mlp_few_bwd(C.byref(d), _ptr(x2), _ptr(da), _ptr(db_), _ptr(w), _ptr(wt), _ptr(b), _ptr(gamma), _ptr(beta),
-                                   0, _ptr(dx), _ptr(rows[0]), _ptr(rows[1]), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
-    _lib.check(rc, "flare_mlp_few_bwd")
+        rc = lib.flare_mlp_few_bwd_res(C.byref(d), _ptr(x2), _ptr(da), _ptr(db_), _ptr(r2), _ptr(w), _ptr(wt), _ptr(b), _ptr(gamma),
+                                       _ptr(beta), 0, _ptr(dx), _ptr(rows[0]), _ptr(rows[1]), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_few_bwd_res")
     dW, db = _weight_grads(d, rows[1], rows[0], any(l.bias is not None for l in layers), gb=gb, gsum=gsum)
     return dx, gsum, dW, db, layers
 
@@ -871,7 +933,7 @@ class _FusedPairFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, mod_a, mod_b, cd, norm, fmt, x, gamma, beta, *wb):
-        out_dtype, y_head = fmt
+        out_dtype, y_head, with_res = fmt
         with torch.no_grad():
             info = _pair_info(x, mod_a, mod_b, cd)
             packed = None if info is None else _packed_few(mod_a, info[0], cd, True)
@@ -879,25 +941,26 @@ class _FusedPairFn(torch.autograd.Function):
             n = len(info[0]) // 2 if ctx.pair else 0
             if y_head and not ctx.pair:
                 raise ValueError("head-padded rows have no backward here: call under torch.no_grad()")
+            pair = [] if ctx.pair else None
             ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
-                                operands=(packed[0][:n], packed[1][:n]) if ctx.pair else None)
+                                operands=(packed[0][:n], packed[1][:n]) if ctx.pair else None, pair=pair)
             yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
-                                operands=(packed[0][n:], packed[1][n:]) if ctx.pair else None)
+                                operands=(packed[0][n:], packed[1][n:]) if ctx.pair else None, pair=pair)
         ctx.mods, ctx.cd, ctx.norm, ctx.y_head = (mod_a, mod_b), cd, norm, y_head
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)
         ctx.save_for_backward(x)
-        return ya, yb
+        return (ya, yb, x.view_as(x)) if with_res else (ya, yb)
 
     @staticmethod
     @once_differentiable
-    def backward(ctx, dya, dyb):
+    def backward(ctx, dya, dyb, dres=None):
         (x,) = ctx.saved_tensors
         if ctx.versions != tuple(None if t is None else t._version for t in ctx.params):
             raise RuntimeError("a parameter of the fused MLP was modified in place between its forward and its backward")
         mod_a, mod_b = ctx.mods
         if ctx.pair:
-            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb, ctx.y_head)
+            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb, ctx.y_head, dres)
             n = len(layers) // 2
             la, lb, dWa, dWb = layers[:n], layers[n:], dW[:n], dW[n:]
             dba, dbb = (None, None) if db is None else (db[:n], db[n:])

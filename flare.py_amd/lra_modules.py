@@ -21,7 +21,7 @@ from torch.nn import functional as F
 
 from .functional import flare_multihead_mixer, triple_attention
 from . import fused, rows
-from .modules import ResidualMLP, _chain_info, _lin, _mlp_block, _norm, _project
+from .modules import ResidualMLP, _chain_info, _lin, _mlp_block, _norm, _prepack, _project
 
 __all__ = ["FLARE", "FLAREBlock", "TripleAttention", "TripleBlock", "make_kernel", "RotaryPositionalEmbeddings"]
 
@@ -91,7 +91,10 @@ class FLARE(nn.Module):
         q = self.latent_q.view(self.num_heads, self.num_latents, self.head_dim)
         cd = self._fusable(x)
         if cd is not None:
-            k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd)
+            if _res is x:
+                k, v, _res = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd, with_res=True)
+            else:
+                k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd)
         else:
             xn = x if _norm is None else rows.norm(_norm, x) if _chain_info(self.k_proj, x) is not None else _norm(x)
             k, v = self.k_proj(xn), self.v_proj(xn)
@@ -126,6 +129,8 @@ class FLAREBlock(nn.Module):
                                input_residual=True, output_residual=True)
 
     def forward(self, x, attention_mask=None):
+        if torch.is_grad_enabled():
+            _prepack(self, x)
         x = self.att(x, attention_mask=attention_mask, _norm=self.norm1, _res=x)
         cd = fused.compute_dtype(x, self.mlp)
         if cd is not None:

@@ -191,6 +191,11 @@ class FLARE(nn.Module):
         cds = {fused.compute_dtype(x, m) for m in (self.k_proj, self.v_proj, self.out_proj)}
         return cds.pop() if len(cds) == 1 else None
 
+    def _project_kv(self, x, cd, norm, res, y_head=0):
+        """(k rows, v rows, the residual), the residual by way of the projections' node where it is their own input."""
+        kv = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=norm, out_dtype=cd, y_head=y_head, with_res=res is x)
+        return kv if res is x else (*kv, res)
+
     def forward(self, x, return_scores: bool = False, _norm=None, _res=None):
         """(y, scores).  _norm / _res are FLAREBlock's pre-norm and residual, folded into the fused
         launches when the fast path applies: then y = _res + out_proj(mixer(.. _norm(x) ..))."""
@@ -208,7 +213,7 @@ class FLARE(nn.Module):
                   and (not torch.is_grad_enabled() or fused.narrow_train_ok(x, self.k_proj, self.v_proj, self.out_proj)))
         if narrow:
             H = self.num_heads
-            k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd, y_head=D)
+            k, v, _res = self._project_kv(x, cd, _norm, _res, D)
             k, v = (t.view(B, N, H, 16).permute(0, 2, 1, 3) for t in (k, v))
             if torch.is_grad_enabled():
                 y = mixer_narrow_heads(q, k, v, self.attn_scale)
@@ -218,7 +223,7 @@ class FLARE(nn.Module):
             out_dtype = _res.dtype if _res is not None else x.dtype
             return fused.project_padded(y, self.out_proj, cd, D, _res, out_dtype), None
         if cd is not None:
-            k, v = fused.fused_mlp_pair(x, self.k_proj, self.v_proj, cd, norm=_norm, out_dtype=cd)
+            k, v, _res = self._project_kv(x, cd, _norm, _res)
             k, v = self._heads(k), self._heads(v)
             if self.qk_norm:
                 q = self.q_norm(q)
@@ -252,6 +257,17 @@ class FLARE(nn.Module):
         return _project(self.out_proj, y, _res), scores
 
 
+def _prepack(block, x, return_scores=False):
+    """One packing launch for the stacks of a training step's block, where its layers take the few-token launches."""
+    att = block.att
+    if (x.is_cuda and not return_scores and 0 < x.numel() // x.shape[-1] <= fused._FEW_TOKENS.get(x.shape[-1], 0)
+            and torch.is_autocast_enabled("cuda") and all(hasattr(att, n) for n in ("k_proj", "v_proj", "out_proj"))):
+        cds = {fused.compute_dtype(x, m) for m in (att.k_proj, att.v_proj, att.out_proj, block.mlp)}
+        cd = cds.pop()
+        if not cds and cd is not None:
+            fused.prepack(x, cd, (att.k_proj, att.v_proj), (att.out_proj,), (block.mlp,))
+
+
 class FLAREBlock(nn.Module):
     """x + att(norm1 x), then x + mlp(norm2 x); returns (x, scores)."""
 
@@ -274,6 +290,8 @@ class FLAREBlock(nn.Module):
             y = block_plan.forward(self, x)      # inference under autocast: the launches below from one call
             if y is not None:
                 return y, None
+        if torch.is_grad_enabled():
+            _prepack(self, x, return_scores)
         x, scores = self.att(x, return_scores=return_scores, _norm=self.norm1, _res=x)
         cd = fused.compute_dtype(x, self.mlp)
         if cd is not None:

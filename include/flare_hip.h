@@ -419,6 +419,14 @@ int flare_mlp_few(const FlareMlpDesc* desc);
 int flare_mlp_few_bwd(const FlareMlpDesc* desc, const void* x, const void* dy_a, const void* dy_b, const void* w, const void* wt,
                       const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in, void* g_out,
                       float* gb_part, void* stream);
+/* The same with dres (or NULL): [T,C] contiguous rows of x's type that are added to dx (the gradient a residual path brings). */
+int flare_mlp_few_bwd_res(const FlareMlpDesc* desc, const void* x, const void* dy_a, const void* dy_b, const void* dres, const void* w,
+                          const void* wt, const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx,
+                          void* a_in, void* g_out, float* gb_part, void* stream);
+/* Forward of two chains of equal L, masks and activation that read the same rows through the same norm, in one launch: desc as for one
+ * of them (FLARE_MLP_W_TILED set), w [2L,C,C] and bias [2L,C] the first chain's tiles followed by the second's. */
+int flare_mlp_few_pair_fwd(const FlareMlpDesc* desc, const void* x, const void* w, const float* bias, const float* gamma,
+                           const float* beta, void* y_a, void* y_b, void* stream);
 /* Weight and bias gradients from the rows flare_mlp_bwd leaves, in one pass over both (the reference gets them from
  * torch's Linear backward: dW = dt^T s, db = column sums of dt; pdebench/models/flare.py:45-59 under autograd).
  * Only T, C, L and w_dtype of the descriptor are read.  a_in, g_out: L arrays of [T,C] rows in the weights' type,

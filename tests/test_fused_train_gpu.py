@@ -572,3 +572,48 @@ def test_padded_rows_beyond_the_few_token_launches_are_refused(dev):
     y = fused.project_padded(torch.randn(16385, 128, device=dev), nn.Linear(64, 64).to(dev), torch.bfloat16, 8, None, torch.float32)
     with pytest.raises(RuntimeError, match="head-padded"):
         y.sum().backward()
+
+
+@pytest.mark.parametrize("lra,C,H,N,kw", [(False, 64, 8, 1000, {}), (True, 64, 8, 1000, {}), (False, 128, 8, 17, {"rmsnorm": True}),
+                                          (False, 32, 2, 4097, {"num_layers_ffn": 1}), (False, 64, 4, 500, {"num_layers_v_proj": 2}),
+                                          (False, 64, 4, 500, {"num_layers_ffn": 0, "ffn_mlp_ratio": 4.0})])
+def test_joint_packing_and_the_residuals_gradient_of_a_block(dev, monkeypatch, lra, C, H, N, kw):
+    """One packing launch for a block's stacks and the residual's gradient added by the projections' launch, against a packing each and
+    autograd's own sum: everything but dx is bit for bit the same, dx (fp32) to the rounding of one more addition."""
+    from flare_py_amd import lra_modules
+
+    torch.manual_seed(N)
+    blk = (lra_modules.FLAREBlock(channel_dim=C, num_heads=H, num_latents=64, kv_proj_hidden_dim=C, ffn_hidden_dim=C) if lra
+           else F.FLAREBlock(channel_dim=C, num_heads=H, num_latents=64, **kw)).to(dev)
+    x = torch.randn(2, N, C, device=dev, requires_grad=True)
+    gy = torch.randn(2, N, C, device=dev)
+
+    def step():
+        for m in blk.modules():
+            fused.drop_operands(m)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = blk(x)
+        y = y if lra else y[0]
+        return [y.detach(), *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
+
+    packs, real = [], fused._pack_launch
+    monkeypatch.setattr(fused, "_pack_launch", lambda *a, **k: (packs.append(len(a[2])), real(*a, **k))[1])
+    got = step()
+    if not kw or "rmsnorm" in kw:
+        assert packs == [16]
+    n = len(packs)                                             # a second step of unchanged weights packs nothing
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        blk(x)
+    assert len(packs) == n
+    monkeypatch.setattr(fused, "prepack", lambda *a: None)
+    monkeypatch.setattr(fused, "_pair_packs", lambda *a: False)
+    want = step()
+    for i, (a, b) in enumerate(zip(got, want)):
+        if i == 1:
+            assert float((a - b).norm() / b.norm()) <= 1e-6
+        else:
+            assert torch.equal(a, b), i
+    # the block's input may be a leaf whose gradient is not asked for, and one gradient of two may be
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x.detach())
+    (y if lra else y[0]).sum().backward()
