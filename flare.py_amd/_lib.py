@@ -17,6 +17,7 @@ DT_F32, DT_BF16, DT_F16 = 0, 1, 2
 FLAG_FORCE_GENERIC = 1
 FLAG_MFMA16 = 2
 FLAG_GRAD_LIKE_KV = 8
+FLAG_ABSENT_TOKENS = 16
 MLP_EXPAND = 1
 MLP_W_TILED = 2
 MLP_BWD_ADD_DY = 1           # bits of flare_mlp_bwd's add_dy argument

@@ -480,7 +480,7 @@ struct BwdPlan { int n_splits, tokens_per_split, n_splits0, tokens_per_split0; s
 
 bool bwd_wants_dz32(const FlareMixerDesc* d)
 {
-    return !(d->flags & FLARE_FLAG_MFMA16) && drop_threshold(d) == 0 && flare::bwd_dz32_supported(d->dtype, d->M, d->D);
+    return !(d->flags & (FLARE_FLAG_MFMA16 | FLARE_FLAG_ABSENT_TOKENS)) && drop_threshold(d) == 0 && flare::bwd_dz32_supported(d->dtype, d->M, d->D);
 }
 
 BwdPlan plan_bwd(const FlareMixerDesc* d)
@@ -590,6 +590,8 @@ int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, co
     a.scale = desc->scale; a.scale_log2 = desc->scale * 1.4426950408889634f;
     a.drop_thr = drop_threshold(desc);
     a.drop_rs = 1.f;
+    a.absent = (desc->flags & FLARE_FLAG_ABSENT_TOKENS) ? 1 : 0;
+    if (a.absent && a.drop_thr != 0) return fail(FLARE_EUNSUPPORTED, "FLARE_FLAG_ABSENT_TOKENS cannot be combined with attention dropout");
     if (a.drop_thr != 0) {
         a.drop_rs = 1.0f / (1.0f - desc->dropout_p);
         a.seed_lo = (uint32_t)(desc->dropout_seed & 0xffffffffu);
@@ -614,6 +616,7 @@ int half_bwd_args(flare::MixerBwdArgs& a, const FlareMixerDesc* desc, void* work
 {
     int rc = check_bwd(desc);
     if (rc != FLARE_OK) return rc;
+    if (desc->flags & FLARE_FLAG_ABSENT_TOKENS) return fail(FLARE_EUNSUPPORTED, "the half backwards do not take FLARE_FLAG_ABSENT_TOKENS");
     if (desc->dtype != FLARE_DT_F32 && drop_threshold(desc) != 0)
         return fail(FLARE_EUNSUPPORTED, "the bf16 / f16 half backwards do not take attention dropout");
     const BwdPlan p = plan_bwd(desc);

@@ -225,7 +225,9 @@ struct MixerBwdArgs {
     // attention dropout of the forward this is the backward of (same fields as MixerArgs; drop_thr == 0: none)
     uint32_t drop_thr, seed_lo, seed_hi;
     float drop_rs;
+    int absent;              // 1: tokens whose lse_tok exceeds kAbsentLse take no part, whatever their rows hold; their dk, dv rows become zeros
 };
+constexpr float kAbsentLse = 1.5e30f;      // (a half backward's own lse_tok of 1e30, see there, is not such a mark)
 
 // Whether a (b,h) takes the form of the backward in which both weights come from exp2(S) alone (kernels on the 32x32x16
 // product): the one-exponential form's own condition (the latents' largest log-sum-exp and the tokens' smallest one at

@@ -58,7 +58,9 @@ template <int Q4> __device__ __forceinline__ f32x4 dot_rows(const f32x4 (&a)[Q4]
 // waves' sums meet in LDS and the workgroup writes one partial [64][D].
 // MODE 0: dz_m += B[n,m] dy_n (values = dY), and delta_n = <dy_n, y_n> from the first latent block.
 // MODE 1: dq_m += dS[m,n] k_n (values = K), dS assembled from three score-like products.
-template <int D, int MODE, int HALF, bool DROP>
+// KIND: 0 plain, 1 the forward dropped weights, 2 absent tokens (a key mask): a token is a row of the score-like products, so only its
+// weights and its row of the value tile have to go.
+template <int D, int MODE, int HALF, int KIND>
 __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_lat_kernel(MixerBwdArgs a)
 {
     constexpr int QL = D / 4, Q4 = QL / 4, RT = D / 16, VS = D + 4, VPT = D / 16;
@@ -80,7 +82,8 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
     const int tps = MODE == 0 ? a.tokens_per_split0 : a.tokens_per_split;
     const int n_parts = MODE == 0 ? a.n_splits0 : a.n_splits;
     constexpr bool use_a = HALF != 2, use_b = HALF != 1;      // gather term, scatter term of dS
-    constexpr bool drop = DROP;                               // the forward dropped weights: the same masks are regenerated here
+    constexpr bool ABSENT = KIND == 2;
+    constexpr bool drop = KIND == 1;                          // the forward dropped weights: the same masks are regenerated here
 
     // latent operands (B of the score-like products): q log2-scaled; for the dq pass also dz and z with their scalars
     f32x4 qb[CT][Q4], dzb[MODE ? CT : 1][Q4], zb[MODE ? CT : 1][Q4];
@@ -116,7 +119,7 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
 
     // rows of the next tile, requested while this one is worked on (rows past the range repeat its last row)
     f32x4 ka[Q4], va[MODE ? Q4 : 1], dya[Q4], ya[MODE ? 1 : Q4], vr[VPT];
-    float rho[4], dt[4];
+    float rho[4], dt[4], ab[ABSENT ? VPT : 1];
     auto fetch = [&](int n0) {
         const int n = max(min(n0 + c16, n_end - 1), 0);
 #pragma unroll
@@ -137,6 +140,7 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
         for (int i = 0; i < VPT; ++i) {
             const int c = lane + 64 * i, tok = c / (D / 4), ch = c % (D / 4);
             const int nv = max(min(n0 + tok, n_end - 1), 0);
+            if constexpr (ABSENT) ab[i] = lse_tok[nv];
             vr[i] = MODE ? *reinterpret_cast<const f32x4*>(k + (int64_t)nv * a.ks[2] + 4 * ch)
                          : *reinterpret_cast<const f32x4*>(dy + (int64_t)nv * a.dys[2] + 4 * ch);
         }
@@ -163,6 +167,7 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
             const int c = lane + 64 * i, tok = c / (D / 4), ch = c % (D / 4);
+            if constexpr (ABSENT) vr[i] = ab[i] > kAbsentLse ? zero4f() : vr[i];
             *reinterpret_cast<f32x4*>(&vt[w][tok][4 * ch]) = vr[i];
         }
         asm volatile("" ::: "memory");
@@ -178,7 +183,7 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
         }
         bool valid[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) valid[r] = n0 + 4 * g + r < n_end;
+        for (int r = 0; r < 4; ++r) valid[r] = n0 + 4 * g + r < n_end && !(ABSENT && rh[r] > kAbsentLse * kLog2e);
         fetch(n0 + 64);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
@@ -322,7 +327,7 @@ __global__ __launch_bounds__(256) void bwd_f32_delta_kernel(MixerBwdArgs a)
 // q (log2-scaled), z and dz rows of latents [m0, m0 + mc) of one (b,h) in LDS with their scalars; a wave takes 16 tokens
 // at a time (lane = token column c16) and walks the latents 16 at a time (rows 4g + r).  8 waves per workgroup share
 // the operands.  dk comes out in units of the log2-scaled q: multiplied by ln 2 at the end.
-template <int D, int HALF>
+template <int D, int HALF, bool ABSENT>
 __global__ __launch_bounds__(512) void bwd_f32_tok_kernel(MixerBwdArgs a)
 {
     constexpr int QL = D / 4, Q4 = QL / 4, RT = D / 16, LS = D + 4;
@@ -453,6 +458,10 @@ __global__ __launch_bounds__(512) void bwd_f32_tok_kernel(MixerBwdArgs a)
                 f32x4* pk = reinterpret_cast<f32x4*>(dk + (int64_t)n * a.dks[2] + 16 * rt + 4 * g);
                 f32x4* pv = reinterpret_cast<f32x4*>(dv + (int64_t)n * a.dvs[2] + 16 * rt + 4 * g);
                 f32x4 ok = dka[rt] * kLn2, ov = dva[rt];
+                if constexpr (ABSENT) {      // a token is a column of its own: whatever its rows held stays in it
+                    ok = rho > kAbsentLse * kLog2e ? zero4f() : ok;
+                    ov = rho > kAbsentLse * kLog2e ? zero4f() : ov;
+                }
                 if (a.accumulate) {
                     ok += *pk;
                     if constexpr (use_a) ov += *pv;
@@ -477,7 +486,7 @@ int tok_chunk(int M, int D)
     return mc;
 }
 
-template <int D, int HALF>
+template <int D, int HALF, int KIND>
 hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
 {
     MixerBwdArgs a = a0;
@@ -486,13 +495,12 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
     if (HALF == 1) {
         hipLaunchKernelGGL(bwd_f32_delta_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, a);
     } else {
-        if (a.drop_thr != 0) hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 0, 0, true>), dim3(a.n_splits0 * mblocks, a.H, a.B), dim3(256), 0, st, a);
-        else                 hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 0, 0, false>), dim3(a.n_splits0 * mblocks, a.H, a.B), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 0, 0, KIND>), dim3(a.n_splits0 * mblocks, a.H, a.B), dim3(256), 0, st, a);
         merge_launch_f32<0>(a, rows * (D / 4), st);
     }
     // token pass, in chunks of latents when their operands do not fit the LDS
     const int mc = tok_chunk(a.M, D);
-    auto kern = bwd_f32_tok_kernel<D, HALF>;
+    auto kern = bwd_f32_tok_kernel<D, HALF, KIND == 2>;
     const size_t lds = (size_t)mc * ((size_t)3 * (D + 4) * 4 + 8);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -506,8 +514,7 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
         a.accumulate = m0 > 0;
         hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, a);
     }
-    if (a.drop_thr != 0) hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 1, HALF, true>), dim3(a.n_splits * mblocks1, a.H, a.B), dim3(256), 0, st, a);
-    else                 hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 1, HALF, false>), dim3(a.n_splits * mblocks1, a.H, a.B), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((bwd_f32_lat_kernel<D, 1, HALF, KIND>), dim3(a.n_splits * mblocks1, a.H, a.B), dim3(256), 0, st, a);
     merge_launch_f32<1>(a, rows * (D / 4), st);
     return hipGetLastError();
 }
@@ -515,7 +522,9 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
 template <int D>
 hipError_t launch_d(const MixerBwdArgs& a, hipStream_t st)
 {
-    return a.half == 1 ? launch_dh<D, 1>(a, st) : a.half == 2 ? launch_dh<D, 2>(a, st) : launch_dh<D, 0>(a, st);
+    if (a.absent) return a.half != 0 || a.drop_thr != 0 ? hipErrorInvalidValue : launch_dh<D, 0, 2>(a, st);
+    if (a.drop_thr != 0) return a.half == 1 ? launch_dh<D, 1, 1>(a, st) : a.half == 2 ? launch_dh<D, 2, 1>(a, st) : launch_dh<D, 0, 1>(a, st);
+    return a.half == 1 ? launch_dh<D, 1, 0>(a, st) : a.half == 2 ? launch_dh<D, 2, 0>(a, st) : launch_dh<D, 0, 0>(a, st);
 }
 
 }  // namespace

@@ -173,9 +173,14 @@ __device__ __forceinline__ float dot8(u32x4 u, u32x4 w)
 constexpr int kBTile = 64;   // tokens per LDS tile
 
 // One workgroup = 4 waves x (16 CT latents) x one token range.  MODE 0: dz partial; MODE 1: dq partial.
-template <typename T, int D, int CT, int MODE, bool DROPK>
+// KIND: 0 plain, 1 the forward dropped weights, 2 absent tokens (a key mask): their rows are staged as zeros, which with their
+// log-sum-exp leaves nothing of them in dz and dq; in the token pass a token is a column of its own and only its stores change.
+// (Around the kernels, in torch, the mask was five passes over [N,D] arrays and seven small launches: forward + backward at B=4, H=8,
+// N=50,000, M=128, D=16 bf16 579 us, 371 us with the mask here, 341 us without one.)
+template <typename T, int D, int CT, int MODE, int KIND>
 __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void bwd_lat_kernel(MixerBwdArgs a)
 {
+    constexpr bool DROPK = KIND == 1, ABSENT = KIND == 2;
     constexpr int KD = (D + 31) / 32, RT = D / 16, CH = D / 8, MB = 64 * CT, ROWB = D * 2, TILEB = kBTile * ROWB;
     constexpr int NT = MODE == 0 ? 2 : 4;          // staged tiles: K rows, dY^T | K rows, K^T, V rows, dY rows
     using M_ = Mb<T>;
@@ -251,6 +256,7 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
     auto v_slot = [](int tok, int ch) { return tok * ROWB + ((CH >= 4 ? (ch ^ (((tok >> 2) & 1) << 1)) : ch) << 4); };
 
     u32x4 kr[CPT], vr[CPT], yr[CPT];
+    float ab[ABSENT ? CPT : 1];      // log-sum-exp of the token a staged chunk belongs to, looked at where the chunk is stored
     float ysc[CPT];    // eR of the token a staged dy chunk belongs to (one-exponential form)
     float rr = 0.f, dd = 0.f;
     float rr_max = -3.0e38f;   // MODE 0: -(smallest rho2_n) over the tokens this thread has loaded
@@ -269,6 +275,7 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
             ysc[i] = 1.f;
             if (c < TCH) {
                 const int n = min(n0 + c / CH, n_end - 1), ch = c % CH;
+                if constexpr (ABSENT) ab[i] = rho[n];
                 if (MODE == 1 && fast) ysc[i] = fast_exp2(lmax2 - rho[n] * kLog2e);
                 kr[i] = load16(k + (int64_t)n * a.ks[2] + ch * 8);
                 yr[i] = load16(dy + (int64_t)n * a.dys[2] + ch * 8);
@@ -287,6 +294,12 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
             const int c = tid + i * 256;
             if (c < TCH) {
                 const int tok = c / CH, ch = c % CH;
+                if constexpr (ABSENT) {
+                    const bool gone = ab[i] > kAbsentLse;
+                    kr[i] = gone ? zero4() : kr[i];
+                    yr[i] = gone ? zero4() : yr[i];
+                    if (MODE == 1 || make_delta) vr[i] = gone ? zero4() : vr[i];
+                }
                 *reinterpret_cast<u32x4*>(&tl[buf][0][k_slot(tok, ch)]) = kr[i];
                 if (MODE == 0) {
                     *reinterpret_cast<u32x4*>(&tl[buf][1][v_slot(tok, ch)]) = to_bf16x8<T>(yr[i]);
@@ -597,9 +610,10 @@ __global__ __launch_bounds__(256) void bwd_half_prep_kernel(MixerBwdArgs a)
 template <int D> constexpr int kTokWaves = D <= 32 ? 12 : 8;
 template <int D> constexpr int kTokTiles = 2;      // 16-token column tiles per wave iteration
 
-template <typename T, int D, bool DROPK>
+template <typename T, int D, int KIND>
 __global__ __launch_bounds__(64 * kTokWaves<D>, 1) void bwd_tok_kernel(MixerBwdArgs a, int tokens_per_wg)
 {
+    constexpr bool DROPK = KIND == 1, ABSENT = KIND == 2;
     constexpr int NTH = 64 * kTokWaves<D>;
     constexpr int KD = (D + 31) / 32, RT = D / 16, CH = D / 8;
     constexpr int kBTW = kTokTiles<D>;
@@ -868,6 +882,7 @@ __global__ __launch_bounds__(64 * kTokWaves<D>, 1) void bwd_tok_kernel(MixerBwdA
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
                     f32x4 t = acc[rt];
+                    if constexpr (ABSENT) t = r2[tw] > kAbsentLse * kLog2e ? zf : t;
                     if (a.accumulate) {       // a later chunk of latents: add to what the earlier launches stored
                         const uint2 old = *reinterpret_cast<const uint2*>(p + 4 * rt);
                         t[0] += M_::unpack(uint16_t(old.x & 0xffffu));
@@ -899,22 +914,23 @@ __global__ __launch_bounds__(64 * kTokWaves<D>, 1) void bwd_tok_kernel(MixerBwdA
     }
 }
 
-template <typename T, int D, int MODE, bool DROPK>
+template <typename T, int D, int MODE, int KIND>
 hipError_t lat_launch(const MixerBwdArgs& a, hipStream_t st)
 {
+    constexpr bool DROPK = KIND == 1;
     // 4 latent tiles per wave need too many registers at D = 64 in the dq pass, and with the keep factors of a forward
     // with dropout everywhere (then 2 tiles, 1 at D = 64 in the dq pass)
     if (a.M % 256 == 0 && !(D == 64 && MODE == 1) && !DROPK) {
-        hipLaunchKernelGGL((bwd_lat_kernel<T, D, DROPK ? 2 : 4, MODE, DROPK>), dim3(a.n_splits * (a.M / 256), a.H, a.B), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_lat_kernel<T, D, DROPK ? 2 : 4, MODE, KIND>), dim3(a.n_splits * (a.M / 256), a.H, a.B), dim3(256), 0, st, a);
     } else if (a.M % 128 == 0 && !(DROPK && D == 64 && MODE == 1)) {
-        hipLaunchKernelGGL((bwd_lat_kernel<T, D, 2, MODE, DROPK>), dim3(a.n_splits * (a.M / 128), a.H, a.B), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_lat_kernel<T, D, 2, MODE, KIND>), dim3(a.n_splits * (a.M / 128), a.H, a.B), dim3(256), 0, st, a);
     } else {
-        hipLaunchKernelGGL((bwd_lat_kernel<T, D, 1, MODE, DROPK>), dim3(a.n_splits * ((a.M + 63) / 64), a.H, a.B), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_lat_kernel<T, D, 1, MODE, KIND>), dim3(a.n_splits * ((a.M + 63) / 64), a.H, a.B), dim3(256), 0, st, a);
     }
     return hipGetLastError();
 }
 
-template <typename T, int D, bool DROPK>
+template <typename T, int D, int KIND>
 hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
 {
     const int64_t lat = (int64_t)a.B * a.H * a.M;
@@ -923,16 +939,16 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
     a0.tokens_per_split = a.tokens_per_split0;
     // bf16 at D = 32 without dropout: the token-parallel passes on the 32x32x16 product.  The scatter half alone stays on
     // the two-exponential form, which only the 16x16x32 token and dq passes run at full speed.
-    const bool mfma32 = !DROPK && !a.no_mfma32 && std::is_same<T, bf16_t>::value && bwd_dz32_supported(1, a.M, D);
+    const bool mfma32 = KIND == 0 && !a.no_mfma32 && std::is_same<T, bf16_t>::value && bwd_dz32_supported(1, a.M, D);
     const bool dz32 = mfma32, dq32 = mfma32 && a.half != 2;
     hipError_t e = hipSuccess;
     if (a.half != 0) {
-        if (DROPK) return hipErrorInvalidValue;
+        if (KIND != 0) return hipErrorInvalidValue;
         const int64_t items = std::max<int64_t>((int64_t)a.B * a.H * (a.half == 1 ? a.N : a.M), lat);
         hipLaunchKernelGGL(bwd_half_prep_kernel, dim3((unsigned)std::min<int64_t>((items + 255) / 256, 4096)), dim3(256), 0, st, a);
     }
     if (a.half != 1) {      // the gather half is handed dz
-        e = dz32 ? launch_bwd_dz32(a0, st) : lat_launch<T, D, 0, DROPK>(a0, st);
+        e = dz32 ? launch_bwd_dz32(a0, st) : lat_launch<T, D, 0, KIND>(a0, st);
         if (e != hipSuccess) return e;
         merge_launch<0>(a0, lat * (D / 4), st);
     }
@@ -944,7 +960,7 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
         if (e != hipSuccess) return e;
     }
     {
-        auto kern = bwd_tok_kernel<T, D, DROPK>;
+        auto kern = bwd_tok_kernel<T, D, KIND>;
         // the latents are covered in 1, 2 or 4 launches, each with the operand sets of its chunk in LDS
         const int chunks = mixer_bwd_tok_chunks(a.M, D);
         if (chunks == 0) return hipErrorInvalidValue;
@@ -969,29 +985,28 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
             hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + tpw - 1) / tpw), a.H, a.B), dim3(64 * kTokWaves<D>), lds, st, ac, (int)tpw);
         }
     }
-    e = dq32 ? launch_bwd_dq32(a, st) : lat_launch<T, D, 1, DROPK>(a, st);
+    e = dq32 ? launch_bwd_dq32(a, st) : lat_launch<T, D, 1, KIND>(a, st);
     if (e != hipSuccess) return e;
     merge_launch<1>(a, lat * (D / 4), st);
     return hipGetLastError();
 }
 
+template <typename T, int KIND>
+hipError_t bwd_k(const MixerBwdArgs& a, hipStream_t st)
+{
+    switch (a.D) {
+        case 16: return bwd_all<T, 16, KIND>(a, st);
+        case 32: return bwd_all<T, 32, KIND>(a, st);
+        case 64: return bwd_all<T, 64, KIND>(a, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 template <typename T>
 hipError_t bwd_d(const MixerBwdArgs& a, hipStream_t st)
 {
-    if (a.drop_thr != 0) {      // the forward dropped weights: kernels that regenerate the keep masks
-        switch (a.D) {
-            case 16: return bwd_all<T, 16, true>(a, st);
-            case 32: return bwd_all<T, 32, true>(a, st);
-            case 64: return bwd_all<T, 64, true>(a, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
-    switch (a.D) {
-        case 16: return bwd_all<T, 16, false>(a, st);
-        case 32: return bwd_all<T, 32, false>(a, st);
-        case 64: return bwd_all<T, 64, false>(a, st);
-        default: return hipErrorInvalidValue;
-    }
+    if (a.drop_thr != 0) return a.absent ? hipErrorInvalidValue : bwd_k<T, 1>(a, st);      // the forward dropped weights: keep masks regenerated
+    return a.absent ? bwd_k<T, 2>(a, st) : bwd_k<T, 0>(a, st);
 }
 
 }  // namespace

@@ -244,7 +244,7 @@ def _hip_backward_ok(q, k, v, key_mask, force_generic, drop=None) -> bool:
     return _lib.load().flare_mixer_bwd_workspace_bytes(C.byref(d), C.byref(need)) == _lib.FLARE_OK
 
 
-def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None):
+def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None, flags=0):
     """dq (fp32), dk, dv from the HIP backward kernels (flare_mixer_bwd); drop = (p, seed) of the forward's attention dropout."""
     lib = _lib.load()
     k, v = _rows_last_contig(k), _rows_last_contig(v)
@@ -256,6 +256,7 @@ def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None):
     if gy.stride(-1) != 1 or any(s % per16 for s in gy.stride()[:3]) or gy.data_ptr() % 16:
         gy = gy.contiguous()
     d = _mixer_desc(q4, k, v, y, scale, 0, False, drop)
+    d.flags |= flags
     dq = torch.empty((B, H, M, D), dtype=torch.float32, device=k.device)
     # k and v that are token-major views ([B,N,H,D] storage, as a projection's output is) get their gradients in the
     # same layout: the projection's backward then reads them as [B*N, H*D] rows without a copy
@@ -418,6 +419,11 @@ def _mixer_torch_grad(q, k, v, scale, key_mask, gy, drop=None, stats=None):
 
 def _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, km, gy, drop=None):
     """_mixer_hip_grad for a problem that may carry a key mask."""
+    if km is not None and drop is None:
+        # The kernels know a padded token by its log-sum-exp; a batch element without a single real token has lse_lat = -inf.
+        lse_tok = torch.where(km.to(torch.bool)[:, None, :], lse_tok, 2e30)
+        return _mixer_hip_grad(q, k, v, y, z, torch.nan_to_num(lse_lat, nan=1e30, posinf=1e30, neginf=1e30), lse_tok, scale, gy,
+                               flags=_lib.FLAG_ABSENT_TOKENS)
     if km is not None:
         # A padded token takes no part in either softmax.  The kernels need no mask for that: with its k, v
         # and dy rows zeroed it adds nothing to dq or dz, with its log-sum-exp set far above any score its

@@ -455,3 +455,39 @@ def test_fp32_torch_recomputation_from_the_forwards_statistics_at_small_sizes(de
             assert err <= 1e-4, f"{name} rel-L2 {err:.3e}"
         else:
             assert float(got.abs().max()) <= 1e-5, name
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 17, 32, 16), (3, 1, 65, 64, 16), (3, 2, 700, 128, 16), (2, 1, 333, 256, 16), (2, 1, 130, 96, 32),
+                                   (2, 1, 500, 256, 32), (3, 1, 129, 128, 64), (2, 1, 200, 256, 64), (2, 1, 300, 512, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_absent_tokens_in_every_kernel(dev, shape, dtype):
+    """A key mask in the backward kernels themselves, over their latent blockings and head dims: the last batch element has no token
+    (from two elements on), padded rows hold NaN in k, v and dy; views with a row stride; tolerances of the unmasked tests."""
+    B, H, N, M, D = shape
+    q, k, v, gy = make(B, H, N, M, D, dtype, seed=N)
+    g = torch.Generator().manual_seed(N)
+    mask = torch.rand(B, N, generator=g) < 0.6
+    mask[0, 0] = True
+    mask[-1] = False
+    m4 = mask[:, None, :, None]
+    nan = torch.full((), float("nan"), dtype=dtype)
+    wide = torch.full((2, B, N, H, D + 8), float("nan"), dtype=dtype)
+    for i, t in enumerate((k, v)):
+        wide[i, ..., :D] = torch.where(m4, t, nan).permute(0, 2, 1, 3)
+    wide = wide.to(dev)
+    qd = q.to(dev).requires_grad_(True)
+    kd, vd = (wide[i, ..., :D].permute(0, 2, 1, 3).requires_grad_(True) for i in (0, 1))
+    assert FN._hip_backward_ok(qd, kd, vd, mask.to(dev), False)
+    y = F.flare_multihead_mixer(qd, kd, vd, scale=0.8, key_mask=mask.to(dev), token_major_out=True)
+    dq, dk, dv = torch.autograd.grad(y, (qd, kd, vd), torch.where(m4, gy, nan).to(dev))
+    qr = q.double().requires_grad_(True)
+    real = [b for b in range(B) if mask[b].any()]
+    kr, vr = (t[real].double().requires_grad_(True) for t in (k, v))
+    yr, _ = O.mixer_explicit(qr, kr, vr, 0.8, mask[real])
+    want = torch.autograd.grad(yr, (qr, kr, vr), (gy.double() * m4)[real])
+    for name, a, r in zip(("dq", "dk", "dv"), (dq, dk[real], dv[real]), want):
+        assert bool(torch.isfinite(a).all()), name
+        err = O.rel_l2(a, r)
+        assert err <= (1e-4 if dtype == torch.float32 else 3e-2), f"{name} rel-L2 {err:.3e}"
+    for t in (dk, dv):
+        assert bool((t.cpu()[~m4.expand_as(k)] == 0).all())
