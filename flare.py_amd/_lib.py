@@ -137,6 +137,7 @@ SYMBOLS = {
     "flare_mlp_few_pair_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_act_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P]),
+    "flare_rows_act_fwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_rows_layer_bwd_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_layer_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_norm_fwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, C.c_float, _P, _P, _P, _P, _P, _P]),

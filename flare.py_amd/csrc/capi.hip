@@ -1417,6 +1417,14 @@ int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const
     return hip_status(flare::launch_rows_act_bwd(act, ds, t, dt, copy, db_part, db, T, C, static_cast<hipStream_t>(stream)), "row activation backward launch");
 }
 
+int flare_rows_act_fwd(int64_t T, int32_t C, int32_t act, const float* t, const float* x, const float* res, float* y, void* stream)
+{
+    const int rc = check_rows(T, C, {t, y}, {x, res});
+    if (rc != FLARE_OK) return rc;
+    if (act != -1 && act != FLARE_ACT_GELU_TANH) return fail(FLARE_EUNSUPPORTED, "activation %d: only none and tanh-GELU", act);
+    return hip_status(flare::launch_rows_act_fwd(act, t, x, res, y, T * C, static_cast<hipStream_t>(stream)), "row activation launch");
+}
+
 int flare_rows_layer_bwd_parts(int64_t T, int32_t C, int32_t* parts)
 {
     if (!parts) return fail(FLARE_EINVAL, "parts is NULL");

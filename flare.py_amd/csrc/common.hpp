@@ -447,6 +447,7 @@ hipError_t launch_mlp_few(const MlpArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_mlp_few_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts, hipStream_t st);   // n a multiple of 4
 hipError_t launch_sum_layer_parts(const float* dw_part, float* dw, const float* db_part, float* db, int C, int parts, hipStream_t st);   // db may be null
+hipError_t launch_rows_act_fwd(int act, const float* t, const float* x, const float* res, float* y, int64_t n, hipStream_t st);   // n a multiple of 4
 bool       rows_layer_bwd_supported(int C);
 int        rows_layer_bwd_parts(int64_t T);
 hipError_t launch_rows_layer_bwd(int act, const RowsLayerArgs& a, float* dw, float* db, hipStream_t st);

@@ -107,20 +107,29 @@ def _layer_parts(T, width):
 
 class _LinearLongRowsPass(torch.autograd.Function):
     """[res +] ([x +] act(x W^T + b)); inputs (act or -1, add, x, w, b, res).  One node per layer, as with torch's layers, and
-    the forward is torch's own calls: a chain's outputs do not depend on whether a call comes here (a norm's in front of it do, in
-    rounding: _NormFn reduces in an order of its own)."""
+    the forward gives their values bit for bit: a chain's outputs do not depend on whether a call comes here (a norm's in front of it
+    do, in rounding: _NormFn reduces in an order of its own)."""
 
     @staticmethod
     def forward(ctx, act, add, x, w, b, res):
         width = x.shape[-1]
         s = _rows(x, width)
         t = torch.nn.functional.linear(s, w, b)
-        y = t if act < 0 else torch.nn.functional.gelu(t, approximate="tanh") if act == 0 else torch.nn.functional.silu(t)
-        if add:
-            y = s + y
-        y = y.view(x.shape)
-        if res is not None:
-            y = res + y
+        if act == 0 or (act < 0 and add and res is not None):      # the activation and the sums in one pass
+            r = None if res is None else _rows(res, width)
+            y = torch.empty_like(t) if act == 0 else t
+            with _on_device(t.device):
+                rc = _lib.load().flare_rows_act_fwd(t.shape[0], width, act, _ptr(t), _ptr(s) if add else None, _ptr(r), _ptr(y),
+                                                    C.c_void_p(_stream_ptr(t.device)))
+            _lib.check(rc, "flare_rows_act_fwd")
+            y = y.view(x.shape)
+        else:
+            y = t if act < 0 else torch.nn.functional.silu(t)
+            if add:
+                y = s + y
+            y = y.view(x.shape)
+            if res is not None:
+                y = res + y
         ctx.act, ctx.add = act, add
         ctx.save_for_backward(s, w, t if act >= 0 else None)
         return y

@@ -455,6 +455,8 @@ int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_l
 int flare_rows_parts(int64_t T, int32_t C, int32_t* parts);
 int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const float* t, float* dt, float* copy, float* db_part,
                        float* db, void* stream);
+/* y = [res +] ([x +] act(t)), act -1 or FLARE_ACT_GELU_TANH (the values of torch's tanh-GELU bit for bit); x, res may be NULL, y may be t. */
+int flare_rows_act_fwd(int64_t T, int32_t C, int32_t act, const float* t, const float* x, const float* res, float* y, void* stream);
 /* Backward of one layer y = [x +] act(x W^T + b) in one pass (C in {64, 128}; flare_rows_layer_bwd_parts answers 0 for the others):
  * dx = [dy if add] + (dy act'(t)) W (or NULL), dw [C,C] (out, in), db [C] (or NULL).  dw_part [parts,C,C] and db_part [parts,C] are scratch. */
 int flare_rows_layer_bwd_parts(int64_t T, int32_t C, int32_t* parts);

@@ -229,3 +229,33 @@ def test_layer_backward_in_one_pass(dev, act, T, C):
         if want_x:
             assert rel(dx, dt @ w.double() + (dy.double() if add else 0)) <= 2e-6
             assert bool((guard[T:] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,C", [(1, 32), (4097, 64), (70001, 128)])
+@pytest.mark.parametrize("act", [-1, 0])
+def test_activation_and_sums_equal_the_torch_layers(dev, act, T, C):
+    """Bit for bit, over every binade, signed zeros, subnormals, infinities and NaN; in place too."""
+    import ctypes
+
+    from flare_py_amd import _lib
+
+    lib = _lib.load()
+    torch.manual_seed(T)
+    t = torch.randint(-2 ** 31, 2 ** 31 - 1, (T, C), device=dev, dtype=torch.int32).view(torch.float32)
+    t[:, :16] = torch.randn(T, 16, device=dev) * 3
+    t.view(-1)[:6] = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), 1e-40], device=dev)
+    x, res = torch.randn(T, C, device=dev), torch.randn(T, C, device=dev)
+    f = (lambda v: v) if act < 0 else (lambda v: nn.functional.gelu(v, approximate="tanh"))
+    p = lambda v: None if v is None else ctypes.c_void_p(v.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for xx, rr in ((None, None), (x, None), (None, res), (x, res)):
+        want = f(t)
+        want = want if xx is None else xx + want
+        want = want if rr is None else rr + want
+        y, again = torch.empty_like(t), t.clone()
+        _lib.check(lib.flare_rows_act_fwd(T, C, act, p(t), p(xx), p(rr), p(y), st), "flare_rows_act_fwd")
+        _lib.check(lib.flare_rows_act_fwd(T, C, act, p(again), p(xx), p(rr), p(again), st), "flare_rows_act_fwd")
+        for a in (y, again):
+            assert torch.equal(torch.nan_to_num(a, nan=0.0, posinf=1e38, neginf=-1e38), torch.nan_to_num(want, nan=0.0, posinf=1e38, neginf=-1e38))
+            assert torch.equal(a.isnan(), want.isnan())
+    assert lib.flare_rows_act_fwd(T, C, 1, p(t), None, None, p(t), st) == _lib.FLARE_EUNSUPPORTED
