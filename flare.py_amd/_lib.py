@@ -65,6 +65,14 @@ class FlareMlpDesc(C.Structure):
     ]
 
 
+class FlareNarrowDesc(C.Structure):
+    _fields_ = [
+        ("T", C.c_int64), ("x_stride", C.c_int64),
+        ("C", C.c_int32), ("K", C.c_int32), ("out", C.c_int32), ("act", C.c_int32),
+        ("w_dtype", C.c_int32), ("x_dtype", C.c_int32), ("y_dtype", C.c_int32),
+    ]
+
+
 class FlareBlockDesc(C.Structure):
     _fields_ = [
         ("mlp", FlareMlpDesc * 4), ("mixer", FlareMixerDesc),
@@ -135,6 +143,9 @@ SYMBOLS = {
     "flare_mlp_few_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_few_bwd_res": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_few_pair_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
+    "flare_mlp_narrow_fwd": (C.c_int, [C.POINTER(FlareNarrowDesc), _P, _P, _P, _P, _P, _P]),
+    "flare_mlp_narrow_parts": (C.c_int, [C.c_int64, C.POINTER(C.c_int32)]),
+    "flare_mlp_narrow_bwd": (C.c_int, [C.POINTER(FlareNarrowDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_act_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_act_fwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P]),

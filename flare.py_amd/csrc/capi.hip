@@ -1386,6 +1386,57 @@ int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img
     return hip_status(flare::launch_mlp_pack(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp pack launch");
 }
 
+// what the narrow layers' entries share
+static int narrow_args(flare::NarrowArgs& a, const FlareNarrowDesc* d, const void* x, const float* w, const float* b)
+{
+    if (!d) return fail(FLARE_EINVAL, "descriptor is NULL");
+    if (d->T < 1 || d->K < 1 || d->K > 4) return fail(FLARE_EINVAL, "T >= 1 and 1 <= K <= 4 required (got %lld, %d)", (long long)d->T, d->K);
+    if (d->w_dtype != FLARE_DT_BF16 && d->w_dtype != FLARE_DT_F16) return fail(FLARE_EINVAL, "w_dtype must be bf16 or f16");
+    if (!flare::mlp_mfma_supported(d->w_dtype, d->C)) return fail(FLARE_EUNSUPPORTED, "C=%d: only 32, 64 and 128 are supported", d->C);
+    if (d->act < -1 || d->act > FLARE_ACT_SILU) return fail(FLARE_EINVAL, "unknown activation %d", d->act);
+    for (int dt : {d->x_dtype, d->y_dtype})
+        if (dt < FLARE_DT_F32 || dt > FLARE_DT_F16) return fail(FLARE_EINVAL, "unknown dtype %d", dt);
+    if (d->out ? d->act != -1 || d->x_dtype != d->w_dtype || d->x_stride != d->C : d->x_stride < d->K || d->y_dtype != d->w_dtype)
+        return fail(FLARE_EINVAL, "the wide rows are contiguous and of w_dtype, narrow x rows K wide or more; no activation behind the last layer");
+    if (!x || !w || !aligned16(d->out ? x : w)) return fail(FLARE_EINVAL, "x and w must not be NULL, wide rows 16-byte aligned");
+    memset(&a, 0, sizeof(a));
+    a.x = x; a.w = w; a.b = b;
+    a.T = d->T; a.xs = d->x_stride; a.C = d->C; a.K = d->K; a.act = d->act; a.x_dtype = d->x_dtype; a.y_dtype = d->y_dtype;
+    return FLARE_OK;
+}
+
+int flare_mlp_narrow_fwd(const FlareNarrowDesc* d, const void* x, const float* w, const float* b, void* t, void* y, void* stream)
+{
+    flare::NarrowArgs a;
+    const int rc = narrow_args(a, d, x, w, b);
+    if (rc != FLARE_OK) return rc;
+    if (!y || (d->act >= 0 && !t) || (!d->out && (!aligned16(y) || (t && !aligned16(t))))) return fail(FLARE_EINVAL, "y (and t with an activation) must not be NULL, wide rows 16-byte aligned");
+    a.y = y; a.t = t;
+    return hip_status(flare::launch_mlp_narrow(a, d->out != 0, false, d->w_dtype, nullptr, nullptr, static_cast<hipStream_t>(stream)), "narrow layer launch");
+}
+
+int flare_mlp_narrow_parts(int64_t T, int32_t* parts)
+{
+    if (!parts || T < 1) return fail(FLARE_EINVAL, "parts must not be NULL, T >= 1");
+    *parts = flare::mlp_narrow_parts(T);
+    return FLARE_OK;
+}
+
+int flare_mlp_narrow_bwd(const FlareNarrowDesc* d, const void* x, const float* w, const void* t, const void* dy, void* dx,
+                         float* dw_part, float* db_part, float* dw, float* db, void* stream)
+{
+    flare::NarrowArgs a;
+    const int rc = narrow_args(a, d, x, w, nullptr);
+    if (rc != FLARE_OK) return rc;
+    if (!dy || !dw_part || !db_part || !dw || !db || (d->act >= 0 && !t)) return fail(FLARE_EINVAL, "dy, t with an activation, dw_part, db_part, dw and db must not be NULL");
+    if (dx && !d->out) return fail(FLARE_EUNSUPPORTED, "no gradient of the narrow input");
+    const void* ptrs[] = {d->out ? dw_part : dy, t, dx, dw_part, db_part, dw, db};
+    for (const void* p : ptrs)
+        if (p && !aligned16(p)) return fail(FLARE_EINVAL, "every buffer must be 16-byte aligned");
+    a.t = const_cast<void*>(t); a.dy = dy; a.dx = dx; a.dw_part = dw_part; a.db_part = db_part;
+    return hip_status(flare::launch_mlp_narrow(a, d->out != 0, true, d->w_dtype, dw, db, static_cast<hipStream_t>(stream)), "narrow layer backward launch");
+}
+
 static int check_rows(int64_t T, int32_t C, std::initializer_list<const void*> must, std::initializer_list<const void*> may)
 {
     if (T < 1) return fail(FLARE_EINVAL, "T >= 1 required (got %lld)", (long long)T);

@@ -365,6 +365,15 @@ struct RowsNormArgs {
     float eps;
 };
 
+// The narrow first / last layer of a model in training (mlp_narrow.hip).  In: x [T,K] any type at a row stride, w [C,K], y and t [T,C];
+// out: x [T,C] contiguous, w [K,C], y [T,K].  Backward: dy of y's shape, dx (out only, or null), partial dW and db ([C]; out: [4]).
+struct NarrowArgs {
+    const void* x; const float* w; const float* b; void* y; void* t;
+    const void* dy; void* dx; float* dw_part; float* db_part;
+    int64_t T, xs, tokens_per_wg;                           // tokens_per_wg: set by the launcher
+    int C, K, act, x_dtype, y_dtype;                        // act: -1 none, 0 tanh-GELU, 1 SiLU
+};
+
 // Backward of one fp32 layer y = [x +] act(x W^T + b) in one pass (rows_layer_f32_mfma.hip)
 struct RowsLayerArgs {
     const float* dy; const float* t; const float* x;        // [T,C]: the gradient of y, x W^T + b (act only), the input
@@ -446,7 +455,9 @@ int        mlp_few_bwd_rows(int64_t T);
 hipError_t launch_mlp_few(const MlpArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_mlp_few_bwd(const MlpBwdArgs& a, int w_dtype, hipStream_t st);
 hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts, hipStream_t st);   // n a multiple of 4
-hipError_t launch_sum_layer_parts(const float* dw_part, float* dw, const float* db_part, float* db, int C, int parts, hipStream_t st);   // db may be null
+hipError_t launch_sum_two_parts(const float* a_part, float* a, int64_t na, const float* b_part, float* b, int64_t nb, int parts, hipStream_t st);   // na, nb multiples of 4; b may be null
+int        mlp_narrow_parts(int64_t T);
+hipError_t launch_mlp_narrow(const NarrowArgs& a, bool out, bool bwd, int dtype, float* dw, float* db, hipStream_t st);
 hipError_t launch_rows_act_fwd(int act, const float* t, const float* x, const float* res, float* y, int64_t n, hipStream_t st);   // n a multiple of 4
 bool       rows_layer_bwd_supported(int C);
 int        rows_layer_bwd_parts(int64_t T);

@@ -293,15 +293,14 @@ hipError_t launch_sum_parts(const float* part, float* out, int64_t n, int parts,
     return hipGetLastError();
 }
 
-hipError_t launch_sum_layer_parts(const float* dw_part, float* dw, const float* db_part, float* db, int C, int parts, hipStream_t st)
+hipError_t launch_sum_two_parts(const float* a_part, float* a, int64_t na, const float* b_part, float* b, int64_t nb, int parts, hipStream_t st)
 {
     SumJobs jobs{};
-    const int64_t n = (int64_t)C * C;
-    const int first = (int)((n / 4 + 15) / 16);            // sixteen ways over the partials (one per compute unit): 64 outputs a workgroup
-    jobs.j[0] = SumJob{dw_part, dw, n, parts, 0, 16};
+    const int first = (int)((na / 4 + 15) / 16);           // sixteen ways over the partials: 64 outputs a workgroup
+    jobs.j[0] = SumJob{a_part, a, na, parts, 0, 16};
     jobs.n = 1;
-    if (db) jobs.j[jobs.n++] = SumJob{db_part, db, C, parts, first, 4};
-    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(first + (db ? (C / 4 + 3) / 4 : 0))), dim3(256), 0, st, jobs);
+    if (b) jobs.j[jobs.n++] = SumJob{b_part, b, nb, parts, first, 4};
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(first + (b ? (nb / 4 + 3) / 4 : 0))), dim3(256), 0, st, jobs);
     return hipGetLastError();
 }
 

@@ -221,7 +221,7 @@ hipError_t launch_rows_layer_bwd(int act, const RowsLayerArgs& a0, float* dw, fl
     a.rows_per_wg = rows_per_wg(a.T);
     const unsigned grid = (unsigned)rows_layer_bwd_parts(a.T);
     const hipError_t e = a.C == 128 ? launch_c<128>(act, a, grid, st) : launch_c<64>(act, a, grid, st);
-    return e != hipSuccess ? e : launch_sum_layer_parts(a.dw_part, dw, a.db_part, db, a.C, (int)grid, st);
+    return e != hipSuccess ? e : launch_sum_two_parts(a.dw_part, dw, (int64_t)a.C * a.C, a.db_part, db, a.C, (int)grid, st);
 }
 
 }  // namespace flare

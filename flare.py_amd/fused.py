@@ -164,6 +164,101 @@ class _NarrowLinearFn(torch.autograd.Function):
         return dx, dw.to(w.dtype), db, None
 
 
+def _narrow_ok(layer, x, cd, act_module=None):
+    """True where the narrow layer (and the activation behind it) can run as one HIP pass each way: plain modules, fp32 parameters, and
+    for the first layer an input that asks for no gradient."""
+    w, b = layer._parameters.get("weight"), layer._parameters.get("bias")
+    return (type(layer) is nn.Linear and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0 and _plain_module(layer)
+            and (act_module is None or (type(act_module) in (nn.GELU, nn.SiLU) and _plain_module(act_module)))
+            and ("bias" in layer._parameters) and all(type(t) in (torch.Tensor, nn.Parameter) and t.dtype is torch.float32 and t.is_cuda
+                                                      and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (w, b) if t is not None)
+            and w is not None)
+
+
+def _plain_module(m):
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
+                or nn.modules.module._has_any_global_hook())
+
+
+def _narrow_desc(x2, w, cd, out, act, y_dtype):
+    d = _lib.FlareNarrowDesc()
+    d.T, d.x_stride, d.out, d.act = x2.shape[0], x2.stride(0), int(out), act
+    d.C, d.K = (w.shape[1], w.shape[0]) if out else (w.shape[0], w.shape[1])
+    d.w_dtype, d.x_dtype, d.y_dtype = _DTYPES[cd], _DTYPES[x2.dtype], _DTYPES[y_dtype]
+    return d
+
+
+def _narrow_backward(d, x2, w, t, dy2, dx, has_bias, dev):
+    lib = _lib.load()
+    parts = C.c_int32(0)
+    _lib.check(lib.flare_mlp_narrow_parts(d.T, C.byref(parts)), "flare_mlp_narrow_parts")
+    nb = 4 if d.out else d.C
+    part = torch.empty(parts.value, w.numel() + nb, dtype=torch.float32, device=dev)
+    dw, db = torch.empty_like(w), torch.empty(nb, dtype=torch.float32, device=dev)
+    with _on_device(dev):
+        rc = lib.flare_mlp_narrow_bwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(t), _ptr(dy2), _ptr(dx), _ptr(part),
+                                      part.data_ptr() + 4 * parts.value * w.numel(), _ptr(dw), _ptr(db), C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_narrow_bwd")
+    return dw, (db if not d.out else db[:d.K]) if has_bias else None
+
+
+class _NarrowInFn(torch.autograd.Function):
+    """act(x W^T + b) of the lift in the compute type (act -1: none); x [T, in_dim] asks for no gradient."""
+
+    @staticmethod
+    def forward(ctx, x2, w, b, cd, act):
+        d = _narrow_desc(x2, w, cd, False, act, cd)
+        y = torch.empty(d.T, d.C, dtype=cd, device=x2.device)
+        t = torch.empty_like(y) if act >= 0 else None
+        with _on_device(x2.device):
+            rc = _lib.load().flare_mlp_narrow_fwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(b), _ptr(t), _ptr(y), C.c_void_p(_stream_ptr(x2.device)))
+        _lib.check(rc, "flare_mlp_narrow_fwd")
+        ctx.cd, ctx.act, ctx.has_bias = cd, act, b is not None
+        ctx.save_for_backward(x2, w, t)
+        return y
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy):
+        x2, w, t = ctx.saved_tensors                      # through saved-tensor hooks in any memory order
+        x2 = x2 if x2.stride(-1) == 1 and x2.stride(0) >= x2.shape[1] else x2.contiguous()
+        d = _narrow_desc(x2, w.contiguous(), ctx.cd, False, ctx.act, ctx.cd)
+        dw, db = _narrow_backward(d, x2, w.contiguous(), None if t is None else _wide(t, ctx.cd), _wide(dy, ctx.cd), None, ctx.has_bias, dy.device)
+        return None, dw, db, None, None
+
+
+class _NarrowOutFn(torch.autograd.Function):
+    """x W^T + b of the last layer in the compute type, handed out in y_dtype."""
+
+    @staticmethod
+    def forward(ctx, x, w, b, cd, y_dtype):
+        x2 = _wide(x, cd)
+        d = _narrow_desc(x2, w, cd, True, -1, y_dtype)
+        y = torch.empty(*x.shape[:-1], d.K, dtype=y_dtype, device=x.device)
+        with _on_device(x.device):
+            rc = _lib.load().flare_mlp_narrow_fwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(b), None, _ptr(y), C.c_void_p(_stream_ptr(x.device)))
+        _lib.check(rc, "flare_mlp_narrow_fwd")
+        ctx.cd, ctx.y_dtype, ctx.has_bias, ctx.shape = cd, y_dtype, b is not None, x.shape
+        ctx.save_for_backward(x2, w)
+        return y
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy):
+        x2, w = ctx.saved_tensors
+        x2, w = _wide(x2, ctx.cd), w.contiguous()
+        d = _narrow_desc(x2, w, ctx.cd, True, -1, ctx.y_dtype)
+        dx = torch.empty_like(x2) if ctx.needs_input_grad[0] else None
+        dw, db = _narrow_backward(d, x2, w, None, dy.contiguous(), dx, ctx.has_bias, dy.device)
+        return None if dx is None else dx.view(ctx.shape), dw, db, None, None
+
+
+def _wide(t, cd):
+    """Contiguous rows [T, C] in the compute type on the 16-byte grid."""
+    t = t.reshape(-1, t.shape[-1]).to(cd).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _train_subchain(mod):
     """_SubChain of a stack with a narrow end (None for every other module); kept on the module."""
     key = _structure_key(mod)
@@ -477,12 +572,20 @@ def fused_mlp(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=
             if sub.first is not None:
                 if hn is not None and not isinstance(hn, nn.Identity):
                     h, hn = hn(h), None
-                h = _NarrowLinearFn.apply(h.reshape(-1, h.shape[-1]), sub.first.weight, sub.first.bias, cd).view(*h.shape[:-1], -1)
-                if sub.first_act:
-                    h = sub.act_module(h)
+                h2 = h.reshape(-1, h.shape[-1])
+                if not h.requires_grad and h2.stride(-1) == 1 and _narrow_ok(sub.first, h, cd, sub.act_module if sub.first_act else None):
+                    act = _layers_of(sub)[3] if sub.first_act else -1
+                    h = _NarrowInFn.apply(h2, sub.first.weight, sub.first.bias, cd, act).view(*h.shape[:-1], -1)
+                else:
+                    h = _NarrowLinearFn.apply(h2, sub.first.weight, sub.first.bias, cd).view(*h.shape[:-1], -1)
+                    if sub.first_act:
+                        h = sub.act_module(h)
             y = _fused_mlp_train(h, sub, cd, hn, None, cd if sub.last is not None else out_dtype)
             if sub.last is not None:
-                y = sub.last(y).to(out_dtype)
+                if out_dtype in _DTYPES and _narrow_ok(sub.last, y, cd):
+                    y = _NarrowOutFn.apply(y, sub.last.weight, sub.last.bias, cd, out_dtype)
+                else:
+                    y = sub.last(y).to(out_dtype)
             return y if res is None else res + y
         return _fused_mlp_train(x, mod, cd, norm, res, out_dtype)
     return _fused_mlp_fwd(x, mod, cd, norm, res, out_dtype, x_head, y_head)

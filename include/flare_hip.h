@@ -444,6 +444,20 @@ int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_
  * the launch that sums the others; gb NULL: nothing. */
 int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream);
+/* The narrow first or last layer of a model in training under autocast (pdebench/models/flare.py:285-310): values are rounded to
+ * w_dtype (bf16 or f16) where separate torch layers round them.  w and b are the fp32 parameters (b may be NULL).
+ *   out == 0: t = x W^T + b, y = act(t) (act -1: y alone); x [T,K] rows at x_stride in any type, w [C,K], t and y [T,C] in w_dtype
+ *   out != 0: y = x W^T + b; x [T,C] in w_dtype (x_stride == C), w [K,C], y [T,K] in y_dtype; act is -1
+ * Backward: dw and db of w's and b's shape (out: db [4], the first K count) in fp32, summed over dw_part, db_part [parts, ...];
+ * dx [T,C] (or NULL) for the last layer only. */
+typedef struct FlareNarrowDesc {
+    int64_t T, x_stride;
+    int32_t C, K, out, act, w_dtype, x_dtype, y_dtype;
+} FlareNarrowDesc;
+int flare_mlp_narrow_fwd(const FlareNarrowDesc* desc, const void* x, const float* w, const float* b, void* t, void* y, void* stream);
+int flare_mlp_narrow_parts(int64_t T, int32_t* parts);
+int flare_mlp_narrow_bwd(const FlareNarrowDesc* desc, const void* x, const float* w, const void* t, const void* dy, void* dx,
+                         float* dw_part, float* db_part, float* dw, float* db, void* stream);
 /* Row passes around fp32 products in training: contiguous [T,C] rows on the 16-byte grid, C in {32, 64, 128, 256}; act -1 none, else
  * FLARE_ACT_*; norm FLARE_NORM_LAYER or FLARE_NORM_RMS.
  *   flare_rows_act_bwd   dt = ds act'(t), db [C] = its column sums (act -1: the column sums of ds, t and dt may be

@@ -617,3 +617,62 @@ def test_joint_packing_and_the_residuals_gradient_of_a_block(dev, monkeypatch, l
     with torch.autocast("cuda", dtype=torch.bfloat16):
         y = blk(x.detach())
     (y if lra else y[0]).sum().backward()
+
+
+@pytest.mark.parametrize("T,C,K", [(1, 32, 1), (63, 64, 3), (65, 128, 4), (4097, 128, 2), (20001, 64, 1), (70001, 32, 3)])
+@pytest.mark.parametrize("cd,act,xd", [(torch.bfloat16, "gelu", torch.float32), (torch.float16, "silu", torch.float16), (torch.bfloat16, "silu", torch.bfloat16)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_narrow_layers_against_the_torch_layers(dev, monkeypatch, T, C, K, cd, act, xd, bias):
+    """The lift with its activation and the last layer as HIP passes, against the same layers run by torch under autocast: both are held
+    to fp64, and the passes may be further off by a quarter (their sums run in another order, the roundings to 16 bits are alike);
+    2e-5 is room for results that torch gets exactly."""
+    torch.manual_seed(T + K)
+    lo, hi = (ResidualMLP(K, C, C, num_layers=1, act=act, input_residual=False, output_residual=True).to(dev),
+              ResidualMLP(C, C, K, num_layers=1, act=act, input_residual=True, output_residual=False).to(dev))
+    for m in (lo, hi):
+        for l in (m.fc1, m.fc2):
+            if min(l.weight.shape) <= 4 and not bias:
+                l.bias = None
+    first, last = lo.fc1, hi.fc2
+    x, h = torch.randn(T, K + 2, device=dev).to(xd)[:, :K], torch.randn(T, C, device=dev).to(cd)
+    g1, g2 = torch.randn(T, C, device=dev).to(cd), torch.randn(T, K, device=dev)
+    assert fused._narrow_ok(first, x, cd, lo.act) and fused._narrow_ok(last, h, cd)
+    h.requires_grad_(True)
+
+    def run(hip):
+        with torch.autocast("cuda", dtype=cd):
+            a = fused._NarrowInFn.apply(x, first.weight, first.bias, cd, 0 if act == "gelu" else 1) if hip else lo.act(fused._NarrowLinearFn.apply(x, first.weight, first.bias, cd))
+            b = fused._NarrowOutFn.apply(h, last.weight, last.bias, cd, torch.float32) if hip else last(h).float()
+        ps = [p for p in (first.weight, first.bias) if p is not None], [p for p in (last.weight, last.bias) if p is not None]
+        return [a.detach(), b.detach(), *torch.autograd.grad(a, ps[0], g1), *torch.autograd.grad(b, [h, *ps[1]], g2)]
+
+    got, other = run(True), run(False)
+    d = lambda t: None if t is None else t.detach().double().requires_grad_(True)
+    w1, b1, w2, b2, h64 = d(first.weight), d(first.bias), d(last.weight), d(last.bias), d(h)
+    f = nn.functional.silu if act == "silu" else (lambda v: nn.functional.gelu(v, approximate="tanh"))
+    a, b = f(nn.functional.linear(x.double(), w1, b1)), nn.functional.linear(h64, w2, b2)
+    want = [a.detach(), b.detach(), *torch.autograd.grad(a, [t for t in (w1, b1) if t is not None], g1.double()),
+            *torch.autograd.grad(b, [t for t in (h64, w2, b2) if t is not None], g2.double())]
+    for i, (p, q, r) in enumerate(zip(got, other, want)):
+        assert p.shape == q.shape and p.dtype == q.dtype, i
+        ep, eq = rel(p.double(), r), rel(q.double(), r)
+        # the last layer's bias gradient is up to four sums of rounded terms: either side is within a rounding (half a unit) of fp64
+        floor = 2e-5 if p.numel() > 4 else 2.0 ** -9 if cd is torch.bfloat16 else 2.0 ** -12
+        assert ep <= 1.25 * eq + floor, (i, ep, eq)
+
+
+def test_narrow_layers_that_keep_the_torch_layers(dev):
+    lin, x = nn.Linear(3, 64).to(dev), torch.randn(10, 3, device=dev)
+    assert fused._narrow_ok(lin, x, torch.bfloat16)
+    seen = []
+    h = lin.register_forward_hook(lambda *a: seen.append(1))
+    assert not fused._narrow_ok(lin, x, torch.bfloat16)
+    h.remove()
+    assert not fused._narrow_ok(nn.Linear(3, 64).to(dev).bfloat16(), x, torch.bfloat16)
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=64).to(dev)
+    h = m.out_proj[1].fc2.register_forward_hook(lambda *a: seen.append(2))
+    xm = torch.randn(2, 100, 3, device=dev, requires_grad=True)      # an input that asks for its gradient: torch's lift
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        m(xm).sum().backward()
+    h.remove()
+    assert seen == [2] and bool(torch.isfinite(xm.grad).all()) and float(xm.grad.abs().sum()) > 0
