@@ -1336,6 +1336,13 @@ int flare_mlp_wgrad(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_str
 int flare_mlp_wgrad_norm(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream)
 {
+    return flare_mlp_wgrad_norms(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, gb_part, nullptr, gb_rows, gb, nullptr, stream);
+}
+
+int flare_mlp_wgrad_norms(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part, int32_t gb_rows,
+                          float* gb, float* gb2, void* stream)
+{
     int rc = check_wgrad_desc(d);
     if (rc != FLARE_OK) return rc;
     if (!a_in || !g_out || !dw_part) return fail(FLARE_EINVAL, "a_in, g_out and dw_part must not be NULL");
@@ -1352,7 +1359,10 @@ int flare_mlp_wgrad_norm(const FlareMlpDesc* d, const void* a_in, int64_t a_laye
     a.dw_part = dw_part; a.db_part = db_part; a.dw = dw; a.db = db;
     if (gb && (!gb_part || gb_rows < 1 || !aligned16(gb_part) || !aligned16(gb)))
         return fail(FLARE_EINVAL, "gb needs gb_part with gb_rows >= 1, both 16-byte aligned");
+    if (gb2 && (!gb2_part || gb_rows < 1 || !aligned16(gb2_part) || !aligned16(gb2)))
+        return fail(FLARE_EINVAL, "gb2 needs gb2_part with gb_rows >= 1, both 16-byte aligned");
     a.gb_part = gb ? gb_part : nullptr; a.gb_rows = gb_rows; a.gb = gb;
+    a.gb2_part = gb2 ? gb2_part : nullptr; a.gb2 = gb2;
     a.T = d->T; a.C = d->C; a.L = d->L;
     return hip_status(flare::launch_mlp_wgrad(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp weight-gradient launch");
 }

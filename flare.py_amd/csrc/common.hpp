@@ -334,6 +334,7 @@ struct MlpWgradArgs {
     float* dw; float* db;                       // [L,C,C], [L,C] out or null: the partials summed in index order
     const float* gb_part; float* gb;            // or null: the norm's partial rows [gb_rows,2,C] of the backward, summed by the same launch
     int gb_rows;
+    const float* gb2_part; float* gb2;          // or null: a second norm's, of as many rows
     int64_t T;
     int C, L;
     int64_t tokens_per_wg;                      // set by the launcher

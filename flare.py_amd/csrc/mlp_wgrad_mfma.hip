@@ -196,12 +196,12 @@ __global__ __launch_bounds__(64 * WO * WI * WK) void mlp_wgrad_kernel(MlpWgradAr
     }
 }
 
-// Up to three sums over partial results in one launch: out[i] = sum over p of part[p][i].  A workgroup owns 4 X outputs of one
+// Up to four sums over partial results in one launch: out[i] = sum over p of part[p][i].  A workgroup owns 4 X outputs of one
 // job: thread (x, y) adds the partials p = y, y + Y, ... of four outputs with four loads in flight (X Y = 256), the Y meet in
 // LDS.  The order of the additions is fixed.  Wide jobs (the weights) take X = 64, narrow ones (biases, norm parameters, whose
 // partials are many) X = 16.  Every sum was a launch of its own before: three of the nine launches of a chain's backward.
 struct SumJob { const float* part; float* out; int64_t n; int parts, first, x; };     // first: its first workgroup
-struct SumJobs { SumJob j[3]; int n; };
+struct SumJobs { SumJob j[4]; int n; };
 __global__ __launch_bounds__(256) void sum_parts_kernel(SumJobs jobs)
 {
     __shared__ f32x4 red[256];
@@ -321,6 +321,7 @@ hipError_t launch_mlp_wgrad(const MlpWgradArgs& a0, int w_dtype, hipStream_t st)
     add(a.dw_part, a.dw, (int64_t)a.L * a.C * a.C, parts, 64);
     add(a.db_part, a.db, (int64_t)a.L * a.C, parts, 16);
     add(a.gb_part, a.gb, 2 * (int64_t)a.C, a.gb_rows, 16);
+    add(a.gb2_part, a.gb2, 2 * (int64_t)a.C, a.gb_rows, 16);
     if (blocks > 0) {
         hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)blocks), dim3(256), 0, st, jobs);
         e = hipGetLastError();

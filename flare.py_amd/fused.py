@@ -841,11 +841,11 @@ def _packed_train_expand(mod, E, cd):
     return w, b, w_img, wt_img
 
 
-def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None):
+def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None, gb2=None, gsum2=None):
     """dW [L, C(out), C(in)] and db [L, C] (or None) in fp32 from the rows the backward launch left: one pass of
     flare_mlp_wgrad over both row arrays, partial results per token range summed in a fixed order.  g_out, a_in:
     [L,T,C], or [T,C] for an array all L layers share.  gb, gsum: the norm's partial rows [rows,2,C], summed into gsum [2,C] by
-    the launch that sums the others."""
+    the launch that sums the others; gb2, gsum2: another norm's."""
     lib = _lib.load()
     T, Cdim = g_out.shape[-2:]
     L = (g_out.shape[0] if g_out.dim() == 3 else a_in.shape[0]) if L is None else L
@@ -860,10 +860,11 @@ def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None):
     dw = torch.empty(L, Cdim, Cdim, dtype=torch.float32, device=dev)
     db = torch.empty(L, Cdim, dtype=torch.float32, device=dev) if want_bias else None
     with _on_device(dev):
-        rc = lib.flare_mlp_wgrad_norm(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
-                                      _ptr(g_out), T * Cdim if g_out.dim() == 3 else 0, _ptr(dwp), _ptr(dbp), _ptr(dw), _ptr(db),
-                                      _ptr(gb), 0 if gb is None else gb.shape[0], _ptr(gsum), C.c_void_p(_stream_ptr(dev)))
-    _lib.check(rc, "flare_mlp_wgrad_norm")
+        rows = 0 if gb is None and gb2 is None else (gb2 if gb is None else gb).shape[0]
+        rc = lib.flare_mlp_wgrad_norms(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
+                                       _ptr(g_out), T * Cdim if g_out.dim() == 3 else 0, _ptr(dwp), _ptr(dbp), _ptr(dw), _ptr(db),
+                                       _ptr(gb), _ptr(gb2), rows, _ptr(gsum), _ptr(gsum2), C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_wgrad_norms")
     return dw, db
 
 
@@ -919,11 +920,12 @@ def _norm_grads(norm, gsum, need_gamma, need_beta):
             gsum[1].to(norm.bias.dtype) if (need_beta and getattr(norm, "bias", None) is not None) else None]
 
 
-def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
+def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, into=None):
     """Backward of y = [x +] chain(norm(x)) for the chain of C x C layers: (dx [T,C], the norm's [2,C] sums or None,
     dW [L,out,in], db [L,C] or None, the layers).  dx_acc: a [T,C] gradient of the same x that another chain left
     (x's dtype, contiguous); the kernel adds its result into it and it is returned as dx.  x_head: rows of x and dx hold padded
-    heads (few tokens only)."""
+    heads (few tokens only).  into: (a_in, g_out) [L,T,C] that take the rows for the weight gradients, which the caller forms (few
+    tokens only): then (dx, the norm's partial rows or None)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _layers_of(mod)
     L = len(layers)
@@ -933,7 +935,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     packed = _packed_few(mod, layers, cd, True) if few else None
     if packed is not None:
         w_img, b, wt_img = packed            # the tiled operands
-    elif x_head:
+    elif x_head or into is not None:
         raise RuntimeError("head-padded rows have a backward in the few-token launches only")
     else:
         few = 0
@@ -954,8 +956,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     if dx_acc is not None and (dx_acc.shape != (T, Cdim) or dx_acc.dtype != x2.dtype or not dx_acc.is_contiguous()):
         raise ValueError("dx_acc must be a contiguous [T, C] tensor of x's dtype")
     dx = dx_acc if dx_acc is not None else torch.empty(T, xw, dtype=x2.dtype, device=dev)
-    a_in = torch.empty(L, T, Cdim, dtype=cd, device=dev)
-    g_out = torch.empty(L, T, Cdim, dtype=cd, device=dev)
+    a_in, g_out = (torch.empty(L, T, Cdim, dtype=cd, device=dev) for _ in range(2)) if into is None else into
     dn = stats = gb = gsum = None
     any_bias = any(l.bias is not None for l in layers)
     if few and d.norm:
@@ -978,13 +979,15 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
                                    bits, _ptr(dx), _ptr(a_in), _ptr(g_out), _ptr(dn), _ptr(stats), _ptr(gb),
                                    None, C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_bwd")
+    if into is not None:
+        return dx, gb
     # weight and bias gradients: one more launch over the rows the kernel left (16-bit products with fp32
     # accumulation, as torch runs a Linear's backward under autocast); norm gradients: partial rows, summed with the others
     dW, db = _weight_grads(d, g_out, a_in, any_bias, gb=gb, gsum=gsum)                 # [L, out, in], [L, C] fp32
     return dx, gsum, dW, db, layers
 
 
-def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None):
+def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None, into=None):
     """Backward of both stacks of a pair in one launch (y_head: dya and dyb are rows of padded heads; dres: another gradient of x,
     added to dx): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
     None, the 2 L layers)."""
@@ -1010,7 +1013,7 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None):
     d.flags = (y_head // 4) << 12
     gamma, beta = _norm_args(d, norm, x, Cdim)
     dx = torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
-    rows = torch.empty(2, L2, T, Cdim, dtype=cd, device=dev)         # a_in, g_out
+    rows = torch.empty(2, L2, T, Cdim, dtype=cd, device=dev) if into is None else into         # a_in, g_out
     gb = gsum = None
     if d.norm:
         gb = torch.empty(_few(T, Cdim, L2 // 2), 2, Cdim, dtype=torch.float32, device=dev)
@@ -1024,6 +1027,8 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None):
         rc = lib.flare_mlp_few_bwd_res(C.byref(d), _ptr(x2), _ptr(da), _ptr(db_), _ptr(r2), _ptr(w), _ptr(wt), _ptr(b), _ptr(gamma),
                                        _ptr(beta), 0, _ptr(dx), _ptr(rows[0]), _ptr(rows[1]), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_few_bwd_res")
+    if into is not None:                       # as _chain_backward's
+        return dx, gb
     dW, db = _weight_grads(d, rows[1], rows[0], any(l.bias is not None for l in layers), gb=gb, gsum=gsum)
     return dx, gsum, dW, db, layers
 

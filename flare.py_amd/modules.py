@@ -19,7 +19,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
-from . import block_plan, fused, rows
+from . import block_plan, block_train, fused, rows
 from .functional import flare_multihead_mixer, mixer_narrow_heads
 
 __all__ = ["ResidualMLP", "FLARE", "FLAREBlock", "FinalLayer", "FLAREModel"]
@@ -287,7 +287,8 @@ class FLAREBlock(nn.Module):
 
     def forward(self, x, return_scores: bool = False):
         if not return_scores and type(self.att) is FLARE:
-            y = block_plan.forward(self, x)      # inference under autocast: the launches below from one call
+            # the launches below from one call (inference under autocast), or as one autograd node (training on few tokens)
+            y = block_train.forward(self, x) if torch.is_grad_enabled() else block_plan.forward(self, x)
             if y is not None:
                 return y, None
         if torch.is_grad_enabled():

@@ -444,6 +444,10 @@ int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_
  * the launch that sums the others; gb NULL: nothing. */
 int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream);
+/* The same with the partial rows of two norms (a block's), gb_rows each; gb and gb2 may be NULL. */
+int flare_mlp_wgrad_norms(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part,
+                          int32_t gb_rows, float* gb, float* gb2, void* stream);
 /* The narrow first or last layer of a model in training under autocast (pdebench/models/flare.py:285-310): values are rounded to
  * w_dtype (bf16 or f16) where separate torch layers round them.  w and b are the fp32 parameters (b may be NULL).
  *   out == 0: t = x W^T + b, y = act(t) (act -1: y alone); x [T,K] rows at x_stride in any type, w [C,K], t and y [T,C] in w_dtype

@@ -11,7 +11,7 @@ import torch
 from torch import nn
 
 import flare_py_amd as F
-from flare_py_amd import fused
+from flare_py_amd import block_train, fused
 from flare_py_amd.modules import ResidualMLP
 from oracle import flare_oracle as O
 
@@ -468,7 +468,7 @@ def test_block_with_16bit_parameters_trains_fused(dev, dtype):
 def test_packed_operands_are_the_stacked_parameters(dev, C, cd, pd):
     """The packing launch against torch's own stack and cast, bit for bit: rows at a stride and off the 16-byte grid, a missing
     bias, a narrow last layer, the expanding MLP's tiles, special values."""
-    from flare_py_amd import fused
+    from flare_py_amd import block_train, fused
 
     g = torch.Generator().manual_seed(C)
     layers = [torch.nn.Linear(C, C, bias=i != 1) for i in range(3)] + [torch.nn.Linear(C, 3)]
@@ -550,17 +550,20 @@ def test_narrow_heads_stay_padded_in_training(dev, monkeypatch, C, H, B, N, cd, 
             y = blk(x)[0]
         return [y.detach(), *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
 
-    got = step()
+    got = [step()]                                             # the block as one node
+    monkeypatch.setattr(block_train, "forward", lambda *a: None)
+    got.append(step())                                         # stack by stack
     monkeypatch.setattr(fused, "narrow_train_ok", lambda *a: False)
     other = step()
     sd = {k: v.detach().cpu().double().requires_grad_(True) for k, v in blk.state_dict().items()}
     x64 = x.detach().cpu().double().requires_grad_(True)
     y64 = O.flare_block(sd, "", x64, H, rmsnorm=rms)
     want = [y64.detach(), *torch.autograd.grad(y64, [x64, *(sd[n] for n, _ in blk.named_parameters())], gy.cpu().double())]
-    for i, (a, b, r) in enumerate(zip(got, other, want)):
-        assert a.shape == b.shape and a.dtype == b.dtype
-        ea, eb = (float((t.cpu().double() - r).norm() / (r.norm() + 1e-300)) for t in (a, b))
-        assert ea <= 1.25 * eb + 2e-3, (i, ea, eb)
+    for g in got:
+        for i, (a, b, r) in enumerate(zip(g, other, want)):
+            assert a.shape == b.shape and a.dtype == b.dtype
+            ea, eb = (float((t.cpu().double() - r).norm() / (r.norm() + 1e-300)) for t in (a, b))
+            assert ea <= 1.25 * eb + 2e-3, (i, ea, eb)
 
 
 def test_padded_rows_beyond_the_few_token_launches_are_refused(dev):
@@ -596,6 +599,7 @@ def test_joint_packing_and_the_residuals_gradient_of_a_block(dev, monkeypatch, l
         y = y if lra else y[0]
         return [y.detach(), *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
 
+    monkeypatch.setattr(block_train, "forward", lambda *a: None)
     packs, real = [], fused._pack_launch
     monkeypatch.setattr(fused, "_pack_launch", lambda *a, **k: (packs.append(len(a[2])), real(*a, **k))[1])
     got = step()
@@ -676,3 +680,78 @@ def test_narrow_layers_that_keep_the_torch_layers(dev):
         m(xm).sum().backward()
     h.remove()
     assert seen == [2] and bool(torch.isfinite(xm.grad).all()) and float(xm.grad.abs().sum()) > 0
+
+
+# head dims 4, 8, 16, 32, 64; one token; the ends of the few-token range; unequal stacks; norms with and without bias
+@pytest.mark.parametrize("C,H,M,B,N,kw", [(64, 16, 32, 1, 1, {}), (64, 8, 64, 2, 1001, {}), (128, 8, 128, 3, 1365, {"rmsnorm": True}), (128, 8, 64, 1, 12288, {}),
+                                          (64, 2, 256, 1, 333, {"num_layers_ffn": 1}), (64, 1, 32, 2, 40, {"num_layers_k_proj": 2, "num_layers_v_proj": 2}),
+                                          (32, 2, 96, 1, 16384, {"num_layers_ffn": -1})])
+@pytest.mark.parametrize("cd,xd", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_block_as_one_node(dev, monkeypatch, C, H, M, B, N, kw, cd, xd):
+    """Against the same launches stack by stack: outputs bit for bit; gradients to the order of the fp32 sums over tokens (1e-5), or to a
+    rounding of the 16-bit operands that such a sum feeds (the latents' gradient and what lies before the mixer: 1e-2)."""
+    torch.manual_seed(N)
+    blk = F.FLAREBlock(channel_dim=C, num_heads=H, num_latents=M, **kw).to(dev)
+    for l in blk.modules():
+        if isinstance(l, nn.Linear):
+            l.reset_parameters()
+    x = torch.randn(B, N, C, device=dev).to(xd).requires_grad_(True)
+    gy = torch.randn(B, N, C, device=dev).to(xd)
+
+    def step(hip=True):
+        with torch.autocast("cuda", dtype=cd):
+            y = blk(x)[0]
+        assert ("BlockFn" in type(y.grad_fn).__name__) == hip
+        return [y.detach(), *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
+
+    got, again = step(), step()
+    monkeypatch.setattr(block_train, "forward", lambda *a: None)
+    want = step(False)
+    names = ["y", "x", *(n for n, _ in blk.named_parameters())]
+    assert torch.equal(got[0], want[0])
+    for n, a, a2, b in zip(names, got, again, want):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, a2), n
+        assert rel(a.float(), b.float()) <= (1e-5 if xd is torch.float32 and n.startswith("mlp") else 1e-2), n
+
+
+def test_calls_that_keep_a_node_per_stack(dev):
+    blk = F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=64).to(dev)
+    x = torch.randn(2, 100, 64, device=dev)
+
+    def names(b=blk, t=x):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return type(b(t)[0].grad_fn).__name__
+
+    assert "BlockFn" in names()
+    assert "BlockFn" not in names(t=torch.randn(2, 100, 72, device=dev)[..., :64]) and "BlockFn" not in names(t=torch.randn(1, 16385, 64, device=dev))
+    seen = []
+    h = blk.att.register_forward_hook(lambda *a: seen.append(1))
+    assert "BlockFn" not in names() and seen
+    h.remove()
+    assert "BlockFn" not in names(F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=64, qk_norm=True).to(dev))
+    assert "BlockFn" not in names(F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=40).to(dev))
+    # frozen parameters get no gradient, the others the same one; a change in place between the passes is an error
+    blk.att.latent_q.requires_grad_(False)
+    blk.mlp.fc1.weight.requires_grad_(False)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x)[0]
+    y.sum().backward()
+    assert blk.att.latent_q.grad is None and blk.mlp.fc1.weight.grad is None and blk.mlp.fc2.weight.grad is not None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x)[0]
+    with torch.no_grad():
+        blk.mlp.fc2.bias.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified in place"):
+        y.sum().backward()
+    # saved tensors may come back in another memory order
+    xg = x.clone().requires_grad_(True)
+    def grads():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = blk(xg)[0]
+        return torch.autograd.grad(y.sum(), [xg, blk.att.k_proj.fc1.weight])
+    want = grads()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.transpose(-1, -2).contiguous().transpose(-1, -2) if t.dim() > 1 else t):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = blk(xg)[0]
+    got = torch.autograd.grad(y.sum(), [xg, blk.att.k_proj.fc1.weight])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
