@@ -496,7 +496,8 @@ BwdPlan plan_bwd(const FlareMixerDesc* d)
     auto split = [&](int per_cu, int& n_splits, int& tokens_per_split) {
         int64_t s = std::max<int64_t>(1, per_cu * flare::device_cus() / (bh * mblocks));
         int64_t tps = ((int64_t)d->N + s - 1) / s;
-        tps = (tps + 63) / 64 * 64;
+        const int tile = !f32 && d->D <= 16 ? 128 : 64;
+        tps = (tps + tile - 1) / tile * tile;
         tokens_per_split = (int)tps;
         n_splits = (int)(((int64_t)d->N + tps - 1) / tps);
     };

@@ -170,7 +170,9 @@ __device__ __forceinline__ float dot8(u32x4 u, u32x4 w)
 }
 
 // ---- latent side ---------------------------------------------------------------------------
-constexpr int kBTile = 64;   // tokens per LDS tile
+// Tokens per LDS tile.  At head dim 16 a tile of 64 is half a row chunk per thread and too little work to cover the next one's trip from
+// memory: dz pass 55 -> 51 us, dq pass 84.5 -> 76 us at B=2, H=8, N=100,003, M=128; 115 -> 112 and 226 -> 205 us at B=1, N=300,000, M=256.
+constexpr int bwd_tile(int D) { return D <= 16 ? 128 : 64; }
 
 // One workgroup = 4 waves x (16 CT latents) x one token range.  MODE 0: dz partial; MODE 1: dq partial.
 // KIND: 0 plain, 1 the forward dropped weights, 2 absent tokens (a key mask): their rows are staged as zeros, which with their
@@ -181,6 +183,7 @@ template <typename T, int D, int CT, int MODE, int KIND>
 __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void bwd_lat_kernel(MixerBwdArgs a)
 {
     constexpr bool DROPK = KIND == 1, ABSENT = KIND == 2;
+    constexpr int kBTile = bwd_tile(D);
     constexpr int KD = (D + 31) / 32, RT = D / 16, CH = D / 8, MB = 64 * CT, ROWB = D * 2, TILEB = kBTile * ROWB;
     constexpr int NT = MODE == 0 ? 2 : 4;          // staged tiles: K rows, dY^T | K rows, K^T, V rows, dY rows
     using M_ = Mb<T>;
@@ -517,7 +520,12 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
 
     if (make_delta) {
         // the smallest token log-sum-exp of this split (log2 units), for the passes that follow
-        const float rm = wave_max(rr_max);      // wave 0 = the threads that read the tokens' scalars
+        float rm = wave_max(rr_max);            // waves 0 .. kBTile / 64 - 1: the threads that read the tokens' scalars
+        if constexpr (kBTile > 64) {            // (the tiles' scalars are read no more)
+            if (lane == 0) tsc[0][0][w] = rm;
+            __syncthreads();
+            rm = fmaxf(tsc[0][0][0], tsc[0][0][1]);
+        }
         if (tid == 0) a.rho_min[bh * a.n_splits + split] = -rm;
     }
 
