@@ -149,6 +149,8 @@ SYMBOLS = {
     "flare_mlp_narrow_bwd": (C.c_int, [C.POINTER(FlareNarrowDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_rows_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_act_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P]),
+    "flare_pad_rows": (C.c_int, [C.c_int32, C.c_int32, C.POINTER(C.c_int64), C.c_int32, C.c_int32, C.POINTER(_P), C.POINTER(C.c_int64),
+                                 C.POINTER(_P), C.POINTER(C.c_int64), _P]),
     "flare_rows_act_fwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_rows_layer_bwd_parts": (C.c_int, [C.c_int64, C.c_int32, C.POINTER(C.c_int32)]),
     "flare_rows_layer_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -1479,6 +1479,34 @@ int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const
     return hip_status(flare::launch_rows_act_bwd(act, ds, t, dt, copy, db_part, db, T, C, static_cast<hipStream_t>(stream)), "row activation backward launch");
 }
 
+int flare_pad_rows(int32_t jobs, int32_t elem_bytes, const int64_t n[3], int32_t src_width, int32_t dst_width, const void* const* src,
+                   const int64_t* src_strides, void* const* dst, const int64_t* dst_strides, void* stream)
+{
+    if (jobs < 1 || jobs > 4 || (elem_bytes != 2 && elem_bytes != 4)) return fail(FLARE_EINVAL, "1 to 4 jobs, elements of 2 or 4 bytes");
+    if (!n || !src || !src_strides || !dst || !dst_strides) return fail(FLARE_EINVAL, "a required array is NULL");
+    if (src_width < 1 || dst_width < 1 || src_width > 4096 || dst_width > 4096) return fail(FLARE_EINVAL, "widths must be in [1, 4096]");
+    flare::PadRowsArgs a;
+    memset(&a, 0, sizeof(a));
+    a.jobs = jobs;
+    for (int x = 0; x < 3; ++x) {
+        if (n[x] < 0) return fail(FLARE_EINVAL, "n must be >= 0");
+        if (n[x] == 0) return FLARE_OK;
+        a.n[x] = n[x];
+    }
+    for (int k = 0; k < jobs; ++k) {
+        if (!src[k] || !dst[k] || reinterpret_cast<uintptr_t>(src[k]) % elem_bytes || reinterpret_cast<uintptr_t>(dst[k]) % elem_bytes)
+            return fail(FLARE_EINVAL, "array %d is NULL or off its elements' grid", k);
+        a.job[k].src = static_cast<const uint8_t*>(src[k]);
+        a.job[k].dst = static_cast<uint8_t*>(dst[k]);
+        for (int x = 0; x < 3; ++x) {
+            a.job[k].ss[x] = src_strides[3 * k + x] * elem_bytes;
+            a.job[k].ds[x] = dst_strides[3 * k + x] * elem_bytes;
+            if (a.job[k].ss[x] < 0 || a.job[k].ds[x] < 0) return fail(FLARE_EINVAL, "strides must be >= 0");
+        }
+    }
+    return hip_status(flare::launch_pad_rows(a, (int64_t)src_width * elem_bytes, (int64_t)dst_width * elem_bytes, static_cast<hipStream_t>(stream)), "pad rows launch");
+}
+
 int flare_rows_act_fwd(int64_t T, int32_t C, int32_t act, const float* t, const float* x, const float* res, float* y, void* stream)
 {
     const int rc = check_rows(T, C, {t, y}, {x, res});

@@ -366,6 +366,18 @@ struct RowsNormArgs {
     float eps;
 };
 
+// Rows filled up with zeros, or cut (rows_pad.hip)
+struct PadRowsJob {
+    const uint8_t* src; uint8_t* dst;
+    int64_t ss[3], ds[3];                                   // bytes
+};
+struct PadRowsArgs {
+    PadRowsJob job[4];
+    int jobs;
+    int64_t n[3];
+    int src_units, dst_units;                               // set by the launcher
+};
+
 // The narrow first / last layer of a model in training (mlp_narrow.hip).  In: x [T,K] any type at a row stride, w [C,K], y and t [T,C];
 // out: x [T,C] contiguous, w [K,C], y [T,K].  Backward: dy of y's shape, dx (out only, or null), partial dW and db ([C]; out: [4]).
 struct NarrowArgs {
@@ -460,6 +472,7 @@ hipError_t launch_sum_two_parts(const float* a_part, float* a, int64_t na, const
 int        mlp_narrow_parts(int64_t T);
 hipError_t launch_mlp_narrow(const NarrowArgs& a, bool out, bool bwd, int dtype, float* dw, float* db, hipStream_t st);
 hipError_t launch_rows_act_fwd(int act, const float* t, const float* x, const float* res, float* y, int64_t n, hipStream_t st);   // n a multiple of 4
+hipError_t launch_pad_rows(PadRowsArgs a, int64_t src_bytes, int64_t dst_bytes, hipStream_t st);
 bool       rows_layer_bwd_supported(int C);
 int        rows_layer_bwd_parts(int64_t T);
 hipError_t launch_rows_layer_bwd(int act, const RowsLayerArgs& a, float* dw, float* db, hipStream_t st);

@@ -441,9 +441,34 @@ def _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, km, gy, drop=None):
     return gq, gk, gv
 
 
+def _pad_rows(ts, width, token_major=None):
+    """[B,H,N,D] tensors as [B,H,N,width], filled up with zeros or cut, in one launch; in memory [B,N,H,width] where the tensor (or
+    token_major) says so, else [B,H,N,width]."""
+    B, H, N, D = ts[0].shape
+    ts = [_rows_last_contig(t) for t in ts]
+    if any(s < 0 for t in ts for s in t.stride()):
+        ts = [t.contiguous() for t in ts]
+    out = []
+    for t in ts:
+        if t.stride(1) < t.stride(2) if token_major is None else token_major:
+            out.append(torch.empty(B, N, H, width, dtype=t.dtype, device=t.device).permute(0, 2, 1, 3))
+        else:
+            out.append(torch.empty(B, H, N, width, dtype=t.dtype, device=t.device))
+    if ts[0].numel() == 0:
+        return [o.zero_() for o in out]
+    n, k = (C.c_int64 * 3)(B, H, N), len(ts)
+    with _on_device(ts[0].device):
+        rc = _lib.load().flare_pad_rows(k, ts[0].element_size(), n, D, width, (C.c_void_p * k)(*(t.data_ptr() for t in ts)),
+                                        (C.c_int64 * (3 * k))(*(s for t in ts for s in t.stride()[:3])), (C.c_void_p * k)(*(t.data_ptr() for t in out)),
+                                        (C.c_int64 * (3 * k))(*(s for t in out for s in t.stride()[:3])), C.c_void_p(_stream_ptr(ts[0].device)))
+    _lib.check(rc, "flare_pad_rows")
+    return out
+
+
 class _MixerFn(torch.autograd.Function):
     """q16: q as the kernels take it (cast for autocast, its heads filled up with zero columns to those of k and v), where that is
-    another tensor; the gradient then goes to q itself, in q's type and width, without the cast's and the padding's own nodes."""
+    another tensor; the gradient then goes to q itself, in q's type and width, without the cast's and the padding's own nodes.  k and v
+    whose heads are narrower than q16's are filled up here, and y comes back at their width."""
 
     @staticmethod
     def forward(ctx, q, k, v, scale, key_mask, n_splits, force_generic, token_major, q16=None):
@@ -452,6 +477,10 @@ class _MixerFn(torch.autograd.Function):
         ctx.set_materialize_grads(False)      # z's gradient, which nobody reads, would be a launch
         if q16 is not None:
             q = q16
+        ctx.kv_width, ctx.kv_major = k.shape[-1], tuple(t.stride(1) < t.stride(2) for t in (k, v))
+        ctx.pad = q.shape[-1] > k.shape[-1]
+        if ctx.pad:
+            k, v = _pad_rows((k, v), q.shape[-1])
         ctx.hip = _hip_backward_ok(q, k, v, key_mask, force_generic)
         if ctx.hip:
             y, z, lse_lat, lse_tok = _mixer_forward(q, k, v, scale, key_mask, n_splits, force_generic, token_major, True)
@@ -464,6 +493,9 @@ class _MixerFn(torch.autograd.Function):
         else:
             y, z = _mixer_forward(q, k, v, scale, key_mask, n_splits, force_generic, token_major)
             ctx.save_for_backward(q, k, v)
+        if ctx.pad:       # token-major rows at their own width, so that merging the heads stays free; else a view
+            y = _pad_rows((y,), ctx.kv_width, True)[0] if token_major else y[..., :ctx.kv_width]
+            z = z[..., :ctx.kv_width]
         ctx.mark_non_differentiable(z)
         return y, z
 
@@ -472,6 +504,8 @@ class _MixerFn(torch.autograd.Function):
     def backward(ctx, gy, _gz):
         if gy is None:
             return (None,) * 9
+        if ctx.pad:
+            gy = _pad_rows((gy,), ctx.saved_tensors[0].shape[-1])[0]
         if ctx.hip:
             q, k, v, y, z, lse_lat, lse_tok = ctx.saved_tensors
             gq, gk, gv = _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, ctx.scale, ctx.key_mask, gy)
@@ -479,6 +513,9 @@ class _MixerFn(torch.autograd.Function):
             q, k, v, *stats = ctx.saved_tensors
             gq, gk, gv = _mixer_torch_grad(q, k, v, ctx.scale, ctx.key_mask, gy,
                                            stats=(stats[1], stats[0], stats[2]) if stats else None)
+        if ctx.pad:
+            gk, gv = (_pad_rows((gk, gv), ctx.kv_width, ctx.kv_major[0]) if ctx.kv_major[0] == ctx.kv_major[1] else
+                      [_pad_rows((t,), ctx.kv_width, m)[0] for t, m in zip((gk, gv), ctx.kv_major)])
         return gq[..., :ctx.q_width].to(ctx.q_dtype), gk, gv, None, None, None, None, None, None
 
 
@@ -596,22 +633,27 @@ def flare_multihead_mixer(q, k, v, scale: float = 1.0, key_mask=None, return_z: 
             and _dead_latent_bias(float(scale), k.dtype) is not None):
         return _mixer_odd_latents(q, k, v, float(scale), key_mask, return_z, n_splits, token_major_out)
     pad = _narrow_head_pad(q, k, force_generic) if q.dtype == k.dtype == v.dtype else 0
-    if pad:
-        q, k, v = _pad_last(q, pad), _pad_last(k, pad), _pad_last(v, pad)
     needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))
+    if pad and not (k.dim() == v.dim() == 4 and k.shape == v.shape and q.device == k.device == v.device):
+        q, k, v, pad = _pad_last(q, pad), _pad_last(k, pad), _pad_last(v, pad), 0      # refused below
     if needs_grad and return_z:
         # z is handed out and may enter a loss of its own: take the two differentiable halves, so that gradients
         # reach q, k, v through z as well as through y (the fused function below treats z as an internal value)
+        if pad:
+            q, k, v = _pad_last(q, pad), _pad_last(k, pad), _pad_last(v, pad)
         z, _ = flare_gather(q, k, v, scale, key_mask, n_splits, force_generic)
         y = flare_scatter(q, k, z, scale, key_mask, force_generic)
         if token_major_out:
             y = y.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
     elif needs_grad:
-        # the cast of the latents for autocast stays inside the function
+        # the cast of the latents for autocast, and zero columns for narrow heads, stay inside the function
         cast = q is q_cast and q is not q_in and q_in.dtype == torch.float32
-        y, z = _MixerFn.apply(q_in if cast else q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out,
-                              q.detach() if cast else None)
+        q16 = _pad_last(q.detach(), pad) if pad else q.detach() if cast else None
+        y, z = _MixerFn.apply(q_in if cast else q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out, q16)
+        return (y, z) if return_z else y
     else:
+        if pad:
+            q, (k, v) = _pad_last(q, pad), _pad_rows((k, v), D + pad)
         y, z = _mixer_forward(q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out)
     if pad:
         y, z = y[..., :D], z[..., :D]

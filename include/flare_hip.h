@@ -473,6 +473,10 @@ int flare_mlp_narrow_bwd(const FlareNarrowDesc* desc, const void* x, const float
 int flare_rows_parts(int64_t T, int32_t C, int32_t* parts);
 int flare_rows_act_bwd(int64_t T, int32_t C, int32_t act, const float* ds, const float* t, float* dt, float* copy, float* db_part,
                        float* db, void* stream);
+/* dst rows = src rows filled up with zeros (dst_width > src_width) or cut: up to four arrays of n[0] x n[1] x n[2] rows in one launch,
+ * strides in elements, three per array, rows contiguous; elements of 2 or 4 bytes.  Arrays must not overlap. */
+int flare_pad_rows(int32_t jobs, int32_t elem_bytes, const int64_t n[3], int32_t src_width, int32_t dst_width, const void* const* src,
+                   const int64_t* src_strides, void* const* dst, const int64_t* dst_strides, void* stream);
 /* y = [res +] ([x +] act(t)), act -1 or FLARE_ACT_GELU_TANH (the values of torch's tanh-GELU bit for bit); x, res may be NULL, y may be t. */
 int flare_rows_act_fwd(int64_t T, int32_t C, int32_t act, const float* t, const float* x, const float* res, float* y, void* stream);
 /* Backward of one layer y = [x +] act(x W^T + b) in one pass (C in {64, 128}; flare_rows_layer_bwd_parts answers 0 for the others):

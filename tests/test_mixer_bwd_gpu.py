@@ -491,3 +491,50 @@ def test_absent_tokens_in_every_kernel(dev, shape, dtype):
         assert err <= (1e-4 if dtype == torch.float32 else 3e-2), f"{name} rel-L2 {err:.3e}"
     for t in (dk, dv):
         assert bool((t.cpu()[~m4.expand_as(k)] == 0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,D,width", [((1, 1, 1), 8, 16), ((2, 3, 67), 8, 16), ((2, 4, 130), 4, 16), ((1, 2, 33), 5, 16), ((3, 2, 70), 24, 32), ((2, 2, 4097), 16, 8),
+                                           ((1, 3, 40), 16, 5)])
+def test_rows_filled_up_and_cut(dev, dtype, shape, D, width):
+    """_pad_rows against torch, for rows in either memory order, on and off the 16-byte grid, expanded ones among them."""
+    B, H, N = shape
+    base = torch.randn(2, B, H, N, D + 3, device=dev).to(dtype)
+    sets = [[base[i, ..., :D].contiguous() for i in (0, 1)],
+            [base[i, ..., :D].permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for i in (0, 1)],
+            [base[0, ..., 1:D + 1], base[1, ..., :D].contiguous()], [base[0, :1, :, :1, :D].expand(B, H, N, D)], [base[0, ..., :D].flip(-1)]]
+    for ts in sets:
+        for major in (None, True, False):
+            for t, o in zip(ts, FN._pad_rows(ts, width, major)):
+                want = torch.nn.functional.pad(t, (0, width - D))
+                assert o.shape == want.shape and torch.equal(o, want)
+                if major is not None and H > 1 and N > 1:
+                    assert (o.stride(1) < o.stride(2)) == major
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 3e-2), (torch.float32, 1e-4)])
+@pytest.mark.parametrize("D", [4, 8, 24])
+@pytest.mark.parametrize("major,masked", [(False, False), (True, False), (True, True)])
+def test_narrow_heads_with_gradients(dev, dtype, tol, D, major, masked):
+    """Heads the kernels take filled up with zeros: outputs and gradients against the oracle, for k and v in either memory order and under
+    autocast from fp32, whose gradients come back in fp32."""
+    q, k, v, gy = make(2, 4, 301, 64, D, torch.float32, seed=D)
+    mask = torch.rand(2, 301, generator=torch.Generator().manual_seed(1)) < 0.7 if masked else None
+    qd = q.to(dev).requires_grad_(True)
+    leaf = [t.permute(0, 2, 1, 3).contiguous().to(dev).requires_grad_(True) if major else t.to(dev).requires_grad_(True) for t in (k, v)]
+    kd, vd = (t.permute(0, 2, 1, 3) if major else t for t in leaf)
+    with torch.autocast("cuda", dtype=dtype, enabled=dtype != torch.float32):
+        y = F.flare_multihead_mixer(qd, kd, vd, scale=0.9, key_mask=None if mask is None else mask.to(dev), token_major_out=major)
+    assert y.dtype == dtype and (not major or y.permute(0, 2, 1, 3).is_contiguous())
+    got = torch.autograd.grad(y, (qd, *leaf), gy.to(dev).to(dtype))
+    assert all(g.dtype == torch.float32 for g in got)
+    rnd = lambda t: t.to(dtype).double().requires_grad_(True)
+    qr, kr, vr = rnd(q), rnd(k), rnd(v)
+    yr, _ = O.mixer_explicit(qr, kr, vr, 0.9, mask)
+    keep = 1.0 if mask is None else mask[:, None, :, None].double()
+    assert O.rel_l2(y.detach().cpu().double() * keep, yr.detach() * keep) <= tol
+    want = torch.autograd.grad(yr, (qr, kr, vr), gy.to(dtype).double() * keep)
+    for name, a, r in zip(("dq", "dk", "dv"), got, want):
+        a = a.permute(0, 2, 1, 3) if major and name != "dq" else a
+        err = O.rel_l2(a, r)
+        assert err <= tol, f"{name} rel-L2 {err:.3e}"
