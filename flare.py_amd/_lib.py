@@ -144,6 +144,8 @@ SYMBOLS = {
     "flare_mlp_few_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_few_bwd_res": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_few_pair_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P]),
+    "flare_mlp_few_tail_fwd": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(FlareMlpDesc)] + [_P] * 11),
+    "flare_mlp_few_tail_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(FlareMlpDesc)] + [_P] * 17),
     "flare_mlp_narrow_fwd": (C.c_int, [C.POINTER(FlareNarrowDesc), _P, _P, _P, _P, _P, _P]),
     "flare_mlp_narrow_parts": (C.c_int, [C.c_int64, C.POINTER(C.c_int32)]),
     "flare_mlp_narrow_bwd": (C.c_int, [C.POINTER(FlareNarrowDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -1,11 +1,12 @@
 """A FLAREBlock's inference forward as one call into the library.
 
 Under autocast and without gradients the block is seven launches (norm + k projection, norm + v projection, three of the mixer,
-output projection + residual, norm + feed-forward + residual; pdebench/models/flare.py:107-215), and on small point clouds enqueueing
-them from Python is what it costs: five calls of 20 to 30 us each, most of it spent deciding again what the last call decided.
-An 8-block model of 64 channels on 3973 points: 1070 us a forward, 380 us
-through the plans (0.31 ms of kernels).  `forward` keeps what depends on the module and the shape only -- descriptors, the packed 16-bit weights the modules hold
-anyway, the layout of one scratch allocation -- and hands the rest to flare_block_fwd.  Nothing about an input is kept.
+output projection + residual, norm + feed-forward + residual; pdebench/models/flare.py:107-215), five on few tokens, where the two
+projections and the block's end are one launch each.  On small point clouds enqueueing them from Python is what it costs: calls of
+20 to 30 us each, most of it spent deciding again what the last call decided.  An 8-block model of 64 channels on 3973 points:
+1070 us a forward, 340 us through the plans (0.3 ms of kernels).  `forward` keeps what depends on the module and the shape only --
+descriptors, the packed 16-bit weights the modules hold anyway, the layout of one scratch allocation -- and hands the rest to
+flare_block_fwd.  Nothing about an input is kept.
 
 A plan is made when a block meets a shape for the second time.  Every call compares what it was made from: the modules' structure,
 every parameter's address and version, the norms' eps, the mixer's scale.  Where any of it changed, a new plan is made, and calls a

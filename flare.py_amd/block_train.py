@@ -1,10 +1,11 @@
 """A FLAREBlock's training step on few tokens as one autograd node.
 
 On small meshes a step is the sum of its launches' latencies.  The block's four token-wise launches and the mixer
-(pdebench/models/flare.py:107-215) run as in modules.py; what one node for all of them saves is in the backward: the rows that the
-launches leave for the weight gradients lie side by side, so that one product launch and one launch of sums serve every
-layer and both norms of the block, instead of one each per stack.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels
-1518 -> 1342 us, 64 channels 1171 -> 1024 us.
+(pdebench/models/flare.py:107-215) run as in modules.py; what one node for all of them saves is launches: the rows that the
+backward leaves for the weight gradients lie side by side, so that one product launch and one launch of sums serve every
+layer and both norms of the block, instead of one each per stack, and the output projection and the feed-forward are one launch each
+way.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels 1518 -> 1342 (weight gradients) -> 1261 us (the block's
+end), 64 channels 1171 -> 1024 -> 966 us.
 
 Used under autocast with gradients enabled, where all stacks are plain chains that the few-token launches take, the parameters can be read
 by the packing launch, and nothing hooks into the attention module; `forward` answers None for every other call.
@@ -76,8 +77,7 @@ class _BlockFn(torch.autograd.Function):
             kh, vh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2))
             y, z, lse_lat, lse_tok = functional._mixer_forward(q16, kh, vh, float(att.attn_scale), None, 0, False, True, True)
             y2 = y.permute(0, 2, 1, 3).reshape(B, N, H * Dp)
-            x1 = fused._fused_mlp_fwd(y2, out, cd, res=x, out_dtype=x.dtype, x_head=head, train=True)
-            o = fused._fused_mlp_fwd(x1, mlp, cd, norm=block.norm2, res=x1, out_dtype=x.dtype, train=True)
+            x1, o = fused.tail_forward(y2, out, x, mlp, cd, block.norm2, head)
         ctx.block, ctx.cd, ctx.layers, ctx.n, ctx.head, ctx.scale = block, cd, layers, n, head, float(att.attn_scale)
         ctx.dims, ctx.norms = (B, N, H, Dp, D), (block.norm1, block.norm2)
         # the backward reads the parameters' packed copies again: as with a saved tensor, changing one in place before is an error
@@ -99,8 +99,7 @@ class _BlockFn(torch.autograd.Function):
         norm1, norm2 = ctx.norms
         a_in, g_out = torch.empty(2, L, T, Cdim, dtype=cd, device=dev)
         m = 2 * n
-        dx1, gb2 = fused._chain_backward(mlp, cd, norm2, x1, do, True, into=(a_in[m + 1:], g_out[m + 1:]))
-        dy, _ = fused._chain_backward(out, cd, None, y2, dx1, False, x_head=head, into=(a_in[m:m + 1], g_out[m:m + 1]))
+        dx1, dy, gb2 = fused.tail_backward(y2, out, x1, mlp, cd, norm2, head, do, a_in[m:], g_out[m:])
         kh, vh, yh, gyh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2, y2, dy))
         dq, dk, dv = functional._mixer_hip_grad(q16, kh, vh, yh, z, lse_lat, lse_tok, ctx.scale, gyh)
         dk, dv = (t.permute(0, 2, 1, 3).reshape(T, H * Dp) for t in (dk, dv))

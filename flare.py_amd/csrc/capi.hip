@@ -1037,7 +1037,7 @@ int flare_causal_linear_bwd(const FlareCausalLinearDesc* desc, const void* q, co
 
 static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const float* w_in, const float* b_in, int out_dim,
                         const void* x, const void* w, const float* bias, const float* gamma, const float* beta,
-                        const void* res, void* y, void* y2, void* stream)
+                        const void* res, void* y, void* y2, void* stream, flare::MlpArgs* args_only = nullptr)
 {
     if (!d) return fail(FLARE_EINVAL, "descriptor is NULL");
     if (d->T < 1 || d->L < 1 || d->L > 16) return fail(FLARE_EINVAL, "T >= 1 and 1 <= L <= 16 required (got %lld, %d)", (long long)d->T, d->L);
@@ -1091,6 +1091,10 @@ static int mlp_fwd_impl(const FlareMlpDesc* d, int in_dim, int in_act, const flo
     a.xs = d->x_stride; a.rs = d->res_stride; a.ys = d->y_stride;
     if (d->flags & FLARE_MLP_W_TILED) {
         if (in_dim || out_dim || !flare_mlp_few(d)) return fail(FLARE_EUNSUPPORTED, "tiled weights: only where flare_mlp_few says so");
+        if (args_only) {
+            *args_only = a;
+            return FLARE_OK;
+        }
         return hip_status(flare::launch_mlp_few(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token launch");
     }
     return hip_status(flare::launch_mlp_mfma(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp launch");
@@ -1102,6 +1106,30 @@ int flare_mlp_few_pair_fwd(const FlareMlpDesc* d, const void* x, const void* w, 
     if (!d || !(d->flags & FLARE_MLP_W_TILED)) return fail(FLARE_EINVAL, "a pair of chains takes tiled weights");
     if (!y_b || !aligned16(y_b)) return fail(FLARE_EINVAL, "y_b must be 16-byte aligned and not NULL");
     return mlp_fwd_impl(d, 0, 0, nullptr, nullptr, 0, x, w, bias, gamma, beta, nullptr, y_a, y_b, stream);
+}
+
+// a Linear with a residual (first) whose result the chain (second) takes as its rows and as its own residual
+static bool tail_ok(const FlareMlpDesc& f, const FlareMlpDesc& s)
+{
+    return (f.flags & FLARE_MLP_W_TILED) && s.flags == FLARE_MLP_W_TILED && f.L == 1 && f.act_mask == 0 && f.add_mask == 0 &&
+           f.norm == FLARE_NORM_NONE && !((f.flags >> 12) & 15) && f.T == s.T && f.C == s.C && f.w_dtype == s.w_dtype && f.x_dtype == f.w_dtype &&
+           f.y_dtype == s.x_dtype && f.y_stride == s.x_stride && s.res_dtype == s.x_dtype && s.res_stride == s.x_stride;
+}
+
+int flare_mlp_few_tail_fwd(const FlareMlpDesc* first, const FlareMlpDesc* second, const void* x, const void* res, const void* w1,
+                           const float* bias1, const void* w2, const float* bias2, const float* gamma, const float* beta, void* x1,
+                           void* y, void* stream)
+{
+    if (!first || !second || !tail_ok(*first, *second)) return fail(FLARE_EUNSUPPORTED, "a Linear and a residual in front of a chain: few tokens, rows that fit");
+    if (!res) return fail(FLARE_EINVAL, "res must not be NULL");
+    flare::MlpArgs f, s;
+    void* mid = x1 ? x1 : y;                   // without x1 the rows between the two are not stored: any address will do
+    int rc = mlp_fwd_impl(first, 0, 0, nullptr, nullptr, 0, x, w1, bias1, nullptr, nullptr, res, mid, nullptr, stream, &f);
+    if (rc == FLARE_OK) rc = mlp_fwd_impl(second, 0, 0, nullptr, nullptr, 0, mid, w2, bias2, gamma, beta, mid, y, nullptr, stream, &s);
+    if (rc != FLARE_OK) return rc;
+    s.x = nullptr; s.res = res; s.res_dtype = first->res_dtype; s.rs = first->res_stride;
+    s.pre_x = x; s.pre_y = x1; s.pre_w = f.w; s.pre_bias = bias1; s.pre_xs = f.xs; s.pre_head = f.x_head;
+    return hip_status(flare::launch_mlp_few(s, second->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token launch");
 }
 
 int flare_mlp_few(const FlareMlpDesc* d)
@@ -1185,6 +1213,8 @@ int flare_block_fwd(const FlareBlockDesc* d, const void* x, void* y, void* scrat
         rc = mlp(1, x, nullptr, v);
     if (rc != FLARE_OK) return rc;
     if ((rc = flare_mixer_fwd(&d->mixer, d->q, k, v, nullptr, ym, nullptr, base + s.ws, s.ws_bytes, stream)) != FLARE_OK) return rc;
+    if (tail_ok(d->mlp[2], d->mlp[3]))
+        return flare_mlp_few_tail_fwd(&d->mlp[2], &d->mlp[3], ym, x, d->w[2], d->b[2], d->w[3], d->b[3], d->gamma[3], d->beta[3], nullptr, y, stream);
     if ((rc = mlp(2, ym, x, x1)) != FLARE_OK) return rc;
     return mlp(3, x1, x1, y);
 }
@@ -1225,7 +1255,7 @@ static int check_mlp_bwd_common(const FlareMlpDesc* d, const void* x, const void
 static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,
                         const float* bias, const float* gamma, const float* beta, int32_t add_dy, void* dx, void* a_in,
                         void* g_out, void* dn, float* stats, float* gb_part, float* gb, void* stream, bool few, const void* dy2,
-                        const void* dres)
+                        const void* dres, const flare::MlpBwdArgs* pre = nullptr)
 {
     int rc = check_mlp_bwd_common(d, x, dy, w_img, wt_img, bias, gamma, beta, dx, dn, stats, gb_part, gb);
     if (rc != FLARE_OK) return rc;
@@ -1254,6 +1284,10 @@ static int mlp_bwd_impl(const FlareMlpDesc* d, const void* x, const void* dy, co
     a.add_dy = add_dy;
     a.xs = d->x_stride; a.dys = d->y_stride; a.dxs = x_width;
     a.x_head = x_head; a.y_head = y_head;
+    if (pre) {
+        a.pre_x = pre->pre_x; a.pre_dx = pre->pre_dx; a.pre_wt = pre->pre_wt; a.pre_a = pre->pre_a; a.pre_g = pre->pre_g;
+        a.pre_xs = pre->pre_xs; a.pre_head = pre->pre_head;
+    }
     if (few) return hip_status(flare::launch_mlp_few_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp few-token backward launch");
     return hip_status(flare::launch_mlp_bwd(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp backward launch");
 }
@@ -1281,6 +1315,27 @@ int flare_mlp_few_bwd_res(const FlareMlpDesc* d, const void* x, const void* dy_a
     if (dy_b && !aligned16(dy_b)) return fail(FLARE_EINVAL, "dy_b must be 16-byte aligned");
     // the shared checks ask for dn and stats, which this launch does without
     return mlp_bwd_impl(d, x, dy_a, w_img, wt_img, bias, gamma, beta, add_dy, dx, a_in, g_out, gb_part, gb_part, gb_part, nullptr, stream, true, dy_b, dres);
+}
+
+int flare_mlp_few_tail_bwd(const FlareMlpDesc* first, const FlareMlpDesc* second, const void* x1, const void* dy, const void* w2,
+                           const void* wt2, const float* bias2, const float* gamma, const float* beta, void* dx1, void* a_in2, void* g_out2,
+                           float* gb_part, const void* x, const void* wt1, void* dx, void* a_in1, void* g_out1, void* stream)
+{
+    if (!first || !second || first->L != 1 || first->act_mask || first->add_mask || first->norm != FLARE_NORM_NONE || first->T != second->T ||
+        first->C != second->C || first->w_dtype != second->w_dtype || first->x_dtype != first->w_dtype || (first->flags & ~0xf00) || second->flags)
+        return fail(FLARE_EUNSUPPORTED, "a Linear and a residual in front of a chain: few tokens, rows that fit");
+    if (!flare_mlp_few(second)) return fail(FLARE_EUNSUPPORTED, "the few-token launch runs only where flare_mlp_few says so");
+    const int head = 4 * ((first->flags >> 8) & 15);
+    if (head > 8) return fail(FLARE_EINVAL, "head-padded rows need a head dim of 4 or 8");
+    if (first->x_stride < (head ? 16 * (first->C / head) : first->C) || first->x_stride % 4) return fail(FLARE_EINVAL, "x: row stride >= the row width, a multiple of 4");
+    for (const void* p : {x, wt1, static_cast<const void*>(dx), static_cast<const void*>(a_in1), static_cast<const void*>(g_out1)})
+        if (!p || !aligned16(p)) return fail(FLARE_EINVAL, "x, wt1, dx, a_in1 and g_out1 must be 16-byte aligned and not NULL");
+    flare::MlpBwdArgs pre;
+    memset(&pre, 0, sizeof(pre));
+    pre.pre_x = x; pre.pre_dx = dx; pre.pre_wt = static_cast<const uint16_t*>(wt1); pre.pre_a = static_cast<uint16_t*>(a_in1);
+    pre.pre_g = static_cast<uint16_t*>(g_out1); pre.pre_xs = first->x_stride; pre.pre_head = head;
+    return mlp_bwd_impl(second, x1, dy, w2, wt2, bias2, gamma, beta, FLARE_MLP_BWD_ADD_DY, dx1, a_in2, g_out2, gb_part, gb_part, gb_part, nullptr,
+                        stream, true, nullptr, nullptr, &pre);
 }
 
 int flare_mlp_expand_bwd(const FlareMlpDesc* d, const void* x, const void* dy, const void* w_img, const void* wt_img,

@@ -294,6 +294,12 @@ struct MlpArgs {
     int out_dim;                                // > 0: only features [0, out_dim <= 4) of the result are stored, y rows are out_dim wide
     int x_head, y_head;                         // > 0: rows of x / y hold heads of x_head / y_head (4 or 8) channels, each padded to 16 columns
     int64_t xs, rs, ys;                         // row strides in elements
+    // few-token launch only, pre_x != null: a Linear in front, x = round(res + pre_x W^T + b) with res the rows of `res`; then x (not read
+    // from memory, stored through pre_y where that is not null) takes the place of both x and res
+    const void* pre_x; void* pre_y;             // pre_x: rows of the weights' type
+    const uint16_t* pre_w; const float* pre_bias;
+    int64_t pre_xs;
+    int pre_head;                               // as x_head, for the rows of pre_x
 };
 
 // backward of the fused MLP chain (mlp_bwd_mfma.hip)
@@ -302,6 +308,12 @@ struct MlpBwdArgs {
     const void* dy2;                            // few-token launch only: gradient of the second chain's output (tiles L .. 2 L - 1), or null
     const void* dres;                           // few-token launch only: [T,C] rows of dx's type that are added to dx, or null
     int x_head, y_head;                         // few-token launch only: as MlpArgs, for the rows of x and dx / of dy
+    // few-token launch of one chain only, pre_x != null: on through the Linear in front (see MlpArgs), whose output's gradient is dx
+    const void* pre_x; void* pre_dx;            // rows of the weights' type, pre_xs elements apart / contiguous
+    const uint16_t* pre_wt;
+    uint16_t* pre_a; uint16_t* pre_g;           // [T,C] out: the rows of pre_x and of dx in the weights' type
+    int64_t pre_xs;
+    int pre_head;
     const uint16_t* w; const uint16_t* wt;      // [L,C,C] 16-bit weights [out][in] and their transposes [in][out]
     const float* bias;                          // [L,C] or null
     const float* gamma; const float* beta;      // [C] norm parameters (beta may be null)

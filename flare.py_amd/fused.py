@@ -758,6 +758,57 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     return y
 
 
+def _tail_descs(y2, out, x, mlp, cd, norm, head):
+    """(Linear, chain) descriptors of a block's end, the norm's vectors."""
+    Cdim, (layers, act_mask, add_mask, act) = out.in_features, _layers_of(mlp)
+    f, s = _lib.FlareMlpDesc(), _lib.FlareMlpDesc()
+    f.T = s.T = y2.shape[0]
+    f.C = s.C = Cdim
+    f.L, s.L = 1, len(layers)
+    f.flags = (head // 4) << 8
+    f.w_dtype = s.w_dtype = f.x_dtype = _DTYPES[cd]
+    f.y_dtype = f.res_dtype = s.x_dtype = s.y_dtype = s.res_dtype = _dtype_code(x)
+    s.act, s.act_mask, s.add_mask = act, act_mask, add_mask
+    f.x_stride = y2.shape[1]
+    f.y_stride = f.res_stride = s.x_stride = s.y_stride = s.res_stride = Cdim
+    return (f, s, *_norm_args(s, norm, x, Cdim))
+
+
+def tail_forward(y2, out, x, mlp, cd, norm, head):
+    """x1 = x + out(y2), x1 + mlp(norm(x1)) in one launch (few tokens; contiguous rows, y2 in the compute type with heads of `head`
+    channels padded): (x1, result)."""
+    y2 = y2.reshape(-1, y2.shape[-1])
+    f, s, gamma, beta = _tail_descs(y2, out, x, mlp, cd, norm, head)
+    f.flags, s.flags = f.flags | _lib.MLP_W_TILED, _lib.MLP_W_TILED
+    w1, b1 = _packed_few(out, [out], cd, True)[:2]
+    w2, b2 = _packed_few(mlp, _layers_of(mlp)[0], cd, True)[:2]
+    x1, y = torch.empty_like(x), torch.empty_like(x)
+    with _on_device(x.device):
+        rc = _lib.load().flare_mlp_few_tail_fwd(C.byref(f), C.byref(s), _ptr(y2), _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(gamma),
+                                                _ptr(beta), _ptr(x1), _ptr(y), C.c_void_p(_stream_ptr(x.device)))
+    _lib.check(rc, "flare_mlp_few_tail_fwd")
+    return x1, y
+
+
+def tail_backward(y2, out, x1, mlp, cd, norm, head, dy, a_in, g_out):
+    """Backward of tail_forward in one launch: (dx1 [T,C], dy2, the norm's partial rows); a_in, g_out take the rows for the weight
+    gradients of out and of mlp's layers, in that order."""
+    Cdim = out.in_features
+    x2, y2, dy = x1.reshape(-1, Cdim), y2.reshape(-1, y2.shape[-1]), _rows2d(dy, Cdim)
+    f, s, gamma, beta = _tail_descs(y2, out, x1, mlp, cd, norm, head)
+    s.y_dtype, s.y_stride = _dtype_code(dy), dy.stride(0)
+    wt1 = _packed_few(out, [out], cd, True)[2]
+    w2, b2, wt2 = _packed_few(mlp, _layers_of(mlp)[0], cd, True)
+    dx1, dy2 = torch.empty_like(x2), torch.empty_like(y2)
+    gb = torch.empty(_few(x2.shape[0], Cdim, s.L), 2, Cdim, dtype=torch.float32, device=x1.device)
+    with _on_device(x1.device):
+        rc = _lib.load().flare_mlp_few_tail_bwd(C.byref(f), C.byref(s), _ptr(x2), _ptr(dy), _ptr(w2), _ptr(wt2), _ptr(b2), _ptr(gamma), _ptr(beta),
+                                                _ptr(dx1), _ptr(a_in[1:]), _ptr(g_out[1:]), _ptr(gb), _ptr(y2), _ptr(wt1), _ptr(dy2),
+                                                _ptr(a_in), _ptr(g_out), C.c_void_p(_stream_ptr(x1.device)))
+    _lib.check(rc, "flare_mlp_few_tail_bwd")
+    return dx1, dy2, gb
+
+
 # --------------------------------------------------------------------------------------
 # training: forward launch + flare_mlp_bwd
 # --------------------------------------------------------------------------------------
@@ -920,12 +971,11 @@ def _norm_grads(norm, gsum, need_gamma, need_beta):
             gsum[1].to(norm.bias.dtype) if (need_beta and getattr(norm, "bias", None) is not None) else None]
 
 
-def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, into=None):
+def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     """Backward of y = [x +] chain(norm(x)) for the chain of C x C layers: (dx [T,C], the norm's [2,C] sums or None,
     dW [L,out,in], db [L,C] or None, the layers).  dx_acc: a [T,C] gradient of the same x that another chain left
     (x's dtype, contiguous); the kernel adds its result into it and it is returned as dx.  x_head: rows of x and dx hold padded
-    heads (few tokens only).  into: (a_in, g_out) [L,T,C] that take the rows for the weight gradients, which the caller forms (few
-    tokens only): then (dx, the norm's partial rows or None)."""
+    heads (few tokens only)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _layers_of(mod)
     L = len(layers)
@@ -935,7 +985,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, into=
     packed = _packed_few(mod, layers, cd, True) if few else None
     if packed is not None:
         w_img, b, wt_img = packed            # the tiled operands
-    elif x_head or into is not None:
+    elif x_head:
         raise RuntimeError("head-padded rows have a backward in the few-token launches only")
     else:
         few = 0
@@ -956,7 +1006,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, into=
     if dx_acc is not None and (dx_acc.shape != (T, Cdim) or dx_acc.dtype != x2.dtype or not dx_acc.is_contiguous()):
         raise ValueError("dx_acc must be a contiguous [T, C] tensor of x's dtype")
     dx = dx_acc if dx_acc is not None else torch.empty(T, xw, dtype=x2.dtype, device=dev)
-    a_in, g_out = (torch.empty(L, T, Cdim, dtype=cd, device=dev) for _ in range(2)) if into is None else into
+    a_in, g_out = (torch.empty(L, T, Cdim, dtype=cd, device=dev) for _ in range(2))
     dn = stats = gb = gsum = None
     any_bias = any(l.bias is not None for l in layers)
     if few and d.norm:
@@ -979,8 +1029,6 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, into=
                                    bits, _ptr(dx), _ptr(a_in), _ptr(g_out), _ptr(dn), _ptr(stats), _ptr(gb),
                                    None, C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_bwd")
-    if into is not None:
-        return dx, gb
     # weight and bias gradients: one more launch over the rows the kernel left (16-bit products with fp32
     # accumulation, as torch runs a Linear's backward under autocast); norm gradients: partial rows, summed with the others
     dW, db = _weight_grads(d, g_out, a_in, any_bias, gb=gb, gsum=gsum)                 # [L, out, in], [L, C] fp32
@@ -1027,7 +1075,7 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None, int
         rc = lib.flare_mlp_few_bwd_res(C.byref(d), _ptr(x2), _ptr(da), _ptr(db_), _ptr(r2), _ptr(w), _ptr(wt), _ptr(b), _ptr(gamma),
                                        _ptr(beta), 0, _ptr(dx), _ptr(rows[0]), _ptr(rows[1]), _ptr(gb), C.c_void_p(_stream_ptr(dev)))
     _lib.check(rc, "flare_mlp_few_bwd_res")
-    if into is not None:                       # as _chain_backward's
+    if into is not None:                       # (dx, the norm's partial rows or None): the caller forms the weight gradients
         return dx, gb
     dW, db = _weight_grads(d, rows[1], rows[0], any(l.bias is not None for l in layers), gb=gb, gsum=gsum)
     return dx, gsum, dW, db, layers

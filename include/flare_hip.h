@@ -429,6 +429,19 @@ int flare_mlp_few_bwd_res(const FlareMlpDesc* desc, const void* x, const void* d
  * of them (FLARE_MLP_W_TILED set), w [2L,C,C] and bias [2L,C] the first chain's tiles followed by the second's. */
 int flare_mlp_few_pair_fwd(const FlareMlpDesc* desc, const void* x, const void* w, const float* bias, const float* gamma,
                            const float* beta, void* y_a, void* y_b, void* stream);
+/* The end of a block in one launch each way (pdebench/models/flare.py:204-215): x1 = res + Linear(x), y = x1 + chain(norm(x1)), the bits
+ * of two launches.  first: the Linear (L = 1, no norm, no masks; x rows of the weights' type, FLARE_MLP_X_HEAD allowed; res_dtype,
+ * res_stride, y_dtype and y_stride are those of res and x1); second: the chain, its x and res rows being x1's; both with
+ * FLARE_MLP_W_TILED.  x1: NULL where its rows are not wanted.
+ * Backward (flags as in flare_mlp_few_bwd): dy is the gradient of y, dx1 [T,C] of x1 (and so of res), dx of x, contiguous rows of the
+ * weights' type as wide as x's; a_in1, g_out1 [T,C] and a_in2, g_out2 [L,T,C] as flare_mlp_bwd leaves them. */
+int flare_mlp_few_tail_fwd(const FlareMlpDesc* first, const FlareMlpDesc* second, const void* x, const void* res, const void* w1,
+                           const float* bias1, const void* w2, const float* bias2, const float* gamma, const float* beta, void* x1,
+                           void* y, void* stream);
+int flare_mlp_few_tail_bwd(const FlareMlpDesc* first, const FlareMlpDesc* second, const void* x1, const void* dy, const void* w2,
+                           const void* wt2, const float* bias2, const float* gamma, const float* beta, void* dx1, void* a_in2,
+                           void* g_out2, float* gb_part, const void* x, const void* wt1, void* dx, void* a_in1, void* g_out1,
+                           void* stream);
 /* Weight and bias gradients from the rows flare_mlp_bwd leaves, in one pass over both (the reference gets them from
  * torch's Linear backward: dW = dt^T s, db = column sums of dt; pdebench/models/flare.py:45-59 under autograd).
  * Only T, C, L and w_dtype of the descriptor are read.  a_in, g_out: L arrays of [T,C] rows in the weights' type,

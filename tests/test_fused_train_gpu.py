@@ -755,3 +755,34 @@ def test_calls_that_keep_a_node_per_stack(dev):
             y = blk(xg)[0]
     got = torch.autograd.grad(y.sum(), [xg, blk.att.k_proj.fc1.weight])
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# one token; a ragged last tile; the ends of the few-token range; chains of 1 to 8 layers; rows of narrow heads
+@pytest.mark.parametrize("C,head,T,layers", [(32, 0, 1, 6), (64, 8, 15, 3), (64, 4, 4097, 3), (128, 0, 17, -1), (128, 8, 12288, 3), (64, 0, 16384, 6)])
+@pytest.mark.parametrize("cd,xd,kind,act", [(torch.bfloat16, torch.float32, "ln", "gelu"), (torch.float16, torch.bfloat16, "rms", "silu"),
+                                            (torch.bfloat16, torch.float16, "ln", "silu"), (torch.float16, torch.float32, None, "gelu")])
+def test_output_projection_and_feed_forward_in_one_launch(dev, monkeypatch, C, head, T, layers, cd, xd, kind, act):
+    """The bits of the two launches, forward and backward, and the rows they leave for the weight gradients."""
+    torch.manual_seed(T)
+    out = nn.Linear(C, C, bias=layers != 6).to(dev)
+    mlp = (nn.Linear(C, C) if layers < 0 else ResidualMLP(C, C, C, num_layers=layers, act=act)).to(dev)
+    norm = {"ln": nn.LayerNorm(C), "rms": nn.RMSNorm(C), None: nn.Identity()}[kind].to(dev)
+    x = torch.randn(T, C, device=dev).to(xd)
+    y = torch.randn(T, C, device=dev).to(cd)
+    if head:
+        y = torch.nn.functional.pad(y.view(T, C // head, head), (0, 16 - head)).reshape(T, -1).contiguous()
+    x1, o = fused.tail_forward(y, out, x, mlp, cd, norm, head)
+    want1 = fused._fused_mlp_fwd(y, out, cd, res=x, out_dtype=xd, x_head=head, train=True)
+    assert torch.equal(x1, want1) and torch.equal(o, fused._fused_mlp_fwd(want1, mlp, cd, norm=norm, res=want1, out_dtype=xd, train=True))
+    do = torch.randn(T, C, device=dev).to(xd)
+    L = len(fused._layers_of(mlp)[0])
+    a, g = torch.zeros(2, L + 1, T, C, dtype=cd, device=dev)
+    dx1, dy, gb = fused.tail_backward(y, out, x1, mlp, cd, norm, head, do, a, g)
+    rows = []
+    monkeypatch.setattr(fused, "_weight_grads", lambda d, g_out, a_in, *r, gb=None, **k: rows.append((a_in, g_out, gb)) or (None, None))
+    want = fused._chain_backward(mlp, cd, norm, x1, do, True)[0]
+    want_dy = fused._chain_backward(out, cd, None, y, want, False, x_head=head)[0]
+    assert torch.equal(dx1, want) and torch.equal(dy, want_dy)
+    for got, w in ((a, (rows[1][0], rows[0][0])), (g, (rows[1][1], rows[0][1]))):
+        assert torch.equal(got, torch.cat(w))
+    assert kind is None or torch.equal(gb, rows[0][2])
