@@ -5,7 +5,7 @@ On small meshes a step is the sum of its launches' latencies.  The block's four 
 backward leaves for the weight gradients lie side by side, so that one product launch and one launch of sums serve every
 layer and both norms of the block, instead of one each per stack, and the output projection and the feed-forward are one launch each
 way.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels 1518 -> 1342 (weight gradients) -> 1261 us (the block's
-end), 64 channels 1171 -> 1024 -> 966 us.
+end; 1238 since two workgroups of the forward share a CU), 64 channels 1171 -> 1024 -> 966 us.
 
 Used under autocast with gradients enabled, where all stacks are plain chains that the few-token launches take, the parameters can be read
 by the packing launch, and nothing hooks into the attention module; `forward` answers None for every other call.

@@ -218,8 +218,11 @@ template <int DT> __device__ __forceinline__ void store_pad(void* base, int64_t 
 // reads then goes from wave to wave through LDS in fp32, in the order row_stats takes it from memory, so the results are the
 // same bits as those of two launches.  What goes away is a launch's latency (start, one trip to memory, end) each way: 8 blocks, bf16, training
 // step at 4096 tokens 1342 -> 1261 us (C = 128) and 1024 -> 966 us (C = 64), inference forward at 3973 tokens, C = 64, 360 -> 340 us.
+// At most 128 registers up to five layers: two workgroups of C = 128 share a CU, which a pair of chains needs from 2049 tokens and a
+// single one from 4097 (with 160 registers they came one after the other: 4 blocks, 9001 tokens, inference 341 -> 282 us; training step at
+// 12,000 tokens 1325 -> 1252 us, of 8 blocks at 4096 tokens 1258 -> 1238 us).
 template <typename T, int C, int LMAX, bool PRE>
-__global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
+__global__ __launch_bounds__(4 * C, LMAX <= 5 ? 4 : 2) void few_mlp_mfma_kernel(MlpArgs a)
 {
     constexpr int FT = C / 16, KS = C / 32;
     using M_ = Mf<T>;
@@ -262,20 +265,22 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
         gm = *reinterpret_cast<const f32x4*>(a.gamma + ch0);
         if (a.beta) bt = *reinterpret_cast<const f32x4*>(a.beta + ch0);
     }
+    // the first layers' weights travel beside the rows, the others take the rows' registers once the norm is done with them
+    constexpr int FIRST = C == 128 ? (LMAX + 1) / 2 : LMAX;
     u32x4 wr[LMAX][KS];
     f32x4 bias[LMAX];
-#pragma unroll
-    for (int l = 0; l < LMAX; ++l) {
+    auto request = [&](int l) {
         const size_t tile = (size_t)chain * L + (l < L ? l : L - 1);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) wr[l][ks] = operand<C>(a.w, tile, w, ks, lane);
         // a missing bias reads the weights instead (any mapped memory will do) and is replaced by zeros where it is used
         bias[l] = *reinterpret_cast<const f32x4*>((has_bias ? a.bias + tile * C : reinterpret_cast<const float*>(a.w)) + ch0);
-    }
-    f32x4 x1 = zero;
+    };
+#pragma unroll
+    for (int l = 0; l < FIRST; ++l) request(l);
     if constexpr (PRE) {
         publish<C>(ex, 1, w, lane, pre.x, pre.y);
-        f32x4 acc = pb;
+        f32x4 x1, acc = pb;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) acc = M_::mma(pw[ks], ex.q[1][ks][lane], acc);
         x1 = acc + own;
@@ -285,8 +290,8 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
             x1 = round4<DT>(x1);
         });
         own = x1;
+        *reinterpret_cast<f32x4*>(&xs[c16][ch0]) = x1;            // also kept there for the residual
         if (a.norm != 0) {
-            *reinterpret_cast<f32x4*>(&xs[c16][ch0]) = x1;
             lds_barrier();
 #pragma unroll
             for (int ft = 0; ft < FT; ++ft) x0[ft] = *reinterpret_cast<const f32x4*>(&xs[c16][16 * ft + 4 * g]);
@@ -298,6 +303,10 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
 #pragma unroll
         for (int r = 0; r < 4; ++r) own[r] = (own[r] - mean) * rstd * gm[r] + bt[r];
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(own[r]));
+#pragma unroll
+    for (int l = FIRST; l < LMAX; ++l) request(l);
     pin(wr);
     pin(bias);
     const ActCoef coef = act_coef(a.act);
@@ -323,15 +332,20 @@ __global__ __launch_bounds__(4 * C) void few_mlp_mfma_kernel(MlpArgs a)
             s[r] = add ? s[r] + u : u;
         }
     }
-    if constexpr (PRE) s += x1;
-    else if (a.res) with_dtype(a.res_dtype, [&](auto dc) { s += load4<decltype(dc)::value>(a.res, tok * a.rs + ch0); });
-    if (live) {
+    // the lane's place again, from its number: kept through the layers it would cost the registers that they need
+    int id = tid;
+    asm volatile("" : "+v"(id));
+    const int g_ = (id & 63) >> 4, c_ = id & 15, f_ = 16 * w + 4 * g_;
+    const int64_t t_ = (int64_t)blockIdx.x * 16 + c_, tok_ = t_ < a.T ? t_ : a.T - 1;
+    if constexpr (PRE) s += *reinterpret_cast<const f32x4*>(&xs[c_][f_]);
+    else if (a.res) with_dtype(a.res_dtype, [&](auto dc) { s += load4<decltype(dc)::value>(a.res, tok_ * a.rs + f_); });
+    if (t_ < a.T) {
         with_dtype(a.y_dtype, [&](auto dc) {
             constexpr int DT = decltype(dc)::value;
-            const int64_t e = tok * a.ys + col_of(a.y_head, w, g);
+            const int64_t e = tok_ * a.ys + col_of(a.y_head, w, g_);
             void* y = chain ? a.y2 : a.y;
             store4<DT>(y, e, s);
-            store_pad<DT>(y, e, a.y_head, g);
+            store_pad<DT>(y, e, a.y_head, g_);
         });
     }
 }
