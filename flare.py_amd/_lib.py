@@ -18,6 +18,7 @@ FLAG_FORCE_GENERIC = 1
 FLAG_MFMA16 = 2
 FLAG_GRAD_LIKE_KV = 8
 FLAG_ABSENT_TOKENS = 16
+FLAG_DQ_PARTS = 32
 MLP_EXPAND = 1
 MLP_W_TILED = 2
 MLP_BWD_ADD_DY = 1           # bits of flare_mlp_bwd's add_dy argument
@@ -140,6 +141,9 @@ SYMBOLS = {
     "flare_mlp_wgrad": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P]),
     "flare_mlp_wgrad_norm": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, C.c_int32, _P, _P]),
     "flare_mlp_wgrad_norms": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P]),
+    "flare_mlp_wgrad_block": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P,
+                                        C.POINTER(FlareMixerDesc), _P, C.c_int32, C.c_int32, _P, _P]),
+    "flare_mixer_bwd_dq_parts": (C.c_int, [C.POINTER(FlareMixerDesc), C.POINTER(_SZ), C.POINTER(C.c_int32)]),
     "flare_mlp_few": (C.c_int, [C.POINTER(FlareMlpDesc)]),
     "flare_mlp_few_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
     "flare_mlp_few_bwd_res": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P]),
@@ -159,6 +163,7 @@ SYMBOLS = {
     "flare_rows_norm_fwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, C.c_float, _P, _P, _P, _P, _P, _P]),
     "flare_rows_norm_bwd": (C.c_int, [C.c_int64, C.c_int32, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_mlp_pack": (C.c_int, [C.POINTER(FlareMlpPackDesc), _P, _P, _P, _P, _P]),
+    "flare_mlp_pack_rows": (C.c_int, [C.POINTER(FlareMlpPackDesc), _P, _P, _P, _P, _P, C.c_int64, C.c_int32, C.c_int32, C.c_int32, _P, _P]),
     "flare_mlp_expand_bwd": (C.c_int, [C.POINTER(FlareMlpDesc), _P, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "flare_triple_workspace_bytes": (C.c_int, [C.POINTER(FlareTripleDesc), C.POINTER(_SZ)]),
     "flare_triple_state_fwd": (C.c_int, [C.POINTER(FlareTripleDesc), _P, _P, _P, _P, _P, _P, _SZ, _P]),

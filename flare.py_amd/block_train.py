@@ -3,9 +3,10 @@
 On small meshes a step is the sum of its launches' latencies.  The block's four token-wise launches and the mixer
 (pdebench/models/flare.py:107-215) run as in modules.py; what one node for all of them saves is launches: the rows that the
 backward leaves for the weight gradients lie side by side, so that one product launch and one launch of sums serve every
-layer and both norms of the block, instead of one each per stack, and the output projection and the feed-forward are one launch each
-way.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels 1518 -> 1342 (weight gradients) -> 1261 us (the block's
-end; 1238 since two workgroups of the forward share a CU), 64 channels 1171 -> 1024 -> 966 us.
+layer, both norms and the latents of the block, instead of one each per stack; the output projection and the feed-forward are one
+launch each way; the latents are cast by the packing launch.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels
+1518 -> 1342 (weight gradients) -> 1261 (the block's end) -> 1238 (two workgroups of the forward on a CU) -> 1208 us (latents), 64
+channels 1171 -> 1024 -> 966 -> 966 -> 894 us.
 
 Used under autocast with gradients enabled, where all stacks are plain chains that the few-token launches take, the parameters can be read
 by the packing launch, and nothing hooks into the attention module; `forward` answers None for every other call.
@@ -62,18 +63,15 @@ class _BlockFn(torch.autograd.Function):
         H, M, D = att.num_heads, att.num_latents, att.head_dim
         head = D if Dp != D else 0
         with torch.no_grad():
-            fused.prepack(x, cd, (k, v), (out,), (mlp,))
+            q = latent_q.view(H, M, D)
+            q16 = torch.empty(H, M, Dp, dtype=cd, device=x.device) if fused._readable(q) and q.is_contiguous() and q.device == x.device else None
+            if not fused.prepack(x, cd, (k, v), (out,), (mlp,), latents=None if q16 is None else (q, q16)) or q16 is None:
+                q16 = torch.nn.functional.pad(q.to(cd), (0, Dp - D)) if head else q.to(cd)
             n = (len(layers) - 1 - len(fused._layers_of(mlp)[0])) // 2
             w, b = fused._packed_few(k, layers[:2 * n], cd, True)[:2]
             pair = []
             k2 = fused._fused_mlp_fwd(x, k, cd, norm=block.norm1, out_dtype=cd, y_head=head, train=True, operands=(w[:n], b[:n]), pair=pair)
             v2 = fused._fused_mlp_fwd(x, v, cd, norm=block.norm1, out_dtype=cd, y_head=head, train=True, operands=(w[n:], b[n:]), pair=pair)
-            q = latent_q.view(H, M, D)
-            if head:
-                q16 = torch.zeros(H, M, Dp, dtype=cd, device=x.device)
-                q16[..., :D].copy_(q)
-            else:
-                q16 = q.to(cd)
             kh, vh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2))
             y, z, lse_lat, lse_tok = functional._mixer_forward(q16, kh, vh, float(att.attn_scale), None, 0, False, True, True)
             y2 = y.permute(0, 2, 1, 3).reshape(B, N, H * Dp)
@@ -101,17 +99,18 @@ class _BlockFn(torch.autograd.Function):
         m = 2 * n
         dx1, dy, gb2 = fused.tail_backward(y2, out, x1, mlp, cd, norm2, head, do, a_in[m:], g_out[m:])
         kh, vh, yh, gyh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2, y2, dy))
-        dq, dk, dv = functional._mixer_hip_grad(q16, kh, vh, yh, z, lse_lat, lse_tok, ctx.scale, gyh)
+        latents, dk, dv = functional._mixer_hip_grad(q16, kh, vh, yh, z, lse_lat, lse_tok, ctx.scale, gyh, dq_parts=True)
+        dq = torch.empty(H, q16.shape[1], D, dtype=torch.float32, device=dev)
         dk, dv = (t.permute(0, 2, 1, 3).reshape(T, H * Dp) for t in (dk, dv))
         dx, gb1 = fused._pair_backward(k, v, cd, norm1, x, dk, dv, head, dx1, into=(a_in[:m], g_out[:m]))
         gs1, gs2 = (None if g is None else torch.empty(2, Cdim, dtype=torch.float32, device=dev) for g in (gb1, gb2))
         d = _lib.FlareMlpDesc()
         d.w_dtype = functional._DTYPES[cd]
-        dW, db = fused._weight_grads(d, g_out, a_in, any(l.bias is not None for l in layers), gb=gb1, gsum=gs1, gb2=gb2, gsum2=gs2)
+        dW, db = fused._weight_grads(d, g_out, a_in, any(l.bias is not None for l in layers), gb=gb1, gsum=gs1, gb2=gb2, gsum2=gs2, latents=latents, dq=dq)
         need = ctx.needs_input_grad            # (block, cd, layers, Dp, x, latent_q, g1, b1, g2, b2, *wb)
         q_like = ctx.params[0]
         grads = [None, None, None, None, dx.view(x.shape) if need[4] else None,
-                 dq[..., :D].reshape(q_like.shape).to(q_like.dtype) if need[5] else None]
+                 dq.reshape(q_like.shape).to(q_like.dtype) if need[5] else None]
         for norm, gs, at in ((norm1, gs1, 6), (norm2, gs2, 8)):
             grads += fused._norm_grads(norm, gs, need[at], need[at + 1])
         grads += [dW[i].to(l.weight.dtype) if need[10 + i] else None for i, l in enumerate(layers)]

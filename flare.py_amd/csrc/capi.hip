@@ -555,6 +555,18 @@ int flare_mixer_bwd_workspace_bytes(const FlareMixerDesc* desc, size_t* bytes)
     return FLARE_OK;
 }
 
+int flare_mixer_bwd_dq_parts(const FlareMixerDesc* desc, size_t* offset, int32_t* splits)
+{
+    if (!offset || !splits) return fail(FLARE_EINVAL, "offset and splits must not be NULL");
+    int rc = check_bwd(desc);
+    if (rc != FLARE_OK) return rc;
+    if (desc->dtype == FLARE_DT_F32) return fail(FLARE_EUNSUPPORTED, "FLARE_FLAG_DQ_PARTS: bf16 and f16 only");
+    const BwdPlan p = plan_bwd(desc);
+    *offset = p.off_part;
+    *splits = p.n_splits;
+    return FLARE_OK;
+}
+
 int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, const void* v, const void* y,
                     const float* z, const float* lse_lat, const float* lse_tok, const void* dy,
                     const int64_t dy_stride[3], float* dq, void* dk, void* dv,
@@ -562,9 +574,10 @@ int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, co
 {
     int rc = check_bwd(desc);
     if (rc != FLARE_OK) return rc;
-    if (!q || !k || !v || !y || !z || !lse_lat || !lse_tok || !dy || !dy_stride || !dq || !dk || !dv)
+    const bool f32 = desc->dtype == FLARE_DT_F32, parts = (desc->flags & FLARE_FLAG_DQ_PARTS) != 0;
+    if (parts && f32) return fail(FLARE_EUNSUPPORTED, "FLARE_FLAG_DQ_PARTS: bf16 and f16 only");
+    if (!q || !k || !v || !y || !z || !lse_lat || !lse_tok || !dy || !dy_stride || !dk || !dv || (!dq && !parts))
         return fail(FLARE_EINVAL, "q, k, v, y, z, lse_lat, lse_tok, dy, dy_stride, dq, dk, dv must not be NULL");
-    const bool f32 = desc->dtype == FLARE_DT_F32;
     if (!(f32 ? strides_mult4(dy_stride) : strides_mult8(dy_stride)) || dy_stride[2] < desc->D)
         return fail(FLARE_EINVAL, "dy strides must be multiples of 16 bytes and its rows >= D");
     const void* ptrs[7] = {q, k, v, y, dy, dk, dv};
@@ -583,7 +596,7 @@ int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, co
     a.delta_lat = reinterpret_cast<float*>(ws + p.off_dl);
     a.rho_min = reinterpret_cast<float*>(ws + p.off_rm);
     a.part = reinterpret_cast<float*>(ws + p.off_part);
-    a.dq = dq; a.dk = dk; a.dv = dv;
+    a.dq = parts ? nullptr : dq; a.dk = dk; a.dv = dv;
     a.B = desc->B; a.H = desc->H; a.N = desc->N; a.M = desc->M; a.D = desc->D;
     a.n_splits = p.n_splits; a.tokens_per_split = p.tokens_per_split;
     a.n_splits0 = p.n_splits0; a.tokens_per_split0 = p.tokens_per_split0;
@@ -1399,6 +1412,15 @@ int flare_mlp_wgrad_norms(const FlareMlpDesc* d, const void* a_in, int64_t a_lay
                           float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part, int32_t gb_rows,
                           float* gb, float* gb2, void* stream)
 {
+    return flare_mlp_wgrad_block(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, gb_part, gb2_part, gb_rows, gb, gb2, nullptr,
+                                 nullptr, 0, 0, nullptr, stream);
+}
+
+int flare_mlp_wgrad_block(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part, int32_t gb_rows,
+                          float* gb, float* gb2, const FlareMixerDesc* m, const float* dq_part, int32_t dq_splits, int32_t dq_cols, float* dq,
+                          void* stream)
+{
     int rc = check_wgrad_desc(d);
     if (rc != FLARE_OK) return rc;
     if (!a_in || !g_out || !dw_part) return fail(FLARE_EINVAL, "a_in, g_out and dw_part must not be NULL");
@@ -1419,6 +1441,14 @@ int flare_mlp_wgrad_norms(const FlareMlpDesc* d, const void* a_in, int64_t a_lay
         return fail(FLARE_EINVAL, "gb2 needs gb2_part with gb_rows >= 1, both 16-byte aligned");
     a.gb_part = gb ? gb_part : nullptr; a.gb_rows = gb_rows; a.gb = gb;
     a.gb2_part = gb2 ? gb2_part : nullptr; a.gb2 = gb2;
+    if (dq) {
+        if (!m || !dq_part || !aligned16(dq_part) || !aligned16(dq)) return fail(FLARE_EINVAL, "dq needs the mixer's descriptor and dq_part, 16-byte aligned");
+        if (m->B < 1 || m->H < 1 || m->M < 1 || dq_splits < 1 || m->D < 4 || m->D % 4 || dq_cols < 4 || dq_cols % 4 || dq_cols > m->D ||
+            (int64_t)m->H * m->M * m->D > INT32_MAX)
+            return fail(FLARE_EINVAL, "dq: B, H, M and dq_splits >= 1, D and dq_cols <= D multiples of 4");
+        a.dq_part = dq_part; a.dq = dq; a.dq_splits = dq_splits; a.dq_cols = dq_cols; a.dq_scale = m->scale;
+        a.B = m->B; a.H = m->H; a.M = m->M; a.D = m->D;
+    }
     a.T = d->T; a.C = d->C; a.L = d->L;
     return hip_status(flare::launch_mlp_wgrad(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp weight-gradient launch");
 }
@@ -1426,6 +1456,12 @@ int flare_mlp_wgrad_norms(const FlareMlpDesc* d, const void* a_in, int64_t a_lay
 static_assert(FLARE_MLP_PACK_MAX == flare::kMlpPackMax, "header and kernel argument block disagree");
 
 int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img, float* bias, void* stream)
+{
+    return flare_mlp_pack_rows(d, w, w_img, wt_img, bias, nullptr, 0, 0, 0, 0, nullptr, stream);
+}
+
+int flare_mlp_pack_rows(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img, float* bias, const void* rows, int64_t n_rows, int32_t cols,
+                        int32_t cols_out, int32_t rows_dtype, void* rows_out, void* stream)
 {
     if (!d) return fail(FLARE_EINVAL, "descriptor is NULL");
     if (d->L < 1 || d->L > FLARE_MLP_PACK_MAX) return fail(FLARE_EINVAL, "1 <= L <= %d required (got %d)", FLARE_MLP_PACK_MAX, d->L);
@@ -1449,6 +1485,13 @@ int flare_mlp_pack(const FlareMlpPackDesc* d, void* w, void* w_img, void* wt_img
     }
     a.w = static_cast<uint16_t*>(w); a.w_img = static_cast<uint16_t*>(w_img); a.wt_img = static_cast<uint16_t*>(wt_img);
     a.bias = bias; a.L = d->L; a.C = d->C; a.tiled = d->tiled ? 1 : 0;
+    if (rows) {
+        if (n_rows < 1 || cols < 1 || cols_out < cols || cols_out % 4) return fail(FLARE_EINVAL, "rows: 1 <= cols <= cols_out, cols_out a multiple of 4");
+        if (rows_dtype < FLARE_DT_F32 || rows_dtype > FLARE_DT_F16) return fail(FLARE_EINVAL, "rows: unknown dtype");
+        if (!rows_out || !aligned16(rows_out)) return fail(FLARE_EINVAL, "rows_out must be 16-byte aligned and not NULL");
+        a.rows_src = rows; a.rows_out = static_cast<uint16_t*>(rows_out);
+        a.n_rows = n_rows; a.cols = cols; a.cols_out = cols_out; a.rows_dtype = rows_dtype;
+    }
     return hip_status(flare::launch_mlp_pack(a, d->w_dtype, static_cast<hipStream_t>(stream)), "mlp pack launch");
 }
 

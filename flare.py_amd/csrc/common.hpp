@@ -347,6 +347,9 @@ struct MlpWgradArgs {
     const float* gb_part; float* gb;            // or null: the norm's partial rows [gb_rows,2,C] of the backward, summed by the same launch
     int gb_rows;
     const float* gb2_part; float* gb2;          // or null: a second norm's, of as many rows
+    const float* dq_part; float* dq;            // or null: the mixer backward's [B,H,dq_splits,M,D] partial results, times dq_scale summed into [H,M,dq_cols]
+    int B, H, M, D, dq_splits, dq_cols;
+    float dq_scale;
     int64_t T;
     int C, L;
     int64_t tokens_per_wg;                      // set by the launcher
@@ -364,6 +367,9 @@ struct MlpPackArgs {
     float* bias;                                // [L,C]
     int L, C;
     int tiled;                                  // 1: w and wt_img in the few-token kernels' operand order (wt_img may be null)
+    const void* rows_src; uint16_t* rows_out;   // rows_src != null: [n_rows,cols] values to [n_rows,cols_out] 16-bit rows, zeros behind a row's end
+    int64_t n_rows;
+    int cols, cols_out, rows_dtype;
 };
 
 // Row passes of fp32 token-wise layers (rows_f32.hip)

@@ -1022,7 +1022,7 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
     }
     e = dq32 ? launch_bwd_dq32(a, st) : lat_launch<T, D, 1, KIND>(a, st);
     if (e != hipSuccess) return e;
-    merge_launch<1>(a, lat * (D / 4), st);
+    if (a.dq) merge_launch<1>(a, lat * (D / 4), st);       // null: the caller adds the partial results up
     return hipGetLastError();
 }
 

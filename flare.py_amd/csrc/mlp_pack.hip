@@ -27,6 +27,19 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPackArgs a)
     typedef V vec4 __attribute__((ext_vector_type(4)));
     const int l = blockIdx.y, what = blockIdx.z;
     const int C = a.C;
+    if (l == a.L) {          // further rows (a block's latents): as a cast of its own every training step it cost 6 us a block
+        if (what != 0) return;
+        const int64_t n = a.n_rows * a.cols_out;
+        for (int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; e < n; e += (int64_t)gridDim.x * 1024) {
+            const int64_t row = e / a.cols_out;
+            const int col = (int)(e % a.cols_out);
+            vec4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = col + j < a.cols ? (V)load_as_float(a.rows_src, row * a.cols + col + j, a.rows_dtype) : (V)0.f;
+            *reinterpret_cast<vec4*>(reinterpret_cast<V*>(a.rows_out) + e) = v;
+        }
+        return;
+    }
     V* out = reinterpret_cast<V*>(what == 0 ? a.w : what == 1 && !a.tiled ? a.w_img : a.wt_img);
     const bool transposed = what == (a.tiled ? 1 : 2);
     const int e = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
@@ -59,7 +72,7 @@ __global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPackArgs a)
 
 hipError_t launch_mlp_pack(const MlpPackArgs& a, int w_dtype, hipStream_t st)
 {
-    const dim3 grid((unsigned)((a.C * a.C / 4 + 255) / 256), (unsigned)a.L, a.tiled ? (a.wt_img ? 2 : 1) : a.w_img ? 3 : 1);
+    const dim3 grid((unsigned)((a.C * a.C / 4 + 255) / 256), (unsigned)(a.L + (a.rows_src ? 1 : 0)), a.tiled ? (a.wt_img ? 2 : 1) : a.w_img ? 3 : 1);
     if (w_dtype == 1) hipLaunchKernelGGL(mlp_pack_kernel<__bf16>, grid, dim3(256), 0, st, a);
     else              hipLaunchKernelGGL(mlp_pack_kernel<_Float16>, grid, dim3(256), 0, st, a);
     return hipGetLastError();

@@ -196,12 +196,22 @@ __global__ __launch_bounds__(64 * WO * WI * WK) void mlp_wgrad_kernel(MlpWgradAr
     }
 }
 
-// Up to four sums over partial results in one launch: out[i] = sum over p of part[p][i].  A workgroup owns 4 X outputs of one
+// Up to five sums over partial results in one launch: out[i] = sum over p of part[p][i].  A workgroup owns 4 X outputs of one
 // job: thread (x, y) adds the partials p = y, y + Y, ... of four outputs with four loads in flight (X Y = 256), the Y meet in
 // LDS.  The order of the additions is fixed.  Wide jobs (the weights) take X = 64, narrow ones (biases, norm parameters, whose
 // partials are many) X = 16.  Every sum was a launch of its own before: three of the nine launches of a chain's backward.
-struct SumJob { const float* part; float* out; int64_t n; int parts, first, x; };     // first: its first workgroup
-struct SumJobs { SumJob j[4]; int n; };
+// The latents' gradient is one of these sums: [B,H,parts,M,D] partial results (inner = M D), so output i belongs to head i / inner, the
+// sum runs over the batch as well, and of a row's cols columns the first cols_out are wanted.  As the mixer's own launch behind every block
+// it cost 6 us (replayed training step of 8 blocks with the latents' cast in the packing launch too, 4096
+// points: C = 128 1244 -> 1208 us, C = 64 with narrow heads 968 -> 894 us).
+struct SumJob {
+    const float* part; float* out; int64_t n;
+    int parts, first, x;                           // first: its first workgroup
+    int batch = 1, heads = 1, inner = 0;           // inner 0: n
+    int cols = 4, cols_out = 4;
+    float scale = 1.f;
+};
+struct SumJobs { SumJob j[5]; int n; };
 __global__ __launch_bounds__(256) void sum_parts_kernel(SumJobs jobs)
 {
     __shared__ f32x4 red[256];
@@ -210,10 +220,12 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(SumJobs jobs)
     const SumJob job = jobs.j[k];
     const int X = job.x, Y = 256 / X;
     const int x = (int)threadIdx.x % X, y = (int)threadIdx.x / X;
-    const int64_t n = job.n, i = ((int64_t)((int)blockIdx.x - job.first) * X + x) * 4;
-    const float* part = job.part;
+    const int64_t i = ((int64_t)((int)blockIdx.x - job.first) * X + x) * 4, n = job.inner ? job.inner : job.n;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    if (i < n) {
+    for (int b = 0; b < job.batch && i < job.n; ++b) {
+        // an ordinary job has one batch element and one head: part[p][i]
+        const int h = job.heads == 1 ? 0 : (int)((uint32_t)i / (uint32_t)job.inner);
+        const float* part = job.part + ((size_t)b * job.heads + h) * job.parts * n - (size_t)h * n;
         int p = y;
         for (; p + 3 * Y < job.parts; p += 4 * Y) {
             const f32x4 v0 = *reinterpret_cast<const f32x4*>(part + (size_t)p * n + i);
@@ -226,9 +238,15 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(SumJobs jobs)
     }
     red[threadIdx.x] = s;
     __syncthreads();
-    if (y == 0 && i < n) {
+    if (y == 0 && i < job.n) {
         for (int q = 1; q < Y; ++q) s += red[q * X + x];
-        *reinterpret_cast<f32x4*>(job.out + i) = s;
+        int64_t o = i;
+        if (job.cols != job.cols_out) {
+            const int row = (int)((uint32_t)i / (uint32_t)job.cols), col = (int)((uint32_t)i % (uint32_t)job.cols);
+            if (col >= job.cols_out) return;
+            o = (int64_t)row * job.cols_out + col;
+        }
+        *reinterpret_cast<f32x4*>(job.out + o) = s * job.scale;
     }
 }
 
@@ -318,6 +336,11 @@ hipError_t launch_mlp_wgrad(const MlpWgradArgs& a0, int w_dtype, hipStream_t st)
         jobs.j[jobs.n++] = SumJob{part, out, n, np, blocks, x};
         blocks += (int)((n / 4 + x - 1) / x);
     };
+    if (a.dq) {
+        add(a.dq_part, a.dq, (int64_t)a.H * a.M * a.D, a.dq_splits, 16);
+        SumJob& j = jobs.j[0];
+        j.batch = a.B; j.heads = a.H; j.inner = a.M * a.D; j.cols = a.D; j.cols_out = a.dq_cols; j.scale = a.dq_scale;
+    }
     add(a.dw_part, a.dw, (int64_t)a.L * a.C * a.C, parts, 64);
     add(a.db_part, a.db, (int64_t)a.L * a.C, parts, 16);
     add(a.gb_part, a.gb, 2 * (int64_t)a.C, a.gb_rows, 16);

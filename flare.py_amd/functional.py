@@ -244,8 +244,9 @@ def _hip_backward_ok(q, k, v, key_mask, force_generic, drop=None) -> bool:
     return _lib.load().flare_mixer_bwd_workspace_bytes(C.byref(d), C.byref(need)) == _lib.FLARE_OK
 
 
-def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None, flags=0):
-    """dq (fp32), dk, dv from the HIP backward kernels (flare_mixer_bwd); drop = (p, seed) of the forward's attention dropout."""
+def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None, flags=0, dq_parts=False):
+    """dq (fp32), dk, dv from the HIP backward kernels (flare_mixer_bwd); drop = (p, seed) of the forward's attention dropout.
+    dq_parts (16-bit types): in dq's place (descriptor, workspace, the partial results' byte offset in it, splits)."""
     lib = _lib.load()
     k, v = _rows_last_contig(k), _rows_last_contig(v)
     B, H, N, D = k.shape
@@ -257,7 +258,9 @@ def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None, flags
         gy = gy.contiguous()
     d = _mixer_desc(q4, k, v, y, scale, 0, False, drop)
     d.flags |= flags
-    dq = torch.empty((B, H, M, D), dtype=torch.float32, device=k.device)
+    dq = None if dq_parts else torch.empty((B, H, M, D), dtype=torch.float32, device=k.device)
+    if dq_parts:
+        d.flags |= _lib.FLAG_DQ_PARTS
     # k and v that are token-major views ([B,N,H,D] storage, as a projection's output is) get their gradients in the
     # same layout: the projection's backward then reads them as [B*N, H*D] rows without a copy
     like_kv = all(t.stride() == (N * H * D, D, H * D, 1) for t in (k, v)) and H > 1
@@ -276,6 +279,10 @@ def _mixer_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, gy, drop=None, flags
                                  _ptr(gy), _s3(gy), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), ws.numel(),
                                  C.c_void_p(_stream_ptr(k.device)))
     _lib.check(rc, "flare_mixer_bwd")
+    if dq_parts:
+        off, splits = C.c_size_t(0), C.c_int32(0)
+        _lib.check(lib.flare_mixer_bwd_dq_parts(C.byref(d), C.byref(off), C.byref(splits)), "flare_mixer_bwd_dq_parts")
+        return (d, ws, off.value, splits.value), dk, dv
     return dq if q.dim() != 3 else dq[0] if B == 1 else dq.sum(0), dk, dv
 
 

@@ -346,10 +346,11 @@ def _readable(*ts):
                              and t.stride(-1) == 1 and (t.dim() == 1 or t.stride(0) >= t.shape[1])) for t in ts)
 
 
-def _pack_launch(Cdim, cd, tiles, dev, images, tiled=False):
+def _pack_launch(Cdim, cd, tiles, dev, images, tiled=False, latents=None):
     """One flare_mlp_pack launch.  tiles: (weight, element offset of the tile, row stride, rows, bias or None, element offset)
     each; returns (w [L,C,C], b [L,C], image of w, image of its transposes), the images None unless asked for.  tiled: w and the
-    last result in the few-token kernels' operand order, no image of w."""
+    last result in the few-token kernels' operand order, no image of w.  latents: (values, 16-bit result [..., columns]) converted and
+    zero-padded on the way."""
     lib = _lib.load()
     L = len(tiles)
     d = _lib.FlareMlpPackDesc()
@@ -364,8 +365,11 @@ def _pack_launch(Cdim, cd, tiles, dev, images, tiled=False):
     with _on_device(dev):
         img = ws[1] if images and not tiled else None
         img_t = ws[-1] if images else None
-        rc = lib.flare_mlp_pack(C.byref(d), _ptr(ws), _ptr(img), _ptr(img_t), _ptr(bias), C.c_void_p(_stream_ptr(dev)))
-    _lib.check(rc, "flare_mlp_pack")
+        src, out = latents or (None, None)
+        n, cols, cols_out, dt = (0, 0, 0, 0) if latents is None else (src.numel() // src.shape[-1], src.shape[-1], out.shape[-1], _DTYPES[src.dtype])
+        rc = lib.flare_mlp_pack_rows(C.byref(d), _ptr(ws), _ptr(img), _ptr(img_t), _ptr(bias), _ptr(src), n, cols, cols_out, dt, _ptr(out),
+                                     C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_pack_rows")
     return ws[0], bias, img, img_t
 
 
@@ -621,10 +625,10 @@ def _pair_packs(x, mod_a, mod_b):
     return info is not None and _chain_tiles(info[0]) is not None
 
 
-def prepack(x, cd, *stacks):
+def prepack(x, cd, *stacks, latents=None):
     """The packed operands of several stacks that the few-token launches of one training step will ask for (a tuple of modules shares
     a packing: a pair), from one packing launch instead of one each.  Does nothing where they are not all plain chains at few
-    tokens, or where fewer than two of them have to be packed again."""
+    tokens, or where fewer than two of them have to be packed again.  latents: see _pack_launch; True if they have been converted."""
     Cdim = x.shape[-1]
     if not 0 < x.numel() // Cdim <= _FEW_TOKENS.get(Cdim, 0):
         return
@@ -651,9 +655,10 @@ def prepack(x, cd, *stacks):
         at += len(t)
     if len(stale) < 2 or at > _lib.MLP_PACK_MAX:
         return
-    w, b, _, wt = _pack_launch(Cdim, cd, tiles, x.device, True, tiled=True)
+    w, b, _, wt = _pack_launch(Cdim, cd, tiles, x.device, True, tiled=True, latents=latents)
     for mod, key, lo, hi in stale:
         mod.__dict__["_flare_packed_few"] = (key, w[lo:hi], b[lo:hi], wt[lo:hi])
+    return True
 
 
 def project_padded(y, out, cd, head, res, out_dtype):
@@ -892,11 +897,12 @@ def _packed_train_expand(mod, E, cd):
     return w, b, w_img, wt_img
 
 
-def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None, gb2=None, gsum2=None):
+def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None, gb2=None, gsum2=None, latents=None, dq=None):
     """dW [L, C(out), C(in)] and db [L, C] (or None) in fp32 from the rows the backward launch left: one pass of
     flare_mlp_wgrad over both row arrays, partial results per token range summed in a fixed order.  g_out, a_in:
     [L,T,C], or [T,C] for an array all L layers share.  gb, gsum: the norm's partial rows [rows,2,C], summed into gsum [2,C] by
-    the launch that sums the others; gb2, gsum2: another norm's."""
+    the launch that sums the others; gb2, gsum2: another norm's; latents, dq: what _mixer_hip_grad left of the latents' gradient,
+    summed into dq [H,M,columns]."""
     lib = _lib.load()
     T, Cdim = g_out.shape[-2:]
     L = (g_out.shape[0] if g_out.dim() == 3 else a_in.shape[0]) if L is None else L
@@ -912,10 +918,13 @@ def _weight_grads(d, g_out, a_in, want_bias, L=None, gb=None, gsum=None, gb2=Non
     db = torch.empty(L, Cdim, dtype=torch.float32, device=dev) if want_bias else None
     with _on_device(dev):
         rows = 0 if gb is None and gb2 is None else (gb2 if gb is None else gb).shape[0]
-        rc = lib.flare_mlp_wgrad_norms(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
+        m, ws, off, splits = (None, None, 0, 0) if latents is None else latents
+        rc = lib.flare_mlp_wgrad_block(C.byref(d), _ptr(a_in), T * Cdim if a_in.dim() == 3 else 0,
                                        _ptr(g_out), T * Cdim if g_out.dim() == 3 else 0, _ptr(dwp), _ptr(dbp), _ptr(dw), _ptr(db),
-                                       _ptr(gb), _ptr(gb2), rows, _ptr(gsum), _ptr(gsum2), C.c_void_p(_stream_ptr(dev)))
-    _lib.check(rc, "flare_mlp_wgrad_norms")
+                                       _ptr(gb), _ptr(gb2), rows, _ptr(gsum), _ptr(gsum2), None if m is None else C.byref(m),
+                                       None if ws is None else C.c_void_p(ws.data_ptr() + off), splits, 0 if dq is None else dq.shape[-1], _ptr(dq),
+                                       C.c_void_p(_stream_ptr(dev)))
+    _lib.check(rc, "flare_mlp_wgrad_block")
     return dw, db
 
 

@@ -68,6 +68,7 @@ extern "C" {
 #define FLARE_FLAG_FORCE_GENERIC 1  /* skip every matrix-core kernel (16-bit and fp32), use the fp32-FMA kernels */
 #define FLARE_FLAG_MFMA16        2  /* keep the 16x16x32 MFMA kernels where the 32x32x16 gather and scatter (bf16, D = 32, no key mask) would run */
 #define FLARE_FLAG_ABSENT_TOKENS 16 /* flare_mixer_bwd, no dropout: a token whose lse_tok is 2e30 takes no part (a key mask's padding): its k, v, dy rows may hold anything, its dk, dv rows become zeros */
+#define FLARE_FLAG_DQ_PARTS      32 /* flare_mixer_bwd, bf16 / f16: dq (may be NULL) is not written, its partial results stay in the workspace (flare_mixer_bwd_dq_parts) */
 #define FLARE_FLAG_GRAD_LIKE_KV  8  /* flare_mixer_bwd: dk has k's strides and dv has v's (default: both [B,H,N,D] contiguous) */
 
 /*
@@ -236,6 +237,9 @@ int flare_scatter_fwd_lse(const FlareMixerDesc* desc, const void* q, const void*
  * A forward that ran with desc->dropout_p > 0 is differentiated by handing the same descriptor (dropout_p and
  * dropout_seed) in here: the kernels regenerate its keep masks. */
 int flare_mixer_bwd_workspace_bytes(const FlareMixerDesc* desc, size_t* bytes);
+/* Where FLARE_FLAG_DQ_PARTS leaves them: fp32 [B,H,splits,M,D], offset bytes into the workspace; dq = scale times their sum over the
+ * splits (flare_mlp_wgrad_block forms it). */
+int flare_mixer_bwd_dq_parts(const FlareMixerDesc* desc, size_t* offset, int32_t* splits);
 int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, const void* v, const void* y,
                     const float* z, const float* lse_lat, const float* lse_tok, const void* dy,
                     const int64_t dy_stride[3], float* dq, void* dk, void* dv,
@@ -461,6 +465,12 @@ int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_l
 int flare_mlp_wgrad_norms(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                           float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part,
                           int32_t gb_rows, float* gb, float* gb2, void* stream);
+/* The same with the gradient of latents that all batch elements share, from the partial results of flare_mixer_bwd (dq NULL: nothing):
+ * dq [H,M,dq_cols] = mixer->scale times the sum of dq_part [B,H,dq_splits,M,D] over the splits and the batch, the first dq_cols columns. */
+int flare_mlp_wgrad_block(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
+                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part,
+                          int32_t gb_rows, float* gb, float* gb2, const FlareMixerDesc* mixer, const float* dq_part, int32_t dq_splits,
+                          int32_t dq_cols, float* dq, void* stream);
 /* The narrow first or last layer of a model in training under autocast (pdebench/models/flare.py:285-310): values are rounded to
  * w_dtype (bf16 or f16) where separate torch layers round them.  w and b are the fp32 parameters (b may be NULL).
  *   out == 0: t = x W^T + b, y = act(t) (act -1: y alone); x [T,K] rows at x_stride in any type, w [C,K], t and y [T,C] in w_dtype
@@ -517,6 +527,10 @@ typedef struct {
     int32_t tiled;
 } FlareMlpPackDesc;
 int flare_mlp_pack(const FlareMlpPackDesc* desc, void* w, void* w_img, void* wt_img, float* bias, void* stream);
+/* The same with n_rows contiguous rows of cols elements (a block's latents) converted to w_dtype by the same launch: rows_out
+ * [n_rows,cols_out], zeros behind column cols. */
+int flare_mlp_pack_rows(const FlareMlpPackDesc* desc, void* w, void* w_img, void* wt_img, float* bias, const void* rows, int64_t n_rows,
+                        int32_t cols, int32_t cols_out, int32_t rows_dtype, void* rows_out, void* stream);
 
 /* Backward of flare_mlp_fwd with FLARE_MLP_EXPAND (y = res + W2 act(W1 norm(x) + b1) + b2, hidden width E C run as E
  * chunks; desc as for the forward: L = 2 E tiles, flags = FLARE_MLP_EXPAND; w_img, wt_img: LDS images of the 2 E tiles

@@ -11,7 +11,7 @@ import torch
 from torch import nn
 
 import flare_py_amd as F
-from flare_py_amd import block_train, fused
+from flare_py_amd import _lib, block_train, functional, fused
 from flare_py_amd.modules import ResidualMLP
 from oracle import flare_oracle as O
 
@@ -786,3 +786,27 @@ def test_output_projection_and_feed_forward_in_one_launch(dev, monkeypatch, C, h
     for got, w in ((a, (rows[1][0], rows[0][0])), (g, (rows[1][1], rows[0][1]))):
         assert torch.equal(got, torch.cat(w))
     assert kind is None or torch.equal(gb, rows[0][2])
+
+
+@pytest.mark.parametrize("B,H,M,N,D,cols", [(1, 2, 32, 1, 16, 16), (3, 4, 64, 333, 16, 8), (2, 8, 128, 1001, 16, 4), (1, 1, 256, 700, 64, 64), (2, 3, 96, 517, 32, 32)])
+@pytest.mark.parametrize("cd", [torch.bfloat16, torch.float16])
+def test_latents_packed_with_the_weights_and_their_gradient_summed_with_theirs(dev, B, H, M, N, D, cols, cd):
+    """The rounded values bit for bit; the gradient to the order of an fp32 sum over the token ranges and the batch (1e-6 of its terms)."""
+    torch.manual_seed(N)
+    lin = nn.Linear(32, 32).to(dev)
+    src, q = torch.randn(H, M, cols, device=dev), torch.full((H, M, D), float("nan"), dtype=cd, device=dev)
+    w, b, _, _ = fused._pack_launch(32, cd, fused._chain_tiles([lin]), dev, True, tiled=True, latents=(src, q))
+    assert torch.equal(q, nn.functional.pad(src.to(cd), (0, D - cols)))
+    assert torch.equal(w, fused._pack_launch(32, cd, fused._chain_tiles([lin]), dev, True, tiled=True)[0]) and torch.equal(b[0], lin.bias)
+    k, v, gy = (torch.randn(B, N, H, D, device=dev).to(cd).permute(0, 2, 1, 3) for _ in range(3))
+    y, z, ll, lt = functional._mixer_forward(q, k, v, 0.5, None, 0, False, True, True)
+    want, dk, dv = functional._mixer_hip_grad(q, k, v, y, z, ll, lt, 0.5, gy)
+    latents, dk2, dv2 = functional._mixer_hip_grad(q, k, v, y, z, ll, lt, 0.5, gy, dq_parts=True)
+    rows = torch.randn(2, 2, 40, 32, device=dev).to(cd)
+    d = _lib.FlareMlpDesc()
+    d.w_dtype = functional._DTYPES[cd]
+    got = torch.full((H, M, cols), float("nan"), device=dev)
+    dw, db = fused._weight_grads(d, rows[0], rows[1], True, latents=latents, dq=got)
+    dw1, db1 = fused._weight_grads(d, rows[0], rows[1], True)
+    assert torch.equal(dk, dk2) and torch.equal(dv, dv2) and torch.equal(dw, dw1) and torch.equal(db, db1)
+    assert float((got - want[..., :cols]).abs().max()) <= 1e-6 * float(want.abs().max()) * max(B, 4)
