@@ -570,3 +570,71 @@ def test_row_pass_validation():
     _refused(bwd(stats=None), "required array is NULL")
     _refused(bwd(part=None), "required array is NULL")
     _refused(bwd(add=odd), "16-byte")
+
+
+def test_block_end_pack_rows_and_partial_gradient_validation():
+    """Argument errors of the few-token launches around a block are found on the host."""
+    lib, fake, odd = _lib.load(), C.c_void_p(1 << 20), C.c_void_p((1 << 20) + 8)
+    f, s = _lib.FlareMlpDesc(), _lib.FlareMlpDesc()
+    for d in (f, s):
+        d.T, d.C, d.L, d.w_dtype, d.x_stride, d.y_stride, d.res_stride = 16, 64, 1, 1, 64, 64, 64
+        d.flags = _lib.MLP_W_TILED
+    s.L, f.x_dtype = 3, 1
+
+    def fwd(f_=f, s_=s, x=fake, res=fake, w1=fake, y=fake, gamma=None):
+        return lib.flare_mlp_few_tail_fwd(f_, s_, x, res, w1, None, fake, None, gamma, None, None, y, None)
+
+    assert fwd(None) == _lib.FLARE_EUNSUPPORTED and fwd(s_=None) == _lib.FLARE_EUNSUPPORTED
+    assert fwd(x=odd) == _lib.FLARE_EINVAL and fwd(res=None) == _lib.FLARE_EINVAL and fwd(w1=None) == _lib.FLARE_EINVAL and fwd(y=odd) == _lib.FLARE_EINVAL
+    for name, bad in (("L", 2), ("act_mask", 1), ("add_mask", 1), ("norm", 1), ("T", 17), ("C", 32), ("w_dtype", 2), ("x_dtype", 0), ("y_stride", 68), ("flags", 0)):
+        old = getattr(f, name)
+        setattr(f, name, bad)
+        assert fwd() == _lib.FLARE_EUNSUPPORTED, name
+        setattr(f, name, old)
+    s.norm = 1
+    assert fwd() == _lib.FLARE_EINVAL and "gamma" in _lib.last_error()
+    s.norm = 0
+    for d in (f, s):
+        d.T = 16385
+    assert fwd() == _lib.FLARE_EUNSUPPORTED
+
+    for d in (f, s):
+        d.T, d.flags = 16, 0
+
+    def bwd(f_=f, s_=s, x1=fake, x=fake, wt1=fake, dx=fake, a=fake, dx1=fake):
+        return lib.flare_mlp_few_tail_bwd(f_, s_, x1, fake, fake, fake, None, None, None, dx1, fake, fake, None, x, wt1, dx, a, fake, None)
+
+    assert bwd(None) == _lib.FLARE_EUNSUPPORTED and bwd(s_=None) == _lib.FLARE_EUNSUPPORTED
+    assert all(bwd(**{n: v}) == _lib.FLARE_EINVAL for n in ("x1", "x", "wt1", "dx", "a", "dx1") for v in (None, odd))
+    f.flags = 3 << 8
+    assert bwd() == _lib.FLARE_EINVAL
+    f.flags = 2 << 8
+    assert bwd() == _lib.FLARE_EINVAL and "row stride" in _lib.last_error()
+    f.flags, s.T = 0, 17
+    assert bwd() == _lib.FLARE_EUNSUPPORTED
+    f.T = s.T = 16385
+    assert bwd() == _lib.FLARE_EUNSUPPORTED
+
+    p = _lib.FlareMlpPackDesc()
+    p.L, p.C, p.w_dtype, p.tiled, p.src[0], p.rows[0], p.ld[0] = 1, 32, 1, 1, 1 << 20, 32, 32
+    for rows in ((fake, 0, 4, 4, 0, fake), (fake, 2, 0, 4, 0, fake), (fake, 2, 8, 4, 0, fake), (fake, 2, 3, 6, 0, fake), (fake, 2, 4, 4, 3, fake),
+                 (fake, 2, 4, 4, 0, None), (fake, 2, 4, 4, 0, odd)):
+        assert lib.flare_mlp_pack_rows(p, fake, None, fake, fake, *rows, None) == _lib.FLARE_EINVAL
+
+    m = _lib.FlareMixerDesc()
+    m.B, m.H, m.N, m.M, m.D, m.dtype, m.scale = 1, 2, 100, 32, 16, 1, 1.0
+    for n in ("q_stride", "k_stride", "v_stride", "y_stride"):
+        setattr(m, n, _lib.I3(3200, 1600, 16))
+    off, splits = C.c_size_t(0), C.c_int32(0)
+    assert lib.flare_mixer_bwd_dq_parts(m, off, splits) == _lib.FLARE_OK and splits.value >= 1 and off.value % 16 == 0
+    assert lib.flare_mixer_bwd_dq_parts(m, None, splits) == _lib.FLARE_EINVAL
+    g = _lib.FlareMlpDesc()
+    g.T, g.C, g.L, g.w_dtype = 100, 32, 1, 1
+
+    def wgrad(m_=m, part=fake, n=1, cols=16, dq=fake):
+        return lib.flare_mlp_wgrad_block(g, fake, 3200, fake, 3200, fake, None, None, None, None, None, 0, None, None, m_, part, n, cols, dq, None)
+
+    assert wgrad(None) == _lib.FLARE_EINVAL and wgrad(part=odd) == _lib.FLARE_EINVAL and wgrad(dq=odd) == _lib.FLARE_EINVAL
+    assert wgrad(n=0) == _lib.FLARE_EINVAL and all(wgrad(cols=c) == _lib.FLARE_EINVAL for c in (0, 6, 20))
+    m.dtype = 0
+    assert lib.flare_mixer_bwd_dq_parts(m, off, splits) == _lib.FLARE_EUNSUPPORTED
