@@ -17,8 +17,8 @@
 // Attention dropout of the forward (MixerBwdArgs::drop_thr != 0): its keep masks are regenerated from the same hash; with
 // K the keep factors (0 or 1 / (1 - p)) the weights the forward used were K A and K B, so dz and dv meet K B and K A,
 // and dS = A (K <dz, v> - Delta) + B (K <dy, z> - delta) with the same Delta and delta (they are sums over kept weights).
-// Every sum has a fixed order: two runs give the same bits.  A key mask needs nothing here: the caller zeroes the
-// padded tokens' rows and raises their log-sum-exp, so that their weights vanish.
+// Every sum has a fixed order: two runs give the same bits.  A padded token is known by its log-sum-exp (see
+// MixerBwdArgs::absent); with dropout the caller zeroes its rows and raises its log-sum-exp, so that its weights vanish.
 #include <algorithm>
 
 #include "common.hpp"

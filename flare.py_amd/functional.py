@@ -432,7 +432,7 @@ def _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, km, gy, drop=None):
         return _mixer_hip_grad(q, k, v, y, z, torch.nan_to_num(lse_lat, nan=1e30, posinf=1e30, neginf=1e30), lse_tok, scale, gy,
                                flags=_lib.FLAG_ABSENT_TOKENS)
     if km is not None:
-        # A padded token takes no part in either softmax.  The kernels need no mask for that: with its k, v
+        # With dropout.  A padded token takes no part in either softmax.  The kernels need no mask for that: with its k, v
         # and dy rows zeroed it adds nothing to dq or dz, with its log-sum-exp set far above any score its
         # scatter weights vanish, and its own dk, dv rows are cleared afterwards.  A batch element without
         # a single real token has lse_lat = -inf; the same treatment turns its gather weights into 0.

@@ -21,8 +21,8 @@ With gradients enabled the chain of C x C layers (the k/v projections, the feed-
 projection of a FLAREBlock at the reference's default ratios) runs through `_FusedMlpFn`: the same forward
 launch, and a backward that recomputes the chain per token tile in one launch (flare_mlp_bwd) and forms the
 parameter gradients from the rows it leaves with one more launch (flare_mlp_wgrad); the expanding two-layer MLP has a
-backward launch of its own (flare_mlp_expand_bwd).  A stack with a narrow first input or last output keeps that one
-layer as a torch layer while gradients are enabled and sends the C x C layers between through the same path.
+backward launch of its own (flare_mlp_expand_bwd).  A stack with a narrow first input or last output runs that one
+layer in a launch of its own while gradients are enabled and sends the C x C layers between through the same path.
 Head-padded rows (narrow heads) have a backward in the few-token launches.
 """
 from __future__ import annotations

@@ -1,8 +1,8 @@
 """Replay of a captured forward + backward for launch-bound training steps.
 
 On short sequences and small meshes a training step of a FLARE block is a few dozen HIP launches whose kernels
-take less time than the host needs to enqueue them (a sequence-benchmark block at B = 32, N = 1024 runs 0.6 ms of
-kernels in a 1.2 ms step).  `GraphedTrainStep` records one step (forward, loss, backward) in a HIP graph per input
+take less time than the host needs to enqueue them (a sequence-benchmark block at B = 32, N = 1024 runs under 0.6 ms
+of kernels in a 0.9 ms step).  `GraphedTrainStep` records one step (forward, loss, backward) in a HIP graph per input
 shape and replays it; there is no tracing compiler behind it and nothing is specialised beyond the shapes.
 
     step = GraphedTrainStep(model, loss_fn, autocast_dtype=torch.bfloat16)
