@@ -6,7 +6,7 @@ backward leaves for the weight gradients lie side by side, so that one product l
 layer, both norms and the latents of the block, instead of one each per stack; the output projection and the feed-forward are one
 launch each way; the latents are cast by the packing launch.  Replayed training step of 8 blocks, 4096 points, bf16: 128 channels
 1518 -> 1342 (weight gradients) -> 1261 (the block's end) -> 1238 (two workgroups of the forward on a CU) -> 1208 us (latents), 64
-channels 1171 -> 1024 -> 966 -> 966 -> 894 us.
+channels 1171 -> 1024 -> 966 -> 966 -> 894 us (1178 and 873 us since the mixer's small launches spread over the chip).
 
 Used under autocast with gradients enabled, where all stacks are plain chains that the few-token launches take, the parameters can be read
 by the packing launch, and nothing hooks into the attention module; `forward` answers None for every other call.

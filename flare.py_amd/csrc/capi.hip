@@ -110,7 +110,10 @@ MixerPlan plan_mixer(const FlareMixerDesc* d, bool want_mfma)
     }
     int64_t tps = ((int64_t)d->N + s - 1) / s;
     tps = ((tps + unit - 1) / unit) * unit;
-    const int min_tokens = p.mfma ? 4 * unit : 8 * unit;  // keep the split overhead small
+    int min_tokens = p.mfma ? 4 * unit : 8 * unit;  // keep the split overhead small
+    // where that leaves half of the CUs without a workgroup: half as many tokens each (8 blocks, 8 heads, 4096 tokens, a replayed
+    // training step 1184 -> 1178 us, 4 blocks on 2 x 1501 tokens 528 -> 521 us; the merge adds 32 partial results instead of 16)
+    if (p.mfma && d->n_splits <= 0 && unit == 64 && (d->N + min_tokens - 1) / min_tokens * (int64_t)d->B * d->H * mblk <= flare::device_cus() / 2) min_tokens = 2 * unit;
     if (tps < min_tokens) tps = min_tokens;
     p.tokens_per_split = (int)tps;
     p.n_splits = (int)(((int64_t)d->N + tps - 1) / tps);

@@ -1009,7 +1009,10 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
         const int64_t per_bh = (device_cus() + (int64_t)a.B * a.H - 1) / ((int64_t)a.B * a.H);
         int64_t tpw = (a.N + per_bh - 1) / per_bh;
         constexpr int pass = kTokWaves<D> * 16 * kTokTiles<D>;
-        tpw = ((tpw + pass - 1) / pass) * pass;
+        // Ranges below one pass: four waves of a workgroup, or eight, on all CUs instead of twelve on some (8 heads, 4096 tokens: 256
+        // workgroups instead of 88; with the scatter's 128 -> 256 a replayed step of 8 blocks 1210 -> 1185 us).
+        const int64_t step = tpw < pass && tpw <= 256 ? 128 : pass;
+        tpw = ((tpw + step - 1) / step) * step;
         for (int c = 0; c < chunks; ++c) {
             MixerBwdArgs ac = a;
             ac.m0 = c * mc;

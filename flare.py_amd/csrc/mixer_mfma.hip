@@ -891,6 +891,10 @@ hipError_t scatter_launch(const MixerArgs& a, hipStream_t st)
     int64_t tpw = (a.N + per_bh - 1) / per_bh;
     tpw = ((tpw + 255) / 256) * 256;
     if (tpw < 256) tpw = 256;       // one 64-token pass per wave: a launch this small is bound by latency, not by the operand set-up
+    // Where that leaves half of the CUs without a workgroup, two waves of each work on twice as many: 8 heads, 4096 tokens were 128
+    // workgroups here, 128 in the gather and 88 of twelve waves in the backward's token pass.  All three spread, replayed training step of 8
+    // blocks: 128 channels 1210 -> 1178 us, 64 channels 896 -> 873; 4 blocks of 64 channels, 2 x 1501 tokens 542 -> 521 us.
+    if (tpw == 256 && (a.N + 255) / 256 * a.H * a.B <= device_cus() / 2) tpw = 128;
     dim3 grid((unsigned)((a.N + tpw - 1) / tpw), a.H, a.B);
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, a, (int)tpw);
     return hipGetLastError();

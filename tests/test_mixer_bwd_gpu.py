@@ -538,3 +538,18 @@ def test_narrow_heads_with_gradients(dev, dtype, tol, D, major, masked):
         a = a.permute(0, 2, 1, 3) if major and name != "dq" else a
         err = O.rel_l2(a, r)
         assert err <= tol, f"{name} rel-L2 {err:.3e}"
+
+
+# token counts on both sides of the lines where a small launch spreads over more workgroups, and off their 128-token ranges
+@pytest.mark.parametrize("shape", [(1, 8, 127, 128, 16), (1, 8, 129, 128, 16), (1, 8, 4096, 64, 16), (1, 8, 4097, 64, 16), (2, 4, 3969, 32, 64),
+                                   (1, 2, 16385, 128, 16), (1, 3, 10881, 96, 32), (1, 1, 33000, 64, 16)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_small_launches_spread_over_the_chip(dev, shape, dtype):
+    """Output and gradients against the oracle, at the bars of the tests above (2e-2 and 3e-2 in 16 bits)."""
+    q, k, v, gy = make(*shape, dtype, seed=5)
+    qd, kd, vd = (t.to(dev).requires_grad_(True) for t in (q, k, v))
+    y = F.flare_multihead_mixer(qd, kd, vd, scale=0.8)
+    y.backward(gy.to(dev))
+    assert O.rel_l2(y.detach(), O.mixer_explicit(q.double(), k.double(), v.double(), 0.8)[0]) <= 2e-2
+    for name, got, ref in zip(("dq", "dk", "dv"), (qd.grad, kd.grad, vd.grad), oracle_grads(q, k, v, gy, 0.8)):
+        assert O.rel_l2(got, ref) <= 3e-2, name
