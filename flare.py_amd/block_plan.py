@@ -8,10 +8,11 @@ projections and the block's end are one launch each.  On small point clouds enqu
 descriptors, the packed 16-bit weights the modules hold anyway, the layout of one scratch allocation -- and hands the rest to
 flare_block_fwd.  Nothing about an input is kept.
 
-A plan is made when a block meets a shape for the second time.  Every call compares what it was made from: the modules' structure,
-every parameter's address and version, the norms' eps, the mixer's scale.  Where any of it changed, a new plan is made, and calls a
-plan does not cover (hooks on the attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer
-pads itself) run the general path of modules.py.
+A plan is made when a block meets a shape for the second time; a shape's first forward runs the general path of modules.py.  Every
+later call compares what the block's plans were made from: the modules' structure, every parameter's address and version, the norms' eps,
+the mixer's scale.  Where any of it changed, all plans of the block go, whatever their shape.  The parameters' memory is held as long as
+plans name its address: another tensor put in a parameter's place then always lies elsewhere.  Calls a plan does not cover (hooks on the
+attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer pads itself) run the general path.
 """
 from __future__ import annotations
 
@@ -22,12 +23,20 @@ from torch import nn
 
 from . import _lib, functional, fused, rows
 
-_MAX_SHAPES = 8           # plans kept per block; a plan holds a descriptor of 0.5 KB and references to the module's packed weights
+_MAX_SHAPES = 8           # plans kept per block; a plan holds a descriptor of 0.5 KB and references to packed weights, which all plans
+                          # of a block share (one packing for few tokens, one for many)
 _X_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
 
 
 class _Plans(dict):
-    """shape -> (key, plan).  A copy of a module, and one read back from a file, begins without plans: they hold addresses."""
+    """shape -> plan, None for a shape met once, False where the general path serves it; all made from the module as `key` describes it.  held: aliases of the parameters whose addresses are in the
+    key.  pair: compute type -> joint packing of the k and v projections.  Never changed to another key: a block whose key differs gets
+    another object, so that a plan under way in one thread cannot join the plans that another thread began.
+    A copy of a module, and one read back from a file, begins without plans: they hold addresses."""
+
+    def __init__(self, key=None, held=()):
+        super().__init__()
+        self.key, self.held, self.pair = key, held, {}
 
     def __deepcopy__(self, memo):
         return _Plans()
@@ -38,6 +47,11 @@ class _Plans(dict):
 
 class _Plan:
     __slots__ = ("desc", "ref", "scratch", "keep")
+
+
+def _parameters(block):
+    m = block._modules
+    return [t for mod in (m["att"], m["mlp"], m["norm1"], m["norm2"]) for t in mod.parameters()]
 
 
 def _key(block):
@@ -68,14 +82,16 @@ def _key(block):
     return key
 
 
-def _mlp(mod, T, cd, x_dtype, y_dtype, x_stride, y_stride, norm=None, res=None, x_head=0, y_head=0):
-    """(descriptor, weights, biases, gamma, beta) of one launch of fused._fused_mlp_fwd, or None."""
+def _mlp(mod, T, cd, x_dtype, y_dtype, x_stride, y_stride, norm=None, res=None, x_head=0, y_head=0, operands=None):
+    """(descriptor, weights, biases, gamma, beta) of one launch of fused._fused_mlp_fwd, or None.  operands: this stack's part of a
+    joint few-token packing."""
     info, io, Cdim, E = fused._forward_plan(mod)
     layers, act_mask, add_mask, act = info
     if io is not None or (E and (x_head or y_head)):
         return None
-    few, w, b = False, None, None
-    if not E and fused._few(T, Cdim, len(layers)):
+    few = operands is not None
+    w, b = operands if few else (None, None)
+    if not few and not E and fused._few(T, Cdim, len(layers)):
         packed = fused._packed_few(mod, layers, cd, False)
         if packed is not None:
             few, (w, b) = True, packed[:2]
@@ -99,7 +115,7 @@ def _mlp(mod, T, cd, x_dtype, y_dtype, x_stride, y_stride, norm=None, res=None, 
     return d, w, b, gamma, beta
 
 
-def _build(block, x, cd):
+def _build(block, x, cd, plans):
     """A plan for inputs of x's shape and type, or None where the general path has to serve them."""
     att, mlp = block.att, block.mlp
     B, N, Cdim = x.shape
@@ -113,19 +129,22 @@ def _build(block, x, cd):
     head = D if D in (4, 8) else 0                        # narrow heads: k, v and the mixer's rows padded to 16 columns
     Dp, T = (16 if head else D), B * N
     width = H * Dp
-    parts = [_mlp(att.k_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head),
-             _mlp(att.v_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head),
+    # few tokens: the projections' weights in one piece, so that one launch serves both
+    info, kv = fused._pair_info(x, att.k_proj, att.v_proj, cd), (None, None)
+    if info is not None:
+        if cd not in plans.pair:
+            tiles = fused._chain_tiles(info[0])
+            plans.pair[cd] = None if tiles is None else fused._pack_launch(Cdim, cd, tiles, x.device, False, tiled=True)
+        packed = plans.pair[cd]
+        if packed is not None:
+            n = len(info[0]) // 2
+            kv = (packed[0][:n], packed[1][:n]), (packed[0][n:], packed[1][n:])
+    parts = [_mlp(att.k_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head, operands=kv[0]),
+             _mlp(att.v_proj, T, cd, x.dtype, cd, Cdim, width, norm=block.norm1, y_head=head, operands=kv[1]),
              _mlp(att.out_proj, T, cd, cd, x.dtype, width, Cdim, res=x.dtype, x_head=head),
              _mlp(mlp, T, cd, x.dtype, x.dtype, Cdim, Cdim, norm=block.norm2, res=x.dtype)]
     if any(p is None for p in parts):
         return None
-    # few tokens: the projections' weights in one piece, so that one launch serves both
-    info = fused._pair_info(x, att.k_proj, att.v_proj, cd)
-    packed = None if info is None else fused._packed_few(att.k_proj, info[0], cd, False)
-    if packed is not None:
-        n = len(info[0]) // 2
-        parts[0] = (parts[0][0], packed[0][:n], packed[1][:n], *parts[0][3:])
-        parts[1] = (parts[1][0], packed[0][n:], packed[1][n:], *parts[1][3:])
     q = att._cached_q(cd, Dp - D)
     plan = _Plan()
     d = plan.desc = _lib.FlareBlockDesc()
@@ -158,20 +177,22 @@ def forward(block, x):
         plans = block.__dict__["_flare_plans"] = _Plans()
     dev = x.device
     shape = (x.shape, x.dtype, cd, dev.index, functional._extra_mixer_flags)
-    entry = plans.get(shape)
-    if entry is None:
+    if shape not in plans:
         if len(plans) >= _MAX_SHAPES:
             plans.clear()
-        plans[shape] = (None, None)
+        plans[shape] = None
         return None
     key = _key(block)
     if key is None:
         return None
-    plan = entry[1]
-    if entry[0] != key:
-        plan = _build(block, x, cd)
-        plans[shape] = (key, plan)
+    if plans.key != key:
+        shapes = dict.fromkeys(plans)
+        plans = block.__dict__["_flare_plans"] = _Plans(key, [t.detach() for t in _parameters(block)])
+        plans.update(shapes)
+    plan = plans.get(shape)
     if plan is None:
+        plan = plans[shape] = _build(block, x, cd, plans) or False
+    if not plan:
         return None
     y = torch.empty_like(x)
     scratch = torch.empty(plan.scratch, dtype=torch.uint8, device=dev)

@@ -285,6 +285,10 @@ class FLAREBlock(nn.Module):
         self.mlp = ResidualMLP(channel_dim, int(channel_dim * ffn_mlp_ratio), channel_dim,
                                num_layers=num_layers_ffn, act=act, input_residual=True, output_residual=True)
 
+    def _apply(self, fn, recurse=True):
+        self.__dict__.pop("_flare_plans", None)          # they hold the memory of parameters that fn may replace
+        return super()._apply(fn, recurse)
+
     def forward(self, x, return_scores: bool = False):
         if not return_scores and type(self.att) is FLARE:
             # the launches below from one call (inference under autocast), or as one autograd node (training on few tokens)

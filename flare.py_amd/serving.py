@@ -56,7 +56,7 @@ class GraphedForward:
                 c = getattr(m, name, None)
                 if c is not None:
                     keep.append(c)
-            keep += [c for _, c in m.__dict__.get("_flare_plans", {}).values()]
+            keep += m.__dict__.get("_flare_plans", {}).values()
         return keep
 
     def _capture(self, x):

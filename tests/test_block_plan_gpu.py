@@ -101,6 +101,41 @@ def test_a_plan_follows_its_module(dev):
     assert len(m._flare_plans) <= block_plan._MAX_SHAPES
 
 
+@pytest.mark.parametrize("how", ["data", "parameter"])
+@pytest.mark.parametrize("what", ["layer", "latents"])
+def test_replaced_weights_reach_the_plans_of_every_shape(dev, how, what):
+    """Weights replaced between calls on two shapes: an earlier one's memory comes back under a later one, at the same version."""
+    m = make(dev)
+    a, b = torch.randn(2, 500, 64, device=dev), torch.randn(1, 700, 64, device=dev)
+    owner, name = (m.mlp.fc1, "weight") if what == "layer" else (m.att, "latent_q")
+    w0 = getattr(owner, name).detach().clone()
+
+    def value(i):
+        return w0 * (1.0 + 0.125 * i)
+
+    def replace(i):
+        if how == "data":
+            getattr(owner, name).data = value(i)
+        else:
+            setattr(owner, name, nn.Parameter(value(i)))
+
+    want = []
+    for i in range(24):
+        n = make(dev)
+        (n.mlp.fc1.weight if what == "layer" else n.att.latent_q).data.copy_(value(i))
+        want.append((general(n, a), general(n, b)))
+    planned(m, a)
+    for i in range(0, 24, 3):
+        replace(i)
+        assert torch.equal(planned(m, b), want[i][1]), i
+        replace(i + 1)
+        assert torch.equal(planned(m, b), want[i + 1][1]), i
+        replace(i + 2)
+        assert torch.equal(planned(m, a), want[i + 2][0]), i
+    m.cpu()
+    assert "_flare_plans" not in m.__dict__
+
+
 def test_calls_that_keep_the_general_path(dev):
     m = make(dev)
     x = torch.randn(2, 300, 64, device=dev)

@@ -312,3 +312,22 @@ def test_row_passes_leave_modules_alone_whose_call_does_more_than_their_class():
         assert not rows._plain(act)
         h.remove()
         assert rows._plain(act)
+
+
+@pytest.mark.parametrize("how", ["data", "parameter"])
+def test_block_plans_hold_the_memory_their_key_names(how):
+    """Replaced weights never get the address of one that plans were made from, so their key always differs."""
+    from torch import nn
+
+    from flare_py_amd import block_plan
+
+    m = FLAREBlock(channel_dim=128, num_heads=8, num_latents=32)
+    plans = block_plan._Plans(block_plan._key(m), [t.detach() for t in block_plan._parameters(m)])
+    for _ in range(12):
+        w = torch.randn(128, 128)
+        if how == "data":
+            m.mlp.fc1.weight.data = w
+        else:
+            m.mlp.fc1.weight = nn.Parameter(w)
+        del w
+        assert block_plan._key(m) != plans.key
