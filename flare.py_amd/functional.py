@@ -449,9 +449,11 @@ def _masked_hip_grad(q, k, v, y, z, lse_lat, lse_tok, scale, km, gy, drop=None):
 
 
 def _pad_rows(ts, width, token_major=None):
-    """[B,H,N,D] tensors as [B,H,N,width], filled up with zeros or cut, in one launch; in memory [B,N,H,width] where the tensor (or
+    """[B,H,N,D] tensors of one shape and type as [B,H,N,width], filled up with zeros or cut, in one launch; in memory [B,N,H,width] where the tensor (or
     token_major) says so, else [B,H,N,width]."""
     B, H, N, D = ts[0].shape
+    if any(t.shape != ts[0].shape or t.dtype != ts[0].dtype or t.device != ts[0].device for t in ts):      # one set of sizes for the launch
+        raise ValueError(f"rows to be filled up must match: {', '.join(f'{tuple(t.shape)} {t.dtype} {t.device}' for t in ts)}")
     ts = [_rows_last_contig(t) for t in ts]
     if any(s < 0 for t in ts for s in t.stride()):
         ts = [t.contiguous() for t in ts]
@@ -474,20 +476,20 @@ def _pad_rows(ts, width, token_major=None):
 
 class _MixerFn(torch.autograd.Function):
     """q16: q as the kernels take it (cast for autocast, its heads filled up with zero columns to those of k and v), where that is
-    another tensor; the gradient then goes to q itself, in q's type and width, without the cast's and the padding's own nodes.  k and v
-    whose heads are narrower than q16's are filled up here, and y comes back at their width."""
+    another tensor; the gradient then goes to q itself, in q's type and width, without the cast's and the padding's own nodes.
+    pad: so many columns of zeros are appended to k and v here (q16 has them), and y comes back at their width."""
 
     @staticmethod
-    def forward(ctx, q, k, v, scale, key_mask, n_splits, force_generic, token_major, q16=None):
+    def forward(ctx, q, k, v, scale, key_mask, n_splits, force_generic, token_major, q16=None, pad=0):
         ctx.scale, ctx.key_mask = scale, key_mask
         ctx.q_dtype, ctx.q_width = q.dtype, q.shape[-1]
         ctx.set_materialize_grads(False)      # z's gradient, which nobody reads, would be a launch
         if q16 is not None:
             q = q16
-        ctx.kv_width, ctx.kv_major = k.shape[-1], tuple(t.stride(1) < t.stride(2) for t in (k, v))
-        ctx.pad = q.shape[-1] > k.shape[-1]
-        if ctx.pad:
-            k, v = _pad_rows((k, v), q.shape[-1])
+        ctx.pad = pad
+        if pad:
+            ctx.kv_width, ctx.kv_major = k.shape[-1], tuple(t.stride(1) < t.stride(2) for t in (k, v))
+            k, v = _pad_rows((k, v), k.shape[-1] + pad)
         ctx.hip = _hip_backward_ok(q, k, v, key_mask, force_generic)
         if ctx.hip:
             y, z, lse_lat, lse_tok = _mixer_forward(q, k, v, scale, key_mask, n_splits, force_generic, token_major, True)
@@ -510,7 +512,7 @@ class _MixerFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, gy, _gz):
         if gy is None:
-            return (None,) * 9
+            return (None,) * 10
         if ctx.pad:
             gy = _pad_rows((gy,), ctx.saved_tensors[0].shape[-1])[0]
         if ctx.hip:
@@ -523,7 +525,7 @@ class _MixerFn(torch.autograd.Function):
         if ctx.pad:
             gk, gv = (_pad_rows((gk, gv), ctx.kv_width, ctx.kv_major[0]) if ctx.kv_major[0] == ctx.kv_major[1] else
                       [_pad_rows((t,), ctx.kv_width, m)[0] for t, m in zip((gk, gv), ctx.kv_major)])
-        return gq[..., :ctx.q_width].to(ctx.q_dtype), gk, gv, None, None, None, None, None, None
+        return gq[..., :ctx.q_width].to(ctx.q_dtype), gk, gv, None, None, None, None, None, None, None
 
 
 def mixer_narrow_heads(q, k, v, scale):
@@ -656,7 +658,7 @@ def flare_multihead_mixer(q, k, v, scale: float = 1.0, key_mask=None, return_z: 
         # the cast of the latents for autocast, and zero columns for narrow heads, stay inside the function
         cast = q is q_cast and q is not q_in and q_in.dtype == torch.float32
         q16 = _pad_last(q.detach(), pad) if pad else q.detach() if cast else None
-        y, z = _MixerFn.apply(q_in if cast else q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out, q16)
+        y, z = _MixerFn.apply(q_in if cast else q, k, v, float(scale), key_mask, n_splits, force_generic, token_major_out, q16, pad)
         return (y, z) if return_z else y
     else:
         if pad:

@@ -553,3 +553,13 @@ def test_small_launches_spread_over_the_chip(dev, shape, dtype):
     assert O.rel_l2(y.detach(), O.mixer_explicit(q.double(), k.double(), v.double(), 0.8)[0]) <= 2e-2
     for name, got, ref in zip(("dq", "dk", "dv"), (qd.grad, kd.grad, vd.grad), oracle_grads(q, k, v, gy, 0.8)):
         assert O.rel_l2(got, ref) <= 3e-2, name
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("q,k,v", [((2, 32, 32), (1, 2, 40, 16), (1, 2, 40, 16)), ((2, 32, 24), (1, 2, 40, 8), (1, 2, 40, 8)), ((2, 32, 4), (1, 2, 40, 8), (1, 2, 40, 8)),
+                                   ((2, 32, 32), (1, 2, 40, 16), (1, 2, 24, 16)), ((2, 32, 8), (1, 2, 40, 8), (1, 2, 24, 8)), ((2, 32, 8), (1, 2, 40, 8), (1, 2, 40, 4))])
+@pytest.mark.parametrize("grad", [False, True])
+def test_operands_that_do_not_match_are_refused(dev, grad, q, k, v, autocast):
+    q, k, v = (torch.randn(s, device=dev, dtype=torch.float32 if autocast else torch.bfloat16, requires_grad=grad) for s in (q, k, v))
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast), pytest.raises(ValueError, match="match"):
+        FN.flare_multihead_mixer(q, k, v)

@@ -331,3 +331,32 @@ def test_block_plans_hold_the_memory_their_key_names(how):
             m.mlp.fc1.weight = nn.Parameter(w)
         del w
         assert block_plan._key(m) != plans.key
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("q,k,v", [((2, 32, 32), (1, 2, 40, 16), (1, 2, 40, 16)), ((2, 32, 8), (1, 2, 40, 16), (1, 2, 40, 16)), ((2, 32, 32), (1, 2, 40, 16), (1, 2, 24, 16)),
+                                   ((2, 32, 32), (1, 2, 40, 16), (1, 2, 40, 8)), ((2, 32, 8), (1, 2, 40, 8), (1, 2, 40, 4)), ((2, 32, 24), (1, 2, 40, 8), (1, 2, 40, 8))])
+def test_mixer_operands_that_do_not_match_are_refused_before_any_launch(monkeypatch, grad, q, k, v):
+    from flare_py_amd import _lib, functional
+
+    class NoLaunch:
+        def __getattr__(self, name):
+            if name.endswith("_bytes"):
+                return lambda *a: 1
+            raise AssertionError(f"{name} called")
+
+    monkeypatch.setattr(functional, "_require_cuda", lambda *a: None)
+    monkeypatch.setattr(_lib, "load", NoLaunch)
+    q, k, v = (torch.randn(s).bfloat16().requires_grad_(grad) for s in (q, k, v))
+    with pytest.raises(ValueError, match="match"):
+        functional.flare_multihead_mixer(q, k, v)
+
+
+def test_rows_to_be_filled_up_must_match(monkeypatch):
+    from flare_py_amd import _lib, functional
+
+    monkeypatch.setattr(_lib, "load", None)
+    k = torch.randn(1, 2, 40, 8)
+    for v in (torch.randn(1, 2, 24, 8), torch.randn(1, 2, 40, 4), torch.randn(1, 2, 40, 8).bfloat16()):
+        with pytest.raises(ValueError, match="match"):
+            functional._pad_rows((k, v), 16)
