@@ -188,6 +188,11 @@ def _narrow_desc(x2, w, cd, out, act, y_dtype):
     return d
 
 
+def _narrow_rows(x2):
+    """Narrow rows as the launches read them: windows over a series, or one point for all tokens, are rows that share memory."""
+    return x2 if x2.stride(-1) == 1 and x2.stride(0) >= x2.shape[1] else x2.clone(memory_format=torch.contiguous_format)
+
+
 def _narrow_backward(d, x2, w, t, dy2, dx, has_bias, dev):
     lib = _lib.load()
     parts = C.c_int32(0)
@@ -207,6 +212,7 @@ class _NarrowInFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, w, b, cd, act):
+        x2 = _narrow_rows(x2)
         d = _narrow_desc(x2, w, cd, False, act, cd)
         y = torch.empty(d.T, d.C, dtype=cd, device=x2.device)
         t = torch.empty_like(y) if act >= 0 else None
@@ -221,7 +227,7 @@ class _NarrowInFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, dy):
         x2, w, t = ctx.saved_tensors                      # through saved-tensor hooks in any memory order
-        x2 = x2 if x2.stride(-1) == 1 and x2.stride(0) >= x2.shape[1] else x2.contiguous()
+        x2 = _narrow_rows(x2)
         d = _narrow_desc(x2, w.contiguous(), ctx.cd, False, ctx.act, ctx.cd)
         dw, db = _narrow_backward(d, x2, w.contiguous(), None if t is None else _wide(t, ctx.cd), _wide(dy, ctx.cd), None, ctx.has_bias, dy.device)
         return None, dw, db, None, None
@@ -577,7 +583,7 @@ def fused_mlp(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=
                 if hn is not None and not isinstance(hn, nn.Identity):
                     h, hn = hn(h), None
                 h2 = h.reshape(-1, h.shape[-1])
-                if not h.requires_grad and h2.stride(-1) == 1 and _narrow_ok(sub.first, h, cd, sub.act_module if sub.first_act else None):
+                if not h.requires_grad and _narrow_ok(sub.first, h, cd, sub.act_module if sub.first_act else None):
                     act = _layers_of(sub)[3] if sub.first_act else -1
                     h = _NarrowInFn.apply(h2, sub.first.weight, sub.first.bias, cd, act).view(*h.shape[:-1], -1)
                 else:

@@ -665,6 +665,26 @@ def test_narrow_layers_against_the_torch_layers(dev, monkeypatch, T, C, K, cd, a
         assert ep <= 1.25 * eq + floor, (i, ep, eq)
 
 
+@pytest.mark.parametrize("B,N", [(1, 1), (1, 700), (2, 300)])
+@pytest.mark.parametrize("how", ["windows", "one point"])
+def test_narrow_input_rows_that_share_memory(dev, how, B, N):
+    """Windows over a series and one point for all tokens as a model's input: rows nearer to each other than they are wide."""
+    torch.manual_seed(3)
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev)
+    if how == "one point":
+        x = torch.randn(B, 1, 3, device=dev).expand(B, N, 3)
+    else:
+        x = torch.randn(B, N + 2, device=dev).unfold(-1, 3, 1)
+
+    def step(x):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(x)
+        return [y.detach(), *torch.autograd.grad(y, list(m.parameters()), torch.ones_like(y))]
+
+    for a, b in zip(step(x), step(x.clone(memory_format=torch.contiguous_format))):
+        assert torch.equal(a, b)
+
+
 def test_narrow_layers_that_keep_the_torch_layers(dev):
     lin, x = nn.Linear(3, 64).to(dev), torch.randn(10, 3, device=dev)
     assert fused._narrow_ok(lin, x, torch.bfloat16)
