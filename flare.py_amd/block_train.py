@@ -79,7 +79,8 @@ class _BlockFn(torch.autograd.Function):
         ctx.block, ctx.cd, ctx.layers, ctx.n, ctx.head, ctx.scale = block, cd, layers, n, head, float(att.attn_scale)
         ctx.dims, ctx.norms = (B, N, H, Dp, D), (block.norm1, block.norm2)
         # the backward reads the parameters' packed copies again: as with a saved tensor, changing one in place before is an error
-        ctx.params = (latent_q, g1, b1, g2, b2, *wb)
+        # (of the latents it reads the saved copy, which stays as it was)
+        ctx.q_like, ctx.params = latent_q, (g1, b1, g2, b2, *wb)
         ctx.versions = tuple(None if t is None else t._version for t in ctx.params)
         ctx.save_for_backward(x, k2, v2, q16, y2, z, lse_lat, lse_tok, x1)
         return o
@@ -108,7 +109,7 @@ class _BlockFn(torch.autograd.Function):
         d.w_dtype = functional._DTYPES[cd]
         dW, db = fused._weight_grads(d, g_out, a_in, any(l.bias is not None for l in layers), gb=gb1, gsum=gs1, gb2=gb2, gsum2=gs2, latents=latents, dq=dq)
         need = ctx.needs_input_grad            # (block, cd, layers, Dp, x, latent_q, g1, b1, g2, b2, *wb)
-        q_like = ctx.params[0]
+        q_like = ctx.q_like
         grads = [None, None, None, None, dx.view(x.shape) if need[4] else None,
                  dq.reshape(q_like.shape).to(q_like.dtype) if need[5] else None]
         for norm, gs, at in ((norm1, gs1, 6), (norm2, gs2, 8)):

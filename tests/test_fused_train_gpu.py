@@ -830,3 +830,26 @@ def test_latents_packed_with_the_weights_and_their_gradient_summed_with_theirs(d
     dw1, db1 = fused._weight_grads(d, rows[0], rows[1], True)
     assert torch.equal(dk, dk2) and torch.equal(dv, dv2) and torch.equal(dw, dw1) and torch.equal(db, db1)
     assert float((got - want[..., :cols]).abs().max()) <= 1e-6 * float(want.abs().max()) * max(B, 4)
+
+
+@pytest.mark.parametrize("again", [False, True])
+@pytest.mark.parametrize("H", [4, 8])
+def test_latents_may_change_between_a_blocks_passes(dev, H, again):
+    """The backward reads the latents' saved 16-bit copy: a change of the parameter in between is none of its business.  again: a second
+    forward on unchanged weights, whose latents are cast by torch."""
+    blk = F.FLAREBlock(channel_dim=64, num_heads=H, num_latents=64).to(dev)
+    x = torch.randn(2, 100, 64, device=dev, requires_grad=True)
+
+    def grads(change):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            if again:
+                blk(x)
+            y = blk(x)[0]
+        assert "BlockFn" in type(y.grad_fn).__name__
+        if change:
+            with torch.no_grad():
+                blk.att.latent_q.mul_(3.0)
+        return torch.autograd.grad(y.sum(), [x, *blk.parameters()])
+
+    for a, b in zip(grads(False), grads(True)):
+        assert torch.equal(a, b)
