@@ -414,8 +414,9 @@ def _param_key(layers):
 
 
 def drop_operands(mod):
-    """Forget the packed weights kept for mod, and for the chain between its narrow ends: that chain's copies live on an object that
-    is no submodule, and a walk over module.modules() alone passes them by."""
+    """Forget the packed weights kept for mod, for the chain between its narrow ends (that chain's copies live on an object that
+    is no submodule, and a walk over module.modules() alone passes them by) and for a block's plans, which hold copies of their own."""
+    mod.__dict__.pop("_flare_plans", None)
     sub = mod.__dict__.get("_flare_subchain")
     for m in (mod, None if sub is None else sub[0]):
         if m is not None:

@@ -191,3 +191,36 @@ def test_refuses_what_a_replay_would_get_wrong(dev):
         F.GraphedTrainStep(_lra_block(dev), _mse)(x.cpu(), None, t.cpu())
     with pytest.raises(ValueError, match="target"):
         F.GraphedTrainStep(_lra_block(dev), _mse)(x)
+
+
+@pytest.mark.parametrize("N", [300, 20000])
+def test_a_block_without_gradients_inside_the_step_sees_parameter_updates(dev, N):
+    """A teacher block that the step runs under no_grad: its weights are packed inside the recorded step like the others'."""
+    class Taught(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.teacher, self.live = (modules.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32) for _ in range(2))
+            self.teacher.requires_grad_(False)
+
+        def forward(self, x):
+            with torch.no_grad():
+                h = self.teacher(x)[0]
+            return self.live(h)[0]
+
+    torch.manual_seed(4)
+    m = Taught().to(dev).train()
+    x, t = torch.randn(1, N, 64, device=dev), torch.randn(1, N, 64, device=dev)
+    params = list(m.live.parameters())
+    step = F.GraphedTrainStep(m, _mse, autocast_dtype=torch.bfloat16)
+    for it in range(4):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss_e = _mse(m(x), t)
+        grads_e = [g.clone() for g in torch.autograd.grad(loss_e, params)]
+        loss_e = loss_e.detach()
+        loss_g = step(x, t).clone()
+        assert torch.equal(loss_g, loss_e), it
+        for p, ge in zip(params, grads_e):
+            assert torch.equal(p.grad, ge), it
+        with torch.no_grad():
+            for p in m.parameters():
+                p.mul_(1.01).add_(0.003)
