@@ -403,20 +403,57 @@ def _few(T, Cdim, L):
 
 
 def _param_key(layers):
-    """What packed copies of these layers' parameters depend on: an in-place change moves a version, another tensor an address.
-    Read from the layers' own tables where the parameters are there (see _structure_key)."""
+    """What packed copies of these layers' parameters depend on: an in-place change moves a version, another tensor an address (see
+    _Key).  Read from the layers' own tables (see _structure_key); a parametrised weight is another tensor at every access, so copies of it
+    serve one call."""
     key = []
     for l in layers:
         p = l._parameters
-        w, b = p["weight"] if "weight" in p else l.weight, p["bias"] if "bias" in p else l.bias
+        if "weight" not in p or "bias" not in p:
+            key.append((object(),))
+            continue
+        w, b = p["weight"], p["bias"]
         key.append((w.data_ptr(), w._version) if b is None else (w.data_ptr(), w._version, b.data_ptr(), b._version))
     return tuple(key)
 
 
+class DropsOperands:
+    """For modules: to(), cpu(), half() and their like drop what is kept of the parameters, which they may replace."""
+
+    def _apply(self, fn, recurse=True):
+        for m in self.modules():
+            drop_operands(m)
+        return super()._apply(fn, recurse)
+
+
+class _Key(tuple):
+    """The key of something kept.  held: aliases of the tensors whose addresses it names, so that no other tensor gets one of them while
+    it is compared.  A copy of a module, and one read back from a file, holds nothing: there the key fits no tensor."""
+
+    def __deepcopy__(self, memo):
+        return ()
+
+    def __reduce__(self):
+        return tuple, ()
+
+
+def _kept(key, layers, cache):
+    """key, whose last entry is _param_key(layers), as the first entry of a cache that replaces `cache`."""
+    kept, old = _Key(key), None if cache is None else cache[0]
+    kept.where = [e[::2] for e in key[-1]]
+    if type(old) is _Key and old.where == kept.where:      # held all the while: an address stands for the same memory
+        kept.held = old.held
+    else:
+        kept.held = [t.detach() for l in layers for t in (l.weight, l.bias) if t is not None]
+    return kept
+
+
 def drop_operands(mod):
     """Forget the packed weights kept for mod, for the chain between its narrow ends (that chain's copies live on an object that
-    is no submodule, and a walk over module.modules() alone passes them by) and for a block's plans, which hold copies of their own."""
+    is no submodule, and a walk over module.modules() alone passes them by), a block's plans, which hold copies of their own, and the
+    latents' cast copy."""
     mod.__dict__.pop("_flare_plans", None)
+    mod.__dict__.pop("_q_cache", None)
     sub = mod.__dict__.get("_flare_subchain")
     for m in (mod, None if sub is None else sub[0]):
         if m is not None:
@@ -435,7 +472,7 @@ def _packed_few(mod, layers, cd, train):
     if tiles is None:
         return None
     w, b, _, wt = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, train, tiled=True)
-    mod.__dict__["_flare_packed_few"] = (key, w, b, wt)
+    mod.__dict__["_flare_packed_few"] = (_kept(key, layers, cache), w, b, wt)
     return w, b, wt
 
 
@@ -448,12 +485,12 @@ def _packed(mod, layers, cd):
     tiles = _chain_tiles(layers)
     if tiles is not None:
         w, b, _, _ = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, False)
-        mod._flare_packed = (key, w, b)
+        mod._flare_packed = (_kept(key, layers, cache), w, b)
         return w, b
     w = torch.stack([l.weight.detach() for l in layers]).to(cd).contiguous()
     Cdim = w.shape[-1]
     b = torch.stack([l.bias.detach().float() if l.bias is not None else w.new_zeros(Cdim, dtype=torch.float32) for l in layers]).contiguous()
-    mod._flare_packed = (key, w, b)
+    mod._flare_packed = (_kept(key, layers, cache), w, b)
     return w, b
 
 
@@ -469,7 +506,7 @@ def _packed_expand(mod, E, cd):
     tiles = _expand_tiles(f1, f2, E, Cdim)
     if tiles is not None:
         w, b, _, _ = _pack_launch(Cdim, cd, tiles, f1.weight.device, False)
-        mod._flare_packed = (key, w, b)
+        mod._flare_packed = (_kept(key, (f1, f2), cache), w, b)
         return w, b
     w1 = f1.weight.detach().to(cd).view(E, Cdim, Cdim)                       # [j][hidden row in chunk][in]
     w2 = f2.weight.detach().to(cd).view(Cdim, E, Cdim).permute(1, 0, 2)      # [j][out][hidden col in chunk]
@@ -479,7 +516,7 @@ def _packed_expand(mod, E, cd):
         b[0::2] = f1.bias.detach().float().view(E, Cdim)
     if f2.bias is not None:
         b[1] = f2.bias.detach().float()
-    mod._flare_packed = (key, w, b)
+    mod._flare_packed = (_kept(key, (f1, f2), cache), w, b)
     return w, b
 
 
@@ -508,7 +545,7 @@ def _packed_io(mod, layers, cd, Cdim, in_dim, out_dim):
         w_in[:, :in_dim] = layers[0].weight.detach().float()
         b_in = (layers[0].bias.detach().float().contiguous() if layers[0].bias is not None
                 else torch.zeros(Cdim, dtype=torch.float32, device=dev))
-    mod._flare_packed = (key, w, b, w_in, b_in)
+    mod._flare_packed = (_kept(key, layers, cache), w, b, w_in, b_in)
     return w, b, w_in, b_in
 
 
@@ -657,7 +694,7 @@ def prepack(x, cd, *stacks, latents=None):
         t = _chain_tiles(layers)
         if t is None:
             return
-        stale.append((mods[0], key, at, at + len(t)))
+        stale.append((mods[0], _kept(key, layers, cache), at, at + len(t)))
         tiles += t
         at += len(t)
     if len(stale) < 2 or at > _lib.MLP_PACK_MAX:
@@ -883,7 +920,7 @@ def _packed_train(mod, layers, cd):
     else:
         w, b = _packed(mod, layers, cd)
         w_img, wt_img = mlp_weight_images(w)
-    mod.__dict__["_flare_packed_train"] = (key, w, b, w_img, wt_img)
+    mod.__dict__["_flare_packed_train"] = (_kept(key, layers, cache), w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
 
@@ -900,7 +937,7 @@ def _packed_train_expand(mod, E, cd):
     else:
         w, b = _packed_expand(mod, E, cd)
         w_img, wt_img = mlp_weight_images(w)
-    mod.__dict__["_flare_packed_train"] = (key, w, b, w_img, wt_img)
+    mod.__dict__["_flare_packed_train"] = (_kept(key, (f1, f2), cache), w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
 

@@ -52,7 +52,7 @@ class RotaryPositionalEmbeddings(nn.Module):
         return x * self.C[:N].to(x.dtype) + partner * self.S[:N].to(x.dtype)
 
 
-class FLARE(nn.Module):
+class FLARE(fused.DropsOperands, nn.Module):
     def __init__(self, channel_dim: int, num_heads: int = 8, num_latents: int = 32, act: str = None,
                  attn_scale: float = 1.0, num_layers_kv_proj: int = 3, kv_proj_hidden_dim: int = 1.0,
                  attn_drop: float = 0.0, proj_drop: float = 0.0, rope=None):
@@ -113,7 +113,7 @@ class FLARE(nn.Module):
         return y if _res is None else _res + y
 
 
-class FLAREBlock(nn.Module):
+class FLAREBlock(fused.DropsOperands, nn.Module):
     def __init__(self, channel_dim: int, num_heads: int = None, num_latents: int = None, act: str = None,
                  rmsnorm: bool = False, attn_scale: float = 1.0, num_layers_kv_proj: int = 3,
                  num_layers_ffn: int = 3, kv_proj_hidden_dim: int = 1.0, ffn_hidden_dim: int = 1.0,
@@ -214,7 +214,7 @@ def make_kernel(kernel: str, head_dim: int, qk_dim: int = None):
                               f"{sorted(_PLAIN_KERNELS)} + {sorted(_LEARNED_KERNELS)}")
 
 
-class TripleAttention(nn.Module):
+class TripleAttention(fused.DropsOperands, nn.Module):
     """Third-order linear attention layer (backends.py:1195-1292): five token-wise projections, the
     feature map on q1, q2, k1, k2, optional unit-norm rows, the padding mask as a multiplication,
     state[i,j,k] = sum_n k1[n,i] v[n,j] k2[n,k] / N and out[n,j] = sum_ik q1[n,i] state[i,j,k] q2[n,k]
@@ -281,7 +281,7 @@ class TripleAttention(nn.Module):
     attn_einsum = attn
 
 
-class TripleBlock(nn.Module):
+class TripleBlock(fused.DropsOperands, nn.Module):
     """Pre-norm residual block around TripleAttention (backends.py:1294-1331)."""
 
     def __init__(self, channel_dim: int, num_heads: int, act: str = None, rmsnorm: bool = False,

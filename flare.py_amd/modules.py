@@ -101,7 +101,7 @@ def _plain_call(mod):
     return type(mod) is ResidualMLP and rows._plain(mod)
 
 
-class ResidualMLP(nn.Module):
+class ResidualMLP(fused.DropsOperands, nn.Module):
     """fc1 -> act -> num_layers x (x + act(fc x)) -> fc2, with optional end residuals.
     num_layers == -1 degenerates to a single Linear named `fc`."""
 
@@ -135,7 +135,7 @@ class ResidualMLP(nn.Module):
         return x + h if self.output_residual else h
 
 
-class FLARE(nn.Module):
+class FLARE(fused.DropsOperands, nn.Module):
     """Latent gather-scatter attention layer: returns (y, scores)."""
 
     def __init__(self, channel_dim: int, num_heads: int = 8, num_latents: int = 32, attn_scale: float = 1.0,
@@ -181,7 +181,8 @@ class FLARE(nn.Module):
             q = self.latent_q.detach().view(self.num_heads, self.num_latents, self.head_dim).to(cd)
             if pad:
                 q = torch.nn.functional.pad(q, (0, pad))
-            c = self._q_cache = (key, q.contiguous())
+            c = self._q_cache = (fused._Key(key), q.contiguous())
+            c[0].held = self.latent_q.detach()
         return c[1]
 
     def _fusable(self, x, return_scores):
@@ -268,7 +269,7 @@ def _prepack(block, x, return_scores=False):
             fused.prepack(x, cd, (att.k_proj, att.v_proj), (att.out_proj,), (block.mlp,))
 
 
-class FLAREBlock(nn.Module):
+class FLAREBlock(fused.DropsOperands, nn.Module):
     """x + att(norm1 x), then x + mlp(norm2 x); returns (x, scores)."""
 
     def __init__(self, channel_dim: int, num_heads: int = None, num_latents: int = None, attn_scale: float = 1.0,
@@ -284,10 +285,6 @@ class FLAREBlock(nn.Module):
                          v_proj_mlp_ratio=v_proj_mlp_ratio, qk_norm=qk_norm, rmsnorm=rmsnorm)
         self.mlp = ResidualMLP(channel_dim, int(channel_dim * ffn_mlp_ratio), channel_dim,
                                num_layers=num_layers_ffn, act=act, input_residual=True, output_residual=True)
-
-    def _apply(self, fn, recurse=True):
-        self.__dict__.pop("_flare_plans", None)          # they hold the memory of parameters that fn may replace
-        return super()._apply(fn, recurse)
 
     def forward(self, x, return_scores: bool = False):
         if not return_scores and type(self.att) is FLARE:
@@ -306,7 +303,7 @@ class FLAREBlock(nn.Module):
         return x, scores
 
 
-class FinalLayer(nn.Module):
+class FinalLayer(fused.DropsOperands, nn.Module):
     def __init__(self, channel_dim: int, out_dim: int, act: str = None, num_layers: int = 2,
                  hidden_dim: int = None, ln: bool = True):
         super().__init__()
@@ -322,7 +319,7 @@ class FinalLayer(nn.Module):
         return self.mlp(self.ln(x))
 
 
-class FLAREModel(nn.Module):
+class FLAREModel(fused.DropsOperands, nn.Module):
     """in_proj -> num_blocks x FLAREBlock -> (norm, out MLP)."""
 
     def __init__(self, in_dim: int, out_dim: int, channel_dim: int = 64, num_blocks: int = 8,

@@ -15,7 +15,8 @@ modules (packed weights, the cast latent queries).  Every graph keeps those tens
 that rebuilds a module's cache (another compute dtype, an optimizer step, `load_state_dict`) can never free
 memory a graph still reads; and every call compares the versions and addresses of the module's parameters and
 buffers with those seen at capture and captures again when any of them changed, so a replay never computes
-with operands packed from old weights.
+with operands packed from old weights.  The parameters' and buffers' memory is held for that comparison until the shape is
+captured again or `reset()` is called: a replaced one then never gets the address of the one it replaced.
 """
 from __future__ import annotations
 
@@ -45,7 +46,10 @@ class GraphedForward:
     def _param_key(self):
         """Versions and addresses of everything the forward reads: an in-place update bumps the version, a
         replaced tensor changes the address."""
-        return tuple((t.data_ptr(), t._version) for t in list(self.module.parameters()) + list(self.module.buffers()))
+        return tuple((t.data_ptr(), t._version) for t in self._tensors())
+
+    def _tensors(self):
+        return list(self.module.parameters()) + list(self.module.buffers())
 
     def _cached_operands(self):
         """The operand caches the fused launches left on the modules during warm-up (their tensors' addresses are
@@ -71,7 +75,7 @@ class GraphedForward:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 static_y = self.module(static_x)
-        return graph, static_x, static_y, self._param_key(), self._cached_operands()
+        return graph, static_x, static_y, self._param_key(), self._cached_operands(), [t.detach() for t in self._tensors()]
 
     def __call__(self, x: torch.Tensor):
         if x.device.type != "cuda":

@@ -91,7 +91,6 @@ class GraphedTrainStep:
         torch.clear_autocast_cache()
         for m in self.module.modules():
             fused.drop_operands(m)
-            m.__dict__.pop("_q_cache", None)
 
     def _capture(self, inputs, params):
         dev = inputs[0].device

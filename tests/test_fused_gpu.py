@@ -504,3 +504,72 @@ def test_cached_operands_follow_parameter_updates(dev, C, H):
                     delattr(mod, name)
         y2 = fresh(x)[0]
     assert not torch.equal(y0, y1) and torch.equal(y1, y2)
+
+
+@pytest.mark.parametrize("how", ["data", "parameter"])
+@pytest.mark.parametrize("what", ["chain", "many tokens", "training", "expand", "narrow ends", "latents", "graph"])
+def test_weights_replaced_twice_between_calls(dev, what, how):
+    """A weight that no call sees between two others: the second one's memory may be that of the weight before, at the same version."""
+    kw = dict(num_layers_ffn=0, ffn_mlp_ratio=4.0) if what == "expand" else {}
+    if what == "narrow ends":
+        make = lambda: F.FLAREModel(in_dim=2, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev).eval()
+        owner, x = (lambda m: (m.in_proj.fc2, "weight")), torch.randn(1, 300, 2, device=dev)
+    else:
+        make = lambda: F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev).eval()
+        owner = (lambda m: (m.att, "latent_q")) if what == "latents" else lambda m: (m.mlp.fc1, "weight")
+        x = torch.randn(1, 20000 if what == "many tokens" else 300, 64, device=dev)
+    if what == "training":
+        x.requires_grad_(True)
+    base = make()
+    state = {k: v.clone() for k, v in base.state_dict().items()}
+    w0 = getattr(*owner(base)).detach().clone()
+
+    def run(m):
+        with torch.autocast("cuda", dtype=torch.bfloat16), torch.set_grad_enabled(what == "training"):
+            y = m(x)
+        y = y[0] if isinstance(y, tuple) else y
+        return torch.autograd.grad(y.float().square().sum(), x)[0] if what == "training" else y
+
+    want = []
+    for i in range(16):
+        m = make()
+        m.load_state_dict(state)
+        getattr(*owner(m)).data.copy_(w0 * (1.0 + 0.125 * i))
+        want.append(run(m).clone())
+    call = F.GraphedForward(base, autocast_dtype=torch.bfloat16) if what == "graph" else None
+    first = lambda y: y[0] if isinstance(y, tuple) else y
+    for i in range(16):
+        o, name = owner(base)
+        value = w0 * (1.0 + 0.125 * i)
+        if how == "data":
+            getattr(o, name).data = value
+        else:
+            setattr(o, name, nn.Parameter(value))
+        del value
+        if i % 2:
+            assert torch.equal(run(base) if call is None else first(call(x)), want[i]), i
+    base.cpu()
+    assert not any(n.startswith(("_flare_packed", "_flare_plans", "_q_cache")) for m in base.modules() for n in m.__dict__)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_parametrised_weight_is_packed_at_every_call(dev, grad):
+    """weight_norm computes the weight anew at every access: its address and version say nothing."""
+    torch.manual_seed(1)
+    blk = F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32).to(dev).eval()
+    torch.nn.utils.parametrizations.weight_norm(blk.mlp.fc1)
+    x = torch.randn(1, 300, 64, device=dev)
+
+    def run():
+        with torch.autocast("cuda", dtype=torch.bfloat16), torch.set_grad_enabled(grad):
+            y = blk(x)[0]
+        return [y.detach(), *(torch.autograd.grad(y.sum(), list(blk.parameters())) if grad else [])]
+
+    for _ in range(6):
+        got = run()
+        for m in blk.modules():
+            fused.drop_operands(m)
+        for a, b in zip(got, run()):
+            assert torch.equal(a, b)
+        with torch.no_grad():
+            blk.mlp.fc1.parametrizations.weight.original0.mul_(1.25)
