@@ -555,6 +555,11 @@ int flare_mixer_bwd_workspace_bytes(const FlareMixerDesc* desc, size_t* bytes)
     int rc = check_bwd(desc);
     if (rc != FLARE_OK) return rc;
     *bytes = plan_bwd(desc).total;
+    if (desc->flags & FLARE_FLAG_ABSENT_TOKENS) {      // the gather half plans without it
+        FlareMixerDesc plain = *desc;
+        plain.flags &= ~FLARE_FLAG_ABSENT_TOKENS;
+        *bytes = std::max(*bytes, plan_bwd(&plain).total);
+    }
     return FLARE_OK;
 }
 
@@ -629,11 +634,15 @@ int flare_mixer_bwd(const FlareMixerDesc* desc, const void* q, const void* k, co
 namespace {
 // Argument block of the half backwards: the whole-mixer workspace layout, one term of dS switched off (fp32: compiled
 // out; bf16 / f16: its softmax weights forced to zero through a log-sum-exp of 1e30, see bwd_half_prep_kernel).
-int half_bwd_args(flare::MixerBwdArgs& a, const FlareMixerDesc* desc, void* workspace, size_t workspace_bytes)
+int half_bwd_args(flare::MixerBwdArgs& a, const FlareMixerDesc* desc, bool gather, void* workspace, size_t workspace_bytes)
 {
     int rc = check_bwd(desc);
     if (rc != FLARE_OK) return rc;
-    if (desc->flags & FLARE_FLAG_ABSENT_TOKENS) return fail(FLARE_EUNSUPPORTED, "the half backwards do not take FLARE_FLAG_ABSENT_TOKENS");
+    const bool absent = (desc->flags & FLARE_FLAG_ABSENT_TOKENS) != 0;
+    if (absent && !gather) return fail(FLARE_EUNSUPPORTED, "the scatter half's backward does not take FLARE_FLAG_ABSENT_TOKENS");
+    FlareMixerDesc plain = *desc;                      // absent tokens are rows of zeros here: any kernel takes them
+    plain.flags &= ~FLARE_FLAG_ABSENT_TOKENS;
+    desc = &plain;
     if (desc->dtype != FLARE_DT_F32 && drop_threshold(desc) != 0)
         return fail(FLARE_EUNSUPPORTED, "the bf16 / f16 half backwards do not take attention dropout");
     const BwdPlan p = plan_bwd(desc);
@@ -651,6 +660,7 @@ int half_bwd_args(flare::MixerBwdArgs& a, const FlareMixerDesc* desc, void* work
     a.n_splits = p.n_splits; a.tokens_per_split = p.tokens_per_split;
     a.n_splits0 = p.n_splits0; a.tokens_per_split0 = p.tokens_per_split0;
     a.no_mfma32 = bwd_wants_dz32(desc) ? 0 : 1;
+    a.absent = absent ? 1 : 0;
     a.scale = desc->scale; a.scale_log2 = desc->scale * 1.4426950408889634f;
     a.drop_thr = drop_threshold(desc);
     a.drop_rs = 1.f;
@@ -675,7 +685,7 @@ int flare_gather_bwd(const FlareMixerDesc* desc, const void* q, const void* k, c
                      void* workspace, size_t workspace_bytes, void* stream)
 {
     flare::MixerBwdArgs a;
-    int rc = half_bwd_args(a, desc, workspace, workspace_bytes);
+    int rc = half_bwd_args(a, desc, true, workspace, workspace_bytes);
     if (rc != FLARE_OK) return rc;
     if (!q || !k || !v || !z || !lse_lat || !dz || !dq || !dk || !dv)
         return fail(FLARE_EINVAL, "q, k, v, z, lse_lat, dz, dq, dk, dv must not be NULL");
@@ -700,7 +710,7 @@ int flare_scatter_bwd(const FlareMixerDesc* desc, const void* q, const void* k, 
                       void* workspace, size_t workspace_bytes, void* stream)
 {
     flare::MixerBwdArgs a;
-    int rc = half_bwd_args(a, desc, workspace, workspace_bytes);
+    int rc = half_bwd_args(a, desc, false, workspace, workspace_bytes);
     if (rc != FLARE_OK) return rc;
     if (!q || !k || !z || !y || !lse_tok || !dy || !dy_stride || !dq || !dk || !dz)
         return fail(FLARE_EINVAL, "q, k, z, y, lse_tok, dy, dy_stride, dq, dk, dz must not be NULL");

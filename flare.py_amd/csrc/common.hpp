@@ -228,6 +228,8 @@ struct MixerBwdArgs {
     int absent;              // 1: tokens whose lse_tok exceeds kAbsentLse take no part, whatever their rows hold; their dk, dv rows become zeros
 };
 constexpr float kAbsentLse = 1.5e30f;      // (a half backward's own lse_tok of 1e30, see there, is not such a mark)
+// Cap of the gather's exponent (log2) where tokens may be absent: a real token's is 0 at most, and 2^60 times what it meets stays finite
+constexpr float kAbsentExpCap = 60.f;
 
 // Whether a (b,h) takes the form of the backward in which both weights come from exp2(S) alone (kernels on the 32x32x16
 // product): the one-exponential form's own condition (the latents' largest log-sum-exp and the tokens' smallest one at

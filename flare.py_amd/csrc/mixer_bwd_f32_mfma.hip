@@ -217,7 +217,10 @@ __global__ __launch_bounds__(256, (D == 64 && MODE == 1) ? 1 : 2) void bwd_f32_l
                 for (int r = 0; r < 4; ++r) {
                     // a half's absent term is left out at compile time: its operands may be anything
                     float ds = 0.f;
-                    if constexpr (use_a) ds = fast_exp2(s[r] - l2[ct]) * (t1[r] - dl[ct]);
+                    // (of a token that the caller zeroed the gather's exponent is -L_m, which nothing bounds)
+                    const float ea = s[r] - l2[ct];
+                    constexpr bool cap = drop || HALF == 1;
+                    if constexpr (use_a) ds = fast_exp2(cap && ea > kAbsentExpCap ? kAbsentExpCap : ea) * (t1[r] - dl[ct]);
                     if constexpr (use_b) ds += fast_exp2(s[r] - rh[r]) * (t2[r] - de[r]);
                     p[r] = valid[r] ? ds : 0.f;
                 }
@@ -522,6 +525,7 @@ hipError_t launch_dh(const MixerBwdArgs& a0, hipStream_t st)
 template <int D>
 hipError_t launch_d(const MixerBwdArgs& a, hipStream_t st)
 {
+    if (a.absent && a.half == 1) return a.drop_thr != 0 ? launch_dh<D, 1, 1>(a, st) : launch_dh<D, 1, 0>(a, st);
     if (a.absent) return a.half != 0 || a.drop_thr != 0 ? hipErrorInvalidValue : launch_dh<D, 0, 2>(a, st);
     if (a.drop_thr != 0) return a.half == 1 ? launch_dh<D, 1, 1>(a, st) : a.half == 2 ? launch_dh<D, 2, 1>(a, st) : launch_dh<D, 0, 1>(a, st);
     return a.half == 1 ? launch_dh<D, 1, 0>(a, st) : a.half == 2 ? launch_dh<D, 2, 0>(a, st) : launch_dh<D, 0, 0>(a, st);

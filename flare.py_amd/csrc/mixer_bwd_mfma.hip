@@ -177,6 +177,8 @@ constexpr int bwd_tile(int D) { return D <= 16 ? 128 : 64; }
 // One workgroup = 4 waves x (16 CT latents) x one token range.  MODE 0: dz partial; MODE 1: dq partial.
 // KIND: 0 plain, 1 the forward dropped weights, 2 absent tokens (a key mask): their rows are staged as zeros, which with their
 // log-sum-exp leaves nothing of them in dz and dq; in the token pass a token is a column of its own and only its stores change.
+// The gather's exponent S - L_m of an absent token (of one that the caller zeroed, under dropout and in the gather half alone) is
+// -L_m, which nothing bounds: it is capped before the exponential, so that the zero row meets a finite weight.
 // (Around the kernels, in torch, the mask was five passes over [N,D] arrays and seven small launches: forward + backward at B=4, H=8,
 // N=50,000, M=128, D=16 bf16 579 us, 371 us with the mask here, 341 us without one.)
 template <typename T, int D, int CT, int MODE, int KIND>
@@ -333,6 +335,7 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
         for (int rt = 0; rt < RT; ++rt) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     const f32x4 zf = {0.f, 0.f, 0.f, 0.f};
 
+    auto gather_exp = [](float x) { return fast_exp2(KIND != 0 && x > kAbsentExpCap ? kAbsentExpCap : x); };
     auto process = [&](auto fast_c, auto drop_c, int n0, int buf) {
         constexpr bool FAST = decltype(fast_c)::value;      // one-exponential form (dq pass only)
         // DROP: the forward dropped weights.  Every additive term is then applied element by element (accumulators start
@@ -401,11 +404,11 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (kFoldLat) {
-                            o[e] = fast_exp2(a0[e]) * fmaf(nel[ct], da[e], g0[e]);
-                            o[e + 4] = fast_exp2(a1[e]) * fmaf(nel[ct], db[e], g1[e]);
+                            o[e] = gather_exp(a0[e]) * fmaf(nel[ct], da[e], g0[e]);
+                            o[e + 4] = gather_exp(a1[e]) * fmaf(nel[ct], db[e], g1[e]);
                         } else {
-                            o[e] = fast_exp2(a0[e] - l2m[ct]) * (fmaf(nel[ct], da[e], g0[e]) - dm[ct]);
-                            o[e + 4] = fast_exp2(a1[e] - l2m[ct]) * (fmaf(nel[ct], db[e], g1[e]) - dm[ct]);
+                            o[e] = gather_exp(a0[e] - l2m[ct]) * (fmaf(nel[ct], da[e], g0[e]) - dm[ct]);
+                            o[e + 4] = gather_exp(a1[e] - l2m[ct]) * (fmaf(nel[ct], db[e], g1[e]) - dm[ct]);
                         }
                     }
                     if (!full) {       // rows past the end of the token range (clamped copies of the last token)
@@ -468,15 +471,15 @@ __global__ __launch_bounds__(256, MODE == 1 ? bwd_dq_wgs_per_cu(D, CT) : 2) void
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (DROP) {
-                            o[e] = fast_exp2(b0[e] - l2m[ct]) * (k1[e] * g10[e] - dm[ct]) + fast_exp2(b0[e] + ra[e]) * (k2[e] * g20[e] + da[e]);
-                            o[e + 4] = fast_exp2(b1[e] - l2m[ct]) * (k1[e + 4] * g11[e] - dm[ct]) +
+                            o[e] = gather_exp(b0[e] - l2m[ct]) * (k1[e] * g10[e] - dm[ct]) + fast_exp2(b0[e] + ra[e]) * (k2[e] * g20[e] + da[e]);
+                            o[e + 4] = gather_exp(b1[e] - l2m[ct]) * (k1[e + 4] * g11[e] - dm[ct]) +
                                        fast_exp2(b1[e] + rb[e]) * (k2[e + 4] * g21[e] + db[e]);
                         } else if constexpr (kFoldLat) {
-                            o[e] = fast_exp2(a0[e]) * g10[e] + fast_exp2(b0[e]) * g20[e];
-                            o[e + 4] = fast_exp2(a1[e]) * g11[e] + fast_exp2(b1[e]) * g21[e];
+                            o[e] = gather_exp(a0[e]) * g10[e] + fast_exp2(b0[e]) * g20[e];
+                            o[e + 4] = gather_exp(a1[e]) * g11[e] + fast_exp2(b1[e]) * g21[e];
                         } else {    // plain products; every term is applied element by element
-                            o[e] = fast_exp2(b0[e] - l2m[ct]) * (g10[e] - dm[ct]) + fast_exp2(b0[e] + ra[e]) * (g20[e] + da[e]);
-                            o[e + 4] = fast_exp2(b1[e] - l2m[ct]) * (g11[e] - dm[ct]) + fast_exp2(b1[e] + rb[e]) * (g21[e] + db[e]);
+                            o[e] = gather_exp(b0[e] - l2m[ct]) * (g10[e] - dm[ct]) + fast_exp2(b0[e] + ra[e]) * (g20[e] + da[e]);
+                            o[e + 4] = gather_exp(b1[e] - l2m[ct]) * (g11[e] - dm[ct]) + fast_exp2(b1[e] + rb[e]) * (g21[e] + db[e]);
                         }
                     }
                 }
@@ -974,11 +977,11 @@ hipError_t bwd_all(const MixerBwdArgs& a, hipStream_t st)
     a0.tokens_per_split = a.tokens_per_split0;
     // bf16 at D = 32 without dropout: the token-parallel passes on the 32x32x16 product.  The scatter half alone stays on
     // the two-exponential form, which only the 16x16x32 token and dq passes run at full speed.
-    const bool mfma32 = KIND == 0 && !a.no_mfma32 && std::is_same<T, bf16_t>::value && bwd_dz32_supported(1, a.M, D);
+    const bool mfma32 = (KIND == 0 || (KIND == 2 && a.half == 1)) && !a.no_mfma32 && std::is_same<T, bf16_t>::value && bwd_dz32_supported(1, a.M, D);
     const bool dz32 = mfma32, dq32 = mfma32 && a.half != 2;
     hipError_t e = hipSuccess;
     if (a.half != 0) {
-        if (KIND != 0) return hipErrorInvalidValue;
+        if (KIND != 0 && !(KIND == 2 && a.half == 1)) return hipErrorInvalidValue;
         const int64_t items = std::max<int64_t>((int64_t)a.B * a.H * (a.half == 1 ? a.N : a.M), lat);
         hipLaunchKernelGGL(bwd_half_prep_kernel, dim3((unsigned)std::min<int64_t>((items + 255) / 256, 4096)), dim3(256), 0, st, a);
     }

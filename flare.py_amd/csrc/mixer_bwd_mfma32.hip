@@ -376,6 +376,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dq32_kernel(MixerBwdArgs a)
     // Which form the (b,h) takes: every wave computes the same answer.
     float lmax2;
     const bool fast = bwd_unshifted_form(a, bh, lane, lmax2);
+    // rows of absent tokens, in the gather half, are zeros whose exponent -L_m nothing bounds but the unshifted form's condition
+    const float cap = a.absent ? kAbsentExpCap : 3.0e38f;
+    auto gather_exp = [&](float x) { return fast_exp2(x > cap ? cap : x); };
 
     // per-latent scalars of the lane's column in every tile
     float l2m[MT], dm[MT];
@@ -642,7 +645,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq32_kernel(MixerBwdArgs a)
                 g2v = mma32(yb[1], z1, g2v);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    o[r] = fast_exp2(s[r] - l2m[mt]) * (g1[r] - dm[mt]) + fast_exp2(s[r] + row0[r]) * g2v[r];
+                    o[r] = gather_exp(s[r] - l2m[mt]) * (g1[r] - dm[mt]) + fast_exp2(s[r] + row0[r]) * g2v[r];
             }
             u32x4 p[2];
 #pragma unroll

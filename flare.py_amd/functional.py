@@ -859,6 +859,8 @@ def _half_hip_grad(which, q, k, x, z, aux, scale, key_mask, g):
             v = v.contiguous()
         gz = g.to(torch.float32).contiguous()
         d = _mixer_desc(q4, k, v, None, scale, 0, False)
+        if keep is not None:
+            d.flags |= _lib.FLAG_ABSENT_TOKENS
         out = torch.empty((B, H, N, D), dtype=k.dtype, device=k.device)
     else:
         y = x.contiguous()

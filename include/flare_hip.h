@@ -67,7 +67,7 @@ extern "C" {
 /* FlareMixerDesc.flags */
 #define FLARE_FLAG_FORCE_GENERIC 1  /* skip every matrix-core kernel (16-bit and fp32), use the fp32-FMA kernels */
 #define FLARE_FLAG_MFMA16        2  /* keep the 16x16x32 MFMA kernels where the 32x32x16 gather and scatter (bf16, D = 32, no key mask) would run */
-#define FLARE_FLAG_ABSENT_TOKENS 16 /* flare_mixer_bwd, no dropout: a token whose lse_tok is 2e30 takes no part (a key mask's padding): its k, v, dy rows may hold anything, its dk, dv rows become zeros */
+#define FLARE_FLAG_ABSENT_TOKENS 16 /* flare_mixer_bwd, no dropout: a token whose lse_tok is 2e30 takes no part (a key mask's padding): its k, v, dy rows may hold anything, its dk, dv rows become zeros.  flare_gather_bwd: some of k's and v's rows are absent tokens that the caller zeroed */
 #define FLARE_FLAG_DQ_PARTS      32 /* flare_mixer_bwd, bf16 / f16: dq (may be NULL) is not written, its partial results stay in the workspace (flare_mixer_bwd_dq_parts) */
 #define FLARE_FLAG_GRAD_LIKE_KV  8  /* flare_mixer_bwd: dk has k's strides and dv has v's (default: both [B,H,N,D] contiguous) */
 
@@ -228,7 +228,8 @@ int flare_scatter_fwd_lse(const FlareMixerDesc* desc, const void* q, const void*
  * (pdebench/__main__.py:1106).  There is no key-mask
  * argument: a padded token is marked by its lse_tok (FLARE_FLAG_ABSENT_TOKENS), a batch element without tokens by 1e30 as its
  * lse_lat.  With dropout, and in the half backwards below: zero the k, v and dy rows of padded tokens, pass 1e30 as their lse_tok,
- * and clear their dk, dv rows afterwards.
+ * and clear their dk, dv rows afterwards (FLARE_FLAG_ABSENT_TOKENS tells flare_gather_bwd of them: a zero row's weight exp(-lse_lat) may
+ * exceed the number range).
  * Inputs: q, k, v as in the forward; y and z its outputs; lse_lat = lse of flare_gather_fwd;
  * lse_tok of flare_scatter_fwd_lse; dy [B,H,N,D] with strides dy_stride.
  * Outputs: dq fp32 [B,H,M,D] contiguous (per batch element: sum over b when q is shared);

@@ -563,3 +563,55 @@ def test_operands_that_do_not_match_are_refused(dev, grad, q, k, v, autocast):
     q, k, v = (torch.randn(s, device=dev, dtype=torch.float32 if autocast else torch.bfloat16, requires_grad=grad) for s in (q, k, v))
     with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast), pytest.raises(ValueError, match="match"):
         FN.flare_multihead_mixer(q, k, v)
+
+
+def low_scores(B, H, N, M, D, dtype):
+    """Operands whose real scores all lie around -122 (-176 in log2 units): a zero row's score is 0, and exp(0 - log-sum-exp of a latent)
+    leaves the number range.  The offset sits in a channel of its own, and scale * log2(e) is 1, so that no rounding of q moves it."""
+    q, k, v, gy = make(B, H, N, M, D, dtype, seed=N + M)
+    q[..., 0], k[..., 0] = -176.0, 1.0
+    mask = torch.rand(B, N, generator=torch.Generator().manual_seed(N)) < 0.6
+    mask[:, 0] = True
+    return q, k, v, gy, 0.6931471805599453, mask
+
+
+LOW_SHAPES = [(2, 2, 333, 128, 16), (1, 2, 500, 256, 16), (2, 1, 97, 32, 16), (2, 1, 700, 256, 32), (1, 2, 130, 64, 32), (2, 1, 300, 128, 64), (1, 1, 210, 256, 64)]
+
+
+@pytest.mark.parametrize("shape", LOW_SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("halves", [False, True])
+def test_absent_tokens_beside_real_scores_far_below_zero(dev, shape, dtype, halves):
+    q, k, v, gy, scale, mask = low_scores(*shape, dtype)
+    qd, kd, vd = (t.to(dev).requires_grad_(True) for t in (q, k, v))
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    yr, zr = O.mixer_explicit(qr, kr, vr, scale, mask)
+    if halves:                            # return_z takes the two halves' backward
+        y, z = F.flare_multihead_mixer(qd, kd, vd, scale=scale, key_mask=mask.to(dev), return_z=True)
+        gz = torch.randn(z.shape, generator=torch.Generator().manual_seed(0))
+        got = torch.autograd.grad((y, z), (qd, kd, vd), (gy.to(dev), gz.to(dev)))
+        zr = O.gather_explicit(qr, kr, vr, scale, mask)
+        zr = zr[0] if isinstance(zr, tuple) else zr
+        want = torch.autograd.grad((O.scatter_explicit(qr, kr, zr, scale, mask), zr), (qr, kr, vr), (gy.double(), gz.double()))
+    else:
+        assert FN._hip_backward_ok(qd, kd, vd, mask.to(dev), False)
+        got = torch.autograd.grad(F.flare_multihead_mixer(qd, kd, vd, scale=scale, key_mask=mask.to(dev)), (qd, kd, vd), gy.to(dev))
+        want = torch.autograd.grad(yr, (qr, kr, vr), gy.double() * mask[:, None, :, None])
+    for name, a, r in zip(("dq", "dk", "dv"), got, want):
+        assert bool(torch.isfinite(a).all()), name
+        err = O.rel_l2(a, r)
+        assert err <= (1e-4 if dtype == torch.float32 else 3e-2), f"{name} rel-L2 {err:.3e}"
+
+
+@pytest.mark.parametrize("shape", LOW_SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_absent_tokens_beside_low_scores_under_dropout(dev, shape, dtype):
+    q, k, v, gy, scale, mask = low_scores(*shape, dtype)
+    qd, kd, vd = (t.to(dev).requires_grad_(True) for t in (q, k, v))
+    y = F.flare_multihead_mixer(qd, kd, vd, scale=scale, key_mask=mask.to(dev), dropout_p=0.25, dropout_seed=7)
+    got = torch.autograd.grad(y, (qd, kd, vd), gy.to(dev))
+    want = FN._mixer_torch_grad(*(t.to(dev).float() for t in (q, k, v)), scale, mask.to(dev), (gy * mask[:, None, :, None]).to(dev).float(), (0.25, 7))
+    for name, a, r in zip(("dq", "dk", "dv"), got, want):
+        assert bool(torch.isfinite(a).all()), name
+        err = O.rel_l2(a, r.cpu())
+        assert err <= (2e-4 if dtype == torch.float32 else 3e-2), f"{name} rel-L2 {err:.3e}"
