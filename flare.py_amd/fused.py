@@ -193,6 +193,15 @@ def _narrow_rows(x2):
     return x2 if x2.stride(-1) == 1 and x2.stride(0) >= x2.shape[1] else x2.clone(memory_format=torch.contiguous_format)
 
 
+def _grid_rows(t):
+    """Rows [T, width] as the launches read them, on the 16-byte grid and a width or more apart; others are copied (contiguous() would
+    give back contiguous rows that begin off the grid)."""
+    step, unit = t.stride()
+    if unit == 1 and step % 4 == 0 and step >= t.shape[1] and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def _narrow_backward(d, x2, w, t, dy2, dx, has_bias, dev):
     lib = _lib.load()
     parts = C.c_int32(0)
@@ -560,8 +569,7 @@ def _fused_mlp_io(x, mod, cd, io, info, norm, out_dtype):
         add_mask >>= 1
     xw = x.shape[-1]
     x2 = x.reshape(-1, xw)
-    if x2.stride(-1) != 1 or (not in_dim and (x2.stride(0) % 4 or x2.data_ptr() % 16)):
-        x2 = x2.contiguous()
+    x2 = _narrow_rows(x2) if in_dim else _grid_rows(x2)
     out_dtype = x.dtype if out_dtype is None else out_dtype
     yw = out_dim if out_dim else Cdim
     y = torch.empty(*x.shape[:-1], yw, dtype=out_dtype, device=x.device)
@@ -773,8 +781,7 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     else:
         w, b = _packed_train(mod, layers, cd)[:2] if train else _packed(mod, layers, cd)
     x2 = x.reshape(-1, x.shape[-1])
-    if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
+    x2 = _grid_rows(x2)
     out_dtype = x.dtype if out_dtype is None else out_dtype
     ywidth = Cdim // y_head * 16 if y_head else Cdim
     y = torch.empty(*x.shape[:-1], ywidth, dtype=out_dtype, device=x.device)
@@ -788,8 +795,7 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     r2 = None
     if res is not None:
         r2 = res.reshape(-1, Cdim)
-        if r2.stride(-1) != 1 or r2.stride(0) % 4 or r2.data_ptr() % 16:
-            r2 = r2.contiguous()
+        r2 = _grid_rows(r2)
         d.res_dtype, d.res_stride = _dtype_code(r2), r2.stride(0)
     if pair is not None:
         pair.append((w, b, y))
@@ -1044,8 +1050,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
         few = 0
         _, b, w_img, wt_img = _packed_train(mod, layers, cd)
     x2 = x
-    if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
+    x2 = _grid_rows(x2)
     dy2 = _rows2d(dy, Cdim)
     T = x2.shape[0]
     dev = x.device
@@ -1097,8 +1102,7 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None, int
     w, b, wt = _packed_few(mod_a, layers, cd, True)
     L2, Cdim, dev = len(layers), x.shape[-1], x.device
     x2 = x.reshape(-1, Cdim)
-    if x2.stride(-1) != 1 or x2.stride(0) % 4 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
+    x2 = _grid_rows(x2)
     yw = Cdim // y_head * 16 if y_head else Cdim
     da, db_ = _rows2d(dya, yw), _rows2d(dyb, yw)
     if da.dtype != db_.dtype:
@@ -1195,9 +1199,7 @@ def _rows2d(t, Cdim):
     t2 = t.reshape(-1, Cdim)
     if t2.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         t2 = t2.float()
-    if t2.stride(-1) != 1 or t2.stride(0) % 4 or t2.data_ptr() % 16:
-        t2 = t2.contiguous()
-    return t2
+    return _grid_rows(t2)
 
 
 def _backward_expand(ctx, dy, x, E):

@@ -142,8 +142,7 @@ def test_calls_that_keep_the_general_path(dev):
     wide = torch.randn(2, 300, 72, device=dev)
     off = torch.randn(2 * 300 * 64 + 1, device=dev)[1:].view(2, 300, 64)
     assert torch.equal(planned(m, wide[..., :64], used=False), general(m, wide[..., :64].contiguous()))
-    with pytest.raises(ValueError):
-        planned(m, off, used=False)
+    assert torch.equal(planned(m, off, used=False), general(m, off.clone()))
     seen = []
     h = m.att.register_forward_hook(lambda *a: seen.append(1))
     planned(m, x, used=False)

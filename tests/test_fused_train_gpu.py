@@ -853,3 +853,43 @@ def test_latents_may_change_between_a_blocks_passes(dev, H, again):
 
     for a, b in zip(grads(False), grads(True)):
         assert torch.equal(a, b)
+
+
+def _off_grid(t):
+    return torch.cat([t.new_zeros(1), t.detach().flatten()])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("kw", [{}, {"num_layers_ffn": 0, "ffn_mlp_ratio": 4.0}, {"qk_norm": True}])
+@pytest.mark.parametrize("N", [200, 20000])
+@pytest.mark.parametrize("xd", [torch.float32, torch.bfloat16])
+def test_rows_off_the_16_byte_grid(dev, xd, N, kw):
+    """Contiguous rows that begin off the grid, as a block's input and as the gradient of its output."""
+    torch.manual_seed(8)
+    blk = F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev)
+    x, gy = torch.randn(1, N, 64, device=dev).to(xd), torch.randn(1, N, 64, device=dev).to(xd)
+
+    def step(x, gy):
+        x = x.requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = blk(x)[0]
+            with torch.no_grad():
+                z = blk(x.detach())[0]
+        return [y.detach(), z, *torch.autograd.grad(y, [x, *blk.parameters()], gy)]
+
+    want = step(x.clone(), gy)
+    assert _off_grid(x).data_ptr() % 16 and _off_grid(x).is_contiguous()
+    for got in (step(x.clone(), _off_grid(gy)), step(_off_grid(x), gy)):
+        for a, b in zip(got, want):
+            assert rel(a, b) <= (1e-5 if xd is torch.float32 else 1e-2)
+    one = torch.randn(1, 1, 64, device=dev).to(xd).expand(1, N, 64)          # one row for all tokens
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(blk(one)[0], blk(one.contiguous())[0])
+
+
+@pytest.mark.parametrize("off", [False, True])
+def test_inference_with_narrow_rows_that_share_memory(dev, off):
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev).eval()
+    t = torch.randn(1, 303, device=dev)
+    x = _off_grid(torch.randn(1, 301, 3, device=dev)) if off else t.unfold(-1, 3, 1)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(m(x), m(x.clone(memory_format=torch.contiguous_format)))
