@@ -243,7 +243,8 @@ class _NarrowInFn(torch.autograd.Function):
 
 
 class _NarrowOutFn(torch.autograd.Function):
-    """x W^T + b of the last layer in the compute type, handed out in y_dtype."""
+    """x W^T + b of the last layer in the compute type, handed out in y_dtype.  The backward of a gradient penalty on this layer's weight
+    is differentiated again: then it is torch's products, with the launch's roundings."""
 
     @staticmethod
     def forward(ctx, x, w, b, cd, y_dtype):
@@ -254,18 +255,21 @@ class _NarrowOutFn(torch.autograd.Function):
             rc = _lib.load().flare_mlp_narrow_fwd(C.byref(d), _ptr(x2), _ptr(w), _ptr(b), None, _ptr(y), C.c_void_p(_stream_ptr(x.device)))
         _lib.check(rc, "flare_mlp_narrow_fwd")
         ctx.cd, ctx.y_dtype, ctx.has_bias, ctx.shape = cd, y_dtype, b is not None, x.shape
-        ctx.save_for_backward(x2, w)
+        ctx.save_for_backward(x, w)
         return y
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy):
-        x2, w = ctx.saved_tensors
-        x2, w = _wide(x2, ctx.cd), w.contiguous()
+        x, w = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            with torch.autocast("cuda", enabled=False):
+                g, xc, wc = (t.to(ctx.cd).float() for t in (dy.reshape(-1, dy.shape[-1]), x.reshape(-1, x.shape[-1]), w))
+                return (g @ wc).to(x.dtype).view(ctx.shape), g.t() @ xc, g.sum(0) if ctx.has_bias else None, None, None
+        x2, w = _wide(x, ctx.cd), w.contiguous()
         d = _narrow_desc(x2, w, ctx.cd, True, -1, ctx.y_dtype)
         dx = torch.empty_like(x2) if ctx.needs_input_grad[0] else None
         dw, db = _narrow_backward(d, x2, w, None, dy.contiguous(), dx, ctx.has_bias, dy.device)
-        return None if dx is None else dx.view(ctx.shape), dw, db, None, None
+        return None if dx is None else dx.to(x.dtype).view(ctx.shape), dw, db, None, None
 
 
 def _wide(t, cd):

@@ -893,3 +893,31 @@ def test_inference_with_narrow_rows_that_share_memory(dev, off):
     x = _off_grid(torch.randn(1, 301, 3, device=dev)) if off else t.unfold(-1, 3, 1)
     with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
         assert torch.equal(m(x), m(x.clone(memory_format=torch.contiguous_format)))
+
+
+def test_a_gradient_of_the_last_layer_can_be_differentiated(dev, monkeypatch):
+    """A penalty on the gradient of the model's last weight: its backward is torch's where it is differentiated again."""
+    torch.manual_seed(12)
+    m = F.FLAREModel(in_dim=3, out_dim=2, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev)
+    x = torch.randn(1, 900, 3, device=dev)
+    last = [l for l in m.modules() if isinstance(l, nn.Linear)]
+    last = [l for l in last if l.out_features == 2][0]
+
+    def run():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(x)
+        names = []
+        f = y.grad_fn
+        while f is not None and len(names) < 6:
+            names.append(type(f).__name__)
+            f = f.next_functions[0][0] if f.next_functions else None
+        gw, gb = torch.autograd.grad(y.float().square().mean(), [last.weight, last.bias], create_graph=True)
+        return any("NarrowOut" in n for n in names), [gw.detach(), gb.detach(), *torch.autograd.grad(gw.square().sum() + gb.square().sum(), [p for p in m.parameters()])]
+
+    hip, got = run()
+    assert hip
+    monkeypatch.setattr(fused, "_narrow_ok", lambda *a: False)
+    hip, want = run()
+    assert not hip
+    for a, b in zip(got, want):
+        assert rel(a, b) <= 3e-2
