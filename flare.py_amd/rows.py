@@ -24,12 +24,13 @@ from . import _lib, fused
 from .functional import _on_device, _ptr, _stream_ptr
 
 LONG_ROWS = 4096      # rows from which the modules' fp32 Linear layers slice their weight gradient (below, one product is as fast)
-# Elements of a row array from which these nodes pay, at the widths whose layer backward is one pass (_ONE_PASS): a layer enqueues less
-# than torch's own nodes, so they win from the smallest arrays on.  A sequence block's step, torch's nodes / these, us: 64 channels,
-# 8192 rows (0.5 Mi) 3047 / 2298, 16,384 rows 3066 / 2259, 98,304 rows (6 Mi) 3083 / 2273, 131,072 rows 3846 / 2341; 128 channels,
-# 8192 rows 2946 / 2122, 65,536 rows 3176 / 2173, 131,072 rows 5548 / 3869.  The other widths keep the separate passes, which enqueue
-# a little more than torch's nodes do: there the line is where a step waits for the kernels (6 Mi).  A step recorded into a graph has
-# no host to wait for, but follows the same rule: its replays give the results of the eager step bit for bit.
+# Elements of a row array from which these nodes are used, at the widths whose layer backward is one pass (_ONE_PASS).  A layer enqueues
+# less than torch's own nodes there, so they are faster at every size that was measured; a sequence block's step, torch's nodes / these,
+# us: 64 channels, 8192 rows (0.5 Mi) 3047 / 2298, 16,384 rows 3066 / 2259, 98,304 rows (6 Mi) 3083 / 2273, 131,072 rows 3846 / 2341; 128
+# channels, 8192 rows (1 Mi) 2946 / 2122, 65,536 rows 3176 / 2173, 131,072 rows 5548 / 3869.  The line is no break-even, then: it leaves
+# arrays of 0.5 Mi elements and less on the torch layers, where they always were.  The other widths keep the separate passes, which
+# enqueue a little more than torch's nodes do: there the line is 6 Mi, where a step waits for the kernels.  A step recorded into a graph
+# has no host to wait for, but follows the same rule: its replays give the results of the eager step bit for bit.
 MIN_ELEMS = 5 << 17
 _ONE_PASS = (64, 128)
 _WIDTHS = (32, 64, 128, 256)
@@ -58,7 +59,7 @@ def _param_ok(p):
 def _call_ok(x, long_rows):
     return (torch.is_grad_enabled() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype is torch.float32
             and x.shape[-1] in _WIDTHS and x.numel() // x.shape[-1] >= long_rows and not torch.is_autocast_enabled()
-            and x.numel() >= (MIN_ELEMS if x.shape[-1] in _ONE_PASS else 10 * MIN_ELEMS)
+            and x.numel() >= (MIN_ELEMS if x.shape[-1] in _ONE_PASS else MIN_ELEMS * 48 // 5)      # 6 Mi
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 

@@ -125,6 +125,14 @@ def test_small_arrays_keep_the_torch_layers_outside_a_capture(dev, monkeypatch):
     assert rows.chain_info(m, torch.empty(rows.MIN_ELEMS // 64, 64, device=dev)) is not None
 
 
+@pytest.mark.parametrize("C,elems", [(64, rows.MIN_ELEMS), (128, rows.MIN_ELEMS), (32, 6 << 20), (256, 6 << 20)])
+def test_the_sizes_from_which_the_row_passes_run(dev, monkeypatch, C, elems):
+    monkeypatch.undo()
+    m = ResidualMLP(C, C, C, num_layers=1, input_residual=True, output_residual=True).to(dev)
+    assert rows.chain_info(m, torch.empty(elems // C, C, device=dev)) is not None
+    assert rows.chain_info(m, torch.empty(elems // C - 1, C, device=dev)) is None
+
+
 def test_saved_tensors_may_come_back_in_another_memory_order(dev):
     """A saved-tensor hook owes the backward the values, not the strides."""
     torch.manual_seed(2)
