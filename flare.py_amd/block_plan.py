@@ -29,9 +29,10 @@ _X_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
 
 
 class _Plans(dict):
-    """shape -> plan, None for a shape met once, False where the general path serves it; all made from the module as `key` describes it.  held: aliases of the parameters whose addresses are in the
-    key.  pair: compute type -> joint packing of the k and v projections.  Never changed to another key: a block whose key differs gets
-    another object, so that a plan under way in one thread cannot join the plans that another thread began.
+    """shape -> plan, None for a shape met once, False where the general path serves it; all made from the module as `key` describes it.
+    held: the parameters' memory, whose addresses are in the key.  pair: compute type -> joint packing of the k and v projections.
+    Never changed to another key: a block whose key differs gets another object, so that a plan under way in one thread cannot join
+    the plans that another thread began.
     A copy of a module, and one read back from a file, begins without plans: they hold addresses."""
 
     def __init__(self, key=None, held=()):
@@ -49,9 +50,13 @@ class _Plan:
     __slots__ = ("desc", "ref", "scratch", "keep")
 
 
-def _parameters(block):
-    m = block._modules
-    return [t for mod in (m["att"], m["mlp"], m["norm1"], m["norm2"]) for t in mod.parameters()]
+def _held(block):
+    """The memory whose addresses are in the block's key (without a walk over the modules, which is slower than the rest of a plan)."""
+    m, a = block._modules, block._modules["att"]._modules
+    owners = [m["att"], m["norm1"], m["norm2"]]
+    for mod in (a["k_proj"], a["v_proj"], a["out_proj"], m["mlp"]):
+        owners += fused._layers_of(mod)[0]
+    return [fused.hold(t) for o in owners for t in o._parameters.values() if t is not None]
 
 
 def _key(block):
@@ -187,7 +192,7 @@ def forward(block, x):
         return None
     if plans.key != key:
         shapes = dict.fromkeys(plans)
-        plans = block.__dict__["_flare_plans"] = _Plans(key, [t.detach() for t in _parameters(block)])
+        plans = block.__dict__["_flare_plans"] = _Plans(key, _held(block))
         plans.update(shapes)
     plan = plans.get(shape)
     if plan is None:

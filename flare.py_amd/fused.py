@@ -394,9 +394,14 @@ def _pack_launch(Cdim, cd, tiles, dev, images, tiled=False, latents=None):
 
 def _chain_tiles(layers):
     """Tiles of a stack of Linears at most C x C, or None where the launch cannot read them."""
-    if not _readable(*(t for l in layers for t in (l.weight, l.bias))):
-        return None
-    return [(l.weight, 0, l.weight.stride(0), l.out_features, l.bias, 0) for l in layers]
+    tiles = []
+    for l in layers:
+        p = l._parameters                      # as in _param_key: a model's first forward comes here for every layer
+        w, b = (p["weight"], p["bias"]) if "weight" in p and "bias" in p else (l.weight, l.bias)
+        if not _readable(w, b):
+            return None
+        tiles.append((w, 0, w.stride(0), l.out_features, b, 0))
+    return tiles
 
 
 def _expand_tiles(f1, f2, E, Cdim):
@@ -440,7 +445,7 @@ class DropsOperands:
 
 
 class _Key(tuple):
-    """The key of something kept.  held: aliases of the tensors whose addresses it names, so that no other tensor gets one of them while
+    """The key of something kept.  held: the memory whose addresses it names (hold()), so that no other tensor gets one of them while
     it is compared.  A copy of a module, and one read back from a file, holds nothing: there the key fits no tensor."""
 
     def __deepcopy__(self, memo):
@@ -450,14 +455,16 @@ class _Key(tuple):
         return tuple, ()
 
 
-def _kept(key, layers, cache):
-    """key, whose last entry is _param_key(layers), as the first entry of a cache that replaces `cache`."""
-    kept, old = _Key(key), None if cache is None else cache[0]
-    kept.where = [e[::2] for e in key[-1]]
-    if type(old) is _Key and old.where == kept.where:      # held all the while: an address stands for the same memory
-        kept.held = old.held
-    else:
-        kept.held = [t.detach() for l in layers for t in (l.weight, l.bias) if t is not None]
+def hold(t):
+    """Something that keeps t's memory from being given to others, also when t is given other memory (a storage, of a plain tensor: a
+    sixth of a detach(), and a model's first forward holds hundreds)."""
+    return t.untyped_storage() if type(t) in (torch.Tensor, nn.Parameter) else t.detach()
+
+
+def _kept(key, layers):
+    """A cache's first entry for key, which names these layers' parameters."""
+    kept = _Key(key)
+    kept.held = [t.untyped_storage() if type(t) is nn.Parameter else hold(t) for l in layers for t in l._parameters.values() if t is not None]
     return kept
 
 
@@ -485,7 +492,7 @@ def _packed_few(mod, layers, cd, train):
     if tiles is None:
         return None
     w, b, _, wt = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, train, tiled=True)
-    mod.__dict__["_flare_packed_few"] = (_kept(key, layers, cache), w, b, wt)
+    mod.__dict__["_flare_packed_few"] = (_kept(key, layers), w, b, wt)
     return w, b, wt
 
 
@@ -498,12 +505,12 @@ def _packed(mod, layers, cd):
     tiles = _chain_tiles(layers)
     if tiles is not None:
         w, b, _, _ = _pack_launch(layers[0].in_features, cd, tiles, layers[0].weight.device, False)
-        mod._flare_packed = (_kept(key, layers, cache), w, b)
+        mod._flare_packed = (_kept(key, layers), w, b)
         return w, b
     w = torch.stack([l.weight.detach() for l in layers]).to(cd).contiguous()
     Cdim = w.shape[-1]
     b = torch.stack([l.bias.detach().float() if l.bias is not None else w.new_zeros(Cdim, dtype=torch.float32) for l in layers]).contiguous()
-    mod._flare_packed = (_kept(key, layers, cache), w, b)
+    mod._flare_packed = (_kept(key, layers), w, b)
     return w, b
 
 
@@ -519,7 +526,7 @@ def _packed_expand(mod, E, cd):
     tiles = _expand_tiles(f1, f2, E, Cdim)
     if tiles is not None:
         w, b, _, _ = _pack_launch(Cdim, cd, tiles, f1.weight.device, False)
-        mod._flare_packed = (_kept(key, (f1, f2), cache), w, b)
+        mod._flare_packed = (_kept(key, (f1, f2)), w, b)
         return w, b
     w1 = f1.weight.detach().to(cd).view(E, Cdim, Cdim)                       # [j][hidden row in chunk][in]
     w2 = f2.weight.detach().to(cd).view(Cdim, E, Cdim).permute(1, 0, 2)      # [j][out][hidden col in chunk]
@@ -529,7 +536,7 @@ def _packed_expand(mod, E, cd):
         b[0::2] = f1.bias.detach().float().view(E, Cdim)
     if f2.bias is not None:
         b[1] = f2.bias.detach().float()
-    mod._flare_packed = (_kept(key, (f1, f2), cache), w, b)
+    mod._flare_packed = (_kept(key, (f1, f2)), w, b)
     return w, b
 
 
@@ -558,7 +565,7 @@ def _packed_io(mod, layers, cd, Cdim, in_dim, out_dim):
         w_in[:, :in_dim] = layers[0].weight.detach().float()
         b_in = (layers[0].bias.detach().float().contiguous() if layers[0].bias is not None
                 else torch.zeros(Cdim, dtype=torch.float32, device=dev))
-    mod._flare_packed = (_kept(key, layers, cache), w, b, w_in, b_in)
+    mod._flare_packed = (_kept(key, layers), w, b, w_in, b_in)
     return w, b, w_in, b_in
 
 
@@ -706,7 +713,7 @@ def prepack(x, cd, *stacks, latents=None):
         t = _chain_tiles(layers)
         if t is None:
             return
-        stale.append((mods[0], _kept(key, layers, cache), at, at + len(t)))
+        stale.append((mods[0], _kept(key, layers), at, at + len(t)))
         tiles += t
         at += len(t)
     if len(stale) < 2 or at > _lib.MLP_PACK_MAX:
@@ -930,7 +937,7 @@ def _packed_train(mod, layers, cd):
     else:
         w, b = _packed(mod, layers, cd)
         w_img, wt_img = mlp_weight_images(w)
-    mod.__dict__["_flare_packed_train"] = (_kept(key, layers, cache), w, b, w_img, wt_img)
+    mod.__dict__["_flare_packed_train"] = (_kept(key, layers), w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
 
@@ -947,7 +954,7 @@ def _packed_train_expand(mod, E, cd):
     else:
         w, b = _packed_expand(mod, E, cd)
         w_img, wt_img = mlp_weight_images(w)
-    mod.__dict__["_flare_packed_train"] = (_kept(key, (f1, f2), cache), w, b, w_img, wt_img)
+    mod.__dict__["_flare_packed_train"] = (_kept(key, (f1, f2)), w, b, w_img, wt_img)
     return w, b, w_img, wt_img
 
 

@@ -182,7 +182,7 @@ class FLARE(fused.DropsOperands, nn.Module):
             if pad:
                 q = torch.nn.functional.pad(q, (0, pad))
             c = self._q_cache = (fused._Key(key), q.contiguous())
-            c[0].held = self.latent_q.detach()
+            c[0].held = fused.hold(self.latent_q)
         return c[1]
 
     def _fusable(self, x, return_scores):

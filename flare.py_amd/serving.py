@@ -24,6 +24,8 @@ import contextlib
 
 import torch
 
+from . import fused
+
 __all__ = ["GraphedForward"]
 
 
@@ -75,7 +77,7 @@ class GraphedForward:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 static_y = self.module(static_x)
-        return graph, static_x, static_y, self._param_key(), self._cached_operands(), [t.detach() for t in self._tensors()]
+        return graph, static_x, static_y, self._param_key(), self._cached_operands(), [fused.hold(t) for t in self._tensors()]
 
     def __call__(self, x: torch.Tensor):
         if x.device.type != "cuda":

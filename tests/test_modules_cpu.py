@@ -322,7 +322,7 @@ def test_block_plans_hold_the_memory_their_key_names(how):
     from flare_py_amd import block_plan
 
     m = FLAREBlock(channel_dim=128, num_heads=8, num_latents=32)
-    plans = block_plan._Plans(block_plan._key(m), [t.detach() for t in block_plan._parameters(m)])
+    plans = block_plan._Plans(block_plan._key(m), block_plan._held(m))
     for _ in range(12):
         w = torch.randn(128, 128)
         if how == "data":
