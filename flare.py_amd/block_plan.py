@@ -62,8 +62,8 @@ def _held(block):
 def _key(block):
     """Everything a plan is made from, or None for a block that the general path serves."""
     m = block._modules
-    att, mlp, n1, n2 = m["att"], m["mlp"], m["norm1"], m["norm2"]
-    if not rows._plain(att) or att.qk_norm or "latent_q" not in att._parameters:
+    att, mlp, n1, n2 = (m.get(name) for name in ("att", "mlp", "norm1", "norm2"))
+    if mlp is None or n1 is None or n2 is None or not rows._plain(att) or att.qk_norm or "latent_q" not in att._parameters:
         return None
     a = att._modules
     layers, key = [], [att.attn_scale, att.num_heads, att.num_latents, att.head_dim]

@@ -164,3 +164,18 @@ def test_calls_that_keep_the_general_path(dev):
         half(x.bfloat16())
         half(x.bfloat16())
     assert not half.__dict__.get("_flare_plans")
+
+
+@pytest.mark.parametrize("how", [None, nn.Identity()])
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_block_without_norms(dev, how, grad):
+    m = make(dev)
+    x = torch.randn(2, 300, 64, device=dev)
+    planned(m, x)
+    m.norm1 = m.norm2 = how
+    if grad:
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(x)[0].detach()
+        assert torch.equal(y, general(m, x))
+    else:
+        assert torch.equal(planned(m, x, used=False), general(m, x))
