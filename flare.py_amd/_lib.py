@@ -140,7 +140,6 @@ SYMBOLS = {
     "flare_mlp_wgrad_partials": (C.c_int, [C.POINTER(FlareMlpDesc), C.POINTER(C.c_int32)]),
     "flare_mlp_wgrad": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P]),
     "flare_mlp_wgrad_norm": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, C.c_int32, _P, _P]),
-    "flare_mlp_wgrad_norms": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P, _P]),
     "flare_mlp_wgrad_block": (C.c_int, [C.POINTER(FlareMlpDesc), _P, C.c_int64, _P, C.c_int64, _P, _P, _P, _P, _P, _P, C.c_int32, _P, _P,
                                         C.POINTER(FlareMixerDesc), _P, C.c_int32, C.c_int32, _P, _P]),
     "flare_mixer_bwd_dq_parts": (C.c_int, [C.POINTER(FlareMixerDesc), C.POINTER(_SZ), C.POINTER(C.c_int32)]),

@@ -1418,14 +1418,7 @@ int flare_mlp_wgrad(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_str
 int flare_mlp_wgrad_norm(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream)
 {
-    return flare_mlp_wgrad_norms(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, gb_part, nullptr, gb_rows, gb, nullptr, stream);
-}
-
-int flare_mlp_wgrad_norms(const FlareMlpDesc* d, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
-                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part, int32_t gb_rows,
-                          float* gb, float* gb2, void* stream)
-{
-    return flare_mlp_wgrad_block(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, gb_part, gb2_part, gb_rows, gb, gb2, nullptr,
+    return flare_mlp_wgrad_block(d, a_in, a_layer_stride, g_out, g_layer_stride, dw_part, db_part, dw, db, gb_part, nullptr, gb_rows, gb, nullptr, nullptr,
                                  nullptr, 0, 0, nullptr, stream);
 }
 

@@ -168,7 +168,8 @@ def _narrow_ok(layer, x, cd, act_module=None):
     """True where the narrow layer (and the activation behind it) can run as one HIP pass each way: plain modules, fp32 parameters, and
     for the first layer an input that asks for no gradient."""
     w, b = layer._parameters.get("weight"), layer._parameters.get("bias")
-    return (type(layer) is nn.Linear and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0 and _plain_module(layer)
+    return (type(layer) is nn.Linear and cd in (torch.bfloat16, torch.float16) and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter)
+            and x.numel() > 0 and _plain_module(layer)
             and (act_module is None or (type(act_module) in (nn.GELU, nn.SiLU) and _plain_module(act_module)))
             and ("bias" in layer._parameters) and all(type(t) in (torch.Tensor, nn.Parameter) and t.dtype is torch.float32 and t.is_cuda
                                                       and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (w, b) if t is not None)

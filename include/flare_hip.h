@@ -462,12 +462,9 @@ int flare_mlp_wgrad(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_
  * the launch that sums the others; gb NULL: nothing. */
 int flare_mlp_wgrad_norm(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, int32_t gb_rows, float* gb, void* stream);
-/* The same with the partial rows of two norms (a block's), gb_rows each; gb and gb2 may be NULL. */
-int flare_mlp_wgrad_norms(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
-                          float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part,
-                          int32_t gb_rows, float* gb, float* gb2, void* stream);
-/* The same with the gradient of latents that all batch elements share, from the partial results of flare_mixer_bwd (dq NULL: nothing):
- * dq [H,M,dq_cols] = mixer->scale times the sum of dq_part [B,H,dq_splits,M,D] over the splits and the batch, the first dq_cols columns. */
+/* The same with the partial rows of two norms (a block's; gb_rows each, gb and gb2 may be NULL) and with the gradient of latents that all
+ * batch elements share, from the partial results of flare_mixer_bwd (dq NULL: nothing): dq [H,M,dq_cols] = mixer->scale times the sum of
+ * dq_part [B,H,dq_splits,M,D] over the splits and the batch, the first dq_cols columns. */
 int flare_mlp_wgrad_block(const FlareMlpDesc* desc, const void* a_in, int64_t a_layer_stride, const void* g_out, int64_t g_layer_stride,
                           float* dw_part, float* db_part, float* dw, float* db, const float* gb_part, const float* gb2_part,
                           int32_t gb_rows, float* gb, float* gb2, const FlareMixerDesc* mixer, const float* dq_part, int32_t dq_splits,
