@@ -884,14 +884,15 @@ hipError_t scatter_launch(const MixerArgs& a, hipStream_t st)
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    // tokens per workgroup (multiple of 256): one full round of resident workgroups when the
-    // problem is large enough, so that every CU finishes at the same time
+    // tokens per workgroup (a multiple of 256: one 64-token pass for each of its four waves, or 128, see below): one full round of
+    // resident workgroups when the problem is large enough, so that every CU finishes at the same time
     const int slots = resident_slots(reinterpret_cast<const void*>(kern), lds);
     const int64_t per_bh = (slots + (int64_t)a.B * a.H - 1) / ((int64_t)a.B * a.H);   // workgroups per (b,h)
     int64_t tpw = (a.N + per_bh - 1) / per_bh;
     tpw = ((tpw + 255) / 256) * 256;
-    if (tpw < 256) tpw = 256;       // one 64-token pass per wave: a launch this small is bound by latency, not by the operand set-up
-    // Where that leaves half of the CUs without a workgroup, two waves of each work on twice as many: 8 heads, 4096 tokens were 128
+    if (tpw < 256) tpw = 256;       // a launch this small is bound by latency, not by the operand set-up
+    // Where that leaves half of the CUs without a workgroup, twice as many work on 128 tokens each, with two of their four waves (all
+    // four still set up the operands): 8 heads, 4096 tokens were 128
     // workgroups here, 128 in the gather and 88 of twelve waves in the backward's token pass.  All three spread, replayed training step of 8
     // blocks: 128 channels 1210 -> 1178 us, 64 channels 896 -> 873; 4 blocks of 64 channels, 2 x 1501 tokens 542 -> 521 us.
     if (tpw == 256 && (a.N + 255) / 256 * a.H * a.B <= device_cus() / 2) tpw = 128;

@@ -202,8 +202,9 @@ template <int C> hipError_t launch_c(int act, const RowsLayerArgs& a, unsigned g
 
 bool rows_layer_bwd_supported(int C) { return C == 64 || C == 128; }
 
-// Rows of a workgroup: an equal share of the compute units' (one workgroup each: the two buffers fill the LDS), a multiple of the
-// 16 rows a product takes, and not fewer than 64, below which writing the partial dW costs more than the rows.
+// Rows of a workgroup: an equal share of the compute units' (one workgroup each: its 16 waves hold 74 to 119 registers a lane, and two
+// workgroups would need 64; of the LDS the two buffers take 70 of 160 KB), a multiple of the 16 rows a product takes, and not fewer
+// than 64, below which writing the partial dW costs more than the rows.
 static int64_t rows_per_wg(int64_t T)
 {
     const int64_t share = (T + device_cus() - 1) / device_cus();
