@@ -42,7 +42,8 @@ _ACTS = {"gelu": 0, "silu": 1}
 
 def _structure_key(mod):
     """Identity of everything the structural caches are built from: the layers, the activation module and the flags
-    that set the masks.  Assigning a new submodule (a LoRA wrap, a re-initialisation by assignment) changes it.
+    that set the masks.  Assigning a new submodule (a LoRA wrap, a re-initialisation by assignment) changes it: modules compare by
+    identity, and a cache that keeps them, and not their ids, keeps another module from getting the id of one it was built from.
     Read from the module's own tables: every fused call asks several times, and attribute access on a Module goes
     through its __getattr__ for submodules."""
     if isinstance(mod, _SubChain):
@@ -53,15 +54,15 @@ def _structure_key(mod):
         return (type(mod),)
     m = d["_modules"]
     if nl == -1:
-        return (-1, id(m["fc"]), bool(d["residual"]))
+        return (-1, m["fc"], bool(d["residual"]))
     act = m["act"] if "act" in m else d.get("act")
-    return (nl, id(m["fc1"]), tuple(map(id, m["fcs"]._modules.values())), id(m["fc2"]), id(act),
+    return (nl, m["fc1"], (*m["fcs"]._modules.values(),), m["fc2"], act,
             getattr(act, "approximate", None), bool(d["input_residual"]), bool(d["output_residual"]))
 
 
 def _layers_of(mod):
     """(linear layers, act_mask, add_mask, act code) of a ResidualMLP or nn.Linear, or None.  The answer is kept on
-    the module together with the identities of the submodules it was read from, and rebuilt when one of them is
+    the module together with the submodules it was read from, and rebuilt when one of them is
     replaced."""
     key = _structure_key(mod)
     cached = mod.__dict__.get("_flare_layers")

@@ -3,6 +3,9 @@ tests/pdebench/test_pdebench_model_contracts.py:23-132 (smoke, determinism, stat
 shape matrix).  On the CPU only the diagnostic return_scores=True branch (plain torch) can run;
 the mixer branch must refuse, loudly.  The same four contracts run on the HIP path in
 tests/test_modules_gpu.py."""
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -360,3 +363,22 @@ def test_rows_to_be_filled_up_must_match(monkeypatch):
     for v in (torch.randn(1, 2, 24, 8), torch.randn(1, 2, 40, 4), torch.randn(1, 2, 40, 8).bfloat16()):
         with pytest.raises(ValueError, match="match"):
             functional._pad_rows((k, v), 16)
+
+
+def test_a_submodule_replaced_twice_is_seen():
+    """The second one's id may be that of the module before."""
+    from torch import nn
+
+    from flare_py_amd import fused
+
+    m = ResidualMLP(64, 64, 64, num_layers=2, act="silu", input_residual=True, output_residual=True)
+    for n in range(1, 6):
+        m.act = nn.SiLU()
+        assert fused._layers_of(m)[3] == 1
+        for _ in range(n):
+            m.act = nn.ReLU()
+        assert fused._layers_of(m) is None, n
+    c = copy.deepcopy(m)
+    c.act = nn.SiLU()
+    assert fused._layers_of(c)[0][0] is c.fc1 and fused._layers_of(m) is None
+    assert fused._layers_of(pickle.loads(pickle.dumps(c)))[0][0] is not c.fc1
