@@ -79,7 +79,7 @@ def _key(block):
             t = p.get(name)
             key.append(None if t is None else (t.data_ptr(), t._version))
         key += (type(n), getattr(n, "eps", None))
-    if any("weight" not in l._parameters for l in layers):      # a parametrised weight is another tensor at every access
+    if any("weight" not in l._parameters or "bias" not in l._parameters for l in layers):      # parametrised: another tensor at every access
         return None
     q = att._parameters["latent_q"]
     key.append((q.data_ptr(), q._version))

@@ -179,3 +179,12 @@ def test_a_block_without_norms(dev, how, grad):
         assert torch.equal(y, general(m, x))
     else:
         assert torch.equal(planned(m, x, used=False), general(m, x))
+
+
+@pytest.mark.parametrize("name", ["weight", "bias"])
+def test_a_parametrised_layer_keeps_the_general_path(dev, name):
+    """Its weight or bias is another tensor at every access: a plan could serve one call only."""
+    m = make(dev)
+    torch.nn.utils.parametrize.register_parametrization(m.mlp.fc1, name, nn.Identity())
+    x = torch.randn(2, 300, 64, device=dev)
+    assert torch.equal(planned(m, x, used=False), general(m, x))
