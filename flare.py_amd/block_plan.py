@@ -13,6 +13,8 @@ later call compares what the block's plans were made from: the modules' structur
 the mixer's scale.  Where any of it changed, all plans of the block go, whatever their shape.  The parameters' memory is held as long as
 plans name its address: another tensor put in a parameter's place then always lies elsewhere.  Calls a plan does not cover (hooks on the
 attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer pads itself) run the general path.
+No plan is made while a graph is recorded: the packing of k and v would be recorded too, and a call before the first replay would read
+weights that nothing has written yet.
 """
 from __future__ import annotations
 
@@ -190,11 +192,13 @@ def forward(block, x):
     key = _key(block)
     if key is None:
         return None
+    plan = plans.get(shape) if plans.key == key else None
+    if plan is None and torch.cuda.is_current_stream_capturing():
+        return None
     if plans.key != key:
         shapes = dict.fromkeys(plans)
         plans = block.__dict__["_flare_plans"] = _Plans(key, _held(block))
         plans.update(shapes)
-    plan = plans.get(shape)
     if plan is None:
         plan = plans[shape] = _build(block, x, cd, plans) or False
     if not plan:

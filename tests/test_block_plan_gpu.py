@@ -188,3 +188,27 @@ def test_a_parametrised_layer_keeps_the_general_path(dev, name):
     torch.nn.utils.parametrize.register_parametrization(m.mlp.fc1, name, nn.Identity())
     x = torch.randn(2, 300, 64, device=dev)
     assert torch.equal(planned(m, x, used=False), general(m, x))
+
+
+@pytest.mark.parametrize("warm_ups", [1, 2, 3])
+@pytest.mark.parametrize("N", [300, 20000])
+def test_a_recorded_forward_leaves_eager_calls_their_weights(dev, N, warm_ups):
+    """What a recording packs is written by its replays alone."""
+    m = make(dev)
+    x = torch.randn(1, N, 64, device=dev)
+    want = general(make(dev), x)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(warm_ups):
+                m(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = m(x)[0]
+        assert torch.equal(m(x)[0], want) and torch.equal(m(x)[0], want)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            assert torch.equal(y, want) and torch.equal(m(x)[0], want)
