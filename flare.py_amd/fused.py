@@ -438,12 +438,16 @@ def _param_key(layers):
 
 
 class DropsOperands:
-    """For modules: to(), cpu(), half() and their like drop what is kept of the parameters, which they may replace."""
+    """For modules: to(), cpu(), half() and their like drop what is kept of parameters that they replace.  Where they leave all of them in
+    place the packed copies stay: a graph that the caller has recorded may read them."""
 
     def _apply(self, fn, recurse=True):
-        for m in self.modules():
-            drop_operands(m)
-        return super()._apply(fn, recurse)
+        before = [(t.data_ptr(), t.dtype) for t in self.parameters()]
+        out = super()._apply(fn, recurse)
+        if before != [(t.data_ptr(), t.dtype) for t in self.parameters()]:
+            for m in self.modules():
+                drop_operands(m)
+        return out
 
 
 class _Key(tuple):

@@ -573,3 +573,22 @@ def test_a_parametrised_weight_is_packed_at_every_call(dev, grad):
             assert torch.equal(a, b)
         with torch.no_grad():
             blk.mlp.fc1.parametrizations.weight.original0.mul_(1.25)
+
+
+def test_a_move_that_moves_nothing_keeps_the_packed_weights(dev):
+    """A graph recorded by hand reads them."""
+    m = F.FLAREModel(in_dim=3, out_dim=1, channel_dim=64, num_blocks=1, num_heads=4, num_latents=32).to(dev).eval()
+    x = torch.randn(1, 300, 3, device=dev)
+
+    def kept():
+        return {(n, k): v for n, s in m.named_modules() for k, v in s.__dict__.items() if k.startswith(("_flare_packed", "_flare_plans", "_q_cache"))}
+
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        for _ in range(3):
+            m(x)
+    before = kept()
+    m.to(dev).cuda().float()
+    after = kept()
+    assert len(before) > 4 and before.keys() == after.keys() and all(before[k] is after[k] for k in before)
+    m.half()
+    assert not kept()
