@@ -437,15 +437,22 @@ def _param_key(layers):
     return tuple(key)
 
 
+_KEPT = frozenset(("_flare_plans", "_q_cache", "_flare_subchain", "_flare_packed", "_flare_packed_train", "_flare_packed_few"))      # see drop_operands
+
+
 class DropsOperands:
     """For modules: to(), cpu(), half() and their like drop what is kept of parameters that they replace.  Where they leave all of them in
     place the packed copies stay: a graph that the caller has recorded may read them."""
 
     def _apply(self, fn, recurse=True):
+        # its own and, for plain layers among them, its children's: every module that keeps more is of this kind itself
+        kept = [m for m in (self, *self._modules.values()) if m is not None and not _KEPT.isdisjoint(m.__dict__)]
+        if not kept:
+            return super()._apply(fn, recurse)
         before = [(t.data_ptr(), t.dtype) for t in self.parameters()]
         out = super()._apply(fn, recurse)
         if before != [(t.data_ptr(), t.dtype) for t in self.parameters()]:
-            for m in self.modules():
+            for m in kept:
                 drop_operands(m)
         return out
 
