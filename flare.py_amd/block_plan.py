@@ -8,8 +8,10 @@ projections and the block's end are one launch each.  On small point clouds enqu
 descriptors, the packed 16-bit weights the modules hold anyway, the layout of one scratch allocation -- and hands the rest to
 flare_block_fwd.  Nothing about an input is kept.
 
-A plan is made when a block meets a shape for the second time; a shape's first forward runs the general path of modules.py.  Every
-later call compares what the block's plans were made from: the modules' structure, every parameter's address and version, the norms' eps,
+A block's first forward runs the general path of modules.py, which packs the weights; from then on a plan is made where a shape is
+new.  Making one takes about as long as the general path's own decisions, so that a loop over meshes of ever new sizes is no
+slower for it (us a forward of the 8 blocks, 1000 to 5000 points, general path / plans: a new size every time 1082 / 986, the next
+forward of that size 1082 / 400, nine sizes in turn 1036 / 325, weights changed before every forward 2290 / 2100).  Every call compares what the block's plans were made from: the modules' structure, every parameter's address and version, the norms' eps,
 the mixer's scale.  Where any of it changed, all plans of the block go, whatever their shape.  The parameters' memory is held as long as
 plans name its address: another tensor put in a parameter's place then always lies elsewhere.  Calls a plan does not cover (hooks on the
 attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer pads itself) run the general path.
@@ -25,13 +27,13 @@ from torch import nn
 
 from . import _lib, functional, fused, rows
 
-_MAX_SHAPES = 8           # plans kept per block; a plan holds a descriptor of 0.5 KB and references to packed weights, which all plans
-                          # of a block share (one packing for few tokens, one for many)
+_MAX_SHAPES = 32          # plans kept per block, the newest; a plan holds a descriptor of 0.5 KB and references to packed weights, which all
+                          # plans of a block share (one packing for few tokens, one for many)
 _X_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
 
 
 class _Plans(dict):
-    """shape -> plan, None for a shape met once, False where the general path serves it; all made from the module as `key` describes it.
+    """shape -> plan, or False where the general path serves it; all made from the module as `key` describes it (None before the first).
     held: the parameters' memory, whose addresses are in the key.  pair: compute type -> joint packing of the k and v projections.
     Never changed to another key: a block whose key differs gets another object, so that a plan under way in one thread cannot join
     the plans that another thread began.
@@ -52,13 +54,13 @@ class _Plan:
     __slots__ = ("desc", "ref", "scratch", "keep")
 
 
-def _held(block):
-    """The memory whose addresses are in the block's key (without a walk over the modules, which is slower than the rest of a plan)."""
+def _parameters(block):
+    """The parameters whose addresses are in the block's key (without a walk over the modules, which is slower than the rest of a plan)."""
     m, a = block._modules, block._modules["att"]._modules
     owners = [m["att"], m["norm1"], m["norm2"]]
     for mod in (a["k_proj"], a["v_proj"], a["out_proj"], m["mlp"]):
         owners += fused._layers_of(mod)[0]
-    return [fused.hold(t) for o in owners for t in o._parameters.values() if t is not None]
+    return [t for o in owners for t in o._parameters.values() if t is not None]
 
 
 def _key(block):
@@ -131,7 +133,8 @@ def _build(block, x, cd, plans):
         return None
     if M % 32 or D not in (4, 8, 16, 32, 64) or any(type(n) not in (nn.LayerNorm, nn.RMSNorm) for n in (block.norm1, block.norm2)):
         return None
-    if any(p.device != x.device for mod in (att, mlp, block.norm1, block.norm2) for p in mod.parameters()):
+    dev = x.device
+    if any(p.device != dev for p in _parameters(block)):
         return None
     head = D if D in (4, 8) else 0                        # narrow heads: k, v and the mixer's rows padded to 16 columns
     Dp, T = (16 if head else D), B * N
@@ -181,25 +184,21 @@ def forward(block, x):
         return None
     plans = block.__dict__.get("_flare_plans")
     if plans is None:
-        plans = block.__dict__["_flare_plans"] = _Plans()
-    dev = x.device
-    shape = (x.shape, x.dtype, cd, dev.index, functional._extra_mixer_flags)
-    if shape not in plans:
-        if len(plans) >= _MAX_SHAPES:
-            plans.clear()
-        plans[shape] = None
+        block.__dict__["_flare_plans"] = _Plans()
         return None
     key = _key(block)
     if key is None:
         return None
+    dev = x.device
+    shape = (x.shape, x.dtype, cd, dev.index, functional._extra_mixer_flags)
     plan = plans.get(shape) if plans.key == key else None
-    if plan is None and torch.cuda.is_current_stream_capturing():
-        return None
-    if plans.key != key:
-        shapes = dict.fromkeys(plans)
-        plans = block.__dict__["_flare_plans"] = _Plans(key, _held(block))
-        plans.update(shapes)
     if plan is None:
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        if plans.key != key:
+            plans = block.__dict__["_flare_plans"] = _Plans(key, [fused.hold(t) for t in _parameters(block)])
+        for oldest in list(plans)[:len(plans) + 1 - _MAX_SHAPES]:
+            plans.pop(oldest, None)
         plan = plans[shape] = _build(block, x, cd, plans) or False
     if not plan:
         return None

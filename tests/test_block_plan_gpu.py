@@ -32,7 +32,7 @@ def general(m, x, cd=torch.bfloat16, **kw):
 
 
 def planned(m, x, cd=torch.bfloat16, used=True):
-    """The second call with a shape is the first one through a plan."""
+    """The second call of a block is the first one through a plan."""
     calls, lib = [], _lib.load()
     real = lib.flare_block_fwd
     lib.flare_block_fwd = lambda *a: (calls.append(1), real(*a))[1]
@@ -134,6 +134,25 @@ def test_replaced_weights_reach_the_plans_of_every_shape(dev, how, what):
         assert torch.equal(planned(m, a), want[i + 2][0]), i
     m.cpu()
     assert "_flare_plans" not in m.__dict__
+
+
+def test_shapes_that_a_block_meets_once(dev):
+    """Each of them takes a plan, right away and after others took its place, and equals the general path."""
+    m = make(dev)
+    xs = [torch.randn(1, 100 + 7 * n, 64, device=dev) for n in range(block_plan._MAX_SHAPES + 3)] + [torch.randn(1, 13000, 64, device=dev)]
+    planned(m, xs[0])
+    calls, lib = [], _lib.load()
+    real = lib.flare_block_fwd
+    lib.flare_block_fwd = lambda *a: (calls.append(1), real(*a))[1]
+    try:
+        for x in (*xs, *xs):
+            n = len(calls)
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+                y = m(x)[0]
+            assert len(calls) == n + 1 and len(m._flare_plans) <= block_plan._MAX_SHAPES
+            assert torch.equal(y, general(m, x))
+    finally:
+        lib.flare_block_fwd = real
 
 
 def test_calls_that_keep_the_general_path(dev):

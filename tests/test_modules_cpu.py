@@ -322,10 +322,10 @@ def test_block_plans_hold_the_memory_their_key_names(how):
     """Replaced weights never get the address of one that plans were made from, so their key always differs."""
     from torch import nn
 
-    from flare_py_amd import block_plan
+    from flare_py_amd import block_plan, fused
 
     m = FLAREBlock(channel_dim=128, num_heads=8, num_latents=32)
-    plans = block_plan._Plans(block_plan._key(m), block_plan._held(m))
+    plans = block_plan._Plans(block_plan._key(m), [fused.hold(t) for t in block_plan._parameters(m)])
     for _ in range(12):
         w = torch.randn(128, 128)
         if how == "data":
