@@ -4,14 +4,16 @@ Under autocast and without gradients the block is seven launches (norm + k proje
 output projection + residual, norm + feed-forward + residual; pdebench/models/flare.py:107-215), five on few tokens, where the two
 projections and the block's end are one launch each.  On small point clouds enqueueing them from Python is what it costs: calls of
 20 to 30 us each, most of it spent deciding again what the last call decided.  An 8-block model of 64 channels on 3973 points:
-1070 us a forward, 340 us through the plans (0.3 ms of kernels).  `forward` keeps what depends on the module and the shape only --
+1070 us a forward, 340 us through the plans (0.24 ms of kernels).  `forward` keeps what depends on the module and the shape only --
 descriptors, the packed 16-bit weights the modules hold anyway, the layout of one scratch allocation -- and hands the rest to
 flare_block_fwd.  Nothing about an input is kept.
 
 A block's first forward runs the general path of modules.py, which packs the weights; from then on a plan is made where a shape is
 new.  Making one takes about as long as the general path's own decisions, so that a loop over meshes of ever new sizes is no
 slower for it (us a forward of the 8 blocks, 1000 to 5000 points, general path / plans: a new size every time 1082 / 986, the next
-forward of that size 1082 / 400, nine sizes in turn 1036 / 325, weights changed before every forward 2290 / 2100).  Every call compares what the block's plans were made from: the modules' structure, every parameter's address and version, the norms' eps,
+forward of that size 1082 / 400, nine sizes in turn 1036 / 325, weights changed before every forward 2290 / 2100).
+
+Every call compares what the block's plans were made from: the modules' structure, every parameter's address and version, the norms' eps,
 the mixer's scale.  Where any of it changed, all plans of the block go, whatever their shape.  The parameters' memory is held as long as
 plans name its address: another tensor put in a parameter's place then always lies elsewhere.  Calls a plan does not cover (hooks on the
 attention module, gradients, rows off the 16-byte grid, head dims or latent counts that the mixer pads itself) run the general path.
