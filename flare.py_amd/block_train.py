@@ -68,18 +68,19 @@ class _BlockFn(torch.autograd.Function):
             if not fused.prepack(x, cd, (k, v), (out,), (mlp,), latents=None if q16 is None else (q, q16)) or q16 is None:
                 q16 = torch.nn.functional.pad(q.to(cd), (0, Dp - D)) if head else q.to(cd)
             n = (len(layers) - 1 - len(fused._layers_of(mlp)[0])) // 2
-            w, b = fused._packed_few(k, layers[:2 * n], cd, True)[:2]
+            ctx.operands = fused._packed_few(k, layers[:2 * n], cd, True), fused.tail_operands(out, mlp, cd)
+            w, b = ctx.operands[0][:2]
             pair = []
             k2 = fused._fused_mlp_fwd(x, k, cd, norm=block.norm1, out_dtype=cd, y_head=head, train=True, operands=(w[:n], b[:n]), pair=pair)
             v2 = fused._fused_mlp_fwd(x, v, cd, norm=block.norm1, out_dtype=cd, y_head=head, train=True, operands=(w[n:], b[n:]), pair=pair)
             kh, vh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2))
             y, z, lse_lat, lse_tok = functional._mixer_forward(q16, kh, vh, float(att.attn_scale), None, 0, False, True, True)
             y2 = y.permute(0, 2, 1, 3).reshape(B, N, H * Dp)
-            x1, o = fused.tail_forward(y2, out, x, mlp, cd, block.norm2, head)
+            x1, o = fused.tail_forward(y2, out, x, mlp, cd, block.norm2, head, ctx.operands[1])
         ctx.block, ctx.cd, ctx.layers, ctx.n, ctx.head, ctx.scale = block, cd, layers, n, head, float(att.attn_scale)
         ctx.dims, ctx.norms = (B, N, H, Dp, D), (block.norm1, block.norm2)
-        # the backward reads the parameters' packed copies again: as with a saved tensor, changing one in place before is an error
-        # (of the latents it reads the saved copy, which stays as it was)
+        # the backward reads the packed copies that the forward read, also where the block has other parameters by then; as with a saved
+        # tensor, changing one in place before is an error (of the latents it reads the saved copy, which stays as it was)
         ctx.q_like, ctx.params = latent_q, (g1, b1, g2, b2, *wb)
         ctx.versions = tuple(None if t is None else t._version for t in ctx.params)
         ctx.save_for_backward(x, k2, v2, q16, y2, z, lse_lat, lse_tok, x1)
@@ -98,12 +99,13 @@ class _BlockFn(torch.autograd.Function):
         norm1, norm2 = ctx.norms
         a_in, g_out = torch.empty(2, L, T, Cdim, dtype=cd, device=dev)
         m = 2 * n
-        dx1, dy, gb2 = fused.tail_backward(y2, out, x1, mlp, cd, norm2, head, do, a_in[m:], g_out[m:])
+        vectors = ctx.params
+        dx1, dy, gb2 = fused.tail_backward(y2, out, x1, mlp, cd, norm2, head, do, a_in[m:], g_out[m:], ctx.operands[1], vectors[2:4])
         kh, vh, yh, gyh = (t.view(B, N, H, Dp).permute(0, 2, 1, 3) for t in (k2, v2, y2, dy))
         latents, dk, dv = functional._mixer_hip_grad(q16, kh, vh, yh, z, lse_lat, lse_tok, ctx.scale, gyh, dq_parts=True)
         dq = torch.empty(H, q16.shape[1], D, dtype=torch.float32, device=dev)
         dk, dv = (t.permute(0, 2, 1, 3).reshape(T, H * Dp) for t in (dk, dv))
-        dx, gb1 = fused._pair_backward(k, v, cd, norm1, x, dk, dv, head, dx1, into=(a_in[:m], g_out[:m]))
+        dx, gb1 = fused._pair_backward(k, v, cd, norm1, x, dk, dv, ctx.operands[0], vectors[:2], head, dx1, into=(a_in[:m], g_out[:m]))
         gs1, gs2 = (None if g is None else torch.empty(2, Cdim, dtype=torch.float32, device=dev) for g in (gb1, gb2))
         d = _lib.FlareMlpDesc()
         d.w_dtype = functional._DTYPES[cd]

@@ -618,19 +618,20 @@ def _vec32(p):
     return v if v.data_ptr() % 16 == 0 else v.clone()
 
 
-def _norm_args(d, norm, x, Cdim):
-    """Fill the descriptor's norm fields; returns (gamma, beta) fp32 tensors or None."""
+def _norm_args(d, norm, x, Cdim, vectors=None):
+    """Fill the descriptor's norm fields; returns (gamma, beta) fp32 tensors or None.  vectors: (weight, bias) in place of the norm's own."""
     gamma = beta = None
     if norm is not None and not isinstance(norm, nn.Identity):
         if isinstance(norm, nn.LayerNorm):
             d.norm, d.eps = 1, float(norm.eps)
-            beta = None if norm.bias is None else _vec32(norm.bias)
+            bias = norm.bias if vectors is None else vectors[1]
+            beta = None if bias is None else _vec32(bias)
         elif isinstance(norm, nn.RMSNorm):
             d.norm = 2
             d.eps = float(norm.eps) if norm.eps is not None else float(torch.finfo(x.dtype).eps)
         else:
             raise TypeError(f"unsupported norm {type(norm).__name__}")
-        weight = norm.weight
+        weight = norm.weight if vectors is None else vectors[0]
         gamma = _vec32(weight) if weight is not None else torch.ones(Cdim, dtype=torch.float32, device=x.device)
     return gamma, beta
 
@@ -781,8 +782,8 @@ def _forward_plan(mod):
 
 
 def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_head=0, train=False, operands=None, pair=None):
-    """pair: a list that the two chains of a few-token pair pass through (operands: their halves of one packing): the first one's
-    launch is left to the second."""
+    """operands: the packed weights to read in place of the module's.  pair: a list that the two chains of a few-token pair pass through
+    (operands: their halves of one packing): the first one's launch is left to the second."""
     lib = _lib.load()
     info, io, Cdim, E = _forward_plan(mod)
     layers, act_mask, add_mask, act = info
@@ -794,16 +795,17 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     few = not E and bool(_few(x.numel() // x.shape[-1], Cdim, len(layers)))
     if operands is None and few:
         operands = _packed_few(mod, layers, cd, train)
-        few = operands is not None
-    if few:
+    few = few and operands is not None and len(operands) < 4
+    if E and (x_head or y_head):
+        raise ValueError("head-padded rows are not available for the expanding two-layer MLP")
+    if operands is not None:
         w, b = operands[:2]
     elif E:
-        if x_head or y_head:
-            raise ValueError("head-padded rows are not available for the expanding two-layer MLP")
         w, b = _packed_train_expand(mod, E, cd)[:2] if train else _packed_expand(mod, E, cd)
-        act_mask, add_mask = 1, 0
     else:
         w, b = _packed_train(mod, layers, cd)[:2] if train else _packed(mod, layers, cd)
+    if E:
+        act_mask, add_mask = 1, 0
     x2 = x.reshape(-1, x.shape[-1])
     x2 = _grid_rows(x2)
     out_dtype = x.dtype if out_dtype is None else out_dtype
@@ -837,7 +839,17 @@ def _fused_mlp_fwd(x, mod, cd, norm=None, res=None, out_dtype=None, x_head=0, y_
     return y
 
 
-def _tail_descs(y2, out, x, mlp, cd, norm, head):
+def _train_operands(x, mod, cd):
+    """What a stack's launches read in a training step, forward and backward: the result of _packed_few (three), or of _packed_train or
+    _packed_train_expand (four)."""
+    info, _, Cdim, E = _forward_plan(mod)
+    if E:
+        return _packed_train_expand(mod, E, cd)
+    packed = _packed_few(mod, info[0], cd, True) if _few(x.numel() // x.shape[-1], Cdim, len(info[0])) else None
+    return _packed_train(mod, info[0], cd) if packed is None else packed
+
+
+def _tail_descs(y2, out, x, mlp, cd, norm, head, vectors=None):
     """(Linear, chain) descriptors of a block's end, the norm's vectors."""
     Cdim, (layers, act_mask, add_mask, act) = out.in_features, _layers_of(mlp)
     f, s = _lib.FlareMlpDesc(), _lib.FlareMlpDesc()
@@ -850,17 +862,21 @@ def _tail_descs(y2, out, x, mlp, cd, norm, head):
     s.act, s.act_mask, s.add_mask = act, act_mask, add_mask
     f.x_stride = y2.shape[1]
     f.y_stride = f.res_stride = s.x_stride = s.y_stride = s.res_stride = Cdim
-    return (f, s, *_norm_args(s, norm, x, Cdim))
+    return (f, s, *_norm_args(s, norm, x, Cdim, vectors))
 
 
-def tail_forward(y2, out, x, mlp, cd, norm, head):
+def tail_operands(out, mlp, cd):
+    """What both launches of a block's end read: the packed weights of out and of mlp."""
+    return _packed_few(out, [out], cd, True), _packed_few(mlp, _layers_of(mlp)[0], cd, True)
+
+
+def tail_forward(y2, out, x, mlp, cd, norm, head, operands=None):
     """x1 = x + out(y2), x1 + mlp(norm(x1)) in one launch (few tokens; contiguous rows, y2 in the compute type with heads of `head`
-    channels padded): (x1, result)."""
+    channels padded): (x1, result).  operands: tail_operands() of these modules."""
     y2 = y2.reshape(-1, y2.shape[-1])
     f, s, gamma, beta = _tail_descs(y2, out, x, mlp, cd, norm, head)
     f.flags, s.flags = f.flags | _lib.MLP_W_TILED, _lib.MLP_W_TILED
-    w1, b1 = _packed_few(out, [out], cd, True)[:2]
-    w2, b2 = _packed_few(mlp, _layers_of(mlp)[0], cd, True)[:2]
+    (w1, b1, _), (w2, b2, _) = tail_operands(out, mlp, cd) if operands is None else operands
     x1, y = torch.empty_like(x), torch.empty_like(x)
     with _on_device(x.device):
         rc = _lib.load().flare_mlp_few_tail_fwd(C.byref(f), C.byref(s), _ptr(y2), _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(gamma),
@@ -869,15 +885,14 @@ def tail_forward(y2, out, x, mlp, cd, norm, head):
     return x1, y
 
 
-def tail_backward(y2, out, x1, mlp, cd, norm, head, dy, a_in, g_out):
+def tail_backward(y2, out, x1, mlp, cd, norm, head, dy, a_in, g_out, operands=None, vectors=None):
     """Backward of tail_forward in one launch: (dx1 [T,C], dy2, the norm's partial rows); a_in, g_out take the rows for the weight
-    gradients of out and of mlp's layers, in that order."""
+    gradients of out and of mlp's layers, in that order.  operands, vectors: what the forward read, of the stacks and of the norm."""
     Cdim = out.in_features
     x2, y2, dy = x1.reshape(-1, Cdim), y2.reshape(-1, y2.shape[-1]), _rows2d(dy, Cdim)
-    f, s, gamma, beta = _tail_descs(y2, out, x1, mlp, cd, norm, head)
+    f, s, gamma, beta = _tail_descs(y2, out, x1, mlp, cd, norm, head, vectors)
     s.y_dtype, s.y_stride = _dtype_code(dy), dy.stride(0)
-    wt1 = _packed_few(out, [out], cd, True)[2]
-    w2, b2, wt2 = _packed_few(mlp, _layers_of(mlp)[0], cd, True)
+    (_, _, wt1), (w2, b2, wt2) = tail_operands(out, mlp, cd) if operands is None else operands
     dx1, dy2 = torch.empty_like(x2), torch.empty_like(y2)
     gb = torch.empty(_few(x2.shape[0], Cdim, s.L), 2, Cdim, dtype=torch.float32, device=x1.device)
     with _on_device(x1.device):
@@ -1010,15 +1025,16 @@ class _FusedMlpFn(torch.autograd.Function):
     def forward(ctx, mod, cd, norm, fmt, x, res, gamma, beta, *wb):
         out_dtype, x_head = fmt
         with torch.no_grad():
-            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype, x_head=x_head, train=True)
+            ctx.operands = _train_operands(x, mod, cd)
+            y = _fused_mlp_fwd(x, mod, cd, norm=norm, res=res, out_dtype=out_dtype, x_head=x_head, train=True, operands=ctx.operands)
         ctx.mod, ctx.cd, ctx.norm, ctx.x_head = mod, cd, norm, x_head
         # res and x one tensor: dy is added to dx inside the kernel.  (Two tensors over the same memory are not
         # enough: one of them may be detached, and then its path carries no gradient.)
         ctx.res_is_x = res is x
         ctx.has_res = res is not None
         ctx.n_wb = len(wb)
-        # the backward reads the parameters again (its packed copies are keyed by their versions) instead of saving
-        # them: as with a saved tensor, changing one in place between forward and backward is an error
+        # the backward reads the packed copies that the forward read, also where the module has other parameters by then (as after
+        # torch.func.functional_call); as with a saved tensor, changing a parameter in place in between is an error
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)
         ctx.save_for_backward(x)
@@ -1033,7 +1049,7 @@ class _FusedMlpFn(torch.autograd.Function):
         mod, cd, norm = ctx.mod, ctx.cd, ctx.norm
         if not ctx.x_head and _expand_factor(mod, x.shape[-1]):
             return _backward_expand(ctx, dy, x, _expand_factor(mod, x.shape[-1]))
-        dx, gsum, dW, db, layers = _chain_backward(mod, cd, norm, x, dy, ctx.res_is_x, x_head=ctx.x_head)
+        dx, gsum, dW, db, layers = _chain_backward(mod, cd, norm, x, dy, ctx.res_is_x, x_head=ctx.x_head, operands=ctx.operands, vectors=ctx.params[:2])
         L = len(layers)
         need = ctx.needs_input_grad            # (mod, cd, norm, fmt, x, res, gamma, beta, *wb)
         grads = [None, None, None, None]
@@ -1054,25 +1070,25 @@ def _norm_grads(norm, gsum, need_gamma, need_beta):
             gsum[1].to(norm.bias.dtype) if (need_beta and getattr(norm, "bias", None) is not None) else None]
 
 
-def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
+def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0, operands=None, vectors=None):
     """Backward of y = [x +] chain(norm(x)) for the chain of C x C layers: (dx [T,C], the norm's [2,C] sums or None,
     dW [L,out,in], db [L,C] or None, the layers).  dx_acc: a [T,C] gradient of the same x that another chain left
     (x's dtype, contiguous); the kernel adds its result into it and it is returned as dx.  x_head: rows of x and dx hold padded
-    heads (few tokens only)."""
+    heads (few tokens only).  operands, vectors: what the forward read, of the stack and of the norm."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _layers_of(mod)
     L = len(layers)
     Cdim, xw = layers[0].in_features, x.shape[-1]
     x = x.reshape(-1, xw)
     few = _few(x.shape[0], Cdim, L)
-    packed = _packed_few(mod, layers, cd, True) if few else None
-    if packed is not None:
-        w_img, b, wt_img = packed            # the tiled operands
+    operands = _train_operands(x, mod, cd) if operands is None else operands
+    if len(operands) == 3:
+        w_img, b, wt_img = operands          # the tiled operands
     elif x_head:
         raise RuntimeError("head-padded rows have a backward in the few-token launches only")
     else:
         few = 0
-        _, b, w_img, wt_img = _packed_train(mod, layers, cd)
+        _, b, w_img, wt_img = operands
     x2 = x
     x2 = _grid_rows(x2)
     dy2 = _rows2d(dy, Cdim)
@@ -1084,7 +1100,7 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
     d.x_stride, d.y_stride = x2.stride(0), dy2.stride(0)
     d.flags = (x_head // 4) << 8
-    gamma, beta = _norm_args(d, norm, x, Cdim)
+    gamma, beta = _norm_args(d, norm, x, Cdim, vectors)
     if dx_acc is not None and (dx_acc.shape != (T, Cdim) or dx_acc.dtype != x2.dtype or not dx_acc.is_contiguous()):
         raise ValueError("dx_acc must be a contiguous [T, C] tensor of x's dtype")
     dx = dx_acc if dx_acc is not None else torch.empty(T, xw, dtype=x2.dtype, device=dev)
@@ -1117,13 +1133,13 @@ def _chain_backward(mod, cd, norm, x, dy, res_is_x, dx_acc=None, x_head=0):
     return dx, gsum, dW, db, layers
 
 
-def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None, into=None):
-    """Backward of both stacks of a pair in one launch (y_head: dya and dyb are rows of padded heads; dres: another gradient of x,
-    added to dx): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
+def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, operands, vectors, y_head=0, dres=None, into=None):
+    """Backward of both stacks of a pair in one launch (operands, vectors: what the forward read, of the stacks and of the norm; y_head: dya
+    and dyb are rows of padded heads; dres: another gradient of x, added to dx): (dx, the norm's [2,C] sums or None, dW [2L,out,in], db [2L,C] or
     None, the 2 L layers)."""
     lib = _lib.load()
     layers, act_mask, add_mask, act = _pair_info(x, mod_a, mod_b, cd)
-    w, b, wt = _packed_few(mod_a, layers, cd, True)
+    w, b, wt = operands
     L2, Cdim, dev = len(layers), x.shape[-1], x.device
     x2 = x.reshape(-1, Cdim)
     x2 = _grid_rows(x2)
@@ -1140,7 +1156,7 @@ def _pair_backward(mod_a, mod_b, cd, norm, x, dya, dyb, y_head=0, dres=None, int
     d.act, d.act_mask, d.add_mask = act, act_mask, add_mask
     d.x_stride, d.y_stride = x2.stride(0), da.stride(0)
     d.flags = (y_head // 4) << 12
-    gamma, beta = _norm_args(d, norm, x, Cdim)
+    gamma, beta = _norm_args(d, norm, x, Cdim, vectors)
     dx = torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
     rows = torch.empty(2, L2, T, Cdim, dtype=cd, device=dev) if into is None else into         # a_in, g_out
     gb = gsum = None
@@ -1179,10 +1195,11 @@ class _FusedPairFn(torch.autograd.Function):
             if y_head and not ctx.pair:
                 raise ValueError("head-padded rows have no backward here: call under torch.no_grad()")
             pair = [] if ctx.pair else None
-            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
-                                operands=(packed[0][:n], packed[1][:n]) if ctx.pair else None, pair=pair)
-            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True,
-                                operands=(packed[0][n:], packed[1][n:]) if ctx.pair else None, pair=pair)
+            a, b = (((packed[0][:n], packed[1][:n]), (packed[0][n:], packed[1][n:])) if ctx.pair else
+                    (_train_operands(x, mod_a, cd), _train_operands(x, mod_b, cd)))
+            ya = _fused_mlp_fwd(x, mod_a, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True, operands=a, pair=pair)
+            yb = _fused_mlp_fwd(x, mod_b, cd, norm=norm, out_dtype=out_dtype, y_head=y_head, train=True, operands=b, pair=pair)
+        ctx.operands = packed if ctx.pair else (a, b)
         ctx.mods, ctx.cd, ctx.norm, ctx.y_head = (mod_a, mod_b), cd, norm, y_head
         ctx.versions = tuple(None if t is None else t._version for t in (gamma, beta, *wb))
         ctx.params = (gamma, beta, *wb)
@@ -1197,13 +1214,14 @@ class _FusedPairFn(torch.autograd.Function):
             raise RuntimeError("a parameter of the fused MLP was modified in place between its forward and its backward")
         mod_a, mod_b = ctx.mods
         if ctx.pair:
-            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb, ctx.y_head, dres)
+            dx, gs, dW, db, layers = _pair_backward(mod_a, mod_b, ctx.cd, ctx.norm, x, dya, dyb, ctx.operands, ctx.params[:2], ctx.y_head, dres)
             n = len(layers) // 2
             la, lb, dWa, dWb = layers[:n], layers[n:], dW[:n], dW[n:]
             dba, dbb = (None, None) if db is None else (db[:n], db[n:])
         else:
-            dx, gs_a, dWa, dba, la = _chain_backward(mod_a, ctx.cd, ctx.norm, x, dya, False)
-            dx, gs_b, dWb, dbb, lb = _chain_backward(mod_b, ctx.cd, ctx.norm, x, dyb, False, dx_acc=dx)
+            (a, b), vectors = ctx.operands, ctx.params[:2]
+            dx, gs_a, dWa, dba, la = _chain_backward(mod_a, ctx.cd, ctx.norm, x, dya, False, operands=a, vectors=vectors)
+            dx, gs_b, dWb, dbb, lb = _chain_backward(mod_b, ctx.cd, ctx.norm, x, dyb, False, dx_acc=dx, operands=b, vectors=vectors)
             gs = None if gs_a is None else gs_a + gs_b
         need = ctx.needs_input_grad            # (mod_a, mod_b, cd, norm, fmt, x, gamma, beta, *wb)
         grads = [None, None, None, None, None, dx.view(x.shape) if need[5] else None]
@@ -1234,7 +1252,7 @@ def _backward_expand(ctx, dy, x, E):
     _, _, _, act = _layers_of(mod)
     f1, f2 = mod.fc1, mod.fc2
     Cdim = x.shape[-1]
-    _, b, w_img, wt_img = _packed_train_expand(mod, E, cd)
+    _, b, w_img, wt_img = ctx.operands
     x2, dy2 = _rows2d(x, Cdim), _rows2d(dy, Cdim)
     T = x2.shape[0]
     dev = x.device
@@ -1243,7 +1261,7 @@ def _backward_expand(ctx, dy, x, E):
     d.w_dtype, d.x_dtype, d.y_dtype = _dtype_code(w_img), _dtype_code(x2), _dtype_code(dy2)
     d.act, d.act_mask, d.add_mask = act, 1, 0
     d.x_stride, d.y_stride = x2.stride(0), dy2.stride(0)
-    gamma, beta = _norm_args(d, norm, x, Cdim)
+    gamma, beta = _norm_args(d, norm, x, Cdim, ctx.params[:2])
     dx = torch.empty(T, Cdim, dtype=x2.dtype, device=dev)
     n_row = torch.empty(T, Cdim, dtype=cd, device=dev)
     dy_row = torch.empty(T, Cdim, dtype=cd, device=dev)

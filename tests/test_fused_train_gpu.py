@@ -921,3 +921,33 @@ def test_a_gradient_of_the_last_layer_can_be_differentiated(dev, monkeypatch):
     assert not hip
     for a, b in zip(got, want):
         assert rel(a, b) <= 3e-2
+
+
+@pytest.mark.parametrize("kw", [{}, {"qk_norm": True}, {"num_layers_ffn": 0, "ffn_mlp_ratio": 2.0}, {"num_layers_v_proj": 1, "rmsnorm": True}])
+@pytest.mark.parametrize("N", [300, 40000])
+def test_the_backward_reads_the_parameters_of_its_forward(dev, N, kw):
+    """A forward with other parameters (torch.func.functional_call), and a parameter replaced before the backward: the module's own are
+    not what the gradients belong to."""
+    torch.manual_seed(21)
+    blk = F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev)
+    other = F.FLAREBlock(channel_dim=64, num_heads=4, num_latents=32, **kw).to(dev)
+    with torch.no_grad():
+        for p in other.parameters():
+            p.mul_(1.5).add_(0.02)
+    x, gy = torch.randn(1, N, 64, device=dev, requires_grad=True), torch.randn(1, N, 64, device=dev)
+
+    def call(f):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return f(x)[0]
+
+    want = torch.autograd.grad(call(other), [x, *other.parameters()], gy)
+    params = {k: v.detach().clone().requires_grad_(True) for k, v in other.named_parameters()}
+    y = call(lambda t: torch.func.functional_call(blk, params, (t,)))
+    for a, b in zip(torch.autograd.grad(y, [x, *params.values()], gy), want):
+        assert rel(a, b) <= 1e-5          # the same 16-bit products; one block node or one node a stack add them up in fp32 in ranges of their own
+    before = list(other.parameters())
+    y = call(other)
+    for mod, name in ((other.mlp.fc1, "weight"), (other.att.k_proj.fc2, "bias"), (other.att.out_proj, "weight"), (other.norm1, "weight"), (other.norm2, "weight")):
+        setattr(mod, name, nn.Parameter(torch.randn_like(getattr(mod, name))))
+    for a, b in zip(torch.autograd.grad(y, [x, *before], gy), want):
+        assert torch.equal(a, b)
